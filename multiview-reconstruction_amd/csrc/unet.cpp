@@ -209,23 +209,16 @@ void UNet::dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t
   if (!launch_conv_fwd(c, stream)) convFailed = true;
 }
 
-int UNet::wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int dout_cs, int dout_co, int N, int D,
-                int H, int W) {
-  const long long nseg = (long long)N * D * H * ((W + 15) / 16);
-  const int nparts = (int)std::max<long long>(1, std::min<long long>(kWgradParts, nseg));
+void UNet::wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int dout_cs, int dout_co, int N, int D,
+                 int H, int W) {
   WgradArgs a{};
   a.in = in; a.in_cs = in_cs; a.cin = kCin[l];
   a.dout = dout; a.dout_cs = dout_cs; a.dout_co = dout_co; a.cout = kCout[l];
   a.N = N; a.D = D; a.H = H; a.W = W;
-  a.taps = 27;
   a.partial = wpart;
-  launch_conv_wgrad(a, nparts, stream);
-  launch_sum_partials(wpart, nparts, layer[l].count, layer[l].g, stream);
-  const size_t nvox = (size_t)N * D * H * W;
-  const int bparts = (int)std::min<size_t>(256, std::max<size_t>(1, nvox / 256));
-  launch_bias_grad(dout, dout_cs, dout_co, kCout[l], nvox, bpart, bparts, stream);
-  launch_sum_partials(bpart, bparts, kCout[l], bias[l].g, stream);
-  return 0;
+  a.bias_partial = bpart;
+  const int nparts = launch_conv_wgrad(a, kWgradParts, stream);
+  launch_sum_partials(wpart, nparts, layer[l].count, layer[l].g, bpart, kCout[l], bias[l].g, stream);
 }
 
 // ------------------------------------------------------------------ forward / backward
@@ -296,7 +289,7 @@ int UNet::backward(Acts& a) {
   HeadArgs h{};
   h.d1 = a.d1; h.d1_cs = 16; h.wo = head.w; h.bias = head.w + 16; h.avg = a.avg; h.dr = a.dr; h.nvox = v0;
   const int hb = launch_head_bwd(h, a.g_d1, bpart, stream);
-  launch_sum_partials(bpart, hb, 17, head.g, stream);
+  launch_sum_partials(bpart, hb, 17, head.g, nullptr, 0, nullptr, stream);
   // decoder level 1
   launch_relu_bwd(a.g_d1, 16, 0, a.d1, 16, 0, 16, v0, stream);
   wgrad(9, a.a5, 16, a.g_d1, 16, 0, N, D0, H0, W0);
@@ -363,8 +356,9 @@ int UNet::adam_step(float lr) {
 int UNet::ensure_scratch() {
   if (!wpart) {
     size_t maxc = 0;
-    for (int l = 0; l < kLayers; ++l) maxc = std::max(maxc, wcount(l));
-    MVR_HIP(hipMalloc(&wpart, (size_t)kWgradParts * maxc * 4));
+    // the widest layers take 1536 / groups partitions (unet_wgrad.hip), the others up to kWgradParts
+    for (int l = 0; l < kLayers; ++l) maxc = std::max(maxc, wgrad_max_parts(kCin[l], kCout[l], kWgradParts) * wcount(l));
+    MVR_HIP(hipMalloc(&wpart, maxc * 4));
     MVR_HIP(hipMalloc(&bpart, (size_t)1024 * 64 * 4));
     MVR_HIP(hipMalloc(&lossPart, 2048 * 8));  // 1024 double2
   }

@@ -8,9 +8,8 @@
 // ranges of one buffer.  Convolution weights are [tap][cout][cin] (cin
 // contiguous), master copies FP32, compute copies bf16.
 //
-// MFMA layout (v_mfma_f32_16x16x16_bf16): A is 16(m) x 16(k), lane l holds
-// A[l%16][4(l/16)..4(l/16)+3]; B is 16(k) x 16(n), lane l holds
-// B[4(l/16)..+3][l%16]; D lane l holds D[4(l/16)+r][l%16], r = 0..3.
+// The MFMA kernels are in unet_conv.hip (convolutions, forward and data
+// gradient) and unet_wgrad.hip (weight and bias gradients).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -18,9 +17,6 @@
 #include "unet.hpp"
 
 namespace mvr {
-
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 __device__ __forceinline__ uint16_t f2bf(float f) {
@@ -32,100 +28,7 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 // The 3^3 convolutions run in the LDS-tiled kernel of unet_conv.hip (launch_conv_tiled).
 
 // ------------------------------------------------------------------ weight gradient
-// dw[tap][co][ci] = sum_v dout[v][co] * in[v + tap][ci], accumulated per work-group
-// over a contiguous range of 16-voxel x-segments; partial[blockIdx.x][tap][co][ci].
-// Grid: x = number of partitions, y = 27 (or 1) taps.  The 16 x 16 tiles
-// (co block, ci block) are spread over the four waves.
-__global__ __launch_bounds__(256) void k_conv_wgrad(WgradArgs a) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int i = lane & 15, g = lane >> 4;
-  const int tap = blockIdx.y;
-  int dz = 0, dy = 0, dx = 0;
-  if (a.taps == 27) { dz = tap / 9 - 1; dy = (tap / 3) % 3 - 1; dx = tap % 3 - 1; }
-  const int ncb = a.cout / 16, nib = a.cin / 16, ntiles = ncb * nib;
-  // tiles handled by this wave: t = wave, wave + 4, ... (at most kMaxWgradTiles)
-  f32x4 acc[kMaxWgradTiles];
-#pragma unroll
-  for (int t = 0; t < kMaxWgradTiles; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int segsPerRow = (a.W + 15) / 16;
-  const long long nseg = (long long)a.N * a.D * a.H * segsPerRow;
-  const long long s0 = nseg * blockIdx.x / gridDim.x, s1 = nseg * (blockIdx.x + 1) / gridDim.x;
-  for (long long s = s0; s < s1; ++s) {
-    const int sx = (int)(s % segsPerRow);
-    const long long row = s / segsPerRow;
-    const int y = (int)(row % a.H);
-    const long long nz = row / a.H;
-    const int z = (int)(nz % a.D), n = (int)(nz / a.D);
-    const int x0 = sx * 16;
-    // A operand: dout^T, A[m = co][k = v] -> lane holds dout[v = 4g + r][co = i]
-    // B operand: in shifted by the tap, B[k = v][n = ci] -> lane holds in[v = 4g + r][ci = i]
-    const int zz = z + dz, yy = y + dy;
-    const bool rowok = (unsigned)zz < (unsigned)a.D && (unsigned)yy < (unsigned)a.H;
-    for (int t = wave, slot = 0; t < ntiles; t += 4, ++slot) {
-      const int cb = t / nib, ib = t % nib;
-      s16x4 av, bv;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int x = x0 + 4 * g + r;
-        uint16_t dv = 0, iv = 0;
-        if (x < a.W) {
-          const size_t vo = (((size_t)n * a.D + z) * a.H + y) * a.W + x;
-          dv = a.dout[vo * a.dout_cs + a.dout_co + cb * 16 + i];
-          const int xx = x + dx;
-          if (rowok && (unsigned)xx < (unsigned)a.W) {
-            const size_t vi = (((size_t)n * a.D + zz) * a.H + yy) * a.W + xx;
-            iv = a.in[vi * a.in_cs + ib * 16 + i];
-          }
-        }
-        av[r] = (short)dv;
-        bv[r] = (short)iv;
-      }
-#pragma unroll
-      for (int q = 0; q < kMaxWgradTiles; ++q)
-        if (q == slot) acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[q], 0, 0, 0);
-    }
-  }
-  // D lane l holds dw[co = cb*16 + 4g + r][ci = ib*16 + i]
-  float* part = a.partial + ((size_t)blockIdx.x * a.taps + tap) * a.cout * a.cin;
-  for (int t = wave, slot = 0; t < ntiles; t += 4, ++slot) {
-    const int cb = t / nib, ib = t % nib;
-#pragma unroll
-    for (int q = 0; q < kMaxWgradTiles; ++q)
-      if (q == slot)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) part[(size_t)(cb * 16 + 4 * g + r) * a.cin + ib * 16 + i] = acc[q][r];
-  }
-}
-
-// sum of partials: grad[j] = sum_p partial[p][j], j < count
-__global__ void k_sum_partials(const float* __restrict__ partial, int nparts, size_t count, float* __restrict__ grad) {
-  for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < count; j += (size_t)gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int p = 0; p < nparts; ++p) s += partial[(size_t)p * count + j];
-    grad[j] = s;
-  }
-}
-
-// bias gradient partials: db[co] = sum_v dout[v][co]; partial[blockIdx.x][co]
-__global__ __launch_bounds__(256) void k_bias_grad(const uint16_t* __restrict__ dout, int cs, int co0, int cout,
-                                                   size_t nvox, float* __restrict__ partial) {
-  __shared__ float red[256];
-  const int c = threadIdx.x % cout;
-  const int lanesPerC = 256 / cout;
-  const int sub = threadIdx.x / cout;
-  float s = 0.f;
-  if (sub < lanesPerC) {
-    const size_t v0 = nvox * blockIdx.x / gridDim.x, v1 = nvox * (blockIdx.x + 1) / gridDim.x;
-    for (size_t v = v0 + sub; v < v1; v += lanesPerC) s += bf2f(dout[v * cs + co0 + c]);
-  }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x < cout) {
-    float t = 0.f;
-    for (int k = 0; k < lanesPerC; ++k) t += red[k * cout + threadIdx.x];
-    partial[(size_t)blockIdx.x * cout + threadIdx.x] = t;
-  }
-}
+// Weight and bias gradients: unet_wgrad.hip.
 
 // ------------------------------------------------------------------ elementwise pieces
 // All work on units of 8 channels (16 bytes); channel counts, strides and offsets are multiples of 16.
@@ -457,16 +360,6 @@ static inline int grid1(size_t n, int cap = 8192) {
 bool launch_conv_fwd(const ConvArgs& a, hipStream_t s) {
   // every layer of the network has cin, cout and channel strides that are multiples of 16
   return launch_conv_tiled(a, s);
-}
-void launch_conv_wgrad(const WgradArgs& a, int nparts, hipStream_t s) {
-  hipLaunchKernelGGL(k_conv_wgrad, dim3(nparts, a.taps), dim3(256), 0, s, a);
-}
-void launch_sum_partials(const float* partial, int nparts, size_t count, float* grad, hipStream_t s) {
-  hipLaunchKernelGGL(k_sum_partials, dim3(grid1(count, 4096)), dim3(256), 0, s, partial, nparts, count, grad);
-}
-void launch_bias_grad(const uint16_t* dout, int cs, int co0, int cout, size_t nvox, float* partial, int nparts,
-                      hipStream_t s) {
-  hipLaunchKernelGGL(k_bias_grad, dim3(nparts), dim3(256), 0, s, dout, cs, co0, cout, nvox, partial);
 }
 void launch_relu_bwd(uint16_t* g, int gcs, int gco, const uint16_t* post, int pcs, int pco, int C, size_t nvox,
                      hipStream_t s) {

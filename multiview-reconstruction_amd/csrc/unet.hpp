@@ -7,8 +7,6 @@
 
 namespace mvr {
 
-constexpr int kMaxWgradTiles = 4;  // (cout/16)*(cin/16) <= 16 tiles spread over 4 waves
-
 struct ConvArgs {
   const uint16_t* in;  // [n][z][y][x][in_cs], channels [0, cin)
   int in_cs;
@@ -37,8 +35,8 @@ struct WgradArgs {
   const uint16_t* dout;  // gradient of the layer output (after the ReLU mask)
   int dout_cs, dout_co, cout;
   int N, D, H, W;
-  int taps;
-  float* partial;        // [parts][taps][cout][cin]
+  float* partial;        // [parts][27][cout][cin]
+  float* bias_partial;   // [parts][cout]
 };
 
 // views the network takes: V view channels + their weighted mean fit the 16 input channels; the input
@@ -91,10 +89,18 @@ bool launch_conv_fwd(const ConvArgs& a, hipStream_t s);  // false: shape not sup
 // LDS-tiled 3^3 convolution (unet_conv.hip); false when the shape is not one it covers
 bool launch_conv_tiled(const ConvArgs& a, hipStream_t s);
 bool conv_fuses_pool(const ConvArgs& a);  // the launch also writes the pooled output (pool_out set, DMA kernel)
-void launch_conv_wgrad(const WgradArgs& a, int nparts, hipStream_t s);
-void launch_sum_partials(const float* partial, int nparts, size_t count, float* grad, hipStream_t s);
-void launch_bias_grad(const uint16_t* dout, int cs, int co0, int cout, size_t nvox, float* partial, int nparts,
-                      hipStream_t s);
+// weight and bias gradient partials of a 3^3 layer (cin and cout multiples of 16); returns how many partitions
+// (at most maxParts) it wrote
+int launch_conv_wgrad(const WgradArgs& a, int maxParts, hipStream_t s);
+// the most partitions launch_conv_wgrad takes for a layer: enough work-groups for two to six per CU over all of the
+// layer's channel blocks
+inline int wgrad_max_parts(int cin, int cout, int maxParts) {
+  const int p = 1536 / ((cin / 16) * (cout % 32 == 0 ? cout / 32 : cout / 16));
+  return p < maxParts ? p : maxParts;
+}
+// grad[j] = sum_p partial[p][j], j < count; with bcount > 0 (at most 64) also bgrad from bpartial
+void launch_sum_partials(const float* partial, int nparts, size_t count, float* grad, const float* bpartial,
+                         int bcount, float* bgrad, hipStream_t s);
 void launch_relu_bwd(uint16_t* g, int gcs, int gco, const uint16_t* post, int pcs, int pco, int C, size_t nvox,
                      hipStream_t s);
 void launch_pool_fwd(const uint16_t* in, int ics, int ico, uint16_t* out, int ocs, int C, int N, int D, int H, int W,

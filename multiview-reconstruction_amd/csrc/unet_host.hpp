@@ -15,7 +15,7 @@
 namespace mvr {
 
 constexpr int kLayers = 10;
-constexpr int kWgradParts = 256;
+constexpr int kWgradParts = 512;
 
 // planes of context on either side of an inference slab: a multiple of 4 above the network's receptive-field
 // radius of 23 planes (4 at full resolution, 8 at half, 8 at quarter resolution, plus the pooling grid's offset)
@@ -87,8 +87,8 @@ struct UNet {
             uint16_t* pool = nullptr, int pool_cs = 0);
   void dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t* din, int din_cs, int din_co, int N,
              int D, int H, int W);
-  int wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int dout_cs, int dout_co, int N, int D, int H,
-            int W);
+  void wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int dout_cs, int dout_co, int N, int D, int H,
+             int W);
   int forward(Acts& a, bool training, const float* psiScale, float* psiOut, const int* outDims, float minValue,
               double* loss);
   int backward(Acts& a);
