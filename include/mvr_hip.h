@@ -303,7 +303,7 @@ int mvr_unet_infer(mvr_unet* u, const float* const* imgs, const float* const* we
 /* Inference of volumes above `voxels` (padded to multiples of 4; default and any value <= 0: 2^28) runs in
  * z slabs that each carry mvr_unet_inference_halo() planes of context on either side; the result equals
  * the single-window result.  Bounds the network's activation memory beside a resident deconvolution
- * (about 285 bytes per window voxel).  No counterpart in the reference (its PsiInit has no network). */
+ * (about 160 bytes per window voxel).  No counterpart in the reference (its PsiInit has no network). */
 int mvr_unet_set_inference_window(mvr_unet* u, long long voxels);
 int mvr_unet_inference_halo(void);
 void mvr_unet_destroy(mvr_unet* u);

@@ -121,17 +121,24 @@ int UNet::copy_params(float* hostOut, const float* hostIn, bool grads) {
 }
 
 // ------------------------------------------------------------------ activations
-int UNet::Acts::alloc(int N_, int D_, int H_, int W_, bool grads) {
+int UNet::Acts::alloc(int N_, int D_, int H_, int W_, int views, bool grads) {
   N = N_; D = D_; H = H_; W = W_;
   Dcap = D_;
+  // Training keeps the concatenations (the weight gradients read them) with the skip tensors behind the upsampled
+  // channels; an inference reads the upsampled part from the coarse tensor, so the skip tensors stand alone, and the
+  // input's channels beyond the first eight are not stored where they are all zero.
+  cs1 = grads ? 48 : 16;
+  cs2 = grads ? 96 : 32;
+  csIn = !grads && views + 1 <= 8 ? 8 : 16;
   const size_t v0 = (size_t)N * D * H * W, v1 = v0 / 8, v2 = v0 / 64;
   struct B { uint16_t** p; uint16_t** gp; size_t n; };
-  const B bufs[] = {{&x0, nullptr, v0 * 16},   {&a1, &g_a1, v0 * 16},  {&cat1, &g_cat1, v0 * 48},
-                    {&p1, &g_p1, v1 * 16},     {&a2, &g_a2, v1 * 32},  {&cat2, &g_cat2, v1 * 96},
+  const B bufs[] = {{&x0, nullptr, v0 * csIn}, {&a1, &g_a1, v0 * 16},  {&cat1, &g_cat1, v0 * cs1},
+                    {&p1, &g_p1, v1 * 16},     {&a2, &g_a2, v1 * 32},  {&cat2, &g_cat2, v1 * cs2},
                     {&p2, &g_p2, v2 * 32},     {&a3, &g_a3, v2 * 64},  {&b3, &g_b3, v2 * 64},
                     {&a4, &g_a4, v1 * 32},     {&d2, &g_d2, v1 * 32},  {&a5, &g_a5, v0 * 16},
                     {&d1, &g_d1, v0 * 16}};
   for (const B& b : bufs) {
+    if (b.p == &d1 && !grads) continue;  // an inference turns the last activations into psi without storing them
     MVR_HIP(hipMalloc(b.p, b.n * 2));
     if (grads && b.gp) MVR_HIP(hipMalloc(b.gp, b.n * 2));
   }
@@ -161,18 +168,21 @@ int UNet::ensure_acts(Acts& a, int N_, int D_, int H_, int W_, bool grads) {
     return 0;
   }
   a.release();
-  return a.alloc(N_, D_, H_, W_, grads);
+  return a.alloc(N_, D_, H_, W_, V, grads);
 }
 
 bool UNet::conv(int l, const uint16_t* in, int in_cs, int in_co, uint16_t* out, int out_cs, int out_co, int N, int D,
-                int H, int W, bool relu, const uint16_t* up, int up_cs, int up_c, uint16_t* pool, int pool_cs) {
+                int H, int W, bool relu, const uint16_t* up, int up_cs, int up_c, uint16_t* pool, int pool_cs,
+                const PsiArgs* psi) {
   ConvArgs c{};
+  if (psi) c.psi = *psi;
   c.up_in = up;
   c.up_cs = up_cs;
   c.up_c = up ? up_c : 0;
   c.in = in + in_co;
   c.in_cs = in_cs;
   c.cin = kCin[l];
+  c.in_half = l == 0 && in_cs == 8;
   c.w = layer[l].wbf;
   c.bias = bias[l].w;
   c.out = out;
@@ -227,13 +237,16 @@ int UNet::forward(Acts& a, bool training, const float* psiScale, float* psiOut, 
   const int N = a.N, D0 = a.D, H0 = a.H, W0 = a.W;
   const int D1 = D0 / 2, H1 = H0 / 2, W1 = W0 / 2, D2 = D0 / 4, H2 = H0 / 4, W2 = W0 / 4;
   convFailed = false;
-  conv(0, a.x0, 16, 0, a.a1, 16, 0, N, D0, H0, W0, true);
-  // e1 -> cat1[32:48), pooled into p1 by the convolution where it can
-  if (!conv(1, a.a1, 16, 0, a.cat1, 48, 32, N, D0, H0, W0, true, nullptr, 0, 0, a.p1, 16))
-    launch_pool_fwd(a.cat1, 48, 32, a.p1, 16, 16, N, D1, H1, W1, stream);
+  // the skip tensors' channels of cat1 and cat2
+  const int cs1 = a.cs1, co1 = cs1 - 16, cs2 = a.cs2, co2 = cs2 - 32;
+  conv(0, a.x0, a.csIn, 0, a.a1, 16, 0, N, D0, H0, W0, true);
+  // e1, pooled into p1 by the convolution where it can
+  if (!conv(1, a.a1, 16, 0, a.cat1, cs1, co1, N, D0, H0, W0, true, nullptr, 0, 0, a.p1, 16))
+    launch_pool_fwd(a.cat1, cs1, co1, a.p1, 16, 16, N, D1, H1, W1, stream);
   conv(2, a.p1, 16, 0, a.a2, 32, 0, N, D1, H1, W1, true);
-  conv(3, a.a2, 32, 0, a.cat2, 96, 64, N, D1, H1, W1, true);                 // e2 -> cat2[64:96)
-  launch_pool_fwd(a.cat2, 96, 64, a.p2, 32, 32, N, D2, H2, W2, stream);
+  // e2, pooled into p2
+  if (!conv(3, a.a2, 32, 0, a.cat2, cs2, co2, N, D1, H1, W1, true, nullptr, 0, 0, a.p2, 32))
+    launch_pool_fwd(a.cat2, cs2, co2, a.p2, 32, 32, N, D2, H2, W2, stream);
   conv(4, a.p2, 32, 0, a.a3, 64, 0, N, D2, H2, W2, true);
   conv(5, a.a3, 64, 0, a.b3, 64, 0, N, D2, H2, W2, true);
   // decoder: training materialises the concatenations (the weight gradients read them); inference
@@ -242,14 +255,28 @@ int UNet::forward(Acts& a, bool training, const float* psiScale, float* psiOut, 
     launch_up_fwd(a.b3, 64, a.cat2, 96, 0, 64, N, D2, H2, W2, stream);      // up(b3) -> cat2[0:64)
     conv(6, a.cat2, 96, 0, a.a4, 32, 0, N, D1, H1, W1, true);
   } else {
-    conv(6, a.cat2, 96, 64, a.a4, 32, 0, N, D1, H1, W1, true, a.b3, 64, 64);
+    conv(6, a.cat2, cs2, 0, a.a4, 32, 0, N, D1, H1, W1, true, a.b3, 64, 64);
   }
   conv(7, a.a4, 32, 0, a.d2, 32, 0, N, D1, H1, W1, true);
   if (training) {
     launch_up_fwd(a.d2, 32, a.cat1, 48, 0, 32, N, D1, H1, W1, stream);      // up(d2) -> cat1[0:32)
     conv(8, a.cat1, 48, 0, a.a5, 16, 0, N, D0, H0, W0, true);
   } else {
-    conv(8, a.cat1, 48, 32, a.a5, 16, 0, N, D0, H0, W0, true, a.d2, 32, 32);
+    conv(8, a.cat1, cs1, 0, a.a5, 16, 0, N, D0, H0, W0, true, a.d2, 32, 32);
+  }
+  if (!training) {
+    // the output head is fused into the last convolution, whose activations are not stored
+    PsiArgs h{};
+    h.out = psiOut;
+    h.w = head.w;
+    h.avg = a.avg;
+    h.scale = *psiScale;
+    h.minValue = minValue;
+    h.ox = outDims[0]; h.oy = outDims[1]; h.oz = outDims[2]; h.zlo = outDims[3];
+    conv(9, a.a5, 16, 0, nullptr, 16, 0, N, D0, H0, W0, true, nullptr, 0, 0, nullptr, 0, &h);
+    UCHECK(!convFailed, "U-Net convolution refused: three x-y planes of the input exceed 32-bit offsets");
+    MVR_HIP(hipGetLastError());
+    return 0;
   }
   conv(9, a.a5, 16, 0, a.d1, 16, 0, N, D0, H0, W0, true);
   UCHECK(!convFailed, "U-Net convolution refused: three x-y planes of the input exceed 32-bit offsets");
@@ -258,26 +285,17 @@ int UNet::forward(Acts& a, bool training, const float* psiScale, float* psiOut, 
   h.wo = head.w; h.bias = head.w + 16;
   h.avg = a.avg;
   h.nvox = (size_t)N * D0 * H0 * W0;
-  h.minValue = minValue;
-  h.scale = psiScale ? *psiScale : 1.f;
-  if (training) {
-    h.target = a.target;
-    h.dr = a.dr;
-    h.loss_partial = lossPart;
-  }
-  h.psi = psiOut;
-  h.W = W0; h.H = H0; h.D = D0;
-  if (outDims) { h.ox = outDims[0]; h.oy = outDims[1]; h.oz = outDims[2]; h.zlo = outDims[3]; }
+  h.target = a.target;
+  h.dr = a.dr;
+  h.loss_partial = lossPart;
   const int nb = launch_head(h, stream);
   MVR_HIP(hipGetLastError());
-  if (training && loss) {
-    std::vector<double> lp(nb);
-    MVR_HIP(hipMemcpyAsync(lp.data(), lossPart, nb * 8, hipMemcpyDeviceToHost, stream));
-    MVR_HIP(hipStreamSynchronize(stream));
-    double s = 0;
-    for (double x : lp) s += x;
-    *loss = s / (double)h.nvox;
-  }
+  std::vector<double> lp(nb);
+  MVR_HIP(hipMemcpyAsync(lp.data(), lossPart, nb * 8, hipMemcpyDeviceToHost, stream));
+  MVR_HIP(hipStreamSynchronize(stream));
+  double s = 0;
+  for (double x : lp) s += x;
+  *loss = s / (double)h.nvox;
   return 0;
 }
 
@@ -400,6 +418,7 @@ int UNet::pack(Acts& a, int sample, const std::vector<float*>& img, const std::v
   in.sample = sample;
   in.inv_scale = invScale;
   in.out = a.x0;
+  in.out_cs = a.csIn;
   in.avg_out = a.avg;
   launch_pack_input(in, stream);
   return 0;

@@ -174,16 +174,15 @@ __global__ void k_pack_input(InputArgs a) {
 #pragma unroll
     for (int c = 0; c < 16; ++c)
       if (c == a.V) val[c] = mean;
-    uint16_t* o = a.out + ((size_t)a.sample * total + v) * 16;
+    uint16_t* o = a.out + ((size_t)a.sample * total + v) * a.out_cs;
     at8w(o) = pack8(val);
-    at8w(o + 8) = pack8(val + 8);
+    if (a.out_cs == 16) at8w(o + 8) = pack8(val + 8);
     if (a.avg_out) a.avg_out[(size_t)a.sample * total + v] = mean;
   }
 }
 
-// output head: r[v] = sum_c wo[c] d1[v][c] + bo; pred = avg[v] + r[v]
-// training: loss partials of (pred - target)^2 and dr[v] = 2 (pred - target) / count
-// inference: psi[v] = max(minValue, scale * pred)
+// output head of a training step (an inference fuses it into the last convolution): r[v] = sum_c wo[c] d1[v][c] + bo;
+// pred = avg[v] + r; loss partials of (pred - target)^2 and dr[v] = 2 (pred - target) / count
 __global__ __launch_bounds__(256) void k_head(HeadArgs a) {
   __shared__ double red[256];
   double ls = 0.0;
@@ -192,18 +191,9 @@ __global__ __launch_bounds__(256) void k_head(HeadArgs a) {
     const uint16_t* p = a.d1 + v * a.d1_cs;
 #pragma unroll
     for (int c = 0; c < 16; ++c) r += a.wo[c] * bf2f(p[c]);
-    const float pred = a.avg[v] + r;
-    if (a.target) {
-      const float e = pred - a.target[v];
-      ls += (double)e * e;
-      a.dr[v] = 2.f * e / (float)a.nvox;
-    }
-    if (a.psi) {
-      // net dims (W, H, D) may be the output dims (ox, oy, oz) padded up; only inner voxels are written
-      const int x = (int)(v % a.W), y = (int)((v / a.W) % a.H), z = (int)(v / ((size_t)a.W * a.H));
-      if (x < a.ox && y < a.oy && z >= a.zlo && z < a.oz)
-        a.psi[((size_t)z * a.oy + y) * a.ox + x] = fmaxf(a.minValue, a.scale * pred);
-    }
+    const float e = a.avg[v] + r - a.target[v];
+    ls += (double)e * e;
+    a.dr[v] = 2.f * e / (float)a.nvox;
   }
   red[threadIdx.x] = ls;
   __syncthreads();
@@ -211,7 +201,7 @@ __global__ __launch_bounds__(256) void k_head(HeadArgs a) {
     if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0 && a.loss_partial) a.loss_partial[blockIdx.x] = red[0];
+  if (threadIdx.x == 0) a.loss_partial[blockIdx.x] = red[0];
 }
 
 // head backward: d_d1[v][c] = dr[v] * wo[c]; partials of dwo[c] = sum dr d1[v][c], dbo = sum dr

@@ -7,10 +7,21 @@
 
 namespace mvr {
 
+// output head of an inference: psi[v] = max(minValue, scale * (avg[v] + sum_c w[c] d1[v][c] + w[16]))
+struct PsiArgs {
+  float* out;            // psi, dims (ox, oy, oz), or null
+  const float* w;        // 16 weights and the bias
+  const float* avg;      // normalised average channel [D][H][W]
+  float scale, minValue;
+  int ox, oy, oz;        // output volume dims, <= net dims; psi holds planes [zlo, oz) of them
+  int zlo;
+};
+
 struct ConvArgs {
   const uint16_t* in;  // [n][z][y][x][in_cs], channels [0, cin)
   int in_cs;
   int cin;             // multiple of 16
+  int in_half;         // 1: a one-chunk input whose channels 8..15 are zero and not stored (in_cs a multiple of 8)
   const uint16_t* w;   // [taps][cout][cin]
   const float* bias;   // [cout] or null
   uint16_t* out;       // [n][z][y][x][out_cs], channels [out_co, out_co + cout)
@@ -24,9 +35,10 @@ struct ConvArgs {
   const uint16_t* up_in;
   int up_cs, up_c;
   // optional fused 2x2x2 average pooling of the stored (bf16) output into pool_out [n][D/2][H/2][W/2][pool_cs],
-  // channels [pool_co, pool_co + cout): done where conv_fuses_pool(args) holds, else left to the caller
+  // channels [0, cout): done where conv_fuses_pool(args) holds, else left to the caller
   uint16_t* pool_out;
-  int pool_cs, pool_co;
+  int pool_cs;
+  PsiArgs psi;           // optional fused output head (psi.out set; 16 -> 16 channels, one sample): out is not written
 };
 
 struct WgradArgs {
@@ -52,25 +64,22 @@ struct InputArgs {
   int W, H, D;           // sample region
   int sample;            // index in the batch
   float inv_scale;
-  uint16_t* out;         // [batch][D][H][W][16]
+  uint16_t* out;         // [batch][D][H][W][out_cs], out_cs 16 or (V < 8) 8
+  int out_cs;
   float* avg_out;        // [batch][D][H][W] (normalised average channel) or null
 };
 
+// output head of a training step
 struct HeadArgs {
   const uint16_t* d1;    // [nvox][d1_cs], 16 channels
   int d1_cs;
   const float* wo;       // 16
   const float* bias;     // 1
   const float* avg;      // normalised average channel
-  const float* target;   // normalised target (training) or null
-  float* dr;             // gradient of r (training)
-  double* loss_partial;  // per work-group sum of squared errors (training) or null
-  float* psi;            // inference output or null, dims (ox, oy, oz)
-  float scale, minValue;
+  const float* target;   // normalised target
+  float* dr;             // gradient of r
+  double* loss_partial;  // per work-group sum of squared errors
   size_t nvox;
-  int W, H, D;           // net dims of one sample (psi output only)
-  int ox, oy, oz;        // output volume dims, <= net dims; psi holds planes [zlo, oz) of them
-  int zlo;
 };
 
 struct AdamArgs {
@@ -88,7 +97,7 @@ struct AdamArgs {
 bool launch_conv_fwd(const ConvArgs& a, hipStream_t s);  // false: shape not supported, nothing launched
 // LDS-tiled 3^3 convolution (unet_conv.hip); false when the shape is not one it covers
 bool launch_conv_tiled(const ConvArgs& a, hipStream_t s);
-bool conv_fuses_pool(const ConvArgs& a);  // the launch also writes the pooled output (pool_out set, DMA kernel)
+bool conv_fuses_pool(const ConvArgs& a);  // the launch also writes the pooled output (pool_out set, even dimensions)
 // weight and bias gradient partials of a 3^3 layer (cin and cout multiples of 16); returns how many partitions
 // (at most maxParts) it wrote
 int launch_conv_wgrad(const WgradArgs& a, int maxParts, hipStream_t s);

@@ -1,21 +1,35 @@
-// unet_conv.hip -- LDS-tiled 3^3 convolution of the U-Net on BF16 MFMA (forward and data gradient).
+// unet_conv.hip -- 3^3 convolutions of the U-Net on BF16 MFMA (forward and data gradient).
 //
 // out[v][co] = act( sum_tap sum_ci in[v + off(tap)][ci] * w[tap][co][ci] + bias[co] ), zero padding,
-// channels-last bf16 tensors (see unet.hip).  One work-group computes an output tile of TY rows x TX
-// voxels of one z plane for NG x 16 output channels (grid.y selects the channel group):
+// channels-last bf16 tensors (see unet.hip).  A work-group computes a column of 16 x 16 voxel tiles (consecutive z
+// planes) for NG x 16 output channels (grid.y selects the channel group):
 //   - an input may be a concatenation [up(coarse), fine] whose first part is read from the coarse
 //     tensor at half the coordinates (nearest x2 upsampling fused into the staging);
-//   - per 16-channel input chunk, the halo tile 3 x (TY+2) x (TX+2) x 16 bf16 and the chunk's weights
-//     [28 taps][NG*16 cout][16 cin] (tap 27 = zeros) are staged into LDS with 16-byte accesses, each
-//     stored as two 8-channel halves [half][...][8] so that the 16 lanes reading one half of 16
-//     consecutive voxels (or output channels) touch 256 contiguous bytes (no bank conflicts);
+//   - the input goes through LDS one 16-channel chunk and one 18 x 18 halo plane at a time, in a ring of four planes:
+//     while the products of one output plane run on three of them, LDS-DMA loads (global_load_lds_dwordx4: 16 bytes
+//     per lane straight into LDS at the wave's base + 16 lane) fill the fourth with the next plane, so each input
+//     plane crosses LDS once per work-group.  Halo voxels outside the volume read a zero in device memory.  Each
+//     plane is stored as two 8-channel halves [half][voxel][8], so that the 16 lanes reading one half of 16
+//     consecutive voxels touch 256 contiguous bytes (no bank conflicts);
 //   - v_mfma_f32_16x16x32_bf16 takes K = 32 as two taps x 16 channels: lanes 0-31 carry tap 2p,
-//     lanes 32-63 tap 2p+1, eight channels per lane;
-//   - the tile's 16-voxel row segments are the M-tiles (16 per work-group, 4 per wave); a wave reads
-//     each A fragment from LDS once per tap pair and reuses it for its NG output tiles, and each B
-//     fragment once for its 4 M-tiles.
-// The sum over K pairs A and B slots the same way, so the kernel relies only on the M/N placement:
+//     lanes 32-63 tap 2p+1 (tap 27 = zeros), eight channels per lane;
+//   - the weights of the chunk stay in registers (14 fragments per output group): only the voxel fragments are read
+//     from LDS;
+//   - the weights are the first operand, the voxels the second: lane l of the result holds channels 4(l/16)..+3 of
+//     voxel l%16, stored with one 8-byte access.
+// The sum over K pairs both operands' slots the same way, so the kernel relies only on the M/N placement:
 // lane l holds rows/columns l%16 of A/B, and D[4(l/16)+r][l%16].
+//
+// One-chunk layers (cin = 16) march a column of planes with one plane's accumulators; layers of several chunks keep
+// the accumulators of ZP planes and take the chunks one after the other (every sum runs over the chunks in order,
+// and over the tap pairs in order within a chunk).
+//
+// Bound by the LDS reads of the voxel fragments: a fragment (1 KB, 8 clocks of the CU's LDS) feeds NG products of 16
+// clocks, so 16 -> 16 layers cannot run faster than 0.75 us per plane tile and CU (191 us at 252 x 250 x 254; 272 measured,
+// 520 with the weights read from LDS and three halo planes staged per output plane); the wide layers lose the rest to
+// the weight reloads between chunks.  One inference at 252 x 250 x 254, 6 views: 4.75 -> 3.05 ms, with the skip tensors
+// stored without the upsampled channels beside them (the pooled layer 734 -> 312 us) and the head fused behind the last
+// layer.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,497 +48,565 @@ __device__ __forceinline__ uint16_t f2bf_rne(float f) {
   const uint32_t u = __float_as_uint(f);
   return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
 }
+__device__ __forceinline__ float bf2f(uint32_t b) { return __uint_as_float(b << 16); }
 
-// planes per work-group: a work-group walks zp consecutive z planes of its (y, x) tile (single-chunk layers
-// stage their weights once); launches with fewer than kConvZPTiles plane tiles use one plane per work-group
-// so that the grid still fills the chip
-constexpr int kConvZP = 4;
-constexpr long long kConvZPTiles = 16384;
+constexpr int TX = 16, TY = 16;               // output tile (one 16-voxel segment per row, four rows per wave)
+constexpr int HX = TX + 2, HY = TY + 2;
+constexpr int HVP = HX * HY;                  // halo voxels of a plane
+constexpr int kDma = 3;                       // DMA instructions per wave and plane: 2 halves x 6 over four waves
+constexpr int kPlane = 2 * HVP * 8;           // elements of one ring plane
+static_assert(HVP > 5 * 64 && HVP <= 6 * 64, "six DMA instructions per half");
 
-// Tile geometry of the 3^3 convolutions (16 x 16 output voxels per work-group at TX = 16) and the halo offsets of
-// the taps; HVP pads each channel half of the halo to whole 256-voxel DMA rounds.
-template <int TX>
-struct ConvTile {
-  static constexpr int TY = 256 / TX;
-  static constexpr int HX = TX + 2, HY = TY + 2;
-  static constexpr int HV = 3 * HY * HX;          // halo voxels
-  static constexpr int NR = (HV + 255) / 256;     // DMA rounds per half
-  static constexpr int HVP = NR * 256;            // halo slots per half
-  static constexpr int WC = 16;
-  // halo offset of tap t (t = 27: the zero-weight tap, whose A reads the centre tap 13)
-  __host__ __device__ static constexpr int shift(int t) {
-    const int tv = t < 27 ? t : 13;
-    return (tv / 9 * HY + tv / 3 % 3) * HX + tv % 3;
-  }
-  // the odd tap of pair p lies one of four offsets beyond the even one
-  static constexpr int DOFF[4] = {1, HX - 2, HX * HY - 2 * HX - 2, shift(27) - shift(26)};
-  __host__ __device__ static constexpr int dkind(int p) {
-    const int d = shift(2 * p + 1) - shift(2 * p);
-    return d == DOFF[0] ? 0 : d == DOFF[1] ? 1 : d == DOFF[2] ? 2 : d == DOFF[3] ? 3 : -1;
-  }
-  __host__ __device__ static constexpr bool pairs_ok() {
-    for (int p = 0; p < 14; ++p)
-      if (dkind(p) < 0) return false;
-    return true;
-  }
+__device__ __attribute__((aligned(16))) uint16_t g_zero[8];  // what halo voxels outside the volume read
+
+// DMA instruction id of a plane fills half id / 6, voxels dma_voxel(id)..+63; a half's last instruction starts early and
+// repeats voxels of the one before it (the same values), so that every lane of every instruction writes
+__device__ __forceinline__ int dma_voxel(int id) { return min(id % 6 * 64, HVP - 64); }
+
+// a 16-channel chunk's source and this lane's halo voxels in it
+struct RingSrc {
+  const uint16_t* base;   // the sample's first plane
+  size_t plane;           // elements between planes
+  int sh;                 // 1: the upsampled (coarse) source
+  int off[kDma];          // element offsets in a plane, -1: zeros (outside the xy extent, or channels not stored)
 };
 
-template <int TX, int NG>
-__global__ __launch_bounds__(256) void k_conv_tile(ConvArgs a, int zp) {
-  constexpr int TY = 256 / TX;          // tile rows
-  constexpr int HX = TX + 2, HY = TY + 2;
-  constexpr int HV = 3 * HY * HX;       // halo voxels
-  constexpr int SEGX = TX / 16;         // 16-voxel segments per row
-  constexpr int WC = NG * 16;           // output channels of this work-group
-  __shared__ __attribute__((aligned(16))) uint16_t tile[HV * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t wl[28 * WC * 16];
+__device__ __forceinline__ RingSrc ring_src(const ConvArgs& a, int n, int x0, int y0, int cb, int wave, int lane) {
+  RingSrc s;
+  const bool up = cb * 16 < a.up_c;
+  s.sh = up ? 1 : 0;
+  const int sH = a.H >> s.sh, sW = a.W >> s.sh, cs = up ? a.up_cs : a.in_cs;
+  const int halves = !up && a.in_half ? 1 : 2;
+  s.plane = (size_t)sH * sW * cs;
+  s.base = (up ? a.up_in + cb * 16 : a.in + (cb * 16 - a.up_c)) + (size_t)n * (a.D >> s.sh) * s.plane;
+#pragma unroll
+  for (int j = 0; j < kDma; ++j) {
+    const int id = wave * kDma + j, v = dma_voxel(id) + lane;
+    const int xx = x0 + v % HX - 1, yy = y0 + v / HX - 1;
+    const bool ok = (unsigned)xx < (unsigned)a.W && (unsigned)yy < (unsigned)a.H && id / 6 < halves;
+    s.off[j] = ok ? ((yy >> s.sh) * sW + (xx >> s.sh)) * cs + (id / 6) * 8 : -1;
+  }
+  return s;
+}
 
+// DMA of the halo of input plane z into the ring plane `dst`: kDma instructions of every wave
+__device__ __forceinline__ void ring_issue(const RingSrc& s, int z, int D, int wave, uint16_t* __restrict__ dst) {
+  const bool zok = (unsigned)z < (unsigned)D;
+  const uint16_t* src = s.base + (zok ? (size_t)(z >> s.sh) * s.plane : 0);
+#pragma unroll
+  for (int j = 0; j < kDma; ++j) {
+    const int id = wave * kDma + j;
+    const uint16_t* p = zok && s.off[j] >= 0 ? src + s.off[j] : g_zero;
+    __builtin_amdgcn_global_load_lds((const void*)p,
+                                     (__attribute__((address_space(3))) void*)(dst + (id / 6 * HVP + dma_voxel(id)) * 8),
+                                     16, 0, 0);
+  }
+}
+
+// The products of one output plane: ring planes s0, s1, s2 (dz = -1, 0, 1) with the weights wf into acc.  Called with
+// the ring planes that DMA loads may be filling as further restrict parameters, so that the compiler can tell the DMA's
+// writes from this plane's reads and does not wait for the DMA before them.  Every fragment address is one of a few
+// per-lane bases plus a constant: the odd tap of a pair lies one voxel, or one row less two voxels, beyond the even
+// one, or is the first tap of the next plane.  LAST: the next chunk's weights replace each pair's after its last use
+// (wnext: the next chunk's weights).
+struct Weights {
+  const uint16_t* base;    // the layer's weights
+  int lane0, lane1;        // this lane's byte offsets for pair 13 (tap 26 and the zero tap) and the others
+  int chunk;               // byte offset of the output group and chunk (uniform)
+  int pair, group;         // bytes between tap pairs, between 16-channel output blocks
+};
+template <int NG>
+__device__ __forceinline__ void load_pair(const Weights& w, int p, bf16x8 (&wf)[NG]) {
+  // a buffer load: the uniform part of the address in a scalar, so that the pairs' addresses take no vector registers
+  const __amdgpu_buffer_rsrc_t r =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w.base), 0, 0xffffffff, 0x00020000);
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int t = 0; t < NG; ++t) {
+    u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, p < 13 ? w.lane1 : w.lane0, w.chunk + p * w.pair + t * w.group, 0);
+    if (p == 13 && (threadIdx.x & 32)) v = u32x4{0u, 0u, 0u, 0u};
+    wf[t] = __builtin_bit_cast(bf16x8, v);
+  }
+}
+
+template <int NG, bool LAST, int AHEAD>
+__device__ __forceinline__ void ring_products(const uint16_t* __restrict__ s0, const uint16_t* __restrict__ s1,
+                                              const uint16_t* __restrict__ s2, bf16x8 (&wf)[14][NG],
+                                              f32x4 (&acc)[4][NG], const Weights& wnext) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int hi = lane >> 5, hsel = (lane >> 4) & 1;
+  int lb = hsel * HVP + 4 * wave * HX + (lane & 15);
+  asm volatile("" : "+v"(lb));  // the addresses are formed here, not kept in registers for every ring position
+  auto frag = [&](int p, int m) {
+    const int t0 = 2 * p, t1 = t0 < 26 ? t0 + 1 : t0;  // tap 27 has zero weights: it reads tap 26
+    const int d0 = t0 / 9, d1 = t1 / 9;
+    const uint16_t* q0 = d0 == 0 ? s0 : d0 == 1 ? s1 : s2;
+    const int sh0 = (t0 / 3 % 3) * HX + t0 % 3, sh1 = (t1 / 3 % 3) * HX + t1 % 3;
+    const uint16_t* q;
+    if (d0 == d1) {
+      q = q0 + (lb + hi * (sh1 - sh0) + sh0) * 8;
+    } else {
+      const uint16_t* q1 = d1 == 1 ? s1 : s2;
+      q = hi ? q1 + (lb + sh1) * 8 : q0 + (lb + sh0) * 8;
+    }
+    return *reinterpret_cast<const bf16x8*>(q + m * HX * 8);
+  };
+  bf16x8 vf[14][4];
+#pragma unroll
+  for (int p = 0; p < 14; ++p)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) vf[p][m] = frag(p, m);
+#pragma unroll
+  for (int p = 0; p < 14; ++p) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int t = 0; t < NG; ++t)
+        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[p][t], vf[p][m], acc[m][t], 0, 0, 0);
+    if (LAST) load_pair<NG>(wnext, p, wf[p]);
+  }
+  // The reads run AHEAD to AHEAD + 1 pairs ahead of the products (left to itself the compiler waits for each read at
+  // its product: 1037 -> 926-968 us for the 48 -> 16 layer at 252 x 250 x 254).  AHEAD = 0 leaves it so: at three
+  // work-groups per CU the registers of reads in flight spill, and the others' reads fill the gaps (16 -> 16 layer: 272 us,
+  // 304 us with two work-groups and reads two pairs ahead).
+  if constexpr (AHEAD > 0) {
+    __builtin_amdgcn_sched_group_barrier(0x100, 4 * AHEAD, 0);  // LDS reads
+#pragma unroll
+    for (int p = 0; p < 14 - AHEAD; ++p) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 4 * NG, 0);  // MFMA
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * NG * AHEAD, 0);
+  }
+  // the products belong before the wait that follows (nothing else orders them with it)
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int t = 0; t < NG; ++t) asm volatile("" : "+v"(acc[m][t]));
+}
+
+// the weights of a chunk: lane l holds output channel l%16 of tap 2p + l/32, channels 8 (l/16 % 2)..+7
+__device__ __forceinline__ Weights ring_weights(const ConvArgs& a, int co0, int cb) {
+  const int lane = threadIdx.x & 63;
+  Weights w;
+  w.base = a.w;
+  w.lane0 = 2 * ((lane & 15) * a.cin + ((lane >> 4) & 1) * 8);
+  w.lane1 = w.lane0 + 2 * (lane >> 5) * a.cout * a.cin;
+  w.chunk = 2 * (co0 * a.cin + cb * 16);
+  w.pair = 4 * a.cout * a.cin;
+  w.group = 32 * a.cin;
+  return w;
+}
+
+// bias and ReLU of output plane z, bf16 stores, and what is fused behind them:
+//   - the 2x2x2 pooling: even lanes sum the stored values of their voxel pair (the odd voxel's from the next lane) in
+//     the order of k_pool_fwd, z, then y, then x, so the fused pooling rounds exactly as the pooling kernel; pool[ky]
+//     carries the sums from an even plane to the odd one after it;
+//   - the output head of an inference (NG = 1, 16 channels): psi of voxel (row 4 wave + l/16, l%16) per lane, the
+//     activations themselves not stored.
+enum Epilogue { kPlain, kPool, kHead };
+template <int NG, int EPI>
+__device__ __forceinline__ void ring_store(const ConvArgs& a, int n, int z, int x0, int y0, int co0,
+                                           const f32x4 (&acc)[4][NG], const f32x4 (&bias)[NG], const f32x4& hw,
+                                           float hb, float avg, float (*pool)[NG][4]) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i = lane & 15, g = lane >> 4;
-  const int hi = g >> 1;                // tap of the pair carried by this lane
-  const int ch8 = (g & 1) * 8;          // first of the lane's eight channels
-  // work-group -> (n, z group, y block, x block); x block fastest.  Consecutive work-groups go to the 8 XCDs
-  // in turn, so the tile order is remapped to give each XCD a contiguous range of tiles (whole z planes
-  // and their neighbours stay in that XCD's L2).
+  const int x = x0 + i;
+  uint16_t* outPlane = a.out + ((size_t)n * a.D + z) * a.H * a.W * a.out_cs + a.out_co + co0 + 4 * g;
+  constexpr bool pooling = EPI == kPool;
+  if (pooling && !(z & 1)) {
+#pragma unroll
+    for (int ky = 0; ky < 2; ++ky)
+#pragma unroll
+      for (int t = 0; t < NG; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pool[ky][t][r] = 0.f;
+  }
+  float head = 0.f;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const int y = y0 + 4 * wave + m;
+    const bool ok = y < a.H && x < a.W;
+#pragma unroll
+    for (int t = 0; t < NG; ++t) {
+      uint32_t b[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = acc[m][t][r] + bias[t][r];
+        if (a.relu) v = fmaxf(v, 0.f);
+        b[r] = f2bf_rne(v);
+      }
+      if constexpr (EPI == kHead) {
+        float h = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h += hw[r] * bf2f(b[r]);
+        h += __shfl_xor(h, 16, 64);
+        h += __shfl_xor(h, 32, 64);
+        head = m == g ? h : head;
+        continue;
+      }
+      if (ok)
+        *reinterpret_cast<uint2*>(outPlane + ((size_t)y * a.W + x) * a.out_cs + t * 16) =
+            make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+      if (pooling) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int own = __float_as_int(bf2f(b[r]));
+          const float next = __int_as_float(__builtin_amdgcn_update_dpp(0, own, 0xB1, 0xf, 0xf, true));  // lane ^ 1
+          pool[m >> 1][t][r] += __int_as_float(own);
+          pool[m >> 1][t][r] += next;
+        }
+      }
+    }
+  }
+  if constexpr (EPI == kHead) {
+    const int y = y0 + 4 * wave + g;
+    if (y < a.psi.oy && x < a.psi.ox && z >= a.psi.zlo && z < a.psi.oz) {
+      const float pred = avg + (head + hb);
+      a.psi.out[((size_t)z * a.psi.oy + y) * a.psi.ox + x] = fmaxf(a.psi.minValue, a.psi.scale * pred);
+    }
+  }
+  if (pooling && (z & 1)) {
+    // the plane pair is complete: output voxel (z / 2, y / 2, x / 2) of the pooled tensor (D, H, W even)
+    const int H2 = a.H / 2, W2 = a.W / 2, x2 = x / 2;
+    uint16_t* pp = a.pool_out + ((size_t)n * (a.D / 2) + z / 2) * H2 * W2 * a.pool_cs + co0 + 4 * g;
+#pragma unroll
+    for (int ky = 0; ky < 2; ++ky) {
+      const int y2 = (y0 + 4 * wave) / 2 + ky;
+      if ((i & 1) || y2 >= H2 || x2 >= W2) continue;
+#pragma unroll
+      for (int t = 0; t < NG; ++t) {
+        uint32_t b[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) b[r] = f2bf_rne(pool[ky][t][r] * 0.125f);
+        *reinterpret_cast<uint2*>(pp + ((size_t)y2 * W2 + x2) * a.pool_cs + t * 16) =
+            make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+      }
+    }
+  }
+}
+
+struct RingTile {
+  int x0, y0, zs, n;
+};
+// work-group -> (n, z group of zp planes, y block, x block); x block fastest.  Consecutive work-groups go to the 8 XCDs
+// in turn, so the tile order is remapped to give each XCD a contiguous range of tiles (whole z planes and their
+// neighbours stay in that XCD's L2).
+__device__ __forceinline__ RingTile ring_tile(const ConvArgs& a, int zp) {
   const int nbx = (a.W + TX - 1) / TX, nby = (a.H + TY - 1) / TY, nzg = (a.D + zp - 1) / zp;
   const int nbt = (int)gridDim.x;
   int b = nbt % 8 == 0 ? (int)(blockIdx.x % 8) * (nbt / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-  const int bx = b % nbx; b /= nbx;
-  const int by = b % nby; b /= nby;
-  const int zg = b % nzg, n = b / nzg;
-  const int x0 = bx * TX, y0 = by * TY;
-  const int zs = zg * zp, ze = min(a.D, zs + zp);
-  const int co0 = blockIdx.y * WC;
+  RingTile t;
+  t.x0 = (b % nbx) * TX;
+  b /= nbx;
+  t.y0 = (b % nby) * TY;
+  b /= nby;
+  t.zs = (b % nzg) * zp;
+  t.n = b / nzg;
+  return t;
+}
 
-  f32x4 acc[4][NG];
+template <int NG>
+__device__ __forceinline__ void ring_bias(const ConvArgs& a, int co0, f32x4 (&bias)[NG]) {
+  const int g = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int t = 0; t < NG; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bias[t][r] = a.bias ? a.bias[co0 + t * 16 + 4 * g + r] : 0.f;
+}
+
+template <int NG>
+__device__ __forceinline__ void zero_acc(f32x4 (&acc)[4][NG]) {
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll
     for (int t = 0; t < NG; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
 
-  // Staging of one (plane, 16-channel chunk) item: every thread issues all of its 16-byte loads (branch-free,
-  // invalid lanes read a valid dummy address) before the first LDS write, so the loads are in flight together.
-  constexpr int NL = (HV * 2 + 255) / 256;         // halo loads per thread
-  constexpr int NW = (28 * WC * 2 + 255) / 256;    // weight loads per thread
-  uint4 hbuf[NL], wbuf[NW];
-  // per-thread halo coordinates of unit k: v = (threadIdx.x >> 1) + 128 k, decomposed incrementally
-  const int half = threadIdx.x & 1;
-  auto issue = [&](int z, int cb, bool weights) {
-    // the chunk comes from the upsampled source (half coordinates) or from in
-    const bool up = cb * 16 < a.up_c;
-    const int sh = up ? 1 : 0;
-    const int sD = a.D >> sh, sH = a.H >> sh, sW = a.W >> sh;
-    const int cs = up ? a.up_cs : a.in_cs;
-    // base of the first source plane the halo touches, in 64 bits; offsets from it span at most three
-    // planes and fit 32 bits (checked at launch).  zb = max(z - 1, 0) >> sh is a valid plane, so the
-    // dummy address of an invalid lane (offset 0) is inside the tensor.
-    const int zb = max(z - 1, 0) >> sh;
-    const uint16_t* src = (up ? a.up_in + cb * 16 : a.in + (cb * 16 - a.up_c)) +
-                          ((size_t)n * sD + zb) * sH * sW * cs + half * 8;
-    int v0 = threadIdx.x >> 1;
-    int hx = v0 % HX, hy = (v0 / HX) % HY, hz = v0 / (HX * HY);
-    constexpr int DX = 128 % HX, DY = (128 / HX) % HY, DZ = 128 / (HX * HY);
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      if (k) {  // advance by 128 halo voxels
-        hx += DX;
-        int cy = hx >= HX;
-        hx -= cy ? HX : 0;
-        hy += DY + cy;
-        int cz = hy >= HY;
-        hy -= cz ? HY : 0;
-        hz += DZ + cz;
-      }
-      const int xx = x0 + hx - 1, yy = y0 + hy - 1, zz = z + hz - 1;
-      const bool ok = (threadIdx.x + 256 * k) < HV * 2 && (unsigned)xx < (unsigned)a.W &&
-                      (unsigned)yy < (unsigned)a.H && (unsigned)zz < (unsigned)a.D;
-      const int gv = (((zz >> sh) - zb) * sH + (yy >> sh)) * sW + (xx >> sh);
-      hbuf[k] = *reinterpret_cast<const uint4*>(src + (ok ? gv * cs : 0));
-      if (!ok) hbuf[k] = make_uint4(0u, 0u, 0u, 0u);
-    }
-    if (!weights) return;
-#pragma unroll
-    for (int k = 0; k < NW; ++k) {
-      const int e = threadIdx.x + 256 * k;
-      const int c = (e >> 1) % WC, tap = (e >> 1) / WC;
-      const bool ok = tap < 27;
-      wbuf[k] = *reinterpret_cast<const uint4*>(a.w + ((ok ? tap : 0) * a.cout + co0 + c) * a.cin + cb * 16 +
-                                               half * 8);
-      if (!ok) wbuf[k] = make_uint4(0u, 0u, 0u, 0u);
-    }
-  };
-  auto park = [&](bool weights) {
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      const int e = threadIdx.x + 256 * k;
-      if (e < HV * 2) *reinterpret_cast<uint4*>(tile + ((e & 1) * HV + (e >> 1)) * 8) = hbuf[k];
-    }
-    if (!weights) return;
-#pragma unroll
-    for (int k = 0; k < NW; ++k) {
-      const int e = threadIdx.x + 256 * k;
-      if (e < 28 * WC * 2) *reinterpret_cast<uint4*>(wl + ((e & 1) * 28 * WC + (e >> 1)) * 8) = wbuf[k];
-    }
-  };
+// All but the wave's last `YOUNGER` memory operations have completed (its DMA among them, in issue order); after the
+// barrier that holds for every wave, and every wave is done with the planes it has read.  The wait is the wave's own
+// s_waitcnt: the barrier's fence would wait for the DMA still wanted in flight.
+template <int YOUNGER>
+__device__ __forceinline__ void ring_wait() {
+  static_assert(YOUNGER < 16, "low vmcnt bits");
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070 | YOUNGER);  // vmcnt(YOUNGER) lgkmcnt(0), no export wait
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 
-  const int nchunk = a.cin / 16;
-  const int nitems = (ze - zs) * nchunk;  // (plane, chunk) items, chunks fastest
-  const int hsel = ch8 ? 1 : 0;  // the lane's channel half
-  // a single-chunk layer stages its weights once per work-group
-  for (int it = 0; it < nitems; ++it) {
-    const int z = zs + it / nchunk, cb = it % nchunk;
-    const bool wts = nchunk > 1 || it == 0;
-    if (it) __syncthreads();  // the previous item's LDS reads are done
-    issue(z, cb, wts);
-    park(wts);
-    __syncthreads();
-    // Every fragment address is one of four per-lane bases plus a constant: the odd tap of a pair lies one of four
-    // offsets beyond the even one, and the B fragment's tap parity is the lane's (no tap arithmetic in the loop).
-    {
-      using G = ConvTile<TX>;
-      static_assert(TX == 16 && G::pairs_ok(), "one 16-voxel segment per tile row, four odd-tap offsets");
-      const int lb = hsel * HV + 4 * wave * HX + i;
-      const uint16_t* ab[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) ab[k] = tile + (lb + hi * G::DOFF[k]) * 8;
-      const uint16_t* wb = wl + (hsel * 28 * WC + hi * WC + i) * 8;
-#pragma unroll
-      for (int p = 0; p < 14; ++p) {
-        bf16x8 bfr[NG];
-#pragma unroll
-        for (int t = 0; t < NG; ++t) bfr[t] = *reinterpret_cast<const bf16x8*>(wb + (2 * p * WC + t * 16) * 8);
-        const uint16_t* a0 = ab[G::dkind(p)] + G::shift(2 * p) * 8;
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          const bf16x8 afr = *reinterpret_cast<const bf16x8*>(a0 + m * HX * 8);
-#pragma unroll
-          for (int t = 0; t < NG; ++t)
-            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr, bfr[t], acc[m][t], 0, 0, 0);
-        }
-      }
-    }
-    if (cb != nchunk - 1) continue;
+// One step of a column: the DMA of input plane zn into `nxt`, the products, the wait for the plane the next step needs
+// (its DMA went out a step earlier; `nxt` stays in flight), the stores, which drain during the next step.
+template <int NG, int EPI>
+__device__ __forceinline__ void column_step(const ConvArgs& a, const RingSrc& src, const RingTile& T, int z, int ze,
+                                            int co0, const uint16_t* __restrict__ s0, const uint16_t* __restrict__ s1,
+                                            const uint16_t* __restrict__ s2, const uint16_t* __restrict__ s3,
+                                            uint16_t* __restrict__ nxt, bf16x8 (&wf)[14][NG],
+                                            const f32x4 (&bias)[NG], const f32x4& hw, float hb, float (*pool)[NG][4]) {
+  (void)s3;  // in flight or landed: distinct from the others for the compiler
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  f32x4 acc[4][NG];
+  zero_acc<NG>(acc);
+  float avg = 0.f;
+  if constexpr (EPI == kHead) {
+    const int y = T.y0 + 4 * wave + (lane >> 4), x = T.x0 + (lane & 15);
+    avg = a.psi.avg[((size_t)z * a.H + min(y, a.H - 1)) * a.W + min(x, a.W - 1)];
+  }
+  const bool more = z + 2 < ze;
+  if (more) ring_issue(src, z + 3, a.D, wave, nxt);
+  __builtin_amdgcn_sched_barrier(0);  // the DMA goes out before the products, not behind them
+  ring_products<NG, false, NG == 1 ? 0 : 1>(s0, s1, s2, wf, acc, Weights{});
+  if (more)
+    ring_wait<kDma>();
+  else if (z + 1 < ze)
+    ring_wait<0>();
+  ring_store<NG, EPI>(a, T.n, z, T.x0, T.y0, co0, acc, bias, hw, hb, avg, pool);
+}
 
-    // epilogue of plane z: bias, ReLU, bf16 stores (voxel 4g + r of the segment, channel co0 + t * 16 + i)
-    float bias[NG];
+// One chunk: a column of zp planes through a ring of five (unrolled by five, so that the ring positions are known at
+// compile time).
+template <int NG, int EPI>
+__global__ __launch_bounds__(256, NG == 1 ? 3 : 2) void k_conv_column(ConvArgs a, int zp) {
+  __shared__ __attribute__((aligned(16))) uint16_t r0[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r1[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r2[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r3[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r4[kPlane];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const RingTile T = ring_tile(a, zp);
+  const int co0 = blockIdx.y * NG * 16, ze = min(a.D, T.zs + zp);
+  bf16x8 wf[14][NG];
+  f32x4 bias[NG];
+  float pool[2][NG][4];
+  const RingSrc src = ring_src(a, T.n, T.x0, T.y0, 0, wave, lane);
+  ring_issue(src, T.zs - 1, a.D, wave, r0);
+  ring_issue(src, T.zs, a.D, wave, r1);
+  ring_issue(src, T.zs + 1, a.D, wave, r2);
+  ring_issue(src, T.zs + 2, a.D, wave, r3);
+  const Weights w = ring_weights(a, co0, 0);
 #pragma unroll
-    for (int t = 0; t < NG; ++t) bias[t] = a.bias ? a.bias[co0 + t * 16 + i] : 0.f;
-    uint16_t* outPlane = a.out + (((size_t)n * a.D + z) * a.H) * a.W * a.out_cs + a.out_co + co0 + i;
+  for (int p = 0; p < 14; ++p) load_pair<NG>(w, p, wf[p]);
+  ring_bias<NG>(a, co0, bias);
+  f32x4 hw{};
+  float hb = 0.f;
+  if constexpr (EPI == kHead) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int s = 4 * wave + m;
-      const int y = y0 + s / SEGX;
-      const int xs = x0 + (s % SEGX) * 16 + 4 * g;
-      if (y < a.H) {
-        uint16_t* orow = outPlane + ((size_t)y * a.W + xs) * a.out_cs;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (xs + r >= a.W) continue;
-#pragma unroll
-          for (int t = 0; t < NG; ++t) {
-            float v = acc[m][t][r] + bias[t];
-            if (a.relu) v = fmaxf(v, 0.f);
-            orow[r * a.out_cs + t * 16] = f2bf_rne(v);
-          }
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < NG; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int r = 0; r < 4; ++r) hw[r] = a.psi.w[4 * (lane >> 4) + r];
+    hb = a.psi.w[16];
+  }
+  ring_wait<0>();
+  for (int z = T.zs;; z += 5) {
+    column_step<NG, EPI>(a, src, T, z, ze, co0, r0, r1, r2, r3, r4, wf, bias, hw, hb, pool);
+    if (z + 1 >= ze) break;
+    column_step<NG, EPI>(a, src, T, z + 1, ze, co0, r1, r2, r3, r4, r0, wf, bias, hw, hb, pool);
+    if (z + 2 >= ze) break;
+    column_step<NG, EPI>(a, src, T, z + 2, ze, co0, r2, r3, r4, r0, r1, wf, bias, hw, hb, pool);
+    if (z + 3 >= ze) break;
+    column_step<NG, EPI>(a, src, T, z + 3, ze, co0, r3, r4, r0, r1, r2, wf, bias, hw, hb, pool);
+    if (z + 4 >= ze) break;
+    column_step<NG, EPI>(a, src, T, z + 4, ze, co0, r4, r0, r1, r2, r3, wf, bias, hw, hb, pool);
+    if (z + 5 >= ze) break;
   }
 }
 
-// Single-chunk layers with 16 output channels (the full-resolution 16 -> 16 layers) on large launches: the
-// work-group walks kConvZPDma planes and stages the next plane's halo into a second LDS buffer with LDS-DMA loads
-// (global_load_lds_dwordx4: 16 bytes per lane into LDS at the wave's base + 16 lane, no registers) while the
-// MFMAs of the current plane run.  One DMA instruction per 8-channel half writes 256 consecutive voxels of
-// that half, so the LDS layout is the same half-major [half][voxel][8] as above (halves padded to HVP voxels,
-// whole DMA rounds; the padding slots take the dummy loads and are never read).  Halo voxels outside the
-// volume load a valid dummy address and are zeroed after the DMA has landed.  The arithmetic is that of
-// k_conv_tile<TX, 1>: the results are bitwise equal.
-constexpr int kConvZPDma = 8;
-
-// per-lane state of the DMA staging: the lane's halo voxels v0 + 256 r (r < NR), their element offsets from the
-// plane before the output plane (the same for every plane), which are inside the xy extent, and their z offsets
-template <int TX>
-struct DmaLane {
-  const uint16_t* nbase;  // this sample's first plane
-  long long planeElems;
-  int x0, y0;
-  int off[ConvTile<TX>::NR];
-  int hz[ConvTile<TX>::NR];
-  unsigned okxy;          // bit r: voxel r inside the halo and the xy extent
-};
-
-// DMA of plane z's halo into `dst` (both halves); returns the mask of rounds whose voxel lies outside the volume
-template <int TX>
-__device__ __forceinline__ unsigned conv_dma_issue(const ConvArgs& a, const DmaLane<TX>& L, int z,
-                                                   uint16_t* __restrict__ dst) {
-  using T = ConvTile<TX>;
-  const int wave = threadIdx.x >> 6;
-  const long long zoff = (long long)(z - 1) * L.planeElems;  // the lane offsets count from plane z - 1
-  unsigned bad = 0;
-#pragma unroll
-  for (int r = 0; r < T::NR; ++r) {
-    const bool ok = ((L.okxy >> r) & 1u) && (unsigned)(z + L.hz[r] - 1) < (unsigned)a.D;
-    // a voxel outside the volume loads the sample's first voxel (a valid address) and is zeroed afterwards
-    const uint16_t* p = L.nbase + (ok ? zoff + L.off[r] : 0ll);
-    bad |= ok ? 0u : 1u << r;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      __builtin_amdgcn_global_load_lds((const void*)(p + h * 8),
-                                       (__attribute__((address_space(3))) void*)(dst + (h * T::HVP + wave * 64 +
-                                                                                       256 * r) * 8),
-                                       16, 0, 0);
-  }
-  return bad;
+// Several chunks, NG = 1: the accumulators of four planes stay in registers while the chunks' six input planes each
+// pass through a ring of six, the next chunk's planes and weights requested during the current one.
+__device__ __forceinline__ void chunk_planes4(const ConvArgs& a, const RingSrc& cur, const RingSrc& nx, bool more,
+                                              int zs, uint16_t* __restrict__ r0, uint16_t* __restrict__ r1,
+                                              uint16_t* __restrict__ r2, uint16_t* __restrict__ r3,
+                                              uint16_t* __restrict__ r4, uint16_t* __restrict__ r5,
+                                              bf16x8 (&wf)[14][1], f32x4 (&acc)[4][4][1], const Weights& wnext) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  ring_issue(cur, zs + 2, a.D, wave, r3);
+  ring_issue(cur, zs + 3, a.D, wave, r4);
+  ring_issue(cur, zs + 4, a.D, wave, r5);
+  __builtin_amdgcn_sched_barrier(0);
+  ring_products<1, false, 2>(r0, r1, r2, wf, acc[0], wnext);
+  ring_wait<2 * kDma>();
+  if (more) ring_issue(nx, zs - 1, a.D, wave, r0);
+  __builtin_amdgcn_sched_barrier(0);
+  ring_products<1, false, 2>(r1, r2, r3, wf, acc[1], wnext);
+  ring_wait<kDma>();
+  if (more) ring_issue(nx, zs, a.D, wave, r1);
+  __builtin_amdgcn_sched_barrier(0);
+  ring_products<1, false, 2>(r2, r3, r4, wf, acc[2], wnext);
+  ring_wait<0>();
+  if (more) ring_issue(nx, zs + 1, a.D, wave, r2);
+  __builtin_amdgcn_sched_barrier(0);
+  ring_products<1, true, 2>(r3, r4, r5, wf, acc[3], wnext);
+  ring_wait<0>();
 }
 
-// after the lane's DMA has landed: zeros into the slots of its voxels outside the volume
-template <int TX>
-__device__ __forceinline__ void conv_dma_fix(unsigned bad, uint16_t* __restrict__ dst) {
-  using T = ConvTile<TX>;
-  if (!bad) return;
+template <int NCHUNK>
+__global__ __launch_bounds__(256, 2) void k_conv_chunks4(ConvArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t r0[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r1[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r2[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r3[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r4[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r5[kPlane];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const RingTile T = ring_tile(a, 4);
+  const int co0 = blockIdx.y * 16;
+  bf16x8 wf[14][1];
+  f32x4 acc[4][4][1];
 #pragma unroll
-  for (int r = 0; r < T::NR; ++r) {
-    if (!((bad >> r) & 1u)) continue;
+  for (int o = 0; o < 4; ++o) zero_acc<1>(acc[o]);
+  RingSrc cur = ring_src(a, T.n, T.x0, T.y0, 0, wave, lane);
+  ring_issue(cur, T.zs - 1, a.D, wave, r0);
+  ring_issue(cur, T.zs, a.D, wave, r1);
+  ring_issue(cur, T.zs + 1, a.D, wave, r2);
+  const Weights w = ring_weights(a, co0, 0);
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      *reinterpret_cast<uint4*>(dst + (h * T::HVP + (int)threadIdx.x + 256 * r) * 8) = make_uint4(0u, 0u, 0u, 0u);
+  for (int p = 0; p < 14; ++p) load_pair<1>(w, p, wf[p]);
+  ring_wait<0>();
+#pragma unroll
+  for (int cb = 0; cb < NCHUNK; ++cb) {
+    const int nb = cb + 1 < NCHUNK ? cb + 1 : cb;
+    const RingSrc nx = ring_src(a, T.n, T.x0, T.y0, nb, wave, lane);
+    chunk_planes4(a, cur, nx, cb + 1 < NCHUNK, T.zs, r0, r1, r2, r3, r4, r5, wf, acc, ring_weights(a, co0, nb));
+    cur = nx;
   }
+  f32x4 bias[1];
+  ring_bias<1>(a, co0, bias);
+#pragma unroll
+  for (int o = 0; o < 4; ++o)
+    if (T.zs + o < a.D) ring_store<1, kPlain>(a, T.n, T.zs + o, T.x0, T.y0, co0, acc[o], bias, f32x4{}, 0.f, 0.f, nullptr);
 }
 
-// One plane's MFMAs: the next plane's DMA into `nxt` (when `more`), then the products of plane z from `cur` with
-// the weights `w` into acc.  The LDS buffers are distinct restrict parameters, so that the compiler can tell the
-// DMA's writes from this plane's reads and does not wait for the DMA before them.  The loop is unrolled and every
-// fragment address is one of four per-lane bases plus a constant (the A bases differ by the odd tap's offset
-// kind, the B base by the lane's tap parity), so the loop issues no address arithmetic.  Returns the mask of the
-// next plane's voxels outside the volume.
-template <int TX>
-__device__ __forceinline__ unsigned conv_dma_mfma(const ConvArgs& a, const DmaLane<TX>& L, int z, bool more,
-                                                  f32x4* acc, const uint16_t* __restrict__ cur,
-                                                  uint16_t* __restrict__ nxt, const uint16_t* __restrict__ w) {
-  using T = ConvTile<TX>;
-  static_assert(TX == 16 && T::pairs_ok(), "one 16-voxel segment per tile row, four odd-tap offsets");
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int i = lane & 15, g = lane >> 4;
-  const int hi = g >> 1;       // tap of the pair carried by this lane
-  const int hsel = g & 1;      // the lane's channel half
-  const unsigned bad = more ? conv_dma_issue<TX>(a, L, z + 1, nxt) : 0u;
-  // A: segment m of this wave at halo row 4 wave + m, voxel i; B: output channel i of the lane's tap
-  const int lb = hsel * T::HVP + 4 * wave * T::HX + i;
-  const uint16_t* ab[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) ab[k] = cur + (lb + hi * T::DOFF[k]) * 8;
-  const uint16_t* wb = w + (hsel * 28 * T::WC + hi * T::WC + i) * 8;
-#pragma unroll
-  for (int m = 0; m < 4; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int p = 0; p < 14; ++p) {
-    const bf16x8 bfr = *reinterpret_cast<const bf16x8*>(wb + 2 * p * T::WC * 8);
-    const uint16_t* a0 = ab[T::dkind(p)] + T::shift(2 * p) * 8;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const bf16x8 afr = *reinterpret_cast<const bf16x8*>(a0 + m * T::HX * 8);
-      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr, bfr, acc[m], 0, 0, 0);
-    }
+// Several chunks, NG = 2: two planes' accumulators; a chunk's four input planes take the ring positions 4 c .. 4 c + 3
+// modulo six, so three chunks are unrolled.
+__device__ __forceinline__ void chunk_planes2(const ConvArgs& a, const RingSrc& cur, const RingSrc& nx, bool more,
+                                              int zs, uint16_t* __restrict__ r0, uint16_t* __restrict__ r1,
+                                              uint16_t* __restrict__ r2, uint16_t* __restrict__ r3,
+                                              uint16_t* __restrict__ r4, uint16_t* __restrict__ r5,
+                                              bf16x8 (&wf)[14][2], f32x4 (&acc)[2][4][2], const Weights& wnext) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  ring_issue(cur, zs + 2, a.D, wave, r3);
+  if (more) {
+    ring_issue(nx, zs - 1, a.D, wave, r4);
+    ring_issue(nx, zs, a.D, wave, r5);
   }
-  return bad;
+  __builtin_amdgcn_sched_barrier(0);
+  ring_products<2, false, 1>(r0, r1, r2, wf, acc[0], wnext);
+  if (more)
+    ring_wait<2 * kDma>();
+  else
+    ring_wait<0>();
+  if (more) ring_issue(nx, zs + 1, a.D, wave, r0);
+  __builtin_amdgcn_sched_barrier(0);
+  ring_products<2, false, 1>(r1, r2, r3, wf, acc[1], wnext);
+  if (more) {
+#pragma unroll
+    for (int p = 0; p < 14; ++p) load_pair<2>(wnext, p, wf[p]);
+  }
+  ring_wait<0>();
 }
 
-// bias (read before any DMA: a load issued after one would wait for it), ReLU and bf16 stores of plane z: voxel
-// 4g + r of the segment, channel i.  With a pooled output, pool[ky][kx] (the lane's 2 x 2 output voxels of the
-// plane pair) sums the stored values in the order of k_pool_fwd: z, then y, then x (even plane first: rows
-// m = 2 ky, 2 ky + 1, voxels r = 2 kx, 2 kx + 1), so the fused pooling rounds exactly as the pooling kernel.
-template <int TX>
-__device__ __forceinline__ void conv_dma_store(const ConvArgs& a, const DmaLane<TX>& L, int n, int z,
-                                               const f32x4* acc, float bias, float (*pool)[2]) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int i = lane & 15, g = lane >> 4;
-  uint16_t* outPlane = a.out + (((size_t)n * a.D + z) * a.H) * a.W * a.out_cs + a.out_co + i;
-  const bool pooling = a.pool_out != nullptr;
-  if (pooling && !(z & 1)) {
+template <int NCHUNK, int EPI>
+__global__ __launch_bounds__(256, 2) void k_conv_chunks2(ConvArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t r0[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r1[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r2[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r3[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r4[kPlane];
+  __shared__ __attribute__((aligned(16))) uint16_t r5[kPlane];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const RingTile T = ring_tile(a, 2);
+  const int co0 = blockIdx.y * 32;
+  bf16x8 wf[14][2];
+  f32x4 acc[2][4][2];
+  zero_acc<2>(acc[0]);
+  zero_acc<2>(acc[1]);
+  RingSrc cur = ring_src(a, T.n, T.x0, T.y0, 0, wave, lane);
+  ring_issue(cur, T.zs - 1, a.D, wave, r0);
+  ring_issue(cur, T.zs, a.D, wave, r1);
+  ring_issue(cur, T.zs + 1, a.D, wave, r2);
+  const Weights w = ring_weights(a, co0, 0);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) pool[k >> 1][k & 1] = 0.f;
+  for (int p = 0; p < 14; ++p) load_pair<2>(w, p, wf[p]);
+  ring_wait<0>();
+#pragma unroll
+  for (int cb = 0; cb < NCHUNK; ++cb) {
+    const int nb = cb + 1 < NCHUNK ? cb + 1 : cb;
+    const RingSrc nx = ring_src(a, T.n, T.x0, T.y0, nb, wave, lane);
+    const Weights wn = ring_weights(a, co0, nb);
+    if (cb % 3 == 0) chunk_planes2(a, cur, nx, cb + 1 < NCHUNK, T.zs, r0, r1, r2, r3, r4, r5, wf, acc, wn);
+    else if (cb % 3 == 1) chunk_planes2(a, cur, nx, cb + 1 < NCHUNK, T.zs, r4, r5, r0, r1, r2, r3, wf, acc, wn);
+    else chunk_planes2(a, cur, nx, cb + 1 < NCHUNK, T.zs, r2, r3, r4, r5, r0, r1, wf, acc, wn);
+    cur = nx;
   }
+  f32x4 bias[2];
+  ring_bias<2>(a, co0, bias);
+  float pool[2][2][4];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int y = L.y0 + 4 * wave + m;
-    const int xs = L.x0 + 4 * g;
-    if (y < a.H) {
-      uint16_t* orow = outPlane + ((size_t)y * a.W + xs) * a.out_cs;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (xs + r >= a.W) continue;
-        float v = acc[m][r] + bias;
-        if (a.relu) v = fmaxf(v, 0.f);
-        const uint16_t b = f2bf_rne(v);
-        orow[r * a.out_cs] = b;
-        if (pooling) pool[m >> 1][r >> 1] += __uint_as_float((uint32_t)b << 16);
-      }
-    }
-  }
-  if (pooling && (z & 1)) {
-    // the plane pair is complete: output voxel (z / 2, y / 2, x / 2) of the pooled tensor (H, W even)
-    const int H2 = a.H / 2, W2 = a.W / 2;
-    uint16_t* pp = a.pool_out + (((size_t)n * (a.D / 2) + z / 2) * H2) * W2 * a.pool_cs + a.pool_co + i;
-#pragma unroll
-    for (int ky = 0; ky < 2; ++ky) {
-      const int y2 = (L.y0 + 4 * wave) / 2 + ky;
-#pragma unroll
-      for (int kx = 0; kx < 2; ++kx) {
-        const int x2 = (L.x0 + 4 * g) / 2 + kx;
-        if (y2 < H2 && x2 < W2) pp[((size_t)y2 * W2 + x2) * a.pool_cs] = f2bf_rne(pool[ky][kx] * 0.125f);
-      }
-    }
-  }
+  for (int o = 0; o < 2; ++o)
+    if (T.zs + o < a.D) ring_store<2, EPI>(a, T.n, T.zs + o, T.x0, T.y0, co0, acc[o], bias, f32x4{}, 0.f, 0.f, pool);
 }
 
-template <int TX>
-__global__ __launch_bounds__(256) void k_conv_tile_dma(ConvArgs a, int zp) {
-  using T = ConvTile<TX>;
-  __shared__ __attribute__((aligned(16))) uint16_t tileA[2 * T::HVP * 8];
-  __shared__ __attribute__((aligned(16))) uint16_t tileB[2 * T::HVP * 8];
-  __shared__ __attribute__((aligned(16))) uint16_t wl[28 * T::WC * 16];
-
-  const int i = threadIdx.x & 15;
-  // work-group -> (n, z group, y block, x block), XCD-remapped as in k_conv_tile
-  const int nbx = (a.W + TX - 1) / TX, nby = (a.H + T::TY - 1) / T::TY, nzg = (a.D + zp - 1) / zp;
-  const int nbt = (int)gridDim.x;
-  int b = nbt % 8 == 0 ? (int)(blockIdx.x % 8) * (nbt / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-  const int bx = b % nbx; b /= nbx;
-  const int by = b % nby; b /= nby;
-  const int zg = b % nzg, n = b / nzg;
-  const int zs = zg * zp, ze = min(a.D, zs + zp);
-
-  DmaLane<TX> L;
-  L.planeElems = (long long)a.H * a.W * a.in_cs;
-  L.nbase = a.in + (size_t)n * a.D * L.planeElems;
-  L.x0 = bx * TX;
-  L.y0 = by * T::TY;
-  L.okxy = 0;
-  {
-    // the lane's halo voxels v = threadIdx.x + 256 r, decomposed incrementally; offsets fit 32 bits (at most
-    // three planes, checked at launch)
-    constexpr int DX = 256 % T::HX, DY = (256 / T::HX) % T::HY, DZ = 256 / (T::HX * T::HY);
-    const int v0 = threadIdx.x;
-    int hx = v0 % T::HX, hy = (v0 / T::HX) % T::HY, hz = v0 / (T::HX * T::HY);
-#pragma unroll
-    for (int r = 0; r < T::NR; ++r) {
-      if (r) {
-        hx += DX;
-        const int cy = hx >= T::HX;
-        hx -= cy ? T::HX : 0;
-        hy += DY + cy;
-        const int cz = hy >= T::HY;
-        hy -= cz ? T::HY : 0;
-        hz += DZ + cz;
-      }
-      const int xx = L.x0 + hx - 1, yy = L.y0 + hy - 1;
-      const bool ok = v0 + 256 * r < T::HV && (unsigned)xx < (unsigned)a.W && (unsigned)yy < (unsigned)a.H;
-      L.okxy |= ok ? 1u << r : 0u;
-      L.off[r] = ok ? ((hz * a.H + yy) * a.W + xx) * a.in_cs : 0;
-      L.hz[r] = hz;
-    }
-  }
-
-  // weights [28 taps][16 cout][16 cin] as two halves, staged once through registers
-  {
-    constexpr int NW = (28 * T::WC * 2 + 255) / 256;
-    uint4 wbuf[NW];
-    const int half = threadIdx.x & 1;
-#pragma unroll
-    for (int k = 0; k < NW; ++k) {
-      const int e = threadIdx.x + 256 * k;
-      const int c = (e >> 1) % T::WC, tap = (e >> 1) / T::WC;
-      const bool ok = tap < 27;
-      wbuf[k] = *reinterpret_cast<const uint4*>(a.w + ((ok ? tap : 0) * a.cout + c) * a.cin + half * 8);
-      if (!ok) wbuf[k] = make_uint4(0u, 0u, 0u, 0u);
-    }
-#pragma unroll
-    for (int k = 0; k < NW; ++k) {
-      const int e = threadIdx.x + 256 * k;
-      if (e < 28 * T::WC * 2) *reinterpret_cast<uint4*>(wl + ((e & 1) * 28 * T::WC + (e >> 1)) * 8) = wbuf[k];
-    }
-  }
-  const float bias = a.bias ? a.bias[i] : 0.f;
-  unsigned bad = conv_dma_issue<TX>(a, L, zs, tileA);
-  __builtin_amdgcn_s_waitcnt(0);
-  conv_dma_fix<TX>(bad, tileA);
-  __syncthreads();
-  // Planes alternate between the buffers.  A step: the next plane's DMA, this plane's MFMAs, the wait for this
-  // lane's DMA (and for the stores of the plane before, issued a step ago), the zeros, a barrier (the next plane is
-  // in LDS for every wave, every wave is done with the buffer the step after refills), and only then this plane's
-  // stores, which drain during the next step.
-  f32x4 acc[4];
-  float pool[2][2];
-  for (int z = zs; z < ze; ++z) {
-    const bool more = z + 1 < ze;
-    const bool odd = (z - zs) & 1;
-    uint16_t* cur = odd ? tileB : tileA;
-    uint16_t* nxt = odd ? tileA : tileB;
-    bad = conv_dma_mfma<TX>(a, L, z, more, acc, cur, nxt, wl);
-    if (more) {
-      __builtin_amdgcn_s_waitcnt(0);
-      conv_dma_fix<TX>(bad, nxt);
-      __syncthreads();
-    }
-    conv_dma_store<TX>(a, L, n, z, acc, bias, pool);
-  }
-}
-
-template <int TX, int NG>
-void launch_tile(const ConvArgs& a, hipStream_t s) {
-  constexpr int TY = 256 / TX;
-  const long long tiles = (long long)((a.W + TX - 1) / TX) * ((a.H + TY - 1) / TY) * a.D * a.N;
-  const int zp = tiles >= kConvZPTiles ? kConvZP : 1;
-  const unsigned nb = (unsigned)((a.W + TX - 1) / TX) * (unsigned)((a.H + TY - 1) / TY) *
-                      (unsigned)((a.D + zp - 1) / zp) * a.N;
-  hipLaunchKernelGGL((k_conv_tile<TX, NG>), dim3(nb, a.cout / (16 * NG)), dim3(256), 0, s, a, zp);
-}
-
-// the 16 -> 16 single-chunk layers of large launches take the DMA kernel (a pooled output needs even dimensions
-// and the work-groups' even-aligned plane pairs, which kConvZPDma gives)
-template <int TX>
-bool takes_dma(const ConvArgs& a) {
-  constexpr int TY = 256 / TX;
-  const long long tiles = (long long)((a.W + TX - 1) / TX) * ((a.H + TY - 1) / TY) * a.D * a.N;
-  return a.cin == 16 && a.cout == 16 && a.up_c == 0 && tiles >= kConvZPTiles &&
-         (!a.pool_out || !((a.D | a.H | a.W) & 1));
-}
-static_assert(kConvZPDma % 2 == 0, "plane pairs of the fused pooling stay in one work-group");
-
-template <int TX>
-void launch_tx(const ConvArgs& a, hipStream_t s) {
-  constexpr int TY = 256 / TX;
-  if (takes_dma<TX>(a)) {
-    const unsigned nb = (unsigned)((a.W + TX - 1) / TX) * (unsigned)((a.H + TY - 1) / TY) *
-                        (unsigned)((a.D + kConvZPDma - 1) / kConvZPDma) * a.N;
-    hipLaunchKernelGGL((k_conv_tile_dma<TX>), dim3(nb), dim3(256), 0, s, a, kConvZPDma);
+template <int NG>
+void launch_ng(const ConvArgs& a, hipStream_t s) {
+  const long long tiles = (long long)((a.W + TX - 1) / TX) * ((a.H + TY - 1) / TY) * a.N;
+  const int groups = a.cout / (16 * NG);
+  auto columns = [&](int zp) { return (unsigned)(tiles * ((a.D + zp - 1) / zp)); };
+  if (a.cin == 16) {
+    // planes per work-group: the longest columns (the first three planes of a column are not overlapped) that still
+    // give every CU its three (NG = 1) or two work-groups a few times over; even, for the pooling's plane pairs
+    int zp = 16;
+    while (zp > 2 && (long long)columns(zp) * groups < 1024) zp /= 2;
+    const dim3 grid(columns(zp), groups);
+    if (a.psi.out)
+      hipLaunchKernelGGL((k_conv_column<1, kHead>), grid, dim3(256), 0, s, a, zp);
+    else if (a.pool_out)
+      hipLaunchKernelGGL((k_conv_column<NG, kPool>), grid, dim3(256), 0, s, a, zp);
+    else
+      hipLaunchKernelGGL((k_conv_column<NG, kPlain>), grid, dim3(256), 0, s, a, zp);
     return;
   }
-  if ((a.cout / 16) % 2 == 0)
-    launch_tile<TX, 2>(a, s);
-  else
-    launch_tile<TX, 1>(a, s);
+  if constexpr (NG == 1) {
+    const dim3 grid(columns(4), groups);
+    if (a.cin == 32)
+      hipLaunchKernelGGL((k_conv_chunks4<2>), grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_conv_chunks4<3>), grid, dim3(256), 0, s, a);
+  } else {
+    const dim3 grid(columns(2), groups);
+    if (a.pool_out)
+      hipLaunchKernelGGL((k_conv_chunks2<2, kPool>), grid, dim3(256), 0, s, a);
+    else if (a.cin == 32)
+      hipLaunchKernelGGL((k_conv_chunks2<2, kPlain>), grid, dim3(256), 0, s, a);
+    else if (a.cin == 64)
+      hipLaunchKernelGGL((k_conv_chunks2<4, kPlain>), grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_conv_chunks2<6, kPlain>), grid, dim3(256), 0, s, a);
+  }
 }
 
 }  // namespace
 
+// pooling is fused into the one-chunk layers and the 32-channel inputs of even output groups
 bool conv_fuses_pool(const ConvArgs& a) {
-  return a.pool_out && a.taps == 27 && a.in_cs % 16 == 0 && takes_dma<16>(a) &&
-         3ll * a.H * a.W * a.in_cs < (1ll << 31);
+  return a.pool_out && !((a.D | a.H | a.W) & 1) && (a.cin == 16 || (a.cin == 32 && a.cout % 32 == 0));
 }
 
-// 3^3 convolutions with cin and cout multiples of 16
+// The network's 3^3 convolutions: cout a multiple of 16; cin 16, or 32 and 48 for an odd number of 16-channel output
+// blocks, 32, 64 and 96 for an even one
 bool launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
-  if (a.taps != 27 || a.cin % 16 != 0 || a.cout % 16 != 0 || a.in_cs % 16 != 0) return false;
-  // the staging's offsets from its first halo plane cover three planes in 32 bits
-  if (3ll * a.H * a.W * std::max(a.in_cs, a.up_cs) >= (1ll << 31)) return false;
+  const bool pairs = a.cout % 32 == 0;
+  const bool known = a.cin == 16 || a.cin == 32 || (pairs ? a.cin == 64 || a.cin == 96 : a.cin == 48);
+  if (a.taps != 27 || !known || a.cout % 16 != 0 || a.in_cs % (a.in_half ? 8 : 16) != 0) return false;
+  // 32-bit offsets within a plane (and the limit callers are told: three planes)
+  if (3ll * a.H * a.W * std::max(a.in_half ? 16 : a.in_cs, a.up_cs) >= (1ll << 31)) return false;
   if (a.up_c && (a.up_c % 16 != 0 || a.up_cs % 16 != 0 || !a.up_in || (a.W | a.H | a.D) & 1)) return false;
-  // 16 x 16 voxel tiles: the smallest halo per output voxel (3 x 18 x 18 staged per 256 outputs; 64 x 4 and
-  // 32 x 8 tiles stage 1188 and 1020 halo voxels for the same outputs and measured 2.4 % / 0.5 % slower at 256^3)
-  launch_tx<16>(a, s);
+  if (a.in_half && a.cin != 16) return false;
+  if (a.pool_out && !conv_fuses_pool(a)) return false;
+  if (a.psi.out && (a.cin != 16 || a.cout != 16 || a.N != 1)) return false;
+  if (pairs)
+    launch_ng<2>(a, s);
+  else
+    launch_ng<1>(a, s);
   return true;
 }
 

@@ -39,7 +39,8 @@ struct UNet {
              *g_p2 = nullptr, *g_a3 = nullptr, *g_b3 = nullptr, *g_a4 = nullptr, *g_d2 = nullptr,
              *g_a5 = nullptr, *g_d1 = nullptr;
     float *avg = nullptr, *target = nullptr, *dr = nullptr;
-    int alloc(int N, int D, int H, int W, bool grads);
+    int cs1 = 0, cs2 = 0, csIn = 0;  // channels of cat1, cat2 and x0 as stored
+    int alloc(int N, int D, int H, int W, int views, bool grads);
     void release();
   };
   struct TrainVolume {
@@ -82,9 +83,10 @@ struct UNet {
   // rest come from in + in_co
   // pool != nullptr: the 2x2x2 average pooling of the output into pool (channel stride pool_cs) where the
   // convolution fuses it; returns whether it did (else the caller pools)
+  // psi != nullptr: the output head of an inference instead of out
   bool conv(int l, const uint16_t* in, int in_cs, int in_co, uint16_t* out, int out_cs, int out_co, int N, int D,
             int H, int W, bool relu, const uint16_t* up = nullptr, int up_cs = 0, int up_c = 0,
-            uint16_t* pool = nullptr, int pool_cs = 0);
+            uint16_t* pool = nullptr, int pool_cs = 0, const PsiArgs* psi = nullptr);
   void dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t* din, int din_cs, int din_co, int N,
              int D, int H, int W);
   void wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int dout_cs, int dout_co, int N, int D, int H,
