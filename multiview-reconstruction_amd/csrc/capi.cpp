@@ -467,6 +467,39 @@ struct DevBuf {
   ~DevBuf() { if (p) (void)hipFree(p); }
 };
 
+// One array of a preparation call.  Device memory of the call's GPU is used where it is (the kernels read and write
+// 4-byte values); anything else, and every array of a call whose arrays overlap, goes through a buffer of the call's.
+struct PrepArray {
+  const void* user = nullptr;
+  size_t bytes = 0;
+  bool direct = false;
+  DevBuf own;
+  void set(const void* p, size_t n) { user = p; bytes = n; }
+  float* dev() const { return static_cast<float*>(direct ? const_cast<void*>(user) : own.p); }
+  int open(bool copyIn) {
+    if (direct) return 0;
+    MVR_HIP(hipMalloc(&own.p, bytes));
+    if (copyIn) MVR_HIP(hipMemcpy(own.p, user, bytes, hipMemcpyDefault));
+    return 0;
+  }
+  int close() {  // an output: back to the caller
+    if (!direct) MVR_HIP(hipMemcpy(const_cast<void*>(user), own.p, bytes, hipMemcpyDefault));
+    return 0;
+  }
+};
+
+// decides which arrays are used directly; `written` of them (the last ones) are outputs, which must not overlap any other
+void decide_direct(PrepArray* const* a, int n, int written, int dev) {
+  bool overlap = false;
+  for (int i = n - written; i < n; ++i)
+    for (int j = 0; j < n; ++j) {
+      const char *p = static_cast<const char*>(a[i]->user), *q = static_cast<const char*>(a[j]->user);
+      overlap = overlap || (i != j && p < q + a[j]->bytes && q < p + a[i]->bytes);
+    }
+  for (int i = 0; i < n; ++i)
+    a[i]->direct = !overlap && !(reinterpret_cast<uintptr_t>(a[i]->user) & 3) && device_memory_of(a[i]->user, dev, false);
+}
+
 }  // namespace
 
 int mvr_transform_view(int dev, const float* img, const int imgXYZ[3], const double affine[12], const long long bbMin[3],
@@ -485,16 +518,19 @@ int mvr_transform_view(int dev, const float* img, const int imgXYZ[3], const dou
   if (invert_affine(affine, inv)) return -1;
   MVR_HIP(hipSetDevice(dev));
   const size_t ni = (size_t)imgXYZ[0] * imgXYZ[1] * imgXYZ[2], no = (size_t)bbXYZ[0] * bbXYZ[1] * bbXYZ[2];
-  DevBuf di, dout;
-  MVR_HIP(hipMalloc(&di.p, ni * 4));
-  MVR_HIP(hipMalloc(&dout.p, no * 4));
-  MVR_HIP(hipMemcpy(di.p, img, ni * 4, hipMemcpyDefault));
-  if (launch_transform_view((const float*)di.p, imgXYZ, inv, bbMin, bbXYZ, hasMinValue, minValue, outsideValue,
-                            interpolation, (float*)dout.p, nullptr)) {
+  PrepArray in, res;
+  in.set(img, ni * 4);
+  res.set(out, no * 4);
+  PrepArray* all[] = {&in, &res};
+  decide_direct(all, 2, 1, dev);
+  if (in.open(true) || res.open(false)) return -1;
+  if (launch_transform_view(in.dev(), imgXYZ, inv, bbMin, bbXYZ, hasMinValue, minValue, outsideValue, interpolation,
+                            res.dev(), nullptr)) {
     set_error("transform kernel launch failed");
     return -1;
   }
-  MVR_HIP(hipMemcpy(out, dout.p, no * 4, hipMemcpyDefault));
+  if (res.close()) return -1;
+  MVR_HIP(hipStreamSynchronize(nullptr));
   return 0;
 }
 
@@ -514,13 +550,17 @@ int mvr_transform_blending(int dev, const int imgXYZ[3], const float border[3], 
   MVR_HIP(hipSetDevice(dev));
   if (ensure_blend_lut(dev)) return -1;
   const size_t no = (size_t)bbXYZ[0] * bbXYZ[1] * bbXYZ[2];
-  DevBuf dout;
-  MVR_HIP(hipMalloc(&dout.p, no * 4));
-  if (launch_transform_blending(imgXYZ, border, blending, inv, bbMin, bbXYZ, (float*)dout.p, nullptr)) {
+  PrepArray res;
+  res.set(out, no * 4);
+  PrepArray* all[] = {&res};
+  decide_direct(all, 1, 1, dev);
+  if (res.open(false)) return -1;
+  if (launch_transform_blending(imgXYZ, border, blending, inv, bbMin, bbXYZ, res.dev(), nullptr)) {
     set_error("blending kernel launch failed");
     return -1;
   }
-  MVR_HIP(hipMemcpy(out, dout.p, no * 4, hipMemcpyDefault));
+  if (res.close()) return -1;
+  MVR_HIP(hipStreamSynchronize(nullptr));
   return 0;
 }
 
@@ -557,28 +597,34 @@ int mvr_fuse_group(int dev, int numViews, const float* const* imgs, const int* i
       v.dBorder[d] = deconBlending ? deconBlending[6 * j + d] : 0.f;
       v.dRange[d] = deconBlending ? deconBlending[6 * j + 3 + d] : 0.f;
     }
+    v.sameBlend = v.fusionBlend && v.deconBlend && !std::memcmp(v.fBorder, v.dBorder, sizeof(v.fBorder)) &&
+                  !std::memcmp(v.fRange, v.dRange, sizeof(v.fRange));
   }
   MVR_HIP(hipSetDevice(dev));
   if (ensure_blend_lut(dev)) return -1;
-  std::vector<DevBuf> dimg(numViews);
-  for (int j = 0; j < numViews; ++j) {
-    const size_t ni = (size_t)fv[j].in[0] * fv[j].in[1] * fv[j].in[2];
-    MVR_HIP(hipMalloc(&dimg[j].p, ni * 4));
-    MVR_HIP(hipMemcpy(dimg[j].p, imgs[j], ni * 4, hipMemcpyDefault));
-    fv[j].img = (const float*)dimg[j].p;
-  }
   const size_t no = (size_t)bbXYZ[0] * bbXYZ[1] * bbXYZ[2];
-  DevBuf dviews, dout, dw;
-  MVR_HIP(hipMalloc(&dviews.p, sizeof(FuseView) * numViews));
-  MVR_HIP(hipMemcpy(dviews.p, fv.data(), sizeof(FuseView) * numViews, hipMemcpyHostToDevice));
-  MVR_HIP(hipMalloc(&dout.p, no * 4));
-  MVR_HIP(hipMalloc(&dw.p, no * 4));
-  if (launch_fuse_group((const FuseView*)dviews.p, numViews, bbMin, bbXYZ, (float*)dout.p, (float*)dw.p, nullptr)) {
+  std::vector<PrepArray> arrays(numViews + 2);
+  std::vector<PrepArray*> all;
+  for (int j = 0; j < numViews; ++j) arrays[j].set(imgs[j], (size_t)fv[j].in[0] * fv[j].in[1] * fv[j].in[2] * 4);
+  arrays[numViews].set(imgOut, no * 4);
+  arrays[numViews + 1].set(weightOut, no * 4);
+  for (auto& x : arrays) all.push_back(&x);
+  decide_direct(all.data(), numViews + 2, 2, dev);
+  for (int j = 0; j < numViews + 2; ++j)
+    if (arrays[j].open(j < numViews)) return -1;
+  for (int j = 0; j < numViews; ++j) fv[j].img = arrays[j].dev();
+  DevBuf dviews;
+  if (numViews > kFuseArgViews) {
+    MVR_HIP(hipMalloc(&dviews.p, sizeof(FuseView) * numViews));
+    MVR_HIP(hipMemcpy(dviews.p, fv.data(), sizeof(FuseView) * numViews, hipMemcpyHostToDevice));
+  }
+  if (launch_fuse_group(fv.data(), (const FuseView*)dviews.p, numViews, bbMin, bbXYZ, arrays[numViews].dev(),
+                        arrays[numViews + 1].dev(), nullptr)) {
     set_error("group fusion kernel launch failed");
     return -1;
   }
-  MVR_HIP(hipMemcpy(imgOut, dout.p, no * 4, hipMemcpyDefault));
-  MVR_HIP(hipMemcpy(weightOut, dw.p, no * 4, hipMemcpyDefault));
+  if (arrays[numViews].close() || arrays[numViews + 1].close()) return -1;
+  MVR_HIP(hipStreamSynchronize(nullptr));
   return 0;
 }
 
@@ -654,19 +700,26 @@ int mvr_normalize_weights(int dev, float* const* weights, int numViews, const in
     if (!weights[v]) { set_error("null weight array"); return -1; }
   MVR_HIP(hipSetDevice(dev));
   const size_t n = (size_t)nXYZ[0] * nXYZ[1] * nXYZ[2];
-  std::vector<DevBuf> bufs(numViews);
+  std::vector<PrepArray> arrays(numViews);
+  std::vector<PrepArray*> all;
+  for (int v = 0; v < numViews; ++v) {
+    arrays[v].set(weights[v], n * 4);
+    all.push_back(&arrays[v]);
+  }
+  decide_direct(all.data(), numViews, numViews, dev);
   std::vector<float*> dp(numViews);
   for (int v = 0; v < numViews; ++v) {
-    MVR_HIP(hipMalloc(&bufs[v].p, n * 4));
-    MVR_HIP(hipMemcpy(bufs[v].p, weights[v], n * 4, hipMemcpyDefault));
-    dp[v] = (float*)bufs[v].p;
+    if (arrays[v].open(true)) return -1;
+    dp[v] = arrays[v].dev();
   }
   if (launch_normalize_weights(dp.data(), numViews, n, osemSpeedup, additionalSmoothBlending, maxDiffRange,
                                scalingRange, nullptr)) {
     set_error("normalisation kernel launch failed");
     return -1;
   }
-  for (int v = 0; v < numViews; ++v) MVR_HIP(hipMemcpy(weights[v], dp[v], n * 4, hipMemcpyDefault));
+  for (int v = 0; v < numViews; ++v)
+    if (arrays[v].close()) return -1;
+  MVR_HIP(hipStreamSynchronize(nullptr));
   return 0;
 }
 

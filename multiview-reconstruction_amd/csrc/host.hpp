@@ -11,6 +11,9 @@ namespace mvr {
 void set_error(const std::string& msg);
 const char* last_error();
 
+// device memory of `dev`, or managed memory if that is wanted
+bool device_memory_of(const void* p, int dev, bool managed);
+
 #define MVR_HIP(call)                                                                                 \
   do {                                                                                                \
     hipError_t e_ = (call);                                                                           \

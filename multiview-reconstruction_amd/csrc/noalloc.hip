@@ -53,16 +53,6 @@ void launch_twiddles(float2* out, int n, int period, hipStream_t s) {
   hipLaunchKernelGGL(k_twiddles, dim3((n + 255) / 256), dim3(256), 0, s, out, n, period);
 }
 
-// device memory of `dev` (device or managed); host memory would fault the kernels
-bool on_device(const void* p, int dev) {
-  hipPointerAttribute_t a{};
-  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();  // an unknown (pageable host) pointer: clear the error it leaves
-    return false;
-  }
-  return (a.type == hipMemoryTypeDevice && a.device == dev) || a.type == hipMemoryTypeManaged || a.isManaged;
-}
-
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 }  // namespace
@@ -89,7 +79,7 @@ extern "C" int mvr_fft_convolve_noalloc(int dev, const float* img, const int n[3
     return -1;
   }
   MVR_HIP(hipSetDevice(dev));
-  if (!on_device(img, dev) || !on_device(kernel, dev) || !on_device(out, dev)) {
+  if (!device_memory_of(img, dev, true) || !device_memory_of(kernel, dev, true) || !device_memory_of(out, dev, true)) {
     set_error("mvr_fft_convolve_noalloc: img, kernel and out must be device memory of the given device");
     return -1;
   }

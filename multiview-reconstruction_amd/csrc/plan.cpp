@@ -11,6 +11,16 @@ static thread_local std::string g_err;
 void set_error(const std::string& msg) { g_err = msg; }
 const char* last_error() { return g_err.c_str(); }
 
+bool device_memory_of(const void* p, int dev, bool managed) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();  // an unknown (pageable host) pointer: clear the error it leaves
+    return false;
+  }
+  if (a.type == hipMemoryTypeManaged || a.isManaged) return managed;
+  return a.type == hipMemoryTypeDevice && a.device == dev;
+}
+
 static int pick_length(int need, bool half) {
   for (const int* p = strided_lengths(); *p; ++p) {
     if (*p < need) continue;

@@ -72,25 +72,28 @@ __global__ void k_transform_view(const float* __restrict__ img, int3 in, Affine3
 
 __constant__ double c_blendLut[1001];
 
-// BlendingRealRandomAccess.computeWeight at the (float) input location l, interval [0, dm]
+// BlendingRealRandomAccess.computeWeight at the (float) input location l, interval [0, dm].  Most voxels of a frame lie
+// a full range inside the view, where the weight is 1 without a division or table look-up: dist >= range decides that
+// exactly as the rounded quotient dist / range >= 1 does (a float quotient of a smaller dist by range is at most
+// 1 - 2^-24, a float).
 __device__ __forceinline__ float blend_weight(const float l[3], const int dm[3], const float bo[3],
                                               const float bl[3]) {
   float dist[3];
-  float w = 1.f;
-  bool zero = false;
+  bool zero = false, full = true;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     dist[d] = fminf(__fsub_rn(l[d], bo[d]), __fsub_rn(__fsub_rn((float)dm[d], l[d]), bo[d]));
     zero |= dist[d] <= 0.f;
+    full &= dist[d] >= bl[d];
   }
-  if (!zero) {
+  if (zero) return 0.f;
+  float w = 1.f;
+  if (!full) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       const float rel = __fdiv_rn(dist[d], bl[d]);
       if (rel < 1.f) w = (float)((double)w * c_blendLut[(int)((double)rel * 1000.0 + 0.5)]);
     }
-  } else {
-    w = 0.f;
   }
   return w;
 }
@@ -113,25 +116,36 @@ __global__ void k_transform_blending(int3 dimMinus1, float3 border, float3 blend
 // adjustment; img = FusedRandomAccess AVG (fusion/transformed/FusedRandomAccess.java:67-88: views whose fusion
 // weight is 0 are skipped, sum I w / sum w in double, 0 when no weight) and weight = CombineWeightsSum
 // (weightcombination/CombineWeightsSumRandomAccess.java:40-50: (float) of the double sum of decon weights)
-__global__ void k_fuse_group(const FuseView* __restrict__ views, int V, long3 off, int3 outDim,
+// Bound by its FP64 instructions.  Views in the kernel arguments (up to kFuseArgViews: no upload before the launch), the
+// blending computed once where both weights share it and skipped inside the ranges: 2 views into 220 x 200 x 180,
+// @@FUSE@@.
+struct FuseArgs { FuseView v[kFuseArgViews]; };
+template <bool ARGS>
+__global__ void k_fuse_group(FuseArgs args, const FuseView* __restrict__ views, int V, long3 off, int3 outDim,
                              float* __restrict__ img, float* __restrict__ weight) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
   if (x >= outDim.x) return;
   const double sx = (double)(x + off.x), sy = (double)(y + off.y), sz = (double)(z + off.z);
   double sumI = 0.0, sumW = 0.0, sumD = 0.0;
-  for (int j = 0; j < V; ++j) {
-    const FuseView& v = views[j];
+  auto add = [&](const FuseView& v) {
     double tx, ty, tz;
     apply_inv(v.inv, sx, sy, sz, tx, ty, tz);
     const float l[3] = {(float)tx, (float)ty, (float)tz};
     const int dm[3] = {v.in[0] - 1, v.in[1] - 1, v.in[2] - 1};
-    sumD += v.deconBlend ? (double)blend_weight(l, dm, v.dBorder, v.dRange) : 1.0;
     const float wf = v.fusionBlend ? blend_weight(l, dm, v.fBorder, v.fRange) : 1.f;
-    if (wf == 0.f) continue;
+    sumD += v.sameBlend ? (double)wf : v.deconBlend ? (double)blend_weight(l, dm, v.dBorder, v.dRange) : 1.0;
+    if (wf == 0.f) return;
     const float iv = sample_view(v.img, v.in[0], v.in[1], v.in[2], tx, ty, tz, 1, 1.0f, 0.0f, 1, v.adjust != 0,
                                  v.adjA, v.adjB);
     sumI += (double)iv * (double)wf;
     sumW += (double)wf;
+  };
+  if constexpr (ARGS) {
+#pragma unroll
+    for (int j = 0; j < kFuseArgViews; ++j)
+      if (j < V) add(args.v[j]);
+  } else {
+    for (int j = 0; j < V; ++j) add(views[j]);
   }
   const size_t o = ((size_t)z * outDim.y + y) * outDim.x + x;
   img[o] = sumW > 0.0 ? (float)(sumI / sumW) : 0.f;
@@ -224,11 +238,18 @@ int launch_transform_blending(const int inXYZ[3], const float border[3], const f
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_fuse_group(const FuseView* views, int V, const long long off[3], const int outXYZ[3], float* img,
-                      float* weight, hipStream_t s) {
+int launch_fuse_group(const FuseView* host, const FuseView* views, int V, const long long off[3], const int outXYZ[3],
+                      float* img, float* weight, hipStream_t s) {
   const dim3 grid((outXYZ[0] + 255) / 256, outXYZ[1], outXYZ[2]);
-  hipLaunchKernelGGL(k_fuse_group, grid, dim3(256), 0, s, views, V, make_long3(off[0], off[1], off[2]),
-                     make_int3(outXYZ[0], outXYZ[1], outXYZ[2]), img, weight);
+  const long3 o = make_long3(off[0], off[1], off[2]);
+  const int3 n = make_int3(outXYZ[0], outXYZ[1], outXYZ[2]);
+  FuseArgs args{};
+  if (V <= kFuseArgViews) {
+    for (int j = 0; j < V; ++j) args.v[j] = host[j];
+    hipLaunchKernelGGL(k_fuse_group<true>, grid, dim3(256), 0, s, args, views, V, o, n, img, weight);
+  } else {
+    hipLaunchKernelGGL(k_fuse_group<false>, grid, dim3(256), 0, s, args, views, V, o, n, img, weight);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

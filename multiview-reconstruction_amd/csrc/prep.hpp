@@ -29,13 +29,16 @@ struct FuseView {
   double adjA, adjB;         // intensity v -> (float)(v * adjA + adjB) when adjust != 0
   int adjust;
   int fusionBlend, deconBlend;  // 0: constant weight 1
+  int sameBlend;                // both, with the same borders and ranges
   float fBorder[3], fRange[3], dBorder[3], dRange[3];
 };
 
 // ProcessInputImages.fuseGroups for one group: per output voxel, AVG fusion of the resampled views weighted
-// by their fusion blending, and the sum of their deconvolution blending weights (views: device array)
-int launch_fuse_group(const FuseView* views, int V, const long long off[3], const int outXYZ[3], float* img,
-                      float* weight, hipStream_t s);
+// by their fusion blending, and the sum of their deconvolution blending weights.  host: the views; more than
+// kFuseArgViews of them also as a device array (views)
+constexpr int kFuseArgViews = 4;
+int launch_fuse_group(const FuseView* host, const FuseView* views, int V, const long long off[3], const int outXYZ[3],
+                      float* img, float* weight, hipStream_t s);
 int launch_normalize_weights(float* const* w, int V, size_t n, double osem, int smooth, float maxDiffRange,
                              float scalingRange, hipStream_t s);
 
