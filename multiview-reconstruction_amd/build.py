@@ -33,10 +33,13 @@ ARCH = "gfx950"
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-Wall", "-Wno-unused-function", "-Wno-unused-result"]
 
-X_FUNCS = """template void launch_x_fwd<{M}>(const Dom&, const GatherParams&, float2*, const float2*, const float2*, hipStream_t);
-template void launch_x_ratio<{M}>(const Dom&, const RatioParams&, const float2*, float2*, const float2*, const float2*, hipStream_t);
-template int launch_x_update<{M}>(const Dom&, const UpdateParams&, const float2*, const float2*, const float2*, hipStream_t);
-template void launch_x_store<{M}>(const Dom&, const StoreParams&, const float2*, const float2*, const float2*, hipStream_t);
+# x passes with planar spectra (engine.hpp: kPlanarMaxM)
+PLANAR_MAX_M = 128
+
+X_FUNCS = """template void launch_x_fwd<{M}, {T}>(const Dom&, const GatherParams&, float2*, const float2*, const float2*, hipStream_t);
+template void launch_x_ratio<{M}, {T}>(const Dom&, const RatioParams&, const float2*, float2*, const float2*, const float2*, hipStream_t);
+template int launch_x_update<{M}, {T}>(const Dom&, const UpdateParams&, const float2*, const float2*, const float2*, hipStream_t);
+template void launch_x_store<{M}, {T}>(const Dom&, const StoreParams&, const float2*, const float2*, const float2*, hipStream_t);
 """
 S_FUNCS = """template void launch_strided<{L}>(const StridedGeom&, int, const float2*, float2*, const float2*, float, const float2*, hipStream_t);
 template int strided_span<{L}>();
@@ -52,23 +55,26 @@ def generate():
     os.makedirs(GEN, exist_ok=True)
     files = []
     for gi, grp in enumerate(_groups(HALF, 10)):
-        body = "".join(X_FUNCS.format(M=m) for m in grp)
+        body = "".join(X_FUNCS.format(M=m, T=t) for m in grp for t in ("false", "true")
+                       if t == "false" or m <= PLANAR_MAX_M)
         files.append((f"x_{gi}.hip", f'#include "xpasses.hpp"\nnamespace mvr {{\n{body}}}\n'))
     for gi, grp in enumerate(_groups(STRIDED, 10)):
         body = "".join(S_FUNCS.format(L=l) for l in grp)
         files.append((f"s_{gi}.hip", f'#include "passes.hpp"\nnamespace mvr {{\n{body}}}\n'))
     # dispatch table (host only: declarations of the explicit instantiations)
     d = ['#include "engine.hpp"', "namespace mvr {",
-         "template <int M> void launch_x_fwd(const Dom&, const GatherParams&, float2*, const float2*, const float2*, hipStream_t);",
-         "template <int M> void launch_x_ratio(const Dom&, const RatioParams&, const float2*, float2*, const float2*, const float2*, hipStream_t);",
-         "template <int M> int launch_x_update(const Dom&, const UpdateParams&, const float2*, const float2*, const float2*, hipStream_t);",
-         "template <int M> void launch_x_store(const Dom&, const StoreParams&, const float2*, const float2*, const float2*, hipStream_t);",
+         "template <int M, bool TR> void launch_x_fwd(const Dom&, const GatherParams&, float2*, const float2*, const float2*, hipStream_t);",
+         "template <int M, bool TR> void launch_x_ratio(const Dom&, const RatioParams&, const float2*, float2*, const float2*, const float2*, hipStream_t);",
+         "template <int M, bool TR> int launch_x_update(const Dom&, const UpdateParams&, const float2*, const float2*, const float2*, hipStream_t);",
+         "template <int M, bool TR> void launch_x_store(const Dom&, const StoreParams&, const float2*, const float2*, const float2*, hipStream_t);",
          "template <int L> void launch_strided(const StridedGeom&, int, const float2*, float2*, const float2*, float, const float2*, hipStream_t);",
          "template <int L> int strided_span();"]
     for name, fn, typ in [("get_x_fwd", "launch_x_fwd", "XFwdFn"), ("get_x_ratio", "launch_x_ratio", "XRatioFn"),
                           ("get_x_update", "launch_x_update", "XUpdateFn"), ("get_x_store", "launch_x_store", "XStoreFn")]:
-        cases = " ".join(f"case {m}: return &{fn}<{m}>;" for m in HALF)
-        d.append(f"{typ} {name}(int M) {{ switch (M) {{ {cases} default: return nullptr; }} }}")
+        rows = " ".join(f"case {m}: return &{fn}<{m}, false>;" for m in HALF)
+        planar = " ".join(f"case {m}: return &{fn}<{m}, true>;" for m in HALF if m <= PLANAR_MAX_M)
+        d.append(f"{typ} {name}(int M, bool planar) {{ if (planar) switch (M) {{ {planar} default: return nullptr; }} "
+                 f"switch (M) {{ {rows} default: return nullptr; }} }}")
     cases = " ".join(f"case {l}: return &launch_strided<{l}>;" for l in STRIDED)
     d.append(f"StridedFn get_strided(int L) {{ switch (L) {{ {cases} default: return nullptr; }} }}")
     cases = " ".join(f"case {l}: return strided_span<{l}>();" for l in STRIDED)

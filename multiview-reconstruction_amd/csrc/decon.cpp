@@ -114,7 +114,9 @@ int Decon::set_block_size(const int B[3]) {
 
 void Decon::free_blocks() {
   for (auto p : btab) if (p) (void)hipFree(p);
+  for (auto p : qtab) if (p) (void)hipFree(p);
   btab.clear();
+  qtab.clear();
   nbView.clear();
   nbAll = 0;
 }
@@ -144,6 +146,7 @@ int Decon::build_blocks() {
   MVR_HIP(hipMalloc(&dFlags, sizeof(int) * nbAll));
   MVR_HIP(hipMemcpyAsync(dInt, interval.data(), interval.size() * sizeof(int), hipMemcpyHostToDevice, stream));
   btab.assign(V, nullptr);
+  qtab.assign(V, nullptr);
   nbView.assign(V, 0);
   std::vector<int> flags(nbAll);
   int rc = 0;
@@ -164,6 +167,20 @@ int Decon::build_blocks() {
     if (nbView[v] == 0) continue;
     if (hipMalloc(&btab[v], tab.size() * sizeof(int)) != hipSuccess ||
         hipMemcpy(btab[v], tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
+      set_error("block table upload failed");
+      rc = -1;
+    }
+    if (!plan.planar || rc) continue;
+    // the blocks' quotient rows: their output regions widened by the second kernel's reach, inside the volume
+    std::vector<int> rows;
+    for (int b = 0; b < nbView[v]; ++b)
+      for (int k = 1; k < 3; ++k) {
+        const int o = tab[kBlockTabInts * b + k], D = tab[kBlockTabInts * b + 3 + k];
+        rows.push_back(plan.dom.m[k] + std::max(-(K[k] - 1 - K[k] / 2), -o));
+        rows.push_back(plan.dom.m[k] + std::min(D + K[k] / 2, N[k] - o));
+      }
+    if (hipMalloc(&qtab[v], rows.size() * sizeof(int)) != hipSuccess ||
+        hipMemcpy(qtab[v], rows.data(), rows.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
       set_error("block table upload failed");
       rc = -1;
     }
@@ -531,16 +548,10 @@ int Decon::reset_psi() {
   return 0;
 }
 
-// geometry of a strided launch whose kernel execution is timed under category c (untimed when c is off)
-static StridedGeom timed(Timer& t, StridedGeom g, int c) {
-  t.kernel(c, &g.evStart, &g.evStop);
-  return g;
-}
-
 // One view of one Seq iteration over the whole psi volume.
 int Decon::view_seq(int v, double2* statOut, int slot) {
   Dom d = plan.dom;
-  StridedGeom gy = plan.geom_y(), gz = plan.geom_z();
+  Plan::Mid m1 = plan.mid();
   double2* part = slot >= 0 ? partial + (size_t)slot * partials_needed() : partial;
   if (blocked()) {
     // every block of this view in one launch per pass
@@ -556,12 +567,9 @@ int Decon::view_seq(int v, double2* statOut, int slot) {
     d.btab = btab[v];
     d.nb = nbView[v];
     d.blockStride = plan.ncpx();
-    for (StridedGeom* gm : {&gy, &gz}) {
-      gm->blockPlanes = gm->nplanes;
-      gm->nplanes *= d.nb;
-      gm->blockStride = plan.ncpx();
-    }
+    plan.set_blocks(m1, d.nb, plan.ncpx());
   }
+  Plan::Mid m2 = m1;
   GatherParams g{};
   g.src = psi;
   for (int k = 0; k < 3; ++k) { g.N[k] = N[k]; g.org[k] = -d.m[k]; }
@@ -579,25 +587,24 @@ int Decon::view_seq(int v, double2* statOut, int slot) {
   // the first convolution is read on the quotient rows, the second on the output rows; on one frame the
   // quotient pass leaves the rows of ones to the z pass after it
   const int zero[3] = {0, 0, 0};
-  StridedGeom gy1 = gy, gz1 = gz, gy2 = gy, gz2 = gz, gzq = gz, gzf = gz;
-  plan.restrict_rows(q.qlo, q.qhi, gy1, gz1);
-  plan.restrict_rows(zero, zero, gy2, gz2);
+  plan.restrict_rows(q.qlo, q.qhi, m1);
+  plan.restrict_rows(zero, zero, m2);
   if (!blocked()) {
-    plan.skip_ones_rows(q, gzq, &gy2);
-    plan.mirror_rows(g, gzf, gy1);  // psi's mirror copies are read from their sources
+    plan.skip_ones_rows(q, m2);
+    plan.mirror_rows(g, m1);  // psi's mirror copies are read from their sources
+  } else if (plan.planar) {
+    plan.skip_ones_rows(q, m2, qtab[v]);
   }
   timer.begin(stream, PASS_X_FWD);
   plan.xf(d, g, S, plan.twM, plan.wr, stream);
   timer.end(stream);
-  plan.sz(timed(timer, gzf, PASS_Z_FWD), 0, S, S, nullptr, 1.f, plan.twZ, stream);
-  plan.sy(timed(timer, gy1, PASS_Y_CONV), 2, S, S, spec1[v], 1.f, plan.twY, stream);
-  plan.sz(timed(timer, gz1, PASS_Z_INV), 1, S, S, nullptr, 1.f, plan.twZ, stream);
+  plan.mid_forward(m1, S, stream, &timer);
+  plan.mid_rest(m1, S, S, spec1[v], stream, &timer);
   timer.begin(stream, PASS_X_RATIO);
   plan.xr(d, q, S, S, plan.twM, plan.wr, stream);
   timer.end(stream);
-  plan.sz(timed(timer, gzq, PASS_Z_FWD), 0, S, S, nullptr, 1.f, plan.twZ, stream);
-  plan.sy(timed(timer, gy2, PASS_Y_CONV), 2, S, S, spec2[v], 1.f, plan.twY, stream);
-  plan.sz(timed(timer, gz2, PASS_Z_INV), 1, S, S, nullptr, 1.f, plan.twZ, stream);
+  plan.mid_forward(m2, S, stream, &timer);
+  plan.mid_rest(m2, S, S, spec2[v], stream, &timer);
   UpdateParams u{};
   u.psi = psi;
   u.w = w[v];
@@ -630,37 +637,34 @@ void Decon::reduce_slots(int n, double2* out) {
 // One Mul iteration (ComputeBlockMulThreadCPU.runIteration semantics on the whole volume).
 int Decon::iteration_mul(double2* statOut) {
   const Dom& d = plan.dom;
-  const StridedGeom gy = plan.geom_y(), gz = plan.geom_z();
   // both convolutions are read on the output rows (the quotient and the stored result)
   const int zero[3] = {0, 0, 0};
-  StridedGeom gyo = gy, gzo = gz;
-  plan.restrict_rows(zero, zero, gyo, gzo);
+  Plan::Mid m1 = plan.mid();
+  plan.restrict_rows(zero, zero, m1);
+  const Plan::Mid rows = m1;
   GatherParams g{};
   g.src = psi;
   for (int k = 0; k < 3; ++k) { g.N[k] = N[k]; g.org[k] = -d.m[k]; }
   g.mode = GATHER_MIRROR;
-  StridedGeom gzf = gz, gyf = gyo;  // psi's mirror copies are read from their sources
-  plan.mirror_rows(g, gzf, gyf);
+  plan.mirror_rows(g, m1);  // psi's mirror copies are read from their sources
   // the forward transform of psi is shared by all views
   timer.begin(stream, PASS_X_FWD);
   plan.xf(d, g, Spsi, plan.twM, plan.wr, stream);
   timer.end(stream);
-  plan.sz(timed(timer, gzf, PASS_Z_FWD), 0, Spsi, Spsi, nullptr, 1.f, plan.twZ, stream);
+  plan.mid_forward(m1, Spsi, stream, &timer);
   std::vector<const float*> t2p(V), wp(V);
   for (int v = 0; v < V; ++v) {
-    plan.sy(timed(timer, gyf, PASS_Y_CONV), 2, Spsi, S, spec1[v], 1.f, plan.twY, stream);
-    plan.sz(timed(timer, gzo, PASS_Z_INV), 1, S, S, nullptr, 1.f, plan.twZ, stream);
+    plan.mid_rest(m1, Spsi, S, spec1[v], stream, &timer);
     RatioParams q{};
     q.img = img[v];
     for (int k = 0; k < 3; ++k) { q.N[k] = N[k]; q.o[k] = 0; }
-    StridedGeom gzq = gz, gyq = gyo;
-    plan.skip_ones_rows(q, gzq, &gyq);
+    Plan::Mid m2 = rows;
+    plan.skip_ones_rows(q, m2);
     timer.begin(stream, PASS_X_RATIO);
     plan.xr(d, q, S, S, plan.twM, plan.wr, stream);
     timer.end(stream);
-    plan.sz(timed(timer, gzq, PASS_Z_FWD), 0, S, S, nullptr, 1.f, plan.twZ, stream);
-    plan.sy(timed(timer, gyq, PASS_Y_CONV), 2, S, S, spec2[v], 1.f, plan.twY, stream);
-    plan.sz(timed(timer, gzo, PASS_Z_INV), 1, S, S, nullptr, 1.f, plan.twZ, stream);
+    plan.mid_forward(m2, S, stream, &timer);
+    plan.mid_rest(m2, S, S, spec2[v], stream, &timer);
     StoreParams st{T2 + nvox() * v};
     timer.begin(stream, PASS_X_STORE);
     plan.xs(d, st, S, plan.twM, plan.wr, stream);
@@ -926,31 +930,27 @@ int BlockThread::set_view_data(int v, const float* im, const float* wt, const in
 // ComputeBlockSeqThreadCPU.runIteration on the device buffers psiB, imgB, wB (stats left in statDev)
 int BlockThread::iterate_seq(int v, float maxI) {
   const Dom& d = plan.dom;
-  const StridedGeom gy = plan.geom_y(), gz = plan.geom_z();
   // both convolutions are read on the block's rows (the quotient over the whole block, the update)
   const int zero[3] = {0, 0, 0};
-  StridedGeom gyo = gy, gzo = gz;
-  plan.restrict_rows(zero, zero, gyo, gzo);
+  Plan::Mid m1 = plan.mid();
+  plan.restrict_rows(zero, zero, m1);
+  Plan::Mid m2 = m1;
   // convolve1: psi block with mirror-single extension of the block itself (ComputeBlockSeqThreadCPU.java:171-189)
   GatherParams g{};
   g.src = psiB;
   for (int k = 0; k < 3; ++k) { g.N[k] = B[k]; g.org[k] = -d.m[k]; }
   g.mode = GATHER_MIRROR;
-  StridedGeom gzf = gz, gyf = gyo;  // the block's mirror copies are read from their sources
-  plan.mirror_rows(g, gzf, gyf);
+  plan.mirror_rows(g, m1);  // the block's mirror copies are read from their sources
   plan.xf(d, g, S, plan.twM, plan.wr, stream);
-  plan.sz(gzf, 0, S, S, nullptr, 1.f, plan.twZ, stream);
-  plan.sy(gyf, 2, S, S, spec1[v], 1.f, plan.twY, stream);
-  plan.sz(gzo, 1, S, S, nullptr, 1.f, plan.twZ, stream);
+  plan.mid_forward(m1, S, stream);
+  plan.mid_rest(m1, S, S, spec1[v], stream);
   RatioParams q{};
   q.img = imgB;
   for (int k = 0; k < 3; ++k) { q.N[k] = B[k]; q.o[k] = 0; }
-  StridedGeom gzq = gz, gyq = gyo;
-  plan.skip_ones_rows(q, gzq, &gyq);
+  plan.skip_ones_rows(q, m2);
   plan.xr(d, q, S, S, plan.twM, plan.wr, stream);
-  plan.sz(gzq, 0, S, S, nullptr, 1.f, plan.twZ, stream);
-  plan.sy(gyq, 2, S, S, spec2[v], 1.f, plan.twY, stream);
-  plan.sz(gzo, 1, S, S, nullptr, 1.f, plan.twZ, stream);
+  plan.mid_forward(m2, S, stream);
+  plan.mid_rest(m2, S, S, spec2[v], stream);
   if (ensure_partials((int)(plan.rows_inner() / 4 + 1))) return -1;
   UpdateParams u{};
   u.psi = psiB;
@@ -1008,31 +1008,28 @@ int BlockThread::run_seq_at(int v, float* psiBlock, const long long off[3], floa
 int BlockThread::iterate_mul(int nv, const float* maxIs) {
   const size_t nb = (size_t)B[0] * B[1] * B[2];
   const Dom& d = plan.dom;
-  const StridedGeom gy = plan.geom_y(), gz = plan.geom_z();
   const int zero[3] = {0, 0, 0};
-  StridedGeom gyo = gy, gzo = gz;
-  plan.restrict_rows(zero, zero, gyo, gzo);
+  Plan::Mid m1 = plan.mid();
+  plan.restrict_rows(zero, zero, m1);
+  const Plan::Mid rows = m1;
   GatherParams g{};
   g.src = psiB;
   for (int k = 0; k < 3; ++k) { g.N[k] = B[k]; g.org[k] = -d.m[k]; }
   g.mode = GATHER_MIRROR;
-  StridedGeom gzf = gz, gyf = gyo;  // the block's mirror copies are read from their sources
-  plan.mirror_rows(g, gzf, gyf);
+  plan.mirror_rows(g, m1);  // the block's mirror copies are read from their sources
   plan.xf(d, g, Spsi, plan.twM, plan.wr, stream);
-  plan.sz(gzf, 0, Spsi, Spsi, nullptr, 1.f, plan.twZ, stream);
+  plan.mid_forward(m1, Spsi, stream);
   std::vector<const float*> t2p(nv), wp(nv);
   for (int v = 0; v < nv; ++v) {
-    plan.sy(gyf, 2, Spsi, S, spec1[v], 1.f, plan.twY, stream);
-    plan.sz(gzo, 1, S, S, nullptr, 1.f, plan.twZ, stream);
+    plan.mid_rest(m1, Spsi, S, spec1[v], stream);
     RatioParams q{};
     q.img = imgV[v];
     for (int k = 0; k < 3; ++k) { q.N[k] = B[k]; q.o[k] = 0; }
-    StridedGeom gzq = gz, gyq = gyo;
-    plan.skip_ones_rows(q, gzq, &gyq);
+    Plan::Mid m2 = rows;
+    plan.skip_ones_rows(q, m2);
     plan.xr(d, q, S, S, plan.twM, plan.wr, stream);
-    plan.sz(gzq, 0, S, S, nullptr, 1.f, plan.twZ, stream);
-    plan.sy(gyq, 2, S, S, spec2[v], 1.f, plan.twY, stream);
-    plan.sz(gzo, 1, S, S, nullptr, 1.f, plan.twZ, stream);
+    plan.mid_forward(m2, S, stream);
+    plan.mid_rest(m2, S, S, spec2[v], stream);
     StoreParams st{T2 + nb * v};
     plan.xs(d, st, S, plan.twM, plan.wr, stream);
     t2p[v] = T2 + nb * v;

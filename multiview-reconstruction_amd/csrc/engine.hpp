@@ -6,7 +6,8 @@
 //   * the FFT grid is P[0] x P[1] x P[2] (P[d] >= D[d] + K[d] - 1); FFT
 //     position p corresponds to volume coordinate o + p - m, m[d] = K[d]-1-K[d]/2
 //     (the left reach of the kernel), so the output region is p in [m, m + D);
-//   * the half spectrum is stored [z][y][hx], hx < P[0]/2 + 1, with row pitch HxP.
+//   * the half spectrum is stored [z][y][hx], hx < P[0]/2 + 1, with row pitch HxP; small grids (Plan::planar)
+//     store it [hx][z][y].
 // A linear convolution evaluated this way is exact on the output region for
 // any extension of the input outside it (util/FFTConvolution.java:508-543 pads
 // to at least N + K - 1 for the same reason).
@@ -57,7 +58,8 @@ struct GatherParams {
 // skipOnes: rows outside the quotient region (a row of ones, whose x spectrum is P0 at frequency 0 and 0
 // elsewhere) are not written; the z pass that reads the result puts them in itself (StridedGeom ones*), and
 // the work-groups are dealt over the quotient rows only: grid rows (y, z) in [rowLo, rowLo + rowN) per axis
-// (k = 1, 2), which are exactly the rows the quotient region selects.
+// (k = 1, 2), which are exactly the rows the quotient region selects.  For batched blocks (planar spectra only) each
+// block's rows are formed from its entry in the block table, and rowN are the most rows of any block.
 struct RatioParams {
   const float* img;
   int N[3];
@@ -124,10 +126,32 @@ struct StridedGeom {
 typedef void (*StridedFn)(const StridedGeom&, int mode, const float2* in, float2* out, const float2* spec,
                           float scale, const float2* tw, hipStream_t s);
 
-XFwdFn get_x_fwd(int M);
-XRatioFn get_x_ratio(int M);
-XUpdateFn get_x_update(int M);
-XStoreFn get_x_store(int M);
+// One pass of y and z transforms over planar spectra [hx][z][y] (plane.hip), in place or not: forward, times spec
+// ([hx][y slot][z slot]), inverse; spec null: forward and scale, stored in slot order.
+struct PlaneGeom {
+  int Py, Pz;          // at most kPlaneMax each
+  int ncols;           // planes (hx)
+  int nb = 1;          // batch entries: entry b reads in + inIdx[b] inStride (null: b) and spec + specIdx[b] specStride
+  size_t inStride = 0, outStride = 0, specStride = 0;   // (null: the shared spectrum), writes out + b outStride
+  const int* inIdx = nullptr;
+  const int* specIdx = nullptr;
+  int mir[2] = {0, 0}, mirN[2] = {0, 0};   // mirror extension along y, z (StridedGeom's mirM, mirN), off at 0
+  float onesDC = 0.f;                      // rows outside [onesLo, onesHi) (y, z) are spectra of ones, as in StridedGeom
+  int onesLo[2] = {0, 0}, onesHi[2] = {0, 0};
+  const int* onesTab = nullptr;            // per batch entry {yLo, yHi, zLo, zHi} instead
+  int lo[2] = {0, 0}, hi[2] = {1 << 30, 1 << 30};  // rows (y, z) stored
+  hipEvent_t evStart = nullptr, evStop = nullptr;
+};
+constexpr int kPlaneMax = 128;     // y and z lengths
+constexpr int kPlanarMaxM = 128;   // x passes with planar spectra are compiled for half lengths up to this
+void launch_plane(const PlaneGeom& g, const float2* in, float2* out, const float2* spec, float scale,
+                  const float2* twY, const float2* twZ, hipStream_t s);
+
+// planar: spectra [hx][z][y] instead of rows [z][y][hx]
+XFwdFn get_x_fwd(int M, bool planar);
+XRatioFn get_x_ratio(int M, bool planar);
+XUpdateFn get_x_update(int M, bool planar);
+XStoreFn get_x_store(int M, bool planar);
 StridedFn get_strided(int L);
 // the largest pencil position a lane of the length-L strided pass addresses with its 32-bit offset, plus one
 int get_strided_span(int L);

@@ -26,10 +26,12 @@ bool device_memory_of(const void* p, int dev, bool managed);
 // ---------------------------------------------------------------------------
 // One FFT-convolution plan: output region D, kernel size K (see engine.hpp).
 // ---------------------------------------------------------------------------
+struct Timer;
 struct Plan {
   Dom dom{};
   int K[3] = {0, 0, 0};
   int M = 0, Hx = 0;
+  bool planar = false;    // spectra [hx][z][y], y and z transforms in one plane pass
   float2* twM = nullptr;  // length-M twiddles (x)
   float2* wr = nullptr;   // exp(-2 pi i k / P0), k = 0..M
   float2* twY = nullptr;
@@ -49,23 +51,35 @@ struct Plan {
   void destroy();
   size_t ncpx() const { return (size_t)dom.HxP * dom.P[1] * dom.P[2]; }
   size_t rows_inner() const { return (size_t)dom.D[1] * dom.D[2]; }
-  StridedGeom geom_y() const;
-  StridedGeom geom_z() const;
-  // Narrows the geometries gy, gz of a convolution's y_conv and z_inv passes to what the next x pass reads: the
-  // grid rows (y, z) in [m - lo, m + D + hi) per axis (within the grid).  y_conv then stores only those y, and
-  // z_inv transforms only those y planes and stores only those z.  Batched geometries stay batched.
-  void restrict_rows(const int lo[3], const int hi[3], StridedGeom& gy, StridedGeom& gz) const;
-  // Sets q.skipOnes, the quotient rows q.rowLo / rowN, and the z geometry gz of the forward pass that reads the
-  // quotient pass's result: the rows outside the quotient region are rows of ones (not written by the quotient
-  // pass, put in by the z pass).  With gy (the y convolution after that z pass) the z pass also leaves out the
-  // y planes outside the quotient region, planes of ones whose spectrum, P0 P2 at x and z frequency 0, the y
-  // convolution puts in.  Not for batched blocks, whose quotient regions differ per block.
-  void skip_ones_rows(RatioParams& q, StridedGeom& gz, StridedGeom* gy = nullptr) const;
-  // For a forward transform of a mirror gather (g.mode MIRROR): sets g.uniqueRows, so that x_fwd transforms only
-  // the rows that are not mirror copies, and makes the z pass after it (gzf) transform only those y planes and
-  // read z through the mirror, and the y convolution after that (gyc) read y through it.  Not for batched
-  // blocks, whose gathers mirror the whole volume, not the block; a no-op for spectra of 4 GiB or more.
-  void mirror_rows(GatherParams& g, StridedGeom& gzf, StridedGeom& gyc) const;
+  // The passes between the x passes of a convolution: forward z, y with the spectrum product, inverse z; on planar
+  // plans one plane pass.  The defaults cover the whole grid.
+  struct Mid {
+    StridedGeom zf, y, zi;
+    PlaneGeom pl;
+  };
+  Mid mid() const;
+  // batched blocks: nb spectra, blockStride complex values apart
+  void set_blocks(Mid& m, int nb, size_t blockStride) const;
+  // Narrows a convolution to what the next x pass reads: the grid rows (y, z) in [m - lo, m + D + hi) per axis (within
+  // the grid).  The y pass then stores only those y, and the inverse z pass transforms only those y planes and
+  // stores only those z.
+  void restrict_rows(const int lo[3], const int hi[3], Mid& m) const;
+  // For a convolution of the quotient: sets q.skipOnes and the quotient rows q.rowLo / rowN; the rows outside the
+  // quotient region are rows of ones, which the quotient pass does not write and the forward z pass puts in.  That
+  // pass also leaves out the y planes outside the quotient region, planes of ones whose spectrum, P0 P2 at x and z
+  // frequency 0, the y pass puts in.  For batched blocks, whose quotient regions differ per block, only on planar
+  // plans, with the blocks' regions in a device table (blockRows).
+  void skip_ones_rows(RatioParams& q, Mid& m, const int* blockRows = nullptr) const;
+  // For a convolution of a mirror gather (g.mode MIRROR): sets g.uniqueRows, so that x_fwd transforms only the rows
+  // that are not mirror copies; the forward z pass transforms only those y planes and reads z through the mirror, and
+  // the y pass reads y through it.  Not for batched blocks, whose gathers mirror the whole volume, not the block; a
+  // no-op for spectra of 4 GiB or more.
+  void mirror_rows(GatherParams& g, Mid& m) const;
+  // the passes of a convolution: the forward part that does not depend on the kernel (in place; nothing on planar
+  // plans), and the rest
+  void mid_forward(const Mid& m, float2* S, hipStream_t s, Timer* t = nullptr) const;
+  void mid_rest(const Mid& m, const float2* in, float2* out, const float2* spec, hipStream_t s,
+                Timer* t = nullptr) const;
   float inv_scale() const { return 2.0f / ((float)dom.P[0] * (float)dom.P[1] * (float)dom.P[2]); }
 
   // spectrum of a device kernel (K layout), scaled by the inverse-FFT factor
@@ -97,12 +111,17 @@ struct Timer {
   int every = 1;                      // time one launch in `every` of each enabled category
   long long seen[PASS_COUNT] = {0};   // launches of each category since the last reset
   std::vector<hipEvent_t> ev;
-  std::vector<int> cat;
+  struct Shot { size_t ev; int cat; double share; };  // events ev, ev + 1; the share of their time that is category cat's
+  std::vector<Shot> shots;
   size_t used = 0;
+  void grow();
   void begin(hipStream_t s, int c);
   void end(hipStream_t s);
   // a start / stop pair for a launch that records its own kernel's execution (both null when c is off)
-  void kernel(int c, hipEvent_t* start, hipEvent_t* stop);
+  void kernel(int c, hipEvent_t* start, hipEvent_t* stop) { kernel(&c, 1, start, stop); }
+  // the same for a launch that does the work of n passes: each is counted, with an nth of the time
+  void kernel(const int* c, int n, hipEvent_t* start, hipEvent_t* stop);
+  bool zForward = false;  // planar plans: the next plane pass does a forward z pass's work too
   int collect(double* ms, long long* n);  // accumulates into arrays of PASS_COUNT
   void release();
   // enable the categories in mask (bit c = category c), timing the first launch of every group of `every`;
@@ -160,6 +179,7 @@ struct Decon {
   int blockE[3] = {0, 0, 0};
   int nbAll = 0;
   std::vector<int*> btab;   // per view: device table {o[3], D[3]} of its blocks with content
+  std::vector<int*> qtab;   // per view (planar plans): device table {yLo, yHi, zLo, zHi} of the blocks' quotient rows
   std::vector<int> nbView;  // blocks per view after DeconView.filterBlocksForContent
   bool blocked() const { return blockB[0] != 0; }
   int set_block_size(const int B[3]);

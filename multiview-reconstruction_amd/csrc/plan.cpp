@@ -68,10 +68,11 @@ int Plan::create_geometry(const int D[3], const int Kd[3], const int* Pmin) {
   M = dom.P[0] / 2;
   Hx = M + 1;
   dom.HxP = (Hx + 15) / 16 * 16;
-  xf = get_x_fwd(M);
-  xr = get_x_ratio(M);
-  xu = get_x_update(M);
-  xs = get_x_store(M);
+  planar = dom.P[1] <= kPlaneMax && dom.P[2] <= kPlaneMax && M <= kPlanarMaxM;
+  xf = get_x_fwd(M, planar);
+  xr = get_x_ratio(M, planar);
+  xu = get_x_update(M, planar);
+  xs = get_x_store(M, planar);
   sy = get_strided(dom.P[1]);
   sz = get_strided(dom.P[2]);
   if (!xf || !xr || !xu || !xs || !sy || !sz) { set_error("plan: missing kernel instantiation"); return -1; }
@@ -89,43 +90,64 @@ void Plan::destroy() {
     if (*p) { (void)hipFree(*p); *p = nullptr; }
 }
 
-StridedGeom Plan::geom_y() const {
-  StridedGeom g;
-  g.planeStride = (size_t)dom.P[1] * dom.HxP;
-  g.lineStride = dom.HxP;
-  g.ncols = Hx;
-  g.nplanes = dom.P[2];
-  g.width = wy;
-  return g;
+Plan::Mid Plan::mid() const {
+  Mid m;
+  m.y.planeStride = (size_t)dom.P[1] * dom.HxP;
+  m.y.lineStride = dom.HxP;
+  m.y.ncols = Hx;
+  m.y.nplanes = dom.P[2];
+  m.y.width = wy;
+  m.zf.planeStride = dom.HxP;
+  m.zf.lineStride = (size_t)dom.P[1] * dom.HxP;
+  m.zf.ncols = Hx;
+  m.zf.nplanes = dom.P[1];
+  m.zf.width = wz;
+  m.zi = m.zf;
+  m.pl.Py = dom.P[1];
+  m.pl.Pz = dom.P[2];
+  m.pl.ncols = Hx;
+  m.pl.lo[0] = m.pl.lo[1] = 0;
+  m.pl.hi[0] = dom.P[1];
+  m.pl.hi[1] = dom.P[2];
+  return m;
 }
 
-StridedGeom Plan::geom_z() const {
-  StridedGeom g;
-  g.planeStride = dom.HxP;
-  g.lineStride = (size_t)dom.P[1] * dom.HxP;
-  g.ncols = Hx;
-  g.nplanes = dom.P[1];
-  g.width = wz;
-  return g;
+void Plan::set_blocks(Mid& m, int nb, size_t blockStride) const {
+  for (StridedGeom* g : {&m.zf, &m.y, &m.zi}) {
+    g->blockPlanes = g->nplanes;
+    g->nplanes *= nb;
+    g->blockStride = blockStride;
+  }
+  m.pl.nb = nb;
+  m.pl.inStride = m.pl.outStride = blockStride;
 }
 
-void Plan::restrict_rows(const int lo[3], const int hi[3], StridedGeom& gy, StridedGeom& gz) const {
+void Plan::restrict_rows(const int lo[3], const int hi[3], Mid& m) const {
   int a[3], b[3];
   for (int k = 1; k < 3; ++k) {
     a[k] = std::max(0, dom.m[k] - lo[k]);
     b[k] = std::min(dom.P[k], dom.m[k] + dom.D[k] + hi[k]);
+    m.pl.lo[k - 1] = a[k];
+    m.pl.hi[k - 1] = b[k];
   }
-  gy.storeLo = a[1];
-  gy.storeHi = b[1];
-  const int nb = gz.blockPlanes ? gz.nplanes / gz.blockPlanes : 1;
-  gz.plane0 = a[1];
-  gz.nplanes = (b[1] - a[1]) * nb;
-  if (gz.blockPlanes) gz.blockPlanes = b[1] - a[1];
-  gz.storeLo = a[2];
-  gz.storeHi = b[2];
+  m.y.storeLo = a[1];
+  m.y.storeHi = b[1];
+  const int nb = m.zi.blockPlanes ? m.zi.nplanes / m.zi.blockPlanes : 1;
+  m.zi.plane0 = a[1];
+  m.zi.nplanes = (b[1] - a[1]) * nb;
+  if (m.zi.blockPlanes) m.zi.blockPlanes = b[1] - a[1];
+  m.zi.storeLo = a[2];
+  m.zi.storeHi = b[2];
 }
 
-void Plan::skip_ones_rows(RatioParams& q, StridedGeom& gz, StridedGeom* gy) const {
+void Plan::skip_ones_rows(RatioParams& q, Mid& m, const int* blockRows) const {
+  if (blockRows) {
+    q.skipOnes = 1;
+    for (int k = 1; k < 3; ++k) q.rowN[k] = std::min(dom.P[k], dom.D[k] + q.qlo[k] + q.qhi[k]);
+    m.pl.onesDC = (float)dom.P[0];
+    m.pl.onesTab = blockRows;
+    return;
+  }
   // quotient rows (y, z) in grid coordinates, as the quotient pass selects them
   int lo[3], hi[3];
   for (int k = 1; k < 3; ++k) {
@@ -136,36 +158,70 @@ void Plan::skip_ones_rows(RatioParams& q, StridedGeom& gz, StridedGeom* gy) cons
   for (int k = 1; k < 3; ++k) {
     q.rowLo[k] = lo[k];
     q.rowN[k] = std::max(0, hi[k] - lo[k]);
+    m.pl.onesLo[k - 1] = lo[k];
+    m.pl.onesHi[k - 1] = hi[k];
   }
-  gz.onesDC = (float)dom.P[0];  // the x transform of a row of ones
-  gz.onesPlaneLo = lo[1];
-  gz.onesPlaneHi = hi[1];
-  gz.onesLo = lo[2];
-  gz.onesHi = hi[2];
-  if (gy) {
-    gz.plane0 = lo[1];
-    gz.nplanes = std::max(0, hi[1] - lo[1]);
-    gy->onesDC = (float)dom.P[0] * (float)dom.P[2];  // the xz transform of a plane of ones
-    gy->onesDCPlane = 0;
-    gy->onesPlaneLo = 0;
-    gy->onesPlaneHi = dom.P[2];
-    gy->onesLo = lo[1];
-    gy->onesHi = hi[1];
-  }
+  m.pl.onesDC = m.zf.onesDC = (float)dom.P[0];  // the x transform of a row of ones
+  m.zf.onesPlaneLo = lo[1];
+  m.zf.onesPlaneHi = hi[1];
+  m.zf.onesLo = lo[2];
+  m.zf.onesHi = hi[2];
+  m.zf.plane0 = lo[1];
+  m.zf.nplanes = std::max(0, hi[1] - lo[1]);
+  m.y.onesDC = (float)dom.P[0] * (float)dom.P[2];  // the xz transform of a plane of ones
+  m.y.onesDCPlane = 0;
+  m.y.onesPlaneLo = 0;
+  m.y.onesPlaneHi = dom.P[2];
+  m.y.onesLo = lo[1];
+  m.y.onesHi = hi[1];
 }
 
-void Plan::mirror_rows(GatherParams& g, StridedGeom& gzf, StridedGeom& gyc) const {
+void Plan::mirror_rows(GatherParams& g, Mid& m) const {
   // the strided passes read the mirror copies with 32-bit byte offsets from the plane: the z pencil's span, the
   // whole spectrum, must fit them (otherwise every row is transformed and read as written)
   if ((ncpx() + 16) * sizeof(float2) > 0xffffffffull) return;
   g.uniqueRows = 1;
   // unique rows: FFT positions [-org, -org + N) per axis, inside the grid
-  gzf.plane0 = -g.org[1];
-  gzf.nplanes = g.N[1];
-  gzf.mirM = -g.org[2];
-  gzf.mirN = g.N[2];
-  gyc.mirM = -g.org[1];
-  gyc.mirN = g.N[1];
+  m.zf.plane0 = -g.org[1];
+  m.zf.nplanes = g.N[1];
+  m.zf.mirM = -g.org[2];
+  m.zf.mirN = g.N[2];
+  m.y.mirM = -g.org[1];
+  m.y.mirN = g.N[1];
+  for (int k = 0; k < 2; ++k) {
+    m.pl.mir[k] = -g.org[k + 1];
+    m.pl.mirN[k] = g.N[k + 1];
+  }
+}
+
+// geometry of a launch whose kernel execution is timed under category c (untimed without a timer, or when c is off)
+template <typename G>
+static G timed(Timer* t, G g, int c) {
+  if (t) t->kernel(c, &g.evStart, &g.evStop);
+  return g;
+}
+
+void Plan::mid_forward(const Mid& m, float2* S, hipStream_t s, Timer* t) const {
+  if (planar) {
+    if (t) t->zForward = true;
+    return;
+  }
+  sz(timed(t, m.zf, PASS_Z_FWD), 0, S, S, nullptr, 1.f, twZ, s);
+}
+
+void Plan::mid_rest(const Mid& m, const float2* in, float2* out, const float2* spec, hipStream_t s, Timer* t) const {
+  if (planar) {
+    PlaneGeom g = m.pl;
+    if (t) {
+      const int passes[3] = {PASS_Y_CONV, PASS_Z_INV, PASS_Z_FWD};
+      t->kernel(passes, t->zForward ? 3 : 2, &g.evStart, &g.evStop);
+      t->zForward = false;
+    }
+    launch_plane(g, in, out, spec, 1.f, twY, twZ, s);
+    return;
+  }
+  sy(timed(t, m.y, PASS_Y_CONV), 2, in, out, spec, 1.f, twY, s);
+  sz(timed(t, m.zi, PASS_Z_INV), 1, out, out, nullptr, 1.f, twZ, s);
 }
 
 int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const {
@@ -174,8 +230,13 @@ int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) con
   for (int d = 0; d < 3; ++d) { g.N[d] = K[d]; g.org[d] = 0; }
   g.mode = GATHER_KERNEL;
   xf(dom, g, spec, twM, wr, s);
-  sy(geom_y(), 0, spec, spec, nullptr, 1.f, twY, s);
-  sz(geom_z(), 3, spec, spec, nullptr, inv_scale(), twZ, s);
+  const Mid m = mid();
+  if (planar) {
+    launch_plane(m.pl, spec, spec, nullptr, inv_scale(), twY, twZ, s);
+  } else {
+    sy(m.y, 0, spec, spec, nullptr, 1.f, twY, s);
+    sz(m.zf, 3, spec, spec, nullptr, inv_scale(), twZ, s);
+  }
   MVR_HIP(hipGetLastError());
   return 0;
 }
@@ -183,14 +244,13 @@ int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) con
 int Plan::convolve(const GatherParams& g, const float2* spec, float2* work, float* out, hipStream_t s) const {
   // the store reads the output rows only
   const int zero[3] = {0, 0, 0};
-  StridedGeom gy = geom_y(), gz = geom_z(), gzo = gz;
-  restrict_rows(zero, zero, gy, gzo);
+  Mid m = mid();
+  restrict_rows(zero, zero, m);
   GatherParams gg = g;
-  if (g.mode == GATHER_MIRROR) mirror_rows(gg, gz, gy);
+  if (g.mode == GATHER_MIRROR) mirror_rows(gg, m);
   xf(dom, gg, work, twM, wr, s);
-  sz(gz, 0, work, work, nullptr, 1.f, twZ, s);
-  sy(gy, 2, work, work, spec, 1.f, twY, s);
-  sz(gzo, 1, work, work, nullptr, 1.f, twZ, s);
+  mid_forward(m, work, s);
+  mid_rest(m, work, work, spec, s);
   StoreParams st{out};
   xs(dom, st, work, twM, wr, s);
   MVR_HIP(hipGetLastError());
@@ -198,35 +258,35 @@ int Plan::convolve(const GatherParams& g, const float2* spec, float2* work, floa
 }
 
 // ------------------------------------------------------------------ timers
+void Timer::grow() {
+  if (used + 2 <= ev.size()) return;
+  const size_t old = ev.size();
+  ev.resize(old + 256);
+  for (size_t i = old; i < ev.size(); ++i) (void)hipEventCreate(&ev[i]);
+}
 void Timer::begin(hipStream_t s, int c) {
   pending = on && ((mask >> c) & 1u) && seen[c]++ % every == 0;
   if (!pending) return;
-  if (used + 2 > ev.size()) {
-    size_t old = ev.size();
-    ev.resize(old + 256);
-    for (size_t i = old; i < ev.size(); ++i) (void)hipEventCreate(&ev[i]);
-  }
+  grow();
   (void)hipEventRecord(ev[used], s);
-  cat.push_back(c);
-  used++;
+  shots.push_back({used, c, 1.0});
 }
-void Timer::kernel(int c, hipEvent_t* start, hipEvent_t* stop) {
+void Timer::kernel(const int* c, int n, hipEvent_t* start, hipEvent_t* stop) {
   *start = *stop = nullptr;
-  if (!on || !((mask >> c) & 1u) || seen[c]++ % every != 0) return;
-  if (used + 2 > ev.size()) {
-    size_t old = ev.size();
-    ev.resize(old + 256);
-    for (size_t i = old; i < ev.size(); ++i) (void)hipEventCreate(&ev[i]);
-  }
+  if (!on) return;
+  const size_t before = shots.size();
+  for (int i = 0; i < n; ++i)
+    if (((mask >> c[i]) & 1u) && seen[c[i]]++ % every == 0) shots.push_back({used, c[i], 1.0 / n});
+  if (shots.size() == before) return;
+  grow();
   *start = ev[used];
   *stop = ev[used + 1];
-  cat.push_back(c);
   used += 2;
 }
 void Timer::end(hipStream_t s) {
   if (!pending) return;
-  (void)hipEventRecord(ev[used], s);
-  used++;
+  (void)hipEventRecord(ev[used + 1], s);
+  used += 2;
   pending = false;
 }
 void Timer::reset(unsigned m, int e) {
@@ -238,14 +298,14 @@ void Timer::reset(unsigned m, int e) {
 int Timer::collect(double* outMs, long long* outN) {
   if (used > 0) {
     (void)hipEventSynchronize(ev[used - 1]);
-    for (size_t i = 0; i + 1 < used; i += 2) {
+    for (const Shot& s : shots) {
       float t = 0.f;
-      (void)hipEventElapsedTime(&t, ev[i], ev[i + 1]);
-      ms[cat[i / 2]] += t;
-      cnt[cat[i / 2]] += 1;
+      (void)hipEventElapsedTime(&t, ev[s.ev], ev[s.ev + 1]);
+      ms[s.cat] += t * s.share;
+      cnt[s.cat] += 1;
     }
     used = 0;
-    cat.clear();
+    shots.clear();
   }
   for (int c = 0; c < PASS_COUNT; ++c) {
     if (outMs) outMs[c] = ms[c];
@@ -256,7 +316,7 @@ int Timer::collect(double* outMs, long long* outN) {
 void Timer::release() {
   for (auto& e : ev) (void)hipEventDestroy(e);
   ev.clear();
-  cat.clear();
+  shots.clear();
   used = 0;
 }
 

@@ -53,6 +53,17 @@ __device__ __forceinline__ void block_reduce_stats_nt(double s, double mx, doubl
   if (threadIdx.x == 0) *out = make_double2(rs[0], rm[0]);
 }
 
+// Where a row's value k lies: rows of HxP consecutive values, or (TR, planar spectra) one value per hx plane, the row
+// (y, z) at z P1 + y of every plane.
+template <bool TR>
+__device__ __forceinline__ size_t x2_row(const Dom& d, int row) {
+  return TR ? (size_t)row : (size_t)row * d.HxP;
+}
+template <bool TR>
+__device__ __forceinline__ unsigned x2_at(int k, unsigned cs) {
+  return TR ? (unsigned)k * cs : (unsigned)k;
+}
+
 constexpr long long kOuterRow = -(1ll << 62);
 constexpr size_t kNoRow = ~(size_t)0;
 
@@ -184,10 +195,10 @@ __device__ __forceinline__ void x2_forward(float2* rb, const float2* tw, int q, 
 
 // R2C post-processing of a row whose complex transform Z lane q holds as z[k2] = Z[q + A k2]:
 // X[k] = (Z[k] + Z*[M - k]) / 2 + W_P0^k (Z[k] - Z*[M - k]) / 2i for k = q + A k2, and X[M] (lane 0), written
-// to dst (the row's start in HBM) when rowOk
-template <int M>
+// to dst (the row's start in HBM; cs: values per hx plane) when rowOk
+template <int M, bool TR>
 __device__ __forceinline__ void x2_post_store_regs(const float2* z, int q, const float2* twr, float2* __restrict__ dst,
-                                                   bool rowOk) {
+                                                   bool rowOk, unsigned cs) {
   using C = XCfg<M>;
   float2 zc[C::B];
   x2_mirror_pairs<M>(z, z[0], q, zc);  // Z[M] = Z[0]
@@ -200,14 +211,14 @@ __device__ __forceinline__ void x2_post_store_regs(const float2* z, int q, const
     const float2 e = make_float2(0.5f * (zk.x + c.x), 0.5f * (zk.y + c.y));
     const float2 dd = csub(zk, c);
     const float2 od = make_float2(0.5f * dd.y, -0.5f * dd.x);
-    dst[k] = cadd(e, cmul(twr[k], od));
+    dst[x2_at<TR>(k, cs)] = cadd(e, cmul(twr[k], od));
   }
   if (q == 0) {
     const float2 zk = z[0], c = cconj(z[0]);
     const float2 e = make_float2(0.5f * (zk.x + c.x), 0.5f * (zk.y + c.y));
     const float2 dd = csub(zk, c);
     const float2 od = make_float2(0.5f * dd.y, -0.5f * dd.x);
-    dst[M] = cadd(e, cmul(twr[M], od));
+    dst[x2_at<TR>(M, cs)] = cadd(e, cmul(twr[M], od));
   }
 }
 
@@ -216,17 +227,17 @@ __device__ __forceinline__ void x2_post_store_regs(const float2* z, int q, const
 // z[q + B n1] in out[n1] (lane q < B)
 // PF: the transforms' coprime splits by the prime-factor algorithm (false: Cooley-Tukey throughout, which the
 // update pass on short rows runs 3 % faster at M = 150)
-template <int M, bool PF = true>
+template <int M, bool TR, bool PF = true>
 __device__ __forceinline__ void x2_inverse_half_regs(const float2* __restrict__ src, float2* rb, const float2* tw,
-                                                     const float2* twr, int q, float2* out) {
+                                                     const float2* twr, int q, float2* out, unsigned cs) {
   using C = XCfg<M>;
   constexpr int A = C::A, B = C::B;
   float2 x[B];
   float2 xM = make_float2(0.f, 0.f);
   const bool ld = src != nullptr && q < A;
 #pragma unroll
-  for (int k2 = 0; k2 < B; ++k2) x[k2] = ld ? src[q + A * k2] : make_float2(0.f, 0.f);
-  if (ld && q == 0) xM = src[M];
+  for (int k2 = 0; k2 < B; ++k2) x[k2] = ld ? src[x2_at<TR>(q + A * k2, cs)] : make_float2(0.f, 0.f);
+  if (ld && q == 0) xM = src[x2_at<TR>(M, cs)];
   float2 xc[B];
   x2_mirror_pairs<M>(x, xM, q, xc);
   float2 u[B];
@@ -274,7 +285,7 @@ __device__ __forceinline__ void x2_park_inverse(float2* rb, int q, const float2*
 }
 
 // ------------------------------------------------------------------ forward with gather
-template <int M>
+template <int M, bool TR>
 __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, float2* __restrict__ S,
                                                          const float2* __restrict__ twM,
                                                          const float2* __restrict__ wr) {
@@ -343,7 +354,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, f
       }
     }
     srcRow[threadIdx.x] = off;   // row start in src (>= 0), -1: no source row
-    dstRow[threadIdx.x] = live ? (size_t)row * d.HxP : kNoRow;
+    dstRow[threadIdx.x] = live ? x2_row<TR>(d, row) : kNoRow;
   }
   __syncthreads();
   // the first transform step reads its values z[q + B a] = (x[2n], x[2n + 1]) straight from the source
@@ -367,13 +378,13 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, f
   float2 z[C::B];
   x2_forward_regs_half<M>(rb, tw, q, v, z);
   const size_t o = dstRow[r];
-  x2_post_store_regs<M>(z, q, twr, S + (o == kNoRow ? 0 : o), o != kNoRow);
+  x2_post_store_regs<M, TR>(z, q, twr, S + (o == kNoRow ? 0 : o), o != kNoRow, (unsigned)(d.P[1] * d.P[2]));
 }
 
 // ------------------------------------------------------------------ inverse, quotient, forward
 // ratio = img > 0 ? img / blurred : 1 on the quotient region, 1 elsewhere
 // (DeconvolutionMethods.computeQuotient, D/iteration/sequential/DeconvolutionMethods.java:46-98)
-template <int M>
+template <int M, bool TR>
 __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(Dom d, RatioParams q_, const float2* __restrict__ Sin,
                                                            float2* __restrict__ Sout,
                                                            const float2* __restrict__ twM,
@@ -405,8 +416,15 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
     // skipOnes: the work-groups cover the quotient rows only, index i -> grid row (rowLo1 + i % rowN1,
     // rowLo2 + i / rowN1)
     int row = row0 + threadIdx.x;
-    const bool live = row < (q_.skipOnes ? q_.rowN[1] * q_.rowN[2] : nrows);
-    if (q_.skipOnes && live) row = (q_.rowLo[2] + row / q_.rowN[1]) * d.P[1] + q_.rowLo[1] + row % q_.rowN[1];
+    int lo1 = q_.rowLo[1], n1 = q_.rowN[1], lo2 = q_.rowLo[2], n2 = q_.rowN[2];
+    if (q_.skipOnes && d.btab) {  // this block's quotient rows
+      lo1 = d.m[1] + max(-q_.qlo[1], -o[1]);
+      n1 = d.m[1] + min(D[1] + q_.qhi[1], q_.N[1] - o[1]) - lo1;
+      lo2 = d.m[2] + max(-q_.qlo[2], -o[2]);
+      n2 = d.m[2] + min(D[2] + q_.qhi[2], q_.N[2] - o[2]) - lo2;
+    }
+    const bool live = row < (q_.skipOnes ? n1 * n2 : nrows);
+    if (q_.skipOnes && live) row = (lo2 + row / n1) * d.P[1] + lo1 + row % n1;
     long long ir = kOuterRow;
     if (live) {
       // quotient rows: the output region widened by qlo / qhi, inside the volume
@@ -416,7 +434,7 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
         ir = ((long long)(o[2] + lz) * q_.N[1] + (o[1] + ly)) * q_.N[0] + o[0] - d.m[0];
     }
     imgRow[threadIdx.x] = ir;
-    outOff[threadIdx.x] = live ? (size_t)row * d.HxP : kNoRow;
+    outOff[threadIdx.x] = live ? x2_row<TR>(d, row) : kNoRow;
   }
   __syncthreads();
   const int r = threadIdx.x / C::T, q = threadIdx.x % C::T;
@@ -427,7 +445,8 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
   const int x0f = d.m[0] + max(-q_.qlo[0], -o[0]), x1f = d.m[0] + min(D[0] + q_.qhi[0], q_.N[0] - o[0]);
   // rows outside the quotient region are a row of ones after the quotient: their blurred values are not read
   float2 z[C::A];
-  x2_inverse_half_regs<M>(ir != kOuterRow ? Sin + so : nullptr, rb, tw, twr, q, z);
+  const unsigned cs = (unsigned)(d.P[1] * d.P[2]);
+  x2_inverse_half_regs<M, TR>(ir != kOuterRow ? Sin + so : nullptr, rb, tw, twr, q, z, cs);
   float2 zf[C::B];
   if constexpr (!C::long_rows) {
     // short rows (only B of T lanes hold values): park the blurred rows in LDS, form the quotient there with the
@@ -489,12 +508,12 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
     __syncthreads();  // the inverse's reads of the row are done before the forward writes it
     x2_forward_regs<M>(rb, tw, q, z, zf);
   }
-  x2_post_store_regs<M>(zf, q, twr, Sout + (so == kNoRow ? 0 : so),
-                        so != kNoRow && !(q_.skipOnes && ir == kOuterRow));
+  x2_post_store_regs<M, TR>(zf, q, twr, Sout + (so == kNoRow ? 0 : so),
+                            so != kNoRow && !(q_.skipOnes && ir == kOuterRow), cs);
 }
 
 // ------------------------------------------------------------------ inverse + psi update (output rows only)
-template <int M>
+template <int M, bool TR>
 __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_update(Dom d, UpdateParams u, FastDiv divD0,
                                                             const float2* __restrict__ S,
                                                             const float2* __restrict__ twM,
@@ -528,7 +547,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_update(Dom d, UpdateParams u
     if (row < nrows) {
       const int ly = row % D[1], lz = row / D[1];
       pr = ((long long)(o[2] + lz) * u.N[1] + (o[1] + ly)) * u.N[0] + o[0];
-      so = ((size_t)(d.m[2] + lz) * d.P[1] + (d.m[1] + ly)) * d.HxP;
+      so = x2_row<TR>(d, (d.m[2] + lz) * d.P[1] + (d.m[1] + ly));
     }
     psiRow[threadIdx.x] = pr;   // >= 0 for output rows (the output region lies inside the volume)
     rowOff[threadIdx.x] = so;
@@ -538,7 +557,8 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_update(Dom d, UpdateParams u
   float2* rb = buf + r * C::RS;
   const size_t so = rowOff[r];
   float2 z[C::A];
-  x2_inverse_half_regs<M, C::long_rows>(so != kNoRow ? S + so : nullptr, rb, tw, twr, q, z);
+  x2_inverse_half_regs<M, TR, C::long_rows>(so != kNoRow ? S + so : nullptr, rb, tw, twr, q, z,
+                                            (unsigned)(d.P[1] * d.P[2]));
   double sum = 0.0;
   float mx = -1.f;
   const RLConsts rc = rl_consts(u.lambda, u.minValue, u.maxI);
@@ -664,7 +684,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_update(Dom d, UpdateParams u
 }
 
 // ------------------------------------------------------------------ inverse + store of the output region
-template <int M>
+template <int M, bool TR>
 __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_store(Dom d, StoreParams st, const float2* __restrict__ S,
                                                            const float2* __restrict__ twM,
                                                            const float2* __restrict__ wr) {
@@ -683,7 +703,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_store(Dom d, StoreParams st,
     size_t so = kNoRow;
     if (row < nrows) {
       const int ly = row % d.D[1], lz = row / d.D[1];
-      so = ((size_t)(d.m[2] + lz) * d.P[1] + (d.m[1] + ly)) * d.HxP;
+      so = x2_row<TR>(d, (d.m[2] + lz) * d.P[1] + (d.m[1] + ly));
     }
     rowOff[threadIdx.x] = so;
   }
@@ -692,7 +712,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_store(Dom d, StoreParams st,
   float2* rb = buf + r * C::RS;
   const size_t so = rowOff[r];
   float2 z[C::A];
-  x2_inverse_half_regs<M>(so != kNoRow ? S + so : nullptr, rb, tw, twr, q, z);
+  x2_inverse_half_regs<M, TR>(so != kNoRow ? S + so : nullptr, rb, tw, twr, q, z, (unsigned)(d.P[1] * d.P[2]));
   const int row = row0 + r;
   if (q < C::B && row < nrows) {
     const int DX = d.D[0], m0 = d.m[0];
@@ -709,7 +729,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_store(Dom d, StoreParams st,
 // ------------------------------------------------------------------ host launchers
 // Batched launches (d.btab set) run d.nb blocks of wgPerBlock work-groups each: work-group w serves block
 // w / wgPerBlock; rows of a block beyond its own extent are skipped inside the kernels.
-template <int M>
+template <int M, bool TR>
 void launch_x_fwd(const Dom& d, const GatherParams& g, float2* S, const float2* twM, const float2* wr,
                   hipStream_t s) {
   static_assert(x2_ok<M>(), "every compiled x length has a two-step split");
@@ -718,9 +738,9 @@ void launch_x_fwd(const Dom& d, const GatherParams& g, float2* S, const float2* 
   const int rows = g.uniqueRows && g.mode == GATHER_MIRROR ? g.N[1] * g.N[2] : d.P[1] * d.P[2];
   dd.wgPerBlock = (rows + C::RW - 1) / C::RW;
   const int nb = d.btab ? d.nb : 1;
-  hipLaunchKernelGGL(k_x2_fwd<M>, dim3(dd.wgPerBlock * nb), dim3(C::NT), 0, s, dd, g, S, twM, wr);
+  hipLaunchKernelGGL((k_x2_fwd<M, TR>), dim3(dd.wgPerBlock * nb), dim3(C::NT), 0, s, dd, g, S, twM, wr);
 }
-template <int M>
+template <int M, bool TR>
 void launch_x_ratio(const Dom& d, const RatioParams& q, const float2* Sin, float2* Sout, const float2* twM,
                     const float2* wr, hipStream_t s) {
   static_assert(x2_ok<M>(), "every compiled x length has a two-step split");
@@ -730,9 +750,9 @@ void launch_x_ratio(const Dom& d, const RatioParams& q, const float2* Sin, float
   if (rows == 0) return;  // no quotient rows: every row is a row of ones, put in by the z pass
   dd.wgPerBlock = (rows + C::RW - 1) / C::RW;
   const int nb = d.btab ? d.nb : 1;
-  hipLaunchKernelGGL(k_x2_ratio<M>, dim3(dd.wgPerBlock * nb), dim3(C::NT), 0, s, dd, q, Sin, Sout, twM, wr);
+  hipLaunchKernelGGL((k_x2_ratio<M, TR>), dim3(dd.wgPerBlock * nb), dim3(C::NT), 0, s, dd, q, Sin, Sout, twM, wr);
 }
-template <int M>
+template <int M, bool TR>
 int launch_x_update(const Dom& d, const UpdateParams& u, const float2* S, const float2* twM, const float2* wr,
                     hipStream_t s) {
   static_assert(x2_ok<M>(), "every compiled x length has a two-step split");
@@ -741,16 +761,16 @@ int launch_x_update(const Dom& d, const UpdateParams& u, const float2* S, const 
   const int rows = d.D[1] * d.D[2];
   dd.wgPerBlock = (rows + C::RW - 1) / C::RW;
   const int nwg = dd.wgPerBlock * (d.btab ? d.nb : 1);
-  hipLaunchKernelGGL(k_x2_update<M>, dim3(nwg), dim3(C::NT), 0, s, dd, u, FastDiv((unsigned)d.D[0]), S, twM, wr);
+  hipLaunchKernelGGL((k_x2_update<M, TR>), dim3(nwg), dim3(C::NT), 0, s, dd, u, FastDiv((unsigned)d.D[0]), S, twM, wr);
   return nwg;
 }
-template <int M>
+template <int M, bool TR>
 void launch_x_store(const Dom& d, const StoreParams& st, const float2* S, const float2* twM, const float2* wr,
                     hipStream_t s) {
   static_assert(x2_ok<M>(), "every compiled x length has a two-step split");
   using C = XCfg<M>;
   const int rows = d.D[1] * d.D[2];
-  hipLaunchKernelGGL(k_x2_store<M>, dim3((rows + C::RW - 1) / C::RW), dim3(C::NT), 0, s, d, st, S, twM, wr);
+  hipLaunchKernelGGL((k_x2_store<M, TR>), dim3((rows + C::RW - 1) / C::RW), dim3(C::NT), 0, s, d, st, S, twM, wr);
 }
 
 }  // namespace mvr
