@@ -9,8 +9,10 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import hashlib
+import math
 import os
 import shutil
+import struct
 import subprocess
 import sys
 
@@ -41,6 +43,8 @@ template void launch_x_ratio<{M}, {T}>(const Dom&, const RatioParams&, const flo
 template int launch_x_update<{M}, {T}>(const Dom&, const UpdateParams&, const float2*, const float2*, const float2*, hipStream_t);
 template void launch_x_store<{M}, {T}>(const Dom&, const StoreParams&, const float2*, const float2*, const float2*, hipStream_t);
 """
+G_FUNCS = """template void launch_x_fwd_groups<{M}>(const Dom&, const XFwdGroup*, int, const float2*, const float2*, hipStream_t);
+"""
 S_FUNCS = """template void launch_strided<{L}>(const StridedGeom&, int, const float2*, float2*, const float2*, float, const float2*, hipStream_t);
 template int strided_span<{L}>();
 """
@@ -51,12 +55,53 @@ def _groups(seq, n):
     return [seq[i:i + k] for i in range(0, len(seq), k)]
 
 
+def _twiddles():
+    """Device tables exp(-2 pi i k / n), k < n, of every compiled length (float roundings of the double values), and the
+    lookup of a table's address on the current device."""
+    lengths = sorted(set(STRIDED) | set(HALF))
+    at, values = {}, []
+    for n in lengths:
+        at[n] = len(values)
+        values += [(math.cos(2 * math.pi * k / n), -math.sin(2 * math.pi * k / n)) for k in range(n)]
+    rows = [", ".join("{(float)%r, (float)%r}" % (_f32(c), _f32(s)) for c, s in values[i:i + 4])
+            for i in range(0, len(values), 4)]
+    body = ",\n".join(rows)
+    cases = " ".join(f"case {n}: at = {at[n]}; break;" for n in lengths)
+    return f"""#include <mutex>
+#include "engine.hpp"
+namespace mvr {{
+// (neither static nor const: no kernel of this file reads it, and the compiler would leave it out)
+__device__ float2 k_twiddles[] = {{
+{body}}};
+const float2* twiddle_table(int n) {{
+  static std::mutex mu;
+  static const float2* base[64] = {{}};
+  int dev = 0, at = -1;
+  switch (n) {{ {cases} default: return nullptr; }}
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+  std::lock_guard<std::mutex> lk(mu);
+  if (!base[dev]) {{
+    void* p = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(k_twiddles)) != hipSuccess) return nullptr;
+    base[dev] = static_cast<const float2*>(p);
+  }}
+  return base[dev] + at;
+}}
+}}  // namespace mvr
+"""
+
+
+def _f32(x):
+    return struct.unpack("f", struct.pack("f", x))[0]
+
+
 def generate():
     os.makedirs(GEN, exist_ok=True)
     files = []
     for gi, grp in enumerate(_groups(HALF, 10)):
         body = "".join(X_FUNCS.format(M=m, T=t) for m in grp for t in ("false", "true")
                        if t == "false" or m <= PLANAR_MAX_M)
+        body += "".join(G_FUNCS.format(M=m) for m in grp if m <= PLANAR_MAX_M)
         files.append((f"x_{gi}.hip", f'#include "xpasses.hpp"\nnamespace mvr {{\n{body}}}\n'))
     for gi, grp in enumerate(_groups(STRIDED, 10)):
         body = "".join(S_FUNCS.format(L=l) for l in grp)
@@ -67,6 +112,7 @@ def generate():
          "template <int M, bool TR> void launch_x_ratio(const Dom&, const RatioParams&, const float2*, float2*, const float2*, const float2*, hipStream_t);",
          "template <int M, bool TR> int launch_x_update(const Dom&, const UpdateParams&, const float2*, const float2*, const float2*, hipStream_t);",
          "template <int M, bool TR> void launch_x_store(const Dom&, const StoreParams&, const float2*, const float2*, const float2*, hipStream_t);",
+         "template <int M> void launch_x_fwd_groups(const Dom&, const XFwdGroup*, int, const float2*, const float2*, hipStream_t);",
          "template <int L> void launch_strided(const StridedGeom&, int, const float2*, float2*, const float2*, float, const float2*, hipStream_t);",
          "template <int L> int strided_span();"]
     for name, fn, typ in [("get_x_fwd", "launch_x_fwd", "XFwdFn"), ("get_x_ratio", "launch_x_ratio", "XRatioFn"),
@@ -75,6 +121,8 @@ def generate():
         planar = " ".join(f"case {m}: return &{fn}<{m}, true>;" for m in HALF if m <= PLANAR_MAX_M)
         d.append(f"{typ} {name}(int M, bool planar) {{ if (planar) switch (M) {{ {planar} default: return nullptr; }} "
                  f"switch (M) {{ {rows} default: return nullptr; }} }}")
+    cases = " ".join(f"case {m}: return &launch_x_fwd_groups<{m}>;" for m in HALF if m <= PLANAR_MAX_M)
+    d.append(f"XFwdGroupsFn get_x_fwd_groups(int M) {{ switch (M) {{ {cases} default: return nullptr; }} }}")
     cases = " ".join(f"case {l}: return &launch_strided<{l}>;" for l in STRIDED)
     d.append(f"StridedFn get_strided(int L) {{ switch (L) {{ {cases} default: return nullptr; }} }}")
     cases = " ".join(f"case {l}: return strided_span<{l}>();" for l in STRIDED)
@@ -85,6 +133,7 @@ def generate():
     d.append("const int* half_lengths() { return kHalf; }")
     d.append("}  // namespace mvr")
     files.append(("dispatch.cpp", "\n".join(d) + "\n"))
+    files.append(("twiddles.hip", _twiddles()))
     paths = []
     for name, text in files:
         p = os.path.join(GEN, name)

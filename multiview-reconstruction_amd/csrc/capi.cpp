@@ -117,7 +117,6 @@ int mvr_fft_convolve(int dev, const float* img, const int n[3], int ext, float e
   for (void* p : {(void*)dImg, (void*)dK, (void*)dOut, (void*)spec, (void*)work})
     if (p) (void)hipFree(p);
   if (s) (void)hipStreamDestroy(s);
-  plan.destroy();
   return rc;
 }
 

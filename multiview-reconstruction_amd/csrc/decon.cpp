@@ -334,7 +334,6 @@ int Decon::init(int psiInit, const float* psiIn) {
 // Plan for the whole volume (FFT lengths >= Pmin where given), kernel spectra of the first nviews views,
 // work spectra.
 int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
-  plan.destroy();
   int nS = 1;  // work spectra: one per block of the largest view list
   if (blocked()) {
     // a block's domain holds its output region plus both kernels' reach on either side, so that both chained
@@ -462,7 +461,6 @@ int Decon::autotune(int candidates, int chosen[3], double* msOut) {
     rc = -1;
   }
   if (!rc) {
-    plan.destroy();
     if (plan.create(N, K, nullptr)) rc = -1;
   }
   if (!rc) {
@@ -839,7 +837,6 @@ void Decon::destroy() {
   img.clear(); w.clear(); spec1.clear(); spec2.clear();
   psi = psi0 = nullptr; S = Spsi = nullptr; T2 = nullptr; partial = nullptr; statsDev = nullptr;
   ref = nullptr; relDev = nullptr;
-  plan.destroy();
   timer.release();
   if (stream) (void)hipStreamDestroy(stream);
   stream = nullptr;
@@ -1110,7 +1107,6 @@ void BlockThread::destroy() {
     if (p) (void)hipFree(p);
   spec1.clear(); spec2.clear(); imgV.clear(); wV.clear(); viewImg.clear(); viewW.clear();
   psiB = imgB = wB = T2 = nullptr; S = Spsi = nullptr; partial = nullptr; statDev = nullptr;
-  plan.destroy();
   if (stream) (void)hipStreamDestroy(stream);
   stream = nullptr;
 }

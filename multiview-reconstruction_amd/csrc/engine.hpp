@@ -46,9 +46,18 @@ struct GatherParams {
   int org[3];
   int mode;
   float value;
-  // MIRROR only: transform only the rows (y, z) that are not mirror copies, FFT positions [-org, -org + N)
-  // per axis (the passes after it read the copies from their sources)
+  // transform only the rows (y, z) that hold source values, FFT positions [-org, -org + N) per axis (KERNEL: the
+  // kernel's rows); the passes after it read mirror copies from their sources and put constant rows in
   int uniqueRows;
+};
+
+// One group of forward x transforms with planar spectra: n sources, srcStride values apart, into spectra dstStride
+// complex values apart.
+struct XFwdGroup {
+  GatherParams g;
+  float2* S;
+  int n;
+  size_t srcStride, dstStride;
 };
 
 // Inverse-transform epilogues.  `o` is the volume coordinate of the output
@@ -83,10 +92,14 @@ struct UpdateParams {
 
 struct StoreParams {
   float* out;        // compact D[0]*D[1]*D[2] array
+  int n = 1;         // planar spectra: n of them, Dom::blockStride apart, into arrays of D[0]*D[1]*D[2] back to back
 };
 
 typedef void (*XFwdFn)(const Dom&, const GatherParams&, float2* S, const float2* twM, const float2* wr,
                        hipStream_t s);
+// ngroups <= 2 groups in one launch (planar spectra)
+typedef void (*XFwdGroupsFn)(const Dom&, const XFwdGroup* groups, int ngroups, const float2* twM, const float2* wr,
+                             hipStream_t s);
 typedef void (*XRatioFn)(const Dom&, const RatioParams&, const float2* Sin, float2* Sout, const float2* twM,
                          const float2* wr, hipStream_t s);
 typedef int (*XUpdateFn)(const Dom&, const UpdateParams&, const float2* S, const float2* twM, const float2* wr,
@@ -109,15 +122,19 @@ struct StridedGeom {
   int plane0 = 0;
   int storeLo = 0, storeHi = 1 << 30;
   // Forward mode over data whose rows outside planes [onesPlaneLo, onesPlaneHi) x positions [onesLo, onesHi) are
-  // spectra of rows (or planes) of ones, never written: the pass reads none of them and uses onesDC at column 0,
-  // 0 at the other columns; with onesDCPlane >= 0 onesDC is on that plane only, 0 on the others.  Off when onesDC
-  // is 0.
+  // spectra of constant rows (or planes), never written: the pass reads none of them and uses onesDC at column 0,
+  // 0 at the other columns; with onesDCPlane >= 0 onesDC is on that plane only, 0 on the others.  Off unless ones.
+  bool ones = false;
   float onesDC = 0.f;
   int onesPlaneLo = 0, onesPlaneHi = 0, onesLo = 0, onesHi = 0, onesDCPlane = -1;
   // Forward modes over data that is a mirror extension along the pencil (mirN > 0): position n holds what
   // position mirM + mirror(n - mirM, mirN) holds, and only those positions were written; the loads read them
   // (byte offsets from the plane up to L lineStride 8 must fit 32 bits).
   int mirM = 0, mirN = 0;
+  // Forward modes 0 and 3 over a kernel placed around the origin (wrapN > 0): only the positions n with (n + wrapN / 2)
+  // mod L < wrapN were written, the others are zero and not read.  planeMod > 0: planes are counted from plane0 modulo
+  // planeMod.
+  int wrapN = 0, planeMod = 0;
   // timing: when set, the launch records the kernel's own start and stop in these events
   hipEvent_t evStart = nullptr, evStop = nullptr;
 };
@@ -127,7 +144,8 @@ typedef void (*StridedFn)(const StridedGeom&, int mode, const float2* in, float2
                           float scale, const float2* tw, hipStream_t s);
 
 // One pass of y and z transforms over planar spectra [hx][z][y] (plane.hip), in place or not: forward, times spec
-// ([hx][y slot][z slot]), inverse; spec null: forward and scale, stored in slot order.
+// ([hx][y slot][z slot]), inverse.  With a kernel (kin) its x transform is first turned into that spectrum, scaled, in
+// specOut (which may be kin), to be used as spec or, without data (in null), on its own.
 struct PlaneGeom {
   int Py, Pz;          // at most kPlaneMax each
   int ncols;           // planes (hx)
@@ -135,8 +153,14 @@ struct PlaneGeom {
   size_t inStride = 0, outStride = 0, specStride = 0;   // (null: the shared spectrum), writes out + b outStride
   const int* inIdx = nullptr;
   const int* specIdx = nullptr;
+  const float2* kin = nullptr;             // entry b: kin + b kStride, specOut + b kStride
+  float2* specOut = nullptr;
+  size_t kStride = 0;
+  float kScale = 1.f;
+  int kK[2] = {0, 0};                      // kernel sizes along y, z: only its rows were written (StridedGeom's wrapN)
   int mir[2] = {0, 0}, mirN[2] = {0, 0};   // mirror extension along y, z (StridedGeom's mirM, mirN), off at 0
-  float onesDC = 0.f;                      // rows outside [onesLo, onesHi) (y, z) are spectra of ones, as in StridedGeom
+  bool ones = false;                       // rows outside [onesLo, onesHi) (y, z) are constant, as in StridedGeom
+  float onesDC = 0.f;
   int onesLo[2] = {0, 0}, onesHi[2] = {0, 0};
   const int* onesTab = nullptr;            // per batch entry {yLo, yHi, zLo, zHi} instead
   int lo[2] = {0, 0}, hi[2] = {1 << 30, 1 << 30};  // rows (y, z) stored
@@ -144,11 +168,12 @@ struct PlaneGeom {
 };
 constexpr int kPlaneMax = 128;     // y and z lengths
 constexpr int kPlanarMaxM = 128;   // x passes with planar spectra are compiled for half lengths up to this
-void launch_plane(const PlaneGeom& g, const float2* in, float2* out, const float2* spec, float scale,
-                  const float2* twY, const float2* twZ, hipStream_t s);
+void launch_plane(const PlaneGeom& g, const float2* in, float2* out, const float2* spec, const float2* twY,
+                   const float2* twZ, hipStream_t s);
 
 // planar: spectra [hx][z][y] instead of rows [z][y][hx]
 XFwdFn get_x_fwd(int M, bool planar);
+XFwdGroupsFn get_x_fwd_groups(int M);
 XRatioFn get_x_ratio(int M, bool planar);
 XUpdateFn get_x_update(int M, bool planar);
 XStoreFn get_x_store(int M, bool planar);
@@ -158,6 +183,9 @@ int get_strided_span(int L);
 // lengths with compiled kernels, ascending; terminated by 0
 const int* strided_lengths();
 const int* half_lengths();
+// exp(-2 pi i k / n), k < n, for every length of the two lists, in the current device's memory (null: no such length, or
+// the device failed)
+const float2* twiddle_table(int n);
 
 // misc kernels (misc.hip)
 void launch_fill(float* dst, size_t n, float v, hipStream_t s);

@@ -32,11 +32,12 @@ struct Plan {
   int K[3] = {0, 0, 0};
   int M = 0, Hx = 0;
   bool planar = false;    // spectra [hx][z][y], y and z transforms in one plane pass
-  float2* twM = nullptr;  // length-M twiddles (x)
-  float2* wr = nullptr;   // exp(-2 pi i k / P0), k = 0..M
-  float2* twY = nullptr;
-  float2* twZ = nullptr;
+  const float2* twM = nullptr;  // length-M twiddles (x); the tables are the library's (twiddle_table)
+  const float2* wr = nullptr;   // exp(-2 pi i k / P0), k = 0..M
+  const float2* twY = nullptr;
+  const float2* twZ = nullptr;
   XFwdFn xf = nullptr;
+  XFwdGroupsFn xfg = nullptr;  // planar plans
   XRatioFn xr = nullptr;
   XUpdateFn xu = nullptr;
   XStoreFn xs = nullptr;
@@ -45,10 +46,8 @@ struct Plan {
 
   // chooses the FFT lengths; P[d] >= D[d] + K[d] - 1 (or the given minimum per axis)
   int create(const int D[3], const int K[3], const int* Pmin = nullptr);
-  // the same geometry and kernel choice without device memory (twiddle pointers stay null): for callers that
-  // place the twiddle tables themselves
+  // the same geometry and kernel choice without a device (twiddle pointers stay null)
   int create_geometry(const int D[3], const int K[3], const int* Pmin = nullptr);
-  void destroy();
   size_t ncpx() const { return (size_t)dom.HxP * dom.P[1] * dom.P[2]; }
   size_t rows_inner() const { return (size_t)dom.D[1] * dom.D[2]; }
   // The passes between the x passes of a convolution: forward z, y with the spectrum product, inverse z; on planar
@@ -64,6 +63,9 @@ struct Plan {
   // the grid).  The y pass then stores only those y, and the inverse z pass transforms only those y planes and
   // stores only those z.
   void restrict_rows(const int lo[3], const int hi[3], Mid& m) const;
+  // The gather of a constant extension (g.mode VALUE): sets g.uniqueRows, so that x_fwd transforms only the rows inside
+  // the source; the passes after it put the constant rows and planes in.
+  void value_rows(GatherParams& g, Mid& m) const;
   // For a convolution of the quotient: sets q.skipOnes and the quotient rows q.rowLo / rowN; the rows outside the
   // quotient region are rows of ones, which the quotient pass does not write and the forward z pass puts in.  That
   // pass also leaves out the y planes outside the quotient region, planes of ones whose spectrum, P0 P2 at x and z
@@ -82,8 +84,18 @@ struct Plan {
                 Timer* t = nullptr) const;
   float inv_scale() const { return 2.0f / ((float)dom.P[0] * (float)dom.P[1] * (float)dom.P[2]); }
 
+  // rows (y, z) outside [lo, hi) (indices 1, 2) are constant rows of `value`
+  void constant_rows(const int lo[3], const int hi[3], float value, Mid& m) const;
+
   // spectrum of a device kernel (K layout), scaled by the inverse-FFT factor
   int kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const;
+  // the gather of a kernel
+  GatherParams kernel_gather(const float* dKernel) const;
+  // one convolution with a kernel used once: kernel_spectrum and convolve, on planar plans in three launches
+  int convolve_once(const float* dKernel, const GatherParams& g, float2* spec, float2* work, float* out,
+                    hipStream_t s) const;
+  // the gather and geometry of one whole convolution of g, whose rows outside the output region are not stored
+  Mid convolve_geometry(GatherParams& g) const;
   // out (compact D) = K (*) ext(src) with src a volume of dims N; org = volume coord of FFT position 0
   int convolve(const GatherParams& g, const float2* spec, float2* work, float* out, hipStream_t s) const;
 };

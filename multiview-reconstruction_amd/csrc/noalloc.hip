@@ -39,20 +39,6 @@ int scratch_address(int dev, unsigned char** out) {
   return 0;
 }
 
-// exp(-2 pi i k / period), k < n (the same table Plan::create uploads from the host)
-__global__ void k_twiddles(float2* __restrict__ out, int n, int period) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) {
-    double s, c;
-    sincospi(-2.0 * (double)k / (double)period, &s, &c);
-    out[k] = make_float2((float)c, (float)s);
-  }
-}
-
-void launch_twiddles(float2* out, int n, int period, hipStream_t s) {
-  hipLaunchKernelGGL(k_twiddles, dim3((n + 255) / 256), dim3(256), 0, s, out, n, period);
-}
-
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 }  // namespace
@@ -68,9 +54,11 @@ extern "C" int mvr_fft_convolve_noalloc(int dev, const float* img, const int n[3
   // geometry and the scratch layout first, on the host: sizes beyond the array are refused before device work
   Plan plan;
   if (plan.create_geometry(n, k)) return -1;
-  const size_t oWr = align256((size_t)plan.M * 8), oTwY = oWr + align256((size_t)(plan.M + 1) * 8);
-  const size_t oTwZ = oTwY + align256((size_t)plan.dom.P[1] * 8), oSpec = oTwZ + align256((size_t)plan.dom.P[2] * 8);
-  const size_t oWork = oSpec + align256(plan.ncpx() * 8), total = oWork + align256(plan.ncpx() * 8);
+  // (the limit counts the transforms' four twiddle tables with the two spectra)
+  const size_t oWork = align256(plan.ncpx() * 8);
+  const size_t tables = align256((size_t)plan.M * 8) + align256((size_t)(plan.M + 1) * 8) +
+                        align256((size_t)plan.dom.P[1] * 8) + align256((size_t)plan.dom.P[2] * 8);
+  const size_t total = tables + 2 * oWork;
   if (total > (size_t)MVR_NOALLOC_SCRATCH_BYTES) {
     set_error("mvr_fft_convolve_noalloc: the FFT grid " + std::to_string(plan.dom.P[0]) + "x" +
               std::to_string(plan.dom.P[1]) + "x" + std::to_string(plan.dom.P[2]) + " needs " +
@@ -86,26 +74,13 @@ extern "C" int mvr_fft_convolve_noalloc(int dev, const float* img, const int n[3
   unsigned char* base = nullptr;
   if (scratch_address(dev, &base)) return -1;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  plan.twM = reinterpret_cast<float2*>(base);
-  plan.wr = reinterpret_cast<float2*>(base + oWr);
-  plan.twY = reinterpret_cast<float2*>(base + oTwY);
-  plan.twZ = reinterpret_cast<float2*>(base + oTwZ);
-  float2* spec = reinterpret_cast<float2*>(base + oSpec);
+  if (plan.create(n, k)) return -1;  // finds the twiddle tables, static too
+  float2* spec = reinterpret_cast<float2*>(base);
   float2* work = reinterpret_cast<float2*>(base + oWork);
-  launch_twiddles(plan.twM, plan.M, plan.M, s);
-  launch_twiddles(plan.wr, plan.M + 1, plan.dom.P[0], s);
-  launch_twiddles(plan.twY, plan.dom.P[1], plan.dom.P[1], s);
-  launch_twiddles(plan.twZ, plan.dom.P[2], plan.dom.P[2], s);
-  int rc = plan.kernel_spectrum(kernel, spec, s);
-  if (!rc) {
-    GatherParams g{};
-    g.src = img;
-    for (int d = 0; d < 3; ++d) { g.N[d] = n[d]; g.org[d] = -plan.dom.m[d]; }
-    g.mode = ext == MVR_EXT_MIRROR_SINGLE ? GATHER_MIRROR : GATHER_VALUE;
-    g.value = extValue;
-    rc = plan.convolve(g, spec, work, out, s);
-  }
-  // the tables belong to the scratch array: the plan must not free them
-  plan.twM = plan.wr = plan.twY = plan.twZ = nullptr;
-  return rc;
+  GatherParams g{};
+  g.src = img;
+  for (int d = 0; d < 3; ++d) { g.N[d] = n[d]; g.org[d] = -plan.dom.m[d]; }
+  g.mode = ext == MVR_EXT_MIRROR_SINGLE ? GATHER_MIRROR : GATHER_VALUE;
+  g.value = extValue;
+  return plan.convolve_once(kernel, g, spec, work, out, s);
 }

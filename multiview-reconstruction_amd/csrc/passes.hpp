@@ -290,6 +290,7 @@ __global__ __launch_bounds__(W * split2(L).A, (s2_min_waves<L, W, MODE>())) void
     blockOff = (size_t)b * gm.blockStride;
   }
   plane += gm.plane0;
+  if (MODE == 0 && gm.planeMod > 0 && plane >= gm.planeMod) plane -= gm.planeMod;
   // Lanes of columns beyond ncols (the last tile) read the row pitch's padding (pitch = 16-column multiple) and
   // compute values that are never stored.
   const size_t ls = gm.lineStride;
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(W * split2(L).A, (s2_min_waves<L, W, MODE>())) void
   if constexpr (MODE != 1) {
     // ---- forward step 1: thread q = b < B
     if (q < B) {
-      if (gm.onesDC != 0.f) {
+      if (gm.ones) {
         // rows of ones outside the written region: their spectrum is known and not read
         const bool planeIn = plane >= gm.onesPlaneLo && plane < gm.onesPlaneHi;
         const bool dc = col0 + w == 0 && (gm.onesDCPlane < 0 || plane == gm.onesDCPlane);
@@ -331,6 +332,14 @@ __global__ __launch_bounds__(W * split2(L).A, (s2_min_waves<L, W, MODE>())) void
             const int n = mirror_index(q + B * a - gm.mirM, gm.mirN);
             v[a] = s2_ld(sb, w8 + (unsigned)(gm.mirM + n) * ls8);
           }
+        }
+      } else if ((MODE == 0 || MODE == 3) && gm.wrapN > 0) {
+        // a kernel around the origin: zeros beyond its rows
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+          int n = q + B * a + gm.wrapN / 2;
+          n -= n >= L ? L : 0;
+          v[a] = n < gm.wrapN ? s2_ld(sb + (size_t)(B * a) * ls, lo) : make_float2(0.f, 0.f);
         }
       } else {
 #pragma unroll

@@ -34,22 +34,13 @@ static int pick_length(int need, bool half) {
   return -1;
 }
 
-static int upload_twiddles(float2** dst, int n, int period) {
-  std::vector<float2> h(n);
-  for (int k = 0; k < n; ++k) {
-    const double a = -2.0 * M_PI * (double)k / (double)period;
-    h[k] = make_float2((float)std::cos(a), (float)std::sin(a));
-  }
-  MVR_HIP(hipMalloc(dst, sizeof(float2) * n));
-  MVR_HIP(hipMemcpy(*dst, h.data(), sizeof(float2) * n, hipMemcpyHostToDevice));
-  return 0;
-}
-
 int Plan::create(const int D[3], const int Kd[3], const int* Pmin) {
   if (create_geometry(D, Kd, Pmin)) return -1;
-  if (upload_twiddles(&twM, M, M) || upload_twiddles(&wr, M + 1, dom.P[0]) || upload_twiddles(&twY, dom.P[1], dom.P[1]) ||
-      upload_twiddles(&twZ, dom.P[2], dom.P[2]))
-    return -1;
+  twM = twiddle_table(M);
+  wr = twiddle_table(dom.P[0]);
+  twY = twiddle_table(dom.P[1]);
+  twZ = twiddle_table(dom.P[2]);
+  if (!twM || !wr || !twY || !twZ) { set_error("plan: twiddle tables not found on the device"); return -1; }
   return 0;
 }
 
@@ -70,6 +61,7 @@ int Plan::create_geometry(const int D[3], const int Kd[3], const int* Pmin) {
   dom.HxP = (Hx + 15) / 16 * 16;
   planar = dom.P[1] <= kPlaneMax && dom.P[2] <= kPlaneMax && M <= kPlanarMaxM;
   xf = get_x_fwd(M, planar);
+  xfg = planar ? get_x_fwd_groups(M) : nullptr;
   xr = get_x_ratio(M, planar);
   xu = get_x_update(M, planar);
   xs = get_x_store(M, planar);
@@ -83,11 +75,6 @@ int Plan::create_geometry(const int D[3], const int Kd[3], const int* Pmin) {
     return -1;
   }
   return 0;
-}
-
-void Plan::destroy() {
-  for (float2** p : {&twM, &wr, &twY, &twZ})
-    if (*p) { (void)hipFree(*p); *p = nullptr; }
 }
 
 Plan::Mid Plan::mid() const {
@@ -144,6 +131,7 @@ void Plan::skip_ones_rows(RatioParams& q, Mid& m, const int* blockRows) const {
   if (blockRows) {
     q.skipOnes = 1;
     for (int k = 1; k < 3; ++k) q.rowN[k] = std::min(dom.P[k], dom.D[k] + q.qlo[k] + q.qhi[k]);
+    m.pl.ones = true;
     m.pl.onesDC = (float)dom.P[0];
     m.pl.onesTab = blockRows;
     return;
@@ -158,22 +146,35 @@ void Plan::skip_ones_rows(RatioParams& q, Mid& m, const int* blockRows) const {
   for (int k = 1; k < 3; ++k) {
     q.rowLo[k] = lo[k];
     q.rowN[k] = std::max(0, hi[k] - lo[k]);
+  }
+  constant_rows(lo, hi, 1.f, m);
+}
+
+void Plan::constant_rows(const int lo[3], const int hi[3], float value, Mid& m) const {
+  for (int k = 1; k < 3; ++k) {
     m.pl.onesLo[k - 1] = lo[k];
     m.pl.onesHi[k - 1] = hi[k];
   }
-  m.pl.onesDC = m.zf.onesDC = (float)dom.P[0];  // the x transform of a row of ones
+  m.pl.ones = m.zf.ones = m.y.ones = true;
+  m.pl.onesDC = m.zf.onesDC = value * (float)dom.P[0];  // the x transform of a constant row
   m.zf.onesPlaneLo = lo[1];
   m.zf.onesPlaneHi = hi[1];
   m.zf.onesLo = lo[2];
   m.zf.onesHi = hi[2];
   m.zf.plane0 = lo[1];
   m.zf.nplanes = std::max(0, hi[1] - lo[1]);
-  m.y.onesDC = (float)dom.P[0] * (float)dom.P[2];  // the xz transform of a plane of ones
+  m.y.onesDC = value * (float)dom.P[0] * (float)dom.P[2];  // the xz transform of a constant plane
   m.y.onesDCPlane = 0;
   m.y.onesPlaneLo = 0;
   m.y.onesPlaneHi = dom.P[2];
   m.y.onesLo = lo[1];
   m.y.onesHi = hi[1];
+}
+
+void Plan::value_rows(GatherParams& g, Mid& m) const {
+  g.uniqueRows = 1;
+  const int lo[3] = {0, -g.org[1], -g.org[2]}, hi[3] = {0, g.N[1] - g.org[1], g.N[2] - g.org[2]};
+  constant_rows(lo, hi, g.value, m);
 }
 
 void Plan::mirror_rows(GatherParams& g, Mid& m) const {
@@ -217,23 +218,37 @@ void Plan::mid_rest(const Mid& m, const float2* in, float2* out, const float2* s
       t->kernel(passes, t->zForward ? 3 : 2, &g.evStart, &g.evStop);
       t->zForward = false;
     }
-    launch_plane(g, in, out, spec, 1.f, twY, twZ, s);
+    launch_plane(g, in, out, spec, twY, twZ, s);
     return;
   }
   sy(timed(t, m.y, PASS_Y_CONV), 2, in, out, spec, 1.f, twY, s);
   sz(timed(t, m.zi, PASS_Z_INV), 1, out, out, nullptr, 1.f, twZ, s);
 }
 
-int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const {
+GatherParams Plan::kernel_gather(const float* dKernel) const {
   GatherParams g{};
   g.src = dKernel;
   for (int d = 0; d < 3; ++d) { g.N[d] = K[d]; g.org[d] = 0; }
   g.mode = GATHER_KERNEL;
-  xf(dom, g, spec, twM, wr, s);
-  const Mid m = mid();
+  g.uniqueRows = 1;  // the passes after it take zeros for the other rows
+  return g;
+}
+
+int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const {
+  xf(dom, kernel_gather(dKernel), spec, twM, wr, s);
+  Mid m = mid();
   if (planar) {
-    launch_plane(m.pl, spec, spec, nullptr, inv_scale(), twY, twZ, s);
+    m.pl.kin = m.pl.specOut = spec;
+    m.pl.kScale = inv_scale();
+    m.pl.kK[0] = K[1];
+    m.pl.kK[1] = K[2];
+    launch_plane(m.pl, nullptr, nullptr, nullptr, twY, twZ, s);
   } else {
+    m.y.plane0 = dom.P[2] - K[2] / 2;  // the kernel's z planes, around 0
+    m.y.planeMod = dom.P[2];
+    m.y.nplanes = K[2];
+    m.y.wrapN = K[1];
+    m.zf.wrapN = K[2];
     sy(m.y, 0, spec, spec, nullptr, 1.f, twY, s);
     sz(m.zf, 3, spec, spec, nullptr, inv_scale(), twZ, s);
   }
@@ -241,16 +256,42 @@ int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) con
   return 0;
 }
 
-int Plan::convolve(const GatherParams& g, const float2* spec, float2* work, float* out, hipStream_t s) const {
+Plan::Mid Plan::convolve_geometry(GatherParams& g) const {
   // the store reads the output rows only
   const int zero[3] = {0, 0, 0};
   Mid m = mid();
   restrict_rows(zero, zero, m);
+  if (g.mode == GATHER_MIRROR)
+    mirror_rows(g, m);
+  else if (g.mode == GATHER_VALUE)
+    value_rows(g, m);
+  return m;
+}
+
+int Plan::convolve(const GatherParams& g, const float2* spec, float2* work, float* out, hipStream_t s) const {
   GatherParams gg = g;
-  if (g.mode == GATHER_MIRROR) mirror_rows(gg, m);
+  const Mid m = convolve_geometry(gg);
   xf(dom, gg, work, twM, wr, s);
   mid_forward(m, work, s);
   mid_rest(m, work, work, spec, s);
+  StoreParams st{out};
+  xs(dom, st, work, twM, wr, s);
+  MVR_HIP(hipGetLastError());
+  return 0;
+}
+
+int Plan::convolve_once(const float* dKernel, const GatherParams& g, float2* spec, float2* work, float* out,
+                        hipStream_t s) const {
+  if (!planar) return kernel_spectrum(dKernel, spec, s) || convolve(g, spec, work, out, s) ? -1 : 0;
+  GatherParams gg = g;
+  Mid m = convolve_geometry(gg);
+  const XFwdGroup groups[2] = {{kernel_gather(dKernel), spec, 1, 0, 0}, {gg, work, 1, 0, 0}};
+  xfg(dom, groups, 2, twM, wr, s);
+  m.pl.kin = m.pl.specOut = spec;
+  m.pl.kScale = inv_scale();
+  m.pl.kK[0] = K[1];
+  m.pl.kK[1] = K[2];
+  launch_plane(m.pl, work, work, nullptr, twY, twZ, s);
   StoreParams st{out};
   xs(dom, st, work, twM, wr, s);
   MVR_HIP(hipGetLastError());

@@ -112,7 +112,6 @@ static int conv_same(const std::vector<float>& input, const std::vector<float>& 
   } while (0);
   for (void* p : {(void*)dIn, (void*)dK, (void*)dOut, (void*)spec, (void*)work})
     if (p) (void)hipFree(p);
-  plan.destroy();
   return rc;
 }
 

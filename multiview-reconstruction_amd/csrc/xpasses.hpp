@@ -285,10 +285,10 @@ __device__ __forceinline__ void x2_park_inverse(float2* rb, int q, const float2*
 }
 
 // ------------------------------------------------------------------ forward with gather
+// work-group `wg` of the transform of one source into one spectrum
 template <int M, bool TR>
-__global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, float2* __restrict__ S,
-                                                         const float2* __restrict__ twM,
-                                                         const float2* __restrict__ wr) {
+__device__ __forceinline__ void x2_fwd_body(const Dom& d, const GatherParams& g, float2* __restrict__ S,
+                                            const float2* __restrict__ twM, const float2* __restrict__ wr, int wg) {
   using C = XCfg<M>;
   __shared__ float2 buf[C::BUF_FWD];
   __shared__ float2 twS[C::TWL_FWD ? M : 1];
@@ -301,7 +301,6 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, f
   if (C::TWL_FWD) x2_load_twiddles<M>(twS, twrS, twM, wr);
   const int nrows = d.P[1] * d.P[2];
   // batched blocks: this work-group's block, its gather origin (output region origin - m) and spectrum
-  int wg = blockIdx.x;
   int org[3] = {g.org[0], g.org[1], g.org[2]};
   if (d.btab) {
     const int b = blockIdx.x / d.wgPerBlock;
@@ -313,8 +312,8 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, f
   const int row0 = wg * C::RW;
   const int r = threadIdx.x / C::T, q = threadIdx.x % C::T;
   float2* rb = buf + r * C::RS_FWD;
-  // unique rows only (mirror gather): row index -> grid row (-org1 + i % N1, -org2 + i / N1)
-  const bool uniq = g.uniqueRows && g.mode == GATHER_MIRROR;
+  // rows with source values only: row index -> grid row (-org1 + i % N1, -org2 + i / N1), the kernel's rows around 0
+  const bool uniq = g.uniqueRows;
   const int nrowsRun = uniq ? g.N[1] * g.N[2] : nrows;
   // source index of FFT position x of a row: row start (srcRow, -1: no source row) + xmap[x] (-1: outside),
   // else g.value.  Mirror: the volume mirrored at its faces; value: the volume, `value` outside; kernel
@@ -336,7 +335,12 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, f
     int row = row0 + threadIdx.x;
     long long off = -1;
     const bool live = row < nrowsRun;
-    if (uniq && live) row = (-org[2] + row / g.N[1]) * d.P[1] + (-org[1] + row % g.N[1]);
+    if (uniq && live) {
+      int y = row % g.N[1], zz = row / g.N[1];
+      y += kern ? (y < g.N[1] / 2 ? d.P[1] : 0) - g.N[1] / 2 : -org[1];
+      zz += kern ? (zz < g.N[2] / 2 ? d.P[2] : 0) - g.N[2] / 2 : -org[2];
+      row = zz * d.P[1] + y;
+    }
     if (live) {
       const int y = row % d.P[1], zz = row / d.P[1];
       if (kern) {
@@ -379,6 +383,28 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, f
   x2_forward_regs_half<M>(rb, tw, q, v, z);
   const size_t o = dstRow[r];
   x2_post_store_regs<M, TR>(z, q, twr, S + (o == kNoRow ? 0 : o), o != kNoRow, (unsigned)(d.P[1] * d.P[2]));
+}
+
+template <int M, bool TR>
+__global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd(Dom d, GatherParams g, float2* __restrict__ S,
+                                                         const float2* __restrict__ twM,
+                                                         const float2* __restrict__ wr) {
+  x2_fwd_body<M, TR>(d, g, S, twM, wr, blockIdx.x);
+}
+
+// two groups of sources (n1 work-groups for the first), wgEntry work-groups per source of a group
+template <int M>
+__global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd_groups(Dom d, XFwdGroup g1, XFwdGroup g2, unsigned n1,
+                                                                unsigned wgEntry1, unsigned wgEntry2,
+                                                                const float2* __restrict__ twM,
+                                                                const float2* __restrict__ wr) {
+  const bool second = blockIdx.x >= n1;
+  const XFwdGroup& u = second ? g2 : g1;
+  const unsigned id = second ? blockIdx.x - n1 : blockIdx.x, per = second ? wgEntry2 : wgEntry1;
+  const unsigned b = id / per;
+  GatherParams g = u.g;
+  g.src += b * u.srcStride;
+  x2_fwd_body<M, true>(d, g, u.S + b * u.dstStride, twM, wr, (int)(id - b * per));
 }
 
 // ------------------------------------------------------------------ inverse, quotient, forward
@@ -697,7 +723,14 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_store(Dom d, StoreParams st,
   __shared__ size_t rowOff[C::RW];
   if (C::TWL) x2_load_twiddles<M>(twS, twrS, twM, wr);
   const int nrows = d.D[1] * d.D[2];
-  const int row0 = blockIdx.x * C::RW;
+  unsigned wg = blockIdx.x;
+  if (TR && st.n > 1) {  // this work-group's spectrum and output array
+    const unsigned b = wg / d.wgPerBlock;
+    wg -= b * d.wgPerBlock;
+    S += b * d.blockStride;
+    st.out += (size_t)b * d.D[0] * nrows;
+  }
+  const int row0 = wg * C::RW;
   if (threadIdx.x < C::RW) {
     const int row = row0 + threadIdx.x;
     size_t so = kNoRow;
@@ -735,10 +768,22 @@ void launch_x_fwd(const Dom& d, const GatherParams& g, float2* S, const float2* 
   static_assert(x2_ok<M>(), "every compiled x length has a two-step split");
   using C = XCfg<M>;
   Dom dd = d;
-  const int rows = g.uniqueRows && g.mode == GATHER_MIRROR ? g.N[1] * g.N[2] : d.P[1] * d.P[2];
+  const int rows = g.uniqueRows ? g.N[1] * g.N[2] : d.P[1] * d.P[2];
   dd.wgPerBlock = (rows + C::RW - 1) / C::RW;
   const int nb = d.btab ? d.nb : 1;
   hipLaunchKernelGGL((k_x2_fwd<M, TR>), dim3(dd.wgPerBlock * nb), dim3(C::NT), 0, s, dd, g, S, twM, wr);
+}
+template <int M>
+void launch_x_fwd_groups(const Dom& d, const XFwdGroup* u, int n, const float2* twM, const float2* wr, hipStream_t s) {
+  using C = XCfg<M>;
+  unsigned per[2] = {1, 1}, wgs[2] = {0, 0};
+  for (int i = 0; i < n; ++i) {
+    const int rows = u[i].g.uniqueRows ? u[i].g.N[1] * u[i].g.N[2] : d.P[1] * d.P[2];
+    per[i] = (unsigned)((rows + C::RW - 1) / C::RW);
+    wgs[i] = per[i] * (unsigned)u[i].n;
+  }
+  hipLaunchKernelGGL(k_x2_fwd_groups<M>, dim3(wgs[0] + wgs[1]), dim3(C::NT), 0, s, d, u[0], u[n - 1], wgs[0], per[0],
+                     per[1], twM, wr);
 }
 template <int M, bool TR>
 void launch_x_ratio(const Dom& d, const RatioParams& q, const float2* Sin, float2* Sout, const float2* twM,
@@ -769,8 +814,10 @@ void launch_x_store(const Dom& d, const StoreParams& st, const float2* S, const 
                     hipStream_t s) {
   static_assert(x2_ok<M>(), "every compiled x length has a two-step split");
   using C = XCfg<M>;
+  Dom dd = d;
   const int rows = d.D[1] * d.D[2];
-  hipLaunchKernelGGL((k_x2_store<M, TR>), dim3((rows + C::RW - 1) / C::RW), dim3(C::NT), 0, s, d, st, S, twM, wr);
+  dd.wgPerBlock = (rows + C::RW - 1) / C::RW;
+  hipLaunchKernelGGL((k_x2_store<M, TR>), dim3(dd.wgPerBlock * st.n), dim3(C::NT), 0, s, dd, st, S, twM, wr);
 }
 
 }  // namespace mvr
