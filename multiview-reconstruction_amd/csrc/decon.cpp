@@ -356,25 +356,44 @@ int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
   }
   plan.wy = tunedW[0];
   plan.wz = tunedW[1];
-  for (auto p : spec1) if (p) (void)hipFree(p);
-  for (auto p : spec2) if (p) (void)hipFree(p);
-  spec1.assign(V, nullptr);
-  spec2.assign(V, nullptr);
-  const size_t nk = (size_t)K[0] * K[1] * K[2];
-  float* dk = nullptr;
-  MVR_HIP(hipMalloc(&dk, nk * 4));
-  for (int v = 0; v < nviews; ++v) {
-    MVR_HIP(hipMalloc(&spec1[v], plan.ncpx() * 8));
-    MVR_HIP(hipMalloc(&spec2[v], plan.ncpx() * 8));
-    MVR_HIP(hipMemcpyAsync(dk, k1[v].data(), nk * 4, hipMemcpyHostToDevice, stream));
-    if (plan.kernel_spectrum(dk, spec1[v], stream)) return -1;
-    MVR_HIP(hipMemcpyAsync(dk, k2[v].data(), nk * 4, hipMemcpyHostToDevice, stream));
-    if (plan.kernel_spectrum(dk, spec2[v], stream)) return -1;
-    MVR_HIP(hipStreamSynchronize(stream));
+  // buffers of another size, or of views this call leaves out, go first
+  const size_t specN = plan.ncpx();
+  for (auto* specs : {&spec1, &spec2}) {
+    for (size_t v = 0; v < specs->size(); ++v)
+      if ((*specs)[v] && (specN != specLen || (int)v >= nviews)) {
+        (void)hipFree((*specs)[v]);
+        (*specs)[v] = nullptr;
+      }
+    specs->resize(V, nullptr);
   }
+  specLen = specN;
+  if (S && specN * nS != workLen) {
+    (void)hipFree(S);
+    S = nullptr;
+  }
+  const size_t nk = (size_t)K[0] * K[1] * K[2];
+  std::vector<float> hk(2 * nviews * nk);
+  for (int v = 0; v < nviews; ++v) {
+    std::copy(k1[v].begin(), k1[v].end(), hk.begin() + 2 * v * nk);
+    std::copy(k2[v].begin(), k2[v].end(), hk.begin() + (2 * v + 1) * nk);
+  }
+  float* dk = nullptr;
+  MVR_HIP(hipMalloc(&dk, hk.size() * 4));
+  int rc = hipMemcpyAsync(dk, hk.data(), hk.size() * 4, hipMemcpyHostToDevice, stream) == hipSuccess ? 0 : -1;
+  for (int i = 0; i < 2 * nviews && !rc; ++i) {
+    float2*& spec = (i % 2 ? spec2 : spec1)[i / 2];
+    if (!spec && hipMalloc(&spec, specN * 8) != hipSuccess) {
+      spec = nullptr;
+      rc = -1;
+      break;
+    }
+    rc = plan.kernel_spectrum(dk + i * nk, spec, stream);
+  }
+  if (hipStreamSynchronize(stream) != hipSuccess) rc = -1;
   (void)hipFree(dk);
-  if (S) (void)hipFree(S);
-  MVR_HIP(hipMalloc(&S, plan.ncpx() * 8 * (size_t)nS));
+  if (rc) { set_error("kernel spectra: allocation, copy or transform failed"); return -1; }
+  if (!S) MVR_HIP(hipMalloc(&S, specN * 8 * (size_t)nS));
+  workLen = specN * nS;
   if (scheme == SCHEME_MUL) {
     if (Spsi) (void)hipFree(Spsi);
     if (T2) (void)hipFree(T2);

@@ -89,6 +89,8 @@ struct Plan {
 
   // spectrum of a device kernel (K layout), scaled by the inverse-FFT factor
   int kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const;
+  // planar plans: the second half of kernel_spectrum for n x transforms, ncpx() apart, in place
+  void kernel_planes(float2* spec, int n, hipStream_t s) const;
   // the gather of a kernel
   GatherParams kernel_gather(const float* dKernel) const;
   // one convolution with a kernel used once: kernel_spectrum and convolve, on planar plans in three launches
@@ -161,6 +163,7 @@ struct Decon {
   float* psi0 = nullptr;
   Plan plan;
   std::vector<float2*> spec1, spec2;
+  size_t specLen = 0, workLen = 0;  // complex values of a kernel spectrum, of S
   float2* S = nullptr;
   float2* Spsi = nullptr;
   float* T2 = nullptr;

@@ -65,6 +65,20 @@ void launch_reduce_stats_batched(const double2* partial, size_t stride, const in
   hipLaunchKernelGGL(k_reduce_stats_batched, dim3(nUpdates), dim3(kThreads), 0, s, partial, stride, c, out);
 }
 
+__global__ __launch_bounds__(kThreads) void k_psf_products(const float* first, const float* __restrict__ factors, int nf,
+                                                           size_t nk, float* out) {
+  const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x, v = blockIdx.y;
+  if (i >= nk) return;
+  float r = first[v * nk + i];  // first may be out
+  for (int j = 0; j < nf; ++j) r = factors[(v * nf + j) * nk + i] * r;
+  out[v * nk + i] = r;
+}
+
+void launch_psf_products(const float* first, const float* factors, int V, int nf, size_t nk, float* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_psf_products, dim3((unsigned)((nk + kThreads - 1) / kThreads), V), dim3(kThreads), 0, s, first,
+                     factors, nf, nk, out);
+}
+
 // PsiInitAvgPrecise per voxel (D/init/PsiInitAvgPreciseThread.java:127-155): the
 // mean of the positive view values is summed (double) over voxels with any
 // positive value; max of the positive values per view.  Per-work-group

@@ -225,6 +225,17 @@ void Plan::mid_rest(const Mid& m, const float2* in, float2* out, const float2* s
   sz(timed(t, m.zi, PASS_Z_INV), 1, out, out, nullptr, 1.f, twZ, s);
 }
 
+void Plan::kernel_planes(float2* spec, int n, hipStream_t s) const {
+  PlaneGeom g = mid().pl;
+  g.nb = n;
+  g.kStride = ncpx();
+  g.kin = g.specOut = spec;
+  g.kScale = inv_scale();
+  g.kK[0] = K[1];
+  g.kK[1] = K[2];
+  launch_plane(g, nullptr, nullptr, nullptr, twY, twZ, s);
+}
+
 GatherParams Plan::kernel_gather(const float* dKernel) const {
   GatherParams g{};
   g.src = dKernel;
@@ -236,14 +247,10 @@ GatherParams Plan::kernel_gather(const float* dKernel) const {
 
 int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const {
   xf(dom, kernel_gather(dKernel), spec, twM, wr, s);
-  Mid m = mid();
   if (planar) {
-    m.pl.kin = m.pl.specOut = spec;
-    m.pl.kScale = inv_scale();
-    m.pl.kK[0] = K[1];
-    m.pl.kK[1] = K[2];
-    launch_plane(m.pl, nullptr, nullptr, nullptr, twY, twZ, s);
+    kernel_planes(spec, 1, s);
   } else {
+    Mid m = mid();
     m.y.plane0 = dom.P[2] - K[2] / 2;  // the kernel's z planes, around 0
     m.y.planeMod = dom.P[2];
     m.y.nplanes = K[2];
