@@ -1,16 +1,27 @@
 // xpasses.hpp -- x (real axis) passes with the two-step register FFT.
 //
-// A work-group owns RW rows of one x-pass; each row is served by T lanes, T the power of two >= A, so that a
-// row never straddles a wave.  The length-M complex transform of a row (M = P0/2, real FFT by the even/odd
-// split) runs as M = A x B with one LDS exchange.  The R2C post-processing and the C2R pre-processing combine
+// A work-group owns RW rows of one x-pass.  The length-M complex transform of a row (M = P0/2, real FFT by the
+// even/odd split) runs as M = A x B with one LDS exchange: one side of it by A lanes per row, the other by B.
+//
+// The passes are bound by their vector instructions as much as by HBM (at M = 432 these took 75 % of the update's time,
+// 65 % of the quotient's), so lanes are packed: where it holds more rows than rows at multiples of 16 or 32 lanes would,
+// a wave of the A side holds rows side by side (a row never straddles a wave), and the B side's tasks lie densely over
+// the work-group where that leaves a wave without any.  Where neither is so the aligned rows are 10 % faster (M = 225:
+// their exchange has fewer LDS conflicts).  Values next to one another in the real rows move in pairs; whether a pair
+// lies inside the row is a question of the register index, not of the lane, except at the row's ends.  Measured, one
+// iteration of two views: M = 200 1.08 x, 288 1.06, 400 1.13, 480 1.08, 640 1.11; M = 432, 767 x 700 x 321: forward
+// 197 -> 144 us, quotient 852 -> 690, update 851 -> 701 (2.9 -> 3.3 TB/s).
+//
+// The R2C post-processing and the C2R pre-processing combine
 // the values k and M - k of a row; after the second forward step (before the first inverse step) lane q holds
 // index q + A k2 in register k2, and M - (q + A k2) = (A - q) + A (B - 1 - k2), so the partner is lane A - q,
 // register B - 1 - k2 of the same row: the pairs are swapped with wave shuffles, and spectra go between HBM
-// and registers directly, coalesced across the row's lanes.  Real-valued data meets the transforms in
-// registers too: psi is read into the first forward step, and the quotient and the psi update work on the
-// values the inverse leaves in lane q < B (x[2n], x[2n + 1] for n = q + B a).  Index arithmetic that depends on
+// and registers directly, coalesced across the row's lanes.  Real-valued data is read into the first forward step
+// directly; the quotient and the psi update work on rows parked in LDS.  Index arithmetic that depends on
 // runtime sizes is done once per row (row tables in LDS), never per element with '/' or '%'.
 #pragma once
+#include <type_traits>
+
 #include "passes.hpp"
 
 namespace mvr {
@@ -71,9 +82,14 @@ template <int M>
 struct XCfg {
   static constexpr Split2 S = split2(M);
   static constexpr int A = S.A, B = S.B;
-  static constexpr int T = A <= 16 ? 16 : A <= 32 ? 32 : 64;  // lanes per row (a power of two, divides 64)
-  static constexpr int RW = 256 / T;                          // rows per work-group
-  static constexpr int NT = RW * T;                           // threads per work-group
+  static constexpr int NT = 256;             // threads per work-group
+  static constexpr int T = A <= 16 ? 16 : A <= 32 ? 32 : 64;  // lanes of a row that start at a multiple of them
+  static constexpr int RPW = 64 / A;         // rows per wave on the A side
+  static constexpr int TA = RPW > 64 / T ? A : T;             // lanes from row to row
+  static constexpr int RW = NT / 64 * RPW;   // rows per work-group
+  static constexpr int TQ = NT / RW;         // lanes per row where rows are walked with every thread (>= A >= B)
+  // lanes from row to row on the B side: dense if that leaves a wave without tasks
+  static constexpr int TB = TA == A || (RW * B + 63) / 64 < NT / 64 ? B : T;
   static constexpr int RS = M + 5;                 // LDS row stride (complex): M used, +5 against bank conflicts
   static constexpr int PX = 2 * M;
   // the exchange rows, at least as large as the stats reduction that reuses them (2 x 256 doubles)
@@ -101,12 +117,52 @@ struct XCfg {
   // SIMD allow; bounded to 6 waves it takes 80 without spilling (x_ratio 4 % faster at M = 150).  Other lengths
   // either fit already or would spill under the bound.
   static constexpr int MINW_RATIO = (M == 100 || M == 120 || M == 150 || M == 200) ? 6 : 1;
+  // The update takes 128 VGPRs and two spilled ones in place of 130-148: 4 waves per SIMD (M = 432: 778 -> 701 us)
+  static constexpr int MINW_UPDATE = (M == 432 || M == 450 || M == 480) ? 4 : 1;
 };
 
 template <int M>
 __host__ __device__ constexpr bool x2_ok() {
   return split2(M).A > 0 && split2(M).B > 1;
 }
+
+// A thread's place on the two sides of a transform: row ra, index qa < A; row rb, index qb < B.  Idle threads have
+// qa = A, qb = B (and a valid row).
+template <int M>
+struct XLane {
+  int ra, qa, rb, qb;
+  __device__ __forceinline__ XLane() {
+    using C = XCfg<M>;
+    const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6), r = lane / C::TA;
+    const bool a = C::TA == C::T || r < C::RPW, b = C::TB == C::T || (int)threadIdx.x < C::RW * C::B;
+    ra = w * C::RPW + (a ? r : 0);
+    qa = a ? lane - r * C::TA : C::A;
+    rb = b ? (int)threadIdx.x / C::TB : 0;
+    qb = b ? (int)threadIdx.x % C::TB : C::B;
+  }
+};
+
+// two consecutive values at any multiple of 4 bytes, in one access
+typedef float PairValue __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ float2 ld_pair(const float* p) {
+  const PairValue v = *reinterpret_cast<const PairValue*>(p);
+  return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void st_pair(float* p, float2 v) {
+  PairValue u;
+  u.x = v.x;
+  u.y = v.y;
+  *reinterpret_cast<PairValue*>(p) = u;
+}
+
+// The x positions of a register index on the B side, [2 B a, 2 B (a + 1)) over the lanes, against a range [lo, hi): the
+// same for every lane, so that only the register indices at the range's ends test their positions one by one.
+template <int B>
+struct XSpan {
+  int lo, hi;
+  __device__ __forceinline__ bool inside(int a) const { return 2 * B * a >= lo && 2 * B * (a + 1) <= hi; }
+  __device__ __forceinline__ bool outside(int a) const { return 2 * B * (a + 1) <= lo || 2 * B * a >= hi; }
+};
 
 __device__ __forceinline__ float2 shfl2(float2 v, int src) {
   return make_float2(__shfl(v.x, src, 64), __shfl(v.y, src, 64));
@@ -119,7 +175,7 @@ template <int M>
 __device__ __forceinline__ void x2_mirror_pairs(const float2* v, float2 vM, int q, float2* out) {
   using C = XCfg<M>;
   const int lane = (int)(threadIdx.x & 63);
-  const int src = (lane & ~(C::T - 1)) + (q > 0 && q < C::A ? C::A - q : q);
+  const int src = q > 0 && q < C::A ? lane - q + (C::A - q) : lane;
 #pragma unroll
   for (int k2 = 0; k2 < C::B; ++k2) {
     const float2 t = shfl2(v[C::B - 1 - k2], src);
@@ -127,21 +183,24 @@ __device__ __forceinline__ void x2_mirror_pairs(const float2* v, float2 vM, int 
   }
 }
 
-// forward transform whose first-step inputs v[a] = z[q + B a] (lane q < B) are in registers; LDS row `rb` is
-// only written -> out[k2] = Z[q + A k2] (lane q < A)
+// forward transform of rows of `buf` (RS values apart) whose first-step inputs v[a] = z[qb + B a] (lanes qb < B) are in
+// registers; the rows are only written -> out[k2] = Z[qa + A k2] (lanes qa < A)
 template <int M>
-__device__ __forceinline__ void x2_forward_regs(float2* rb, const float2* tw, int q, float2* v, float2* out) {
+__device__ __forceinline__ void x2_forward_regs(float2* buf, const float2* tw, const XLane<M>& l, float2* v, float2* out) {
   using C = XCfg<M>;
   constexpr int A = C::A, B = C::B;
-  if (q < B) {
+  if (l.qb < B) {
+    float2* rb = buf + l.rb * C::RS;
+    const int q = l.qb;
     rdft<A, -1>(v);
 #pragma unroll
     for (int k1 = 0; k1 < A; ++k1) rb[q + B * k1] = k1 == 0 ? v[k1] : cmul(v[k1], tw[q * k1]);
   }
   __syncthreads();
-  if (q < A) {
+  if (l.qa < A) {
+    const float2* rb = buf + l.ra * C::RS;
 #pragma unroll
-    for (int b = 0; b < B; ++b) out[b] = rb[b + B * q];
+    for (int b = 0; b < B; ++b) out[b] = rb[b + B * l.qa];
     rdft<B, -1>(out);
   } else {
 #pragma unroll
@@ -149,12 +208,16 @@ __device__ __forceinline__ void x2_forward_regs(float2* rb, const float2* tw, in
   }
 }
 
-// x2_forward_regs with the exchange in two rounds through a row `rb` of AH * B values: round r carries the
-// first-step results k1 in [r AH, r AH + AH), read by the lanes q = k1 of that range
+// x2_forward_regs with the exchange in two rounds through rows of AH * B values (RS_FWD apart): round r carries the
+// first-step results k1 in [r AH, r AH + AH), read by the lanes qa = k1 of that range
 template <int M>
-__device__ __forceinline__ void x2_forward_regs_half(float2* rb, const float2* tw, int q, float2* v, float2* out) {
+__device__ __forceinline__ void x2_forward_regs_half(float2* buf, const float2* tw, const XLane<M>& l, float2* v,
+                                                     float2* out) {
   using C = XCfg<M>;
   constexpr int A = C::A, B = C::B, AH = C::AH;
+  const int q = l.qb, qa = l.qa;
+  float2* wb = buf + l.rb * C::RS_FWD;
+  const float2* rb = buf + l.ra * C::RS_FWD;
   if (q < B) {
     rdft<A, -1>(v);
 #pragma unroll
@@ -169,28 +232,29 @@ __device__ __forceinline__ void x2_forward_regs_half(float2* rb, const float2* t
     if (q < B) {
 #pragma unroll
       for (int j = 0; j < AH; ++j)
-        if (j < kn) rb[q + B * j] = v[k0 + j];
+        if (j < kn) wb[q + B * j] = v[k0 + j];
     }
     __syncthreads();
-    if (q >= k0 && q < k0 + kn) {
+    if (qa >= k0 && qa < k0 + kn) {
 #pragma unroll
-      for (int b = 0; b < B; ++b) out[b] = rb[b + B * (q - k0)];
+      for (int b = 0; b < B; ++b) out[b] = rb[b + B * (qa - k0)];
     }
   }
-  if (q < A) rdft<B, -1>(out);
+  if (qa < A) rdft<B, -1>(out);
 }
 
-// forward transform of LDS row `rb` (natural order) -> out[k2] = Z[q + A k2] (lane q < A)
+// forward transform of the rows of `buf` (natural order) -> out[k2] = Z[qa + A k2] (lanes qa < A)
 template <int M>
-__device__ __forceinline__ void x2_forward(float2* rb, const float2* tw, int q, float2* out) {
+__device__ __forceinline__ void x2_forward(float2* buf, const float2* tw, const XLane<M>& l, float2* out) {
   using C = XCfg<M>;
   float2 v[C::A];
-  if (q < C::B) {
+  if (l.qb < C::B) {
+    const float2* rb = buf + l.rb * C::RS;
 #pragma unroll
-    for (int a = 0; a < C::A; ++a) v[a] = rb[q + C::B * a];
+    for (int a = 0; a < C::A; ++a) v[a] = rb[l.qb + C::B * a];
   }
-  __syncthreads();  // every lane has read its values before the row is overwritten
-  x2_forward_regs<M>(rb, tw, q, v, out);
+  __syncthreads();  // every lane has read its values before the rows are overwritten
+  x2_forward_regs<M>(buf, tw, l, v, out);
 }
 
 // R2C post-processing of a row whose complex transform Z lane q holds as z[k2] = Z[q + A k2]:
@@ -223,15 +287,18 @@ __device__ __forceinline__ void x2_post_store_regs(const float2* z, int q, const
 }
 
 // inverse of the half spectrum X[0..M] of one row (src: its start in HBM; null: a row of zeros), read straight
-// into registers: the C2R pre-processing Z[k] = E[k] + i O[k] combines X[k] and X*[M - k]; returns
-// z[q + B n1] in out[n1] (lane q < B)
+// into registers by the lanes qa of row ra: the C2R pre-processing Z[k] = E[k] + i O[k] combines X[k] and X*[M - k];
+// returns z[qb + B n1] of row rb in out[n1] (lanes qb < B)
 // PF: the transforms' coprime splits by the prime-factor algorithm (false: Cooley-Tukey throughout, which the
 // update pass on short rows runs 3 % faster at M = 150)
 template <int M, bool TR, bool PF = true>
-__device__ __forceinline__ void x2_inverse_half_regs(const float2* __restrict__ src, float2* rb, const float2* tw,
-                                                     const float2* twr, int q, float2* out, unsigned cs) {
+__device__ __forceinline__ void x2_inverse_half_regs(const float2* __restrict__ src, float2* buf, const float2* tw,
+                                                     const float2* twr, const XLane<M>& l, float2* out, unsigned cs) {
   using C = XCfg<M>;
   constexpr int A = C::A, B = C::B;
+  const int q = l.qa;
+  float2* wb = buf + l.ra * C::RS;
+  const float2* rb = buf + l.rb * C::RS;
   float2 x[B];
   float2 xM = make_float2(0.f, 0.f);
   const bool ld = src != nullptr && q < A;
@@ -255,12 +322,12 @@ __device__ __forceinline__ void x2_inverse_half_regs(const float2* __restrict__ 
   __syncthreads();  // the row buffer is free (previous readers are done)
   if (q < A) {
 #pragma unroll
-    for (int n2 = 0; n2 < B; ++n2) rb[q + A * n2] = n2 == 0 ? u[n2] : cmul(u[n2], cconj(tw[n2 * q]));
+    for (int n2 = 0; n2 < B; ++n2) wb[q + A * n2] = n2 == 0 ? u[n2] : cmul(u[n2], cconj(tw[n2 * q]));
   }
   __syncthreads();
-  if (q < B) {
+  if (l.qb < B) {
 #pragma unroll
-    for (int k1 = 0; k1 < A; ++k1) out[k1] = rb[k1 + A * q];
+    for (int k1 = 0; k1 < A; ++k1) out[k1] = rb[k1 + A * l.qb];
     rdft<A, 1, PF>(out);
   }
 }
@@ -272,14 +339,15 @@ __device__ __forceinline__ void x2_load_twiddles(float2* tw, float2* twr, const 
   for (int i = threadIdx.x; i <= M; i += C::NT) twr[i] = wr[i];
 }
 
-// the inverse result z[q + B n1] (lane q < B, register n1) into LDS row `rb` in natural order
+// the inverse result z[qb + B n1] (lanes qb < B, register n1) into the LDS rows in natural order
 template <int M>
-__device__ __forceinline__ void x2_park_inverse(float2* rb, int q, const float2* z) {
+__device__ __forceinline__ void x2_park_inverse(float2* buf, const XLane<M>& l, const float2* z) {
   using C = XCfg<M>;
-  __syncthreads();  // every lane has read the row's exchange values
-  if (q < C::B) {
+  __syncthreads();  // every lane has read the rows' exchange values
+  if (l.qb < C::B) {
+    float2* rb = buf + l.rb * C::RS;
 #pragma unroll
-    for (int n1 = 0; n1 < C::A; ++n1) rb[q + C::B * n1] = z[n1];
+    for (int n1 = 0; n1 < C::A; ++n1) rb[l.qb + C::B * n1] = z[n1];
   }
   __syncthreads();
 }
@@ -310,8 +378,7 @@ __device__ __forceinline__ void x2_fwd_body(const Dom& d, const GatherParams& g,
     S += (size_t)b * d.blockStride;
   }
   const int row0 = wg * C::RW;
-  const int r = threadIdx.x / C::T, q = threadIdx.x % C::T;
-  float2* rb = buf + r * C::RS_FWD;
+  const XLane<M> l;
   // rows with source values only: row index -> grid row (-org1 + i % N1, -org2 + i / N1), the kernel's rows around 0
   const bool uniq = g.uniqueRows;
   const int nrowsRun = uniq ? g.N[1] * g.N[2] : nrows;
@@ -363,26 +430,27 @@ __device__ __forceinline__ void x2_fwd_body(const Dom& d, const GatherParams& g,
   __syncthreads();
   // the first transform step reads its values z[q + B a] = (x[2n], x[2n + 1]) straight from the source
   float2 v[C::A];
-  if (q < C::B) {
-    const long long off = srcRow[r];
+  if (l.qb < C::B) {
+    const long long off = srcRow[l.rb];
+    const float* row = g.src + (off + org[0] + 2 * l.qb);  // the value of position x of an inner register index
+    const XSpan<C::B> src{-org[0], g.N[0] - org[0]};
+    const bool plain = !kern && !__any(off < 0);
 #pragma unroll
     for (int a = 0; a < C::A; ++a) {
-      const int x = 2 * (q + C::B * a);
-      const int g0 = xmap[x], g1 = xmap[x + 1];
-      const bool ok0 = off >= 0 && g0 >= 0, ok1 = off >= 0 && g1 >= 0;
-      const float* p0 = g.src + (ok0 ? off + g0 : 0);
-      if (ok0 && g1 == g0 + 1 && !(reinterpret_cast<uintptr_t>(p0) & 7)) {
-        v[a] = *reinterpret_cast<const float2*>(p0);  // an aligned contiguous pair: one 8-byte load
+      if (plain && src.inside(a)) {
+        v[a] = ld_pair(row + 2 * C::B * a);
       } else {
-        v[a].x = ok0 ? *p0 : fill;
-        v[a].y = ok1 ? g.src[off + g1] : fill;
+        const int x = 2 * (l.qb + C::B * a);
+        const int g0 = xmap[x], g1 = xmap[x + 1];
+        v[a].x = off >= 0 && g0 >= 0 ? g.src[off + g0] : fill;
+        v[a].y = off >= 0 && g1 >= 0 ? g.src[off + g1] : fill;
       }
     }
   }
   float2 z[C::B];
-  x2_forward_regs_half<M>(rb, tw, q, v, z);
-  const size_t o = dstRow[r];
-  x2_post_store_regs<M, TR>(z, q, twr, S + (o == kNoRow ? 0 : o), o != kNoRow, (unsigned)(d.P[1] * d.P[2]));
+  x2_forward_regs_half<M>(buf, tw, l, v, z);
+  const size_t o = dstRow[l.ra];
+  x2_post_store_regs<M, TR>(z, l.qa, twr, S + (o == kNoRow ? 0 : o), o != kNoRow, (unsigned)(d.P[1] * d.P[2]));
 }
 
 template <int M, bool TR>
@@ -463,84 +531,81 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
     outOff[threadIdx.x] = live ? x2_row<TR>(d, row) : kNoRow;
   }
   __syncthreads();
-  const int r = threadIdx.x / C::T, q = threadIdx.x % C::T;
-  float2* rb = buf + r * C::RS;
-  const long long ir = imgRow[r];
-  const size_t so = outOff[r];
+  const XLane<M> l;
+  const bool rowOnes = imgRow[l.ra] == kOuterRow;
+  const size_t so = outOff[l.ra];
   // FFT positions x of the row whose image value is read: the quotient region, inside the volume
   const int x0f = d.m[0] + max(-q_.qlo[0], -o[0]), x1f = d.m[0] + min(D[0] + q_.qhi[0], q_.N[0] - o[0]);
   // rows outside the quotient region are a row of ones after the quotient: their blurred values are not read
   float2 z[C::A];
   const unsigned cs = (unsigned)(d.P[1] * d.P[2]);
-  x2_inverse_half_regs<M, TR>(ir != kOuterRow ? Sin + so : nullptr, rb, tw, twr, q, z, cs);
-  float2 zf[C::B];
-  if constexpr (!C::long_rows) {
-    // short rows (only B of T lanes hold values): park the blurred rows in LDS, form the quotient there with the
-    // row's T lanes over positions x = q + T i, all of a lane's image values in flight at once (offsets from the
-    // lane's row pointers known at compile time; at M = 150 4 % faster than a flat mapping over the work-group,
-    // 9 % faster than a wave walking its rows one by one), and run the forward transform from LDS
-    x2_park_inverse<M>(rb, q, z);
-    float* fr = reinterpret_cast<float*>(rb);
-    constexpr int NI = (C::PX + C::T - 1) / C::T;
+  x2_inverse_half_regs<M, TR>(!rowOnes ? Sin + so : nullptr, buf, tw, twr, l, z, cs);
+  // park the blurred rows in LDS, form the quotient there with TQ lanes per row, all of a lane's image values in flight
+  // at once at offsets from the lane's row pointers known at compile time, and run the forward transform from LDS.
+  // Positions x = q + TQ i, or on long rows pairs (at M = 432 16 % faster than the quotient on the B side's registers;
+  // at M = 150 and 225 pairs are 3-5 % slower, a flat mapping over the work-group 4 %, a wave walking its rows 9 %)
+  x2_park_inverse<M>(buf, l, z);
+  const int r = (int)threadIdx.x / C::TQ, q = (int)threadIdx.x % C::TQ;
+  if (C::RW * C::TQ == C::NT || r < C::RW) {
+    const long long ir = imgRow[r];
     const bool rowIn = ir != kOuterRow;
     const float* imr = q_.img + (rowIn ? ir : 0);  // image value of FFT position x: imr[x], x in [x0f, x1f)
-    float im[NI];
+    if constexpr (!C::long_rows) {
+      float* fr = reinterpret_cast<float*>(buf + r * C::RS);
+      constexpr int NI = (C::PX + C::TQ - 1) / C::TQ;
+      float im[NI];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int x = q + C::T * i;
-      im[i] = rowIn && x >= x0f && x < x1f ? imr[x] : 0.f;
-    }
+      for (int i = 0; i < NI; ++i) {
+        const int x = q + C::TQ * i;
+        im[i] = rowIn && x >= x0f && x < x1f ? imr[x] : 0.f;
+      }
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int x = q + C::T * i;
-      if (x < C::PX) fr[x] = im[i] > 0.f ? im[i] / fr[x] : 1.f;
-    }
-    __syncthreads();
-    x2_forward<M>(rb, tw, q, zf);
-  } else {
-    // long rows: lane q < B holds blurred values z[a] = (x[2n], x[2n + 1]), n = q + B a, exactly the inputs of its
-    // first forward step: the quotient is formed there, with the image read straight from HBM
-    if (q < C::B) {
-      constexpr int H = (C::A + 1) / 2;  // two halves of loads in flight
+      for (int i = 0; i < NI; ++i) {
+        const int x = q + C::TQ * i;
+        if (x < C::PX) fr[x] = im[i] > 0.f ? im[i] / fr[x] : 1.f;
+      }
+    } else {
+      float2* fr = buf + r * C::RS + q;
+      if (rowIn) imr += 2 * q;
+      constexpr int NI = (M + C::TQ - 1) / C::TQ;
+      const XSpan<C::TQ> quot{x0f, x1f};
+      const bool plain = __all(rowIn);
+      float2 im[NI];
 #pragma unroll
-      for (int a0 = 0; a0 < C::A; a0 += H) {
-        // pair h: image values of FFT positions x, x + 1 (x = 2 (q + B a)); one 8-byte load where both are read
-        // and the address is aligned
-        float2 im[H];
-#pragma unroll
-        for (int h = 0; h < H; ++h) {
-          const int a = a0 + h;
-          const int x = 2 * (q + C::B * a);
-          const bool ok0 = a < C::A && ir != kOuterRow && x >= x0f && x < x1f;
-          const bool ok1 = a < C::A && ir != kOuterRow && x + 1 >= x0f && x + 1 < x1f;
-          const float* p = q_.img + (ok0 ? ir + x : 0);
-          if (ok0 && ok1 && !(reinterpret_cast<uintptr_t>(p) & 7)) {
-            im[h] = *reinterpret_cast<const float2*>(p);
-          } else {
-            im[h].x = ok0 ? *p : 0.f;
-            im[h].y = ok1 ? q_.img[ir + x + 1] : 0.f;
-          }
-        }
-#pragma unroll
-        for (int h = 0; h < H; ++h) {
-          const int a = a0 + h;
-          if (a < C::A) {
-            z[a].x = im[h].x > 0.f ? im[h].x / z[a].x : 1.f;
-            z[a].y = im[h].y > 0.f ? im[h].y / z[a].y : 1.f;
-          }
+      for (int i = 0; i < NI; ++i) {
+        const int x = 2 * (q + C::TQ * i);
+        im[i] = make_float2(0.f, 0.f);
+        if (quot.outside(i)) continue;
+        if (plain && quot.inside(i)) {
+          im[i] = ld_pair(imr + 2 * C::TQ * i);
+        } else if (rowIn) {
+          if (x >= x0f && x < x1f) im[i].x = imr[2 * C::TQ * i];
+          if (x + 1 >= x0f && x + 1 < x1f) im[i].y = imr[2 * C::TQ * i + 1];
         }
       }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if (C::TQ * (i + 1) > M && q + C::TQ * i >= M) continue;
+        float2 f = make_float2(1.f, 1.f);
+        if (!quot.outside(i)) {
+          const float2 b = fr[C::TQ * i];
+          f.x = im[i].x > 0.f ? im[i].x / b.x : 1.f;
+          f.y = im[i].y > 0.f ? im[i].y / b.y : 1.f;
+        }
+        fr[C::TQ * i] = f;
+      }
     }
-    __syncthreads();  // the inverse's reads of the row are done before the forward writes it
-    x2_forward_regs<M>(rb, tw, q, z, zf);
   }
-  x2_post_store_regs<M, TR>(zf, q, twr, Sout + (so == kNoRow ? 0 : so),
-                            so != kNoRow && !(q_.skipOnes && ir == kOuterRow), cs);
+  __syncthreads();
+  float2 zf[C::B];
+  x2_forward<M>(buf, tw, l, zf);
+  x2_post_store_regs<M, TR>(zf, l.qa, twr, Sout + (so == kNoRow ? 0 : so),
+                            so != kNoRow && !(q_.skipOnes && rowOnes), cs);
 }
 
 // ------------------------------------------------------------------ inverse + psi update (output rows only)
 template <int M, bool TR>
-__global__ __launch_bounds__(XCfg<M>::NT) void k_x2_update(Dom d, UpdateParams u, FastDiv divD0,
+__global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_UPDATE) void k_x2_update(Dom d, UpdateParams u, FastDiv divPairs,
                                                             const float2* __restrict__ S,
                                                             const float2* __restrict__ twM,
                                                             const float2* __restrict__ wr) {
@@ -562,7 +627,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_update(Dom d, UpdateParams u
     const int* t = d.btab + kBlockTabInts * b;
     for (int k = 0; k < 3; ++k) { o[k] = t[k]; D[k] = t[3 + k]; }
     S += (size_t)b * d.blockStride;
-    if (D[0] != d.D[0]) divD0 = FastDiv((unsigned)D[0]);  // a tail block's row length
+    if (D[0] != d.D[0]) divPairs = FastDiv((unsigned)(D[0] + 1) / 2);  // a tail block's row length
   }
   const int nrows = D[1] * D[2];
   const int row0 = wg * C::RW;
@@ -579,127 +644,108 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_update(Dom d, UpdateParams u
     rowOff[threadIdx.x] = so;
   }
   __syncthreads();
-  const int r = threadIdx.x / C::T, q = threadIdx.x % C::T;
-  float2* rb = buf + r * C::RS;
-  const size_t so = rowOff[r];
+  const XLane<M> l;
+  const size_t so = rowOff[l.ra];
   float2 z[C::A];
-  x2_inverse_half_regs<M, TR, C::long_rows>(so != kNoRow ? S + so : nullptr, rb, tw, twr, q, z,
+  x2_inverse_half_regs<M, TR, C::long_rows>(so != kNoRow ? S + so : nullptr, buf, tw, twr, l, z,
                                             (unsigned)(d.P[1] * d.P[2]));
   double sum = 0.0;
   float mx = -1.f;
   const RLConsts rc = rl_consts(u.lambda, u.minValue, u.maxI);
   const int DX = D[0];
+  // park the rows in LDS and update pairs of positions there, U pairs in flight (the last pair of an odd row holds one)
+  x2_park_inverse<M>(buf, l, z);
+  const float* fb = reinterpret_cast<const float*>(buf) + d.m[0];
+  auto one = [&](float last, float integral, float weight) {
+    const float next = rl_next_value(last, integral, weight, rc), ch = next - last;
+    sum += (double)ch;
+    mx = java_maxf(mx, ch);
+    return next;
+  };
+  constexpr int U = 4;
   if constexpr (C::long_rows) {
-    // long rows: lane q < B holds the values z[a] = (x[2n], x[2n + 1]), n = q + B a, of its row and updates psi
-    // there (at M = 576 faster than a flat pass)
-    const long long pr = psiRow[r];
-    if (q < C::B && pr >= 0) {
-      const int m0 = d.m[0];
-      float* psiRowPtr = u.psi + pr;
-      const float* wRowPtr = u.w + pr;
-      constexpr int H = (C::A + 3) / 4;  // loads of a quarter of the row's values in flight
+    // long rows: TQ lanes per row at offsets uniform over the work-group; only a row's last pairs test their positions.
+    // At M = 432 778 us for 225 000 rows, 807 with the flat mapping below, 855 on the B side's registers
+    const int r = (int)threadIdx.x / C::TQ, q = (int)threadIdx.x % C::TQ;
+    const long long pr = C::RW * C::TQ == C::NT || r < C::RW ? psiRow[r] : -1;
+    if (pr >= 0) {
+      const float* f = fb + r * 2 * C::RS + 2 * q;
+      float* psi = u.psi + (pr + 2 * q);
+      const float* w = u.w + (pr + 2 * q);
+      for (int i0 = 0; 2 * C::TQ * i0 < DX; i0 += U) {
+        float2 last[U], wt[U];
 #pragma unroll
-      for (int a0 = 0; a0 < C::A; a0 += H) {
-        float last[2 * H], wt[2 * H];
-        int lx[2 * H];
-#pragma unroll
-        for (int j = 0; j < 2 * H; ++j) {
-          const int a = a0 + (j >> 1);
-          lx[j] = 2 * (q + C::B * a) + (j & 1) - m0;
-          if (a >= C::A || lx[j] < 0 || lx[j] >= DX) lx[j] = -1;
-          last[j] = psiRowPtr[max(lx[j], 0)];
-          wt[j] = wRowPtr[max(lx[j], 0)];
+        for (int j = 0; j < U; ++j) {
+          const int at = 2 * C::TQ * (i0 + j), lx = at + 2 * q;
+          last[j] = wt[j] = make_float2(0.f, 0.f);
+          if (at + 2 * C::TQ <= DX) {
+            last[j] = ld_pair(psi + at);
+            wt[j] = ld_pair(w + at);
+          } else {
+            if (lx < DX) { last[j].x = psi[at]; wt[j].x = w[at]; }
+            if (lx + 1 < DX) { last[j].y = psi[at + 1]; wt[j].y = w[at + 1]; }
+          }
         }
 #pragma unroll
-        for (int j = 0; j < 2 * H; ++j) {
-          if (lx[j] < 0) continue;
-          const int a = min(a0 + (j >> 1), C::A - 1);
-          const float next = rl_next_value(last[j], (j & 1) ? z[a].y : z[a].x, wt[j], rc);
-          psiRowPtr[lx[j]] = next;
-          const float ch = next - last[j];
-          sum += (double)ch;
-          mx = java_maxf(mx, ch);
+        for (int j = 0; j < U; ++j) {
+          const int at = 2 * C::TQ * (i0 + j), lx = at + 2 * q;
+          if (lx >= DX) continue;
+          float2 next;
+          next.x = one(last[j].x, f[at], wt[j].x);
+          if (lx + 1 < DX) {
+            next.y = one(last[j].y, f[at + 1], wt[j].y);
+            st_pair(psi + at, next);
+          } else {
+            psi[at] = next.x;
+          }
         }
       }
     }
   } else {
-    // short rows (only B of T lanes hold values): park the rows in LDS and update them with a flat mapping over
-    // every thread, six psi / weight pairs in flight (at M = 150 35 % faster than the register update; the
-    // row's lanes over positions q + T j with 8 pairs in flight were 8 % slower, a wave walking its rows one by
-    // one 12-37 % slower, fewer instructions notwithstanding: the loop is bound by its rounds of loads)
-    x2_park_inverse<M>(rb, q, z);
-    const float* fb = reinterpret_cast<const float*>(buf);
-    const unsigned total = (unsigned)(C::RW * DX);
-    constexpr int U = 6;
-    if (!(DX & 1) && !(u.N[0] & 1) && !(o[0] & 1)) {
-      // even rows in an even-width volume at an even x origin: every pair of positions (2k, 2k + 1) lies in one
-      // row and is 8-byte aligned in psi and the weights, so a thread takes U2 such pairs per round (one row
-      // lookup and one address per pair, 8-byte loads and stores)
-      constexpr int U2 = 4;
-      const unsigned total2 = total / 2;
-      for (unsigned base = threadIdx.x; base < total2; base += U2 * C::NT) {
-        float2 last[U2], wt[U2];
-        size_t gi[U2];
-        unsigned rr[U2];
-        bool ok[U2];
-#pragma unroll
-        for (int j = 0; j < U2; ++j) {
-          const unsigned e = 2 * (base + j * C::NT);  // first position of the pair
-          rr[j] = min(divD0.div(e), (unsigned)C::RW - 1);
-          const int lx = (int)(e - rr[j] * (unsigned)DX);
-          const long long prr = psiRow[rr[j]];
-          ok[j] = e < total && prr >= 0;
-          gi[j] = ok[j] ? (size_t)(prr + lx) : 0;
-          last[j] = *reinterpret_cast<const float2*>(u.psi + gi[j]);
-          wt[j] = *reinterpret_cast<const float2*>(u.w + gi[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < U2; ++j) {
-          if (!ok[j]) continue;
-          const unsigned e = 2 * (base + j * C::NT);
-          const int lx = (int)(e - rr[j] * (unsigned)DX);
-          const float* f = fb + rr[j] * 2 * C::RS + d.m[0] + lx;
-          float2 next;
-          next.x = rl_next_value(last[j].x, f[0], wt[j].x, rc);
-          next.y = rl_next_value(last[j].y, f[1], wt[j].y, rc);
-          *reinterpret_cast<float2*>(u.psi + gi[j]) = next;
-          const float c0 = next.x - last[j].x, c1 = next.y - last[j].y;
-          sum += (double)c0;
-          mx = java_maxf(mx, c0);
-          sum += (double)c1;
-          mx = java_maxf(mx, c1);
-        }
-      }
-    } else {
+    // short rows: a flat mapping of the pairs over every thread (at M = 150 35 % faster than on the B side's registers,
+    // 12 % faster than TQ lanes per row, 12-37 % than a wave walking its rows)
+    const unsigned perRow = divPairs.d, total = (unsigned)C::RW * perRow;
+    auto update_rows = [&](auto odd) {
       for (unsigned base = threadIdx.x; base < total; base += U * C::NT) {
-        float last[U], wt[U];
+        float2 last[U], wt[U];
         size_t gi[U];
-        unsigned rr[U];
-        bool ok[U];
+        unsigned at[U];  // the pair's first value in the rows
+        bool ok[U], two[U];
 #pragma unroll
         for (int j = 0; j < U; ++j) {
-          const unsigned idx = base + j * C::NT;
-          rr[j] = min(divD0.div(idx), (unsigned)C::RW - 1);
-          const int lx = (int)(idx - rr[j] * (unsigned)DX);
-          const long long prr = psiRow[rr[j]];
-          ok[j] = idx < total && prr >= 0;
-          gi[j] = ok[j] ? (size_t)(prr + lx) : 0;
-          last[j] = u.psi[gi[j]];
-          wt[j] = u.w[gi[j]];
+          const unsigned e = base + j * C::NT, r = min(divPairs.div(e), (unsigned)C::RW - 1);
+          const unsigned lx = 2 * (e - r * perRow);
+          const long long pr = psiRow[r];
+          ok[j] = e < total && pr >= 0;
+          two[j] = !odd || (ok[j] && (int)lx + 1 < DX);
+          gi[j] = ok[j] ? (size_t)(pr + lx) : 0;
+          at[j] = r * 2 * C::RS + lx;
+          if (two[j]) {
+            last[j] = ld_pair(u.psi + gi[j]);
+            wt[j] = ld_pair(u.w + gi[j]);
+          } else {
+            last[j] = make_float2(u.psi[gi[j]], 0.f);
+            wt[j] = make_float2(u.w[gi[j]], 0.f);
+          }
         }
 #pragma unroll
         for (int j = 0; j < U; ++j) {
           if (!ok[j]) continue;
-          const unsigned idx = base + j * C::NT;
-          const int lx = (int)(idx - rr[j] * (unsigned)DX);
-          const float next = rl_next_value(last[j], fb[rr[j] * 2 * C::RS + d.m[0] + lx], wt[j], rc);
-          u.psi[gi[j]] = next;
-          const float ch = next - last[j];
-          sum += (double)ch;
-          mx = java_maxf(mx, ch);
+          float2 next;
+          next.x = one(last[j].x, fb[at[j]], wt[j].x);
+          if (two[j]) {
+            next.y = one(last[j].y, fb[at[j] + 1], wt[j].y);
+            st_pair(u.psi + gi[j], next);
+          } else {
+            u.psi[gi[j]] = next.x;
+          }
         }
       }
-    }
+    };
+    if (DX & 1)
+      update_rows(std::true_type{});
+    else
+      update_rows(std::false_type{});
   }
   // the stats reduction reuses the row buffer once every thread has read its rows
   static_assert(C::BUF * sizeof(float2) >= 2 * reduce_width<C::NT>() * sizeof(double),
@@ -741,20 +787,24 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_store(Dom d, StoreParams st,
     rowOff[threadIdx.x] = so;
   }
   __syncthreads();
-  const int r = threadIdx.x / C::T, q = threadIdx.x % C::T;
-  float2* rb = buf + r * C::RS;
-  const size_t so = rowOff[r];
+  const XLane<M> l;
+  const size_t so = rowOff[l.ra];
   float2 z[C::A];
-  x2_inverse_half_regs<M, TR>(so != kNoRow ? S + so : nullptr, rb, tw, twr, q, z, (unsigned)(d.P[1] * d.P[2]));
-  const int row = row0 + r;
+  x2_inverse_half_regs<M, TR>(so != kNoRow ? S + so : nullptr, buf, tw, twr, l, z, (unsigned)(d.P[1] * d.P[2]));
+  const int row = row0 + l.rb, q = l.qb;
   if (q < C::B && row < nrows) {
     const int DX = d.D[0], m0 = d.m[0];
     float* out = st.out + (size_t)row * DX;
+    const XSpan<C::B> span{m0, m0 + DX};
 #pragma unroll
     for (int a = 0; a < C::A; ++a) {
       const int lx = 2 * (q + C::B * a) - m0;
-      if (lx >= 0 && lx < DX) out[lx] = z[a].x;
-      if (lx + 1 >= 0 && lx + 1 < DX) out[lx + 1] = z[a].y;
+      if (span.inside(a)) {
+        st_pair(out + lx, z[a]);
+      } else {
+        if (lx >= 0 && lx < DX) out[lx] = z[a].x;
+        if (lx + 1 >= 0 && lx + 1 < DX) out[lx + 1] = z[a].y;
+      }
     }
   }
 }
@@ -806,7 +856,8 @@ int launch_x_update(const Dom& d, const UpdateParams& u, const float2* S, const 
   const int rows = d.D[1] * d.D[2];
   dd.wgPerBlock = (rows + C::RW - 1) / C::RW;
   const int nwg = dd.wgPerBlock * (d.btab ? d.nb : 1);
-  hipLaunchKernelGGL((k_x2_update<M, TR>), dim3(nwg), dim3(C::NT), 0, s, dd, u, FastDiv((unsigned)d.D[0]), S, twM, wr);
+  hipLaunchKernelGGL((k_x2_update<M, TR>), dim3(nwg), dim3(C::NT), 0, s, dd, u, FastDiv((unsigned)(d.D[0] + 1) / 2), S,
+                     twM, wr);
   return nwg;
 }
 template <int M, bool TR>
