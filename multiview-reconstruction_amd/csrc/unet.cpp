@@ -28,10 +28,34 @@ int UNet::create(int dev_, int V_, unsigned long long seed) {
   V = V_;
   MVR_HIP(hipSetDevice(dev));
   MVR_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+  // master weights, moments and gradients, each in the order of copy_params
+  for (int l = 0; l < kLayers; ++l) {
+    layer[l].count = wcount(l);
+    bias[l].count = kCout[l];
+  }
+  head.count = 17;  // 16 weights + bias
+  const size_t section = (param_count() + 63) / 64 * 64;
+  MVR_HIP(hipMalloc(&params, 4 * section * 4));
+  MVR_HIP(hipMemset(params, 0, 4 * section * 4));
+  size_t at = 0;
+  auto place = [&](Param& p, bool conv) -> int {
+    p.w = params + at;
+    p.m = p.w + section;
+    p.v = p.m + section;
+    p.g = p.v + section;
+    at += p.count;
+    if (conv) {
+      MVR_HIP(hipMalloc(&p.wbf, p.count * 2));
+      MVR_HIP(hipMalloc(&p.wt, p.count * 2));
+    }
+    return 0;
+  };
+  for (int l = 0; l < kLayers; ++l)
+    if (place(layer[l], true) || place(bias[l], false)) return -1;
+  if (place(head, false)) return -1;
   std::mt19937_64 rng(seed);
   for (int l = 0; l < kLayers; ++l) {
     Param& p = layer[l];
-    p.count = wcount(l);
     std::vector<float> h(p.count, 0.f);
     const int fanin = 27 * (l == 0 ? (V + 1) : kCin[l]);
     std::normal_distribution<float> nd(0.f, std::sqrt(2.f / (float)fanin));
@@ -41,14 +65,8 @@ int UNet::create(int dev_, int V_, unsigned long long seed) {
           const bool real = l != 0 || ci < V + 1;
           h[((size_t)t * kCout[l] + co) * kCin[l] + ci] = real ? nd(rng) : 0.f;
         }
-    if (p.alloc(true)) return -1;
     MVR_HIP(hipMemcpy(p.w, h.data(), p.count * 4, hipMemcpyHostToDevice));
-    Param& b = bias[l];
-    b.count = kCout[l];
-    if (b.alloc(false)) return -1;
   }
-  head.count = 17;  // 16 weights + bias
-  if (head.alloc(false)) return -1;
   {
     std::vector<float> h(17, 0.f);
     std::normal_distribution<float> nd(0.f, 0.01f);
@@ -58,39 +76,20 @@ int UNet::create(int dev_, int V_, unsigned long long seed) {
   return refresh_copies();
 }
 
-int UNet::Param::alloc(bool conv) {
-  MVR_HIP(hipMalloc(&w, count * 4));
-  MVR_HIP(hipMalloc(&m, count * 4));
-  MVR_HIP(hipMalloc(&v, count * 4));
-  MVR_HIP(hipMalloc(&g, count * 4));
-  MVR_HIP(hipMemset(w, 0, count * 4));
-  MVR_HIP(hipMemset(m, 0, count * 4));
-  MVR_HIP(hipMemset(v, 0, count * 4));
-  MVR_HIP(hipMemset(g, 0, count * 4));
-  if (conv) {
-    MVR_HIP(hipMalloc(&wbf, count * 2));
-    MVR_HIP(hipMalloc(&wt, count * 2));
-  }
-  return 0;
-}
-
-void UNet::Param::release() {
-  for (void* p : {(void*)w, (void*)m, (void*)v, (void*)g, (void*)wbf, (void*)wt})
-    if (p) (void)hipFree(p);
-  w = m = v = g = nullptr;
-  wbf = wt = nullptr;
+// a parameter tensor (of layer l, or -1: without compute copies) of an Adam step
+void UNet::add_tensor(AdamArgs& a, const Param& p, int l) {
+  static_assert(2 * kLayers + 1 <= kAdamTensors, "every tensor in one launch");
+  AdamTensor& t = a.t[a.n++];
+  t.w = p.w; t.m = p.m; t.v = p.v; t.grad = p.g; t.wbf = p.wbf; t.wt = p.wt; t.count = (unsigned)p.count;
+  t.taps = 27; t.cout = l >= 0 ? kCout[l] : 0; t.cin = l >= 0 ? kCin[l] : 0;
 }
 
 // bf16 compute copies of the FP32 masters (an Adam step with learning rate 0 does exactly that)
 int UNet::refresh_copies() {
-  for (int l = 0; l < kLayers; ++l) {
-    AdamArgs a{};
-    a.w = layer[l].w; a.m = layer[l].m; a.v = layer[l].v; a.grad = layer[l].g;
-    a.wbf = layer[l].wbf; a.wt = layer[l].wt; a.count = layer[l].count;
-    a.taps = 27; a.cout = kCout[l]; a.cin = kCin[l];
-    a.lr = 0.f; a.beta1 = 1.f; a.beta2 = 1.f; a.eps = 1.f; a.c1 = 0.f; a.c2 = 0.f;
-    launch_adam(a, stream);
-  }
+  AdamArgs a{};
+  a.lr = 0.f; a.beta1 = 1.f; a.beta2 = 1.f; a.eps = 1.f; a.c1 = 0.f; a.c2 = 0.f;
+  for (int l = 0; l < kLayers; ++l) add_tensor(a, layer[l], l);
+  launch_adam(a, stream);
   MVR_HIP(hipGetLastError());
   MVR_HIP(hipStreamSynchronize(stream));
   return 0;
@@ -104,18 +103,9 @@ size_t UNet::param_count() const {
 
 int UNet::copy_params(float* hostOut, const float* hostIn, bool grads) {
   MVR_HIP(hipSetDevice(dev));
-  size_t off = 0;
-  auto one = [&](Param& p) -> int {
-    float* dev = grads ? p.g : p.w;
-    if (hostOut) MVR_HIP(hipMemcpy(hostOut + off, dev, p.count * 4, hipMemcpyDeviceToHost));
-    if (hostIn) MVR_HIP(hipMemcpy(dev, hostIn + off, p.count * 4, hipMemcpyHostToDevice));
-    off += p.count;
-    return 0;
-  };
-  for (int l = 0; l < kLayers; ++l) {
-    if (one(layer[l]) || one(bias[l])) return -1;
-  }
-  if (one(head)) return -1;
+  float* p = grads ? layer[0].g : layer[0].w;
+  if (hostOut) MVR_HIP(hipMemcpy(hostOut, p, param_count() * 4, hipMemcpyDeviceToHost));
+  if (hostIn) MVR_HIP(hipMemcpy(p, hostIn, param_count() * 4, hipMemcpyHostToDevice));
   if (hostIn && !grads) return refresh_copies();
   return 0;
 }
@@ -201,8 +191,9 @@ bool UNet::conv(int l, const uint16_t* in, int in_cs, int in_co, uint16_t* out, 
 }
 
 // data gradient of layer l: din = conv(dout, flipped transposed weights), no bias
-void UNet::dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t* din, int din_cs, int din_co, int N,
-                 int D, int H, int W) {
+// and, with the layer's input activations `post` (strided as din), the backward ReLU below it
+void UNet::dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t* din, int din_cs, int N, int D, int H,
+                 int W, const uint16_t* post) {
   ConvArgs c{};
   c.in = dout + dout_co;
   c.in_cs = dout_cs;
@@ -211,7 +202,8 @@ void UNet::dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t
   c.bias = nullptr;
   c.out = din;
   c.out_cs = din_cs;
-  c.out_co = din_co;
+  c.mask = post;
+  c.mask_cs = din_cs;
   c.cout = kCin[l];
   c.N = N; c.D = D; c.H = H; c.W = W;
   c.taps = 27;
@@ -232,8 +224,7 @@ void UNet::wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int
 }
 
 // ------------------------------------------------------------------ forward / backward
-int UNet::forward(Acts& a, bool training, const float* psiScale, float* psiOut, const int* outDims, float minValue,
-                  double* loss) {
+int UNet::forward(Acts& a, bool training, const float* psiScale, float* psiOut, const int* outDims, float minValue) {
   const int N = a.N, D0 = a.D, H0 = a.H, W0 = a.W;
   const int D1 = D0 / 2, H1 = H0 / 2, W1 = W0 / 2, D2 = D0 / 4, H2 = H0 / 4, W2 = W0 / 4;
   convFailed = false;
@@ -288,63 +279,58 @@ int UNet::forward(Acts& a, bool training, const float* psiScale, float* psiOut, 
   h.target = a.target;
   h.dr = a.dr;
   h.loss_partial = lossPart;
-  const int nb = launch_head(h, stream);
+  lossParts = launch_head(h, stream);
   MVR_HIP(hipGetLastError());
-  std::vector<double> lp(nb);
-  MVR_HIP(hipMemcpyAsync(lp.data(), lossPart, nb * 8, hipMemcpyDeviceToHost, stream));
+  return 0;
+}
+
+// the loss of the last training forward pass, waiting for everything enqueued since
+int UNet::read_loss(const Acts& a, double* loss) {
+  std::vector<double> lp(lossParts);
+  MVR_HIP(hipMemcpyAsync(lp.data(), lossPart, lossParts * 8, hipMemcpyDeviceToHost, stream));
   MVR_HIP(hipStreamSynchronize(stream));
   double s = 0;
   for (double x : lp) s += x;
-  *loss = s / (double)h.nvox;
+  *loss = s / (double)((size_t)a.N * a.D * a.H * a.W);
   return 0;
 }
 
 int UNet::backward(Acts& a) {
   const int N = a.N, D0 = a.D, H0 = a.H, W0 = a.W;
   const int D1 = D0 / 2, H1 = H0 / 2, W1 = W0 / 2, D2 = D0 / 4, H2 = H0 / 4, W2 = W0 / 4;
-  const size_t v0 = (size_t)N * D0 * H0 * W0, v1 = v0 / 8, v2 = v0 / 64;
+  const size_t v0 = (size_t)N * D0 * H0 * W0;
   convFailed = false;
   HeadArgs h{};
   h.d1 = a.d1; h.d1_cs = 16; h.wo = head.w; h.bias = head.w + 16; h.avg = a.avg; h.dr = a.dr; h.nvox = v0;
   const int hb = launch_head_bwd(h, a.g_d1, bpart, stream);
   launch_sum_partials(bpart, hb, 17, head.g, nullptr, 0, nullptr, stream);
   // decoder level 1
-  launch_relu_bwd(a.g_d1, 16, 0, a.d1, 16, 0, 16, v0, stream);
   wgrad(9, a.a5, 16, a.g_d1, 16, 0, N, D0, H0, W0);
-  dgrad(9, a.g_d1, 16, 0, a.g_a5, 16, 0, N, D0, H0, W0);
-  launch_relu_bwd(a.g_a5, 16, 0, a.a5, 16, 0, 16, v0, stream);
+  dgrad(9, a.g_d1, 16, 0, a.g_a5, 16, N, D0, H0, W0, a.a5);
   wgrad(8, a.cat1, 48, a.g_a5, 16, 0, N, D0, H0, W0);
-  dgrad(8, a.g_a5, 16, 0, a.g_cat1, 48, 0, N, D0, H0, W0);
+  dgrad(8, a.g_a5, 16, 0, a.g_cat1, 48, N, D0, H0, W0);
   // decoder level 2
-  launch_up_bwd(a.g_cat1, 48, 0, a.g_d2, 32, 32, N, D1, H1, W1, stream);
-  launch_relu_bwd(a.g_d2, 32, 0, a.d2, 32, 0, 32, v1, stream);
+  launch_up_bwd(a.g_cat1, 48, 0, a.g_d2, 32, 32, N, D1, H1, W1, a.d2, stream);
   wgrad(7, a.a4, 32, a.g_d2, 32, 0, N, D1, H1, W1);
-  dgrad(7, a.g_d2, 32, 0, a.g_a4, 32, 0, N, D1, H1, W1);
-  launch_relu_bwd(a.g_a4, 32, 0, a.a4, 32, 0, 32, v1, stream);
+  dgrad(7, a.g_d2, 32, 0, a.g_a4, 32, N, D1, H1, W1, a.a4);
   wgrad(6, a.cat2, 96, a.g_a4, 32, 0, N, D1, H1, W1);
-  dgrad(6, a.g_a4, 32, 0, a.g_cat2, 96, 0, N, D1, H1, W1);
+  dgrad(6, a.g_a4, 32, 0, a.g_cat2, 96, N, D1, H1, W1);
   // bottleneck
-  launch_up_bwd(a.g_cat2, 96, 0, a.g_b3, 64, 64, N, D2, H2, W2, stream);
-  launch_relu_bwd(a.g_b3, 64, 0, a.b3, 64, 0, 64, v2, stream);
+  launch_up_bwd(a.g_cat2, 96, 0, a.g_b3, 64, 64, N, D2, H2, W2, a.b3, stream);
   wgrad(5, a.a3, 64, a.g_b3, 64, 0, N, D2, H2, W2);
-  dgrad(5, a.g_b3, 64, 0, a.g_a3, 64, 0, N, D2, H2, W2);
-  launch_relu_bwd(a.g_a3, 64, 0, a.a3, 64, 0, 64, v2, stream);
+  dgrad(5, a.g_b3, 64, 0, a.g_a3, 64, N, D2, H2, W2, a.a3);
   wgrad(4, a.p2, 32, a.g_a3, 64, 0, N, D2, H2, W2);
-  dgrad(4, a.g_a3, 64, 0, a.g_p2, 32, 0, N, D2, H2, W2);
+  dgrad(4, a.g_a3, 64, 0, a.g_p2, 32, N, D2, H2, W2);
   // encoder level 2: e2 receives the skip gradient (g_cat2[64:96)) plus the pooled path
-  launch_pool_bwd(a.g_p2, 32, a.g_cat2, 96, 64, 32, N, D2, H2, W2, 1, stream);
-  launch_relu_bwd(a.g_cat2, 96, 64, a.cat2, 96, 64, 32, v1, stream);
+  launch_pool_bwd(a.g_p2, 32, a.g_cat2, 96, 64, 32, N, D2, H2, W2, a.cat2, stream);
   wgrad(3, a.a2, 32, a.g_cat2, 96, 64, N, D1, H1, W1);
-  dgrad(3, a.g_cat2, 96, 64, a.g_a2, 32, 0, N, D1, H1, W1);
-  launch_relu_bwd(a.g_a2, 32, 0, a.a2, 32, 0, 32, v1, stream);
+  dgrad(3, a.g_cat2, 96, 64, a.g_a2, 32, N, D1, H1, W1, a.a2);
   wgrad(2, a.p1, 16, a.g_a2, 32, 0, N, D1, H1, W1);
-  dgrad(2, a.g_a2, 32, 0, a.g_p1, 16, 0, N, D1, H1, W1);
+  dgrad(2, a.g_a2, 32, 0, a.g_p1, 16, N, D1, H1, W1);
   // encoder level 1
-  launch_pool_bwd(a.g_p1, 16, a.g_cat1, 48, 32, 16, N, D1, H1, W1, 1, stream);
-  launch_relu_bwd(a.g_cat1, 48, 32, a.cat1, 48, 32, 16, v0, stream);
+  launch_pool_bwd(a.g_p1, 16, a.g_cat1, 48, 32, 16, N, D1, H1, W1, a.cat1, stream);
   wgrad(1, a.a1, 16, a.g_cat1, 48, 32, N, D0, H0, W0);
-  dgrad(1, a.g_cat1, 48, 32, a.g_a1, 16, 0, N, D0, H0, W0);
-  launch_relu_bwd(a.g_a1, 16, 0, a.a1, 16, 0, 16, v0, stream);
+  dgrad(1, a.g_cat1, 48, 32, a.g_a1, 16, N, D0, H0, W0, a.a1);
   wgrad(0, a.x0, 16, a.g_a1, 16, 0, N, D0, H0, W0);
   UCHECK(!convFailed, "U-Net convolution refused: three x-y planes of the input exceed 32-bit offsets");
   MVR_HIP(hipGetLastError());
@@ -355,18 +341,14 @@ int UNet::adam_step(float lr) {
   ++step;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.f / (1.f - std::pow(b1, (float)step)), c2 = 1.f / (1.f - std::pow(b2, (float)step));
-  auto one = [&](Param& p, int l) {
-    AdamArgs a{};
-    a.w = p.w; a.m = p.m; a.v = p.v; a.grad = p.g; a.wbf = p.wbf; a.wt = p.wt; a.count = p.count;
-    a.taps = 27; a.cout = l >= 0 ? kCout[l] : 0; a.cin = l >= 0 ? kCin[l] : 0;
-    a.lr = lr; a.beta1 = b1; a.beta2 = b2; a.eps = 1e-8f; a.c1 = c1; a.c2 = c2;
-    launch_adam(a, stream);
-  };
+  AdamArgs a{};
+  a.lr = lr; a.beta1 = b1; a.beta2 = b2; a.eps = 1e-8f; a.c1 = c1; a.c2 = c2;
   for (int l = 0; l < kLayers; ++l) {
-    one(layer[l], l);
-    one(bias[l], -1);
+    add_tensor(a, layer[l], l);
+    add_tensor(a, bias[l], -1);
   }
-  one(head, -1);
+  add_tensor(a, head, -1);
+  launch_adam(a, stream);
   MVR_HIP(hipGetLastError());
   return 0;
 }
@@ -407,7 +389,7 @@ int UNet::add_volume(const float* const* imgs, const float* const* ws, const flo
   return (int)vols.size() - 1;
 }
 
-int UNet::pack(Acts& a, int sample, const std::vector<float*>& img, const std::vector<float*>& w, const int N3[3],
+int UNet::pack(Acts& a, const std::vector<float*>& img, const std::vector<float*>& w, const int N3[3],
                const int o[3], float invScale) {
   InputArgs in{};
   for (int v = 0; v < V; ++v) { in.img[v] = img[v]; in.w[v] = w[v]; }
@@ -415,7 +397,6 @@ int UNet::pack(Acts& a, int sample, const std::vector<float*>& img, const std::v
   for (int d = 0; d < 3; ++d) in.N3[d] = N3[d];
   in.x0 = o[0]; in.y0 = o[1]; in.z0 = o[2];
   in.W = a.W; in.H = a.H; in.D = a.D;
-  in.sample = sample;
   in.inv_scale = invScale;
   in.out = a.x0;
   in.out_cs = a.csIn;
@@ -431,17 +412,31 @@ int UNet::train_step(const int* volIdx, const int* origins, int batch, int P, fl
   const size_t pv = (size_t)P * P * P;
   for (int b = 0; b < batch; ++b) {
     UCHECK(volIdx[b] >= 0 && volIdx[b] < (int)vols.size(), "bad training volume index");
-    TrainVolume& tv = vols[volIdx[b]];
-    const int* o = origins + 3 * b;
-    for (int d = 0; d < 3; ++d) UCHECK(o[d] >= 0 && o[d] + P <= tv.N[d], "patch outside its volume");
-    pack(train, b, tv.img, tv.w, tv.N, o, 1.f / tv.scale);
-    launch_gather_target(tv.target, tv.N, o, P, 1.f / tv.scale, train.target + pv * b, stream);
+    for (int d = 0; d < 3; ++d)
+      UCHECK(origins[3 * b + d] >= 0 && origins[3 * b + d] + P <= vols[volIdx[b]].N[d], "patch outside its volume");
   }
-  if (forward(train, true, nullptr, nullptr, nullptr, 0.f, loss)) return -1;
+  for (int b0 = 0; b0 < batch; b0 += kPatches) {
+    const int n = std::min(kPatches, batch - b0);
+    PatchArgs pa{};
+    for (int b = 0; b < n; ++b) {
+      const TrainVolume& tv = vols[volIdx[b0 + b]];
+      PatchArgs::Patch& p = pa.p[b];
+      for (int v = 0; v < V; ++v) { p.img[v] = tv.img[v]; p.w[v] = tv.w[v]; }
+      p.target = tv.target;
+      for (int d = 0; d < 3; ++d) { p.N3[d] = tv.N[d]; p.o[d] = origins[3 * (b0 + b) + d]; }
+      p.inv_scale = 1.f / tv.scale;
+    }
+    pa.V = V;
+    pa.P = P;
+    pa.out = train.x0 + pv * 16 * b0;
+    pa.avg_out = train.avg + pv * b0;
+    pa.target_out = train.target + pv * b0;
+    launch_pack_patches(pa, n, stream);
+  }
+  if (forward(train, true, nullptr, nullptr, nullptr, 0.f)) return -1;
   if (backward(train)) return -1;
   if (update && adam_step(lr)) return -1;
-  MVR_HIP(hipStreamSynchronize(stream));
-  return 0;
+  return read_loss(train, loss);
 }
 
 // weighted mean intensity sum w_v img_v / sum w_v over voxels and views (FP64 device partials,
@@ -492,10 +487,10 @@ int UNet::infer(const std::vector<float*>& img, const std::vector<float*>& w, co
     const int ws = std::max(0, zs - kInferHalo), we = std::min(N3[2], ze + kInferHalo);
     if (ensure_acts(inf, 1, up4(we - ws), Y, X, false)) return -1;
     const int o[3] = {0, 0, ws};
-    pack(inf, 0, img, w, N3, o, 1.f / scale);
+    pack(inf, img, w, N3, o, 1.f / scale);
     // psi planes [zs, ze) = window planes [zs - ws, ze - ws)
     const int od[4] = {N3[0], N3[1], ze - ws, zs - ws};
-    if (forward(inf, false, &scale, psiDev + (size_t)ws * N3[1] * N3[0], od, minValue, nullptr)) return -1;
+    if (forward(inf, false, &scale, psiDev + (size_t)ws * N3[1] * N3[0], od, minValue)) return -1;
   }
   MVR_HIP(hipStreamSynchronize(stream));
   return 0;
@@ -516,11 +511,13 @@ int UNet::clear_volumes() {
 void UNet::destroy() {
   (void)hipSetDevice(dev);
   if (stream) (void)hipStreamSynchronize(stream);
-  for (int l = 0; l < kLayers; ++l) {
-    layer[l].release();
-    bias[l].release();
+  for (Param& p : layer) {
+    if (p.wbf) (void)hipFree(p.wbf);
+    if (p.wt) (void)hipFree(p.wt);
+    p = Param{};
   }
-  head.release();
+  if (params) (void)hipFree(params);
+  params = nullptr;
   clear_volumes();
   inf.release();
   for (void* p : {(void*)wpart, (void*)bpart, (void*)lossPart})

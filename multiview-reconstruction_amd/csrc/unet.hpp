@@ -38,6 +38,10 @@ struct ConvArgs {
   // channels [0, cout): done where conv_fuses_pool(args) holds, else left to the caller
   uint16_t* pool_out;
   int pool_cs;
+  // optional ReLU of a backward pass: the activations [n][z][y][x][mask_cs], channels [0, cout), behind the output; cin and
+  // cout 16, 32 or 64 alike
+  const uint16_t* mask;
+  int mask_cs;
   PsiArgs psi;           // optional fused output head (psi.out set; 16 -> 16 channels, one sample): out is not written
 };
 
@@ -62,11 +66,10 @@ struct InputArgs {
   int N3[3];             // dims of the source volumes (x, y, z)
   int x0, y0, z0;        // origin of the sample region
   int W, H, D;           // sample region
-  int sample;            // index in the batch
   float inv_scale;
-  uint16_t* out;         // [batch][D][H][W][out_cs], out_cs 16 or (V < 8) 8
+  uint16_t* out;         // [D][H][W][out_cs], out_cs 16 or (V < 8) 8
   int out_cs;
-  float* avg_out;        // [batch][D][H][W] (normalised average channel) or null
+  float* avg_out;        // [D][H][W] (normalised average channel) or null
 };
 
 // output head of a training step
@@ -82,16 +85,38 @@ struct HeadArgs {
   size_t nvox;
 };
 
-struct AdamArgs {
+// one tensor of an Adam step
+struct AdamTensor {
   float* w;
   float* m;
   float* v;
   const float* grad;
   uint16_t* wbf;   // bf16 copy [taps][cout][cin] or null
   uint16_t* wt;    // flipped transpose [taps][cin][cout] or null
-  size_t count;
+  unsigned count, first;   // elements; its first work-group (set by the launch)
   int taps, cout, cin;
+};
+constexpr int kAdamTensors = 24;
+struct AdamArgs {
+  AdamTensor t[kAdamTensors];
+  int n;
   float lr, beta1, beta2, eps, c1, c2;  // c1 = 1/(1-beta1^t), c2 = 1/(1-beta2^t)
+};
+
+// patches of P^3 voxels of training volumes as network input and target, up to kPatches in a launch
+constexpr int kPatches = 8;
+struct PatchArgs {
+  struct Patch {
+    const float* img[kNetMaxViews];
+    const float* w[kNetMaxViews];
+    const float* target;
+    int N3[3], o[3];     // dims of the volume, origin of the patch (inside it)
+    float inv_scale;
+  } p[kPatches];
+  int V, P;
+  uint16_t* out;         // of the first patch: [P][P][P][16]
+  float* avg_out;        // [P][P][P]
+  float* target_out;
 };
 
 bool launch_conv_fwd(const ConvArgs& a, hipStream_t s);  // false: shape not supported, nothing launched
@@ -110,16 +135,15 @@ inline int wgrad_max_parts(int cin, int cout, int maxParts) {
 // grad[j] = sum_p partial[p][j], j < count; with bcount > 0 (at most 64) also bgrad from bpartial
 void launch_sum_partials(const float* partial, int nparts, size_t count, float* grad, const float* bpartial,
                          int bcount, float* bgrad, hipStream_t s);
-void launch_relu_bwd(uint16_t* g, int gcs, int gco, const uint16_t* post, int pcs, int pco, int C, size_t nvox,
-                     hipStream_t s);
 void launch_pool_fwd(const uint16_t* in, int ics, int ico, uint16_t* out, int ocs, int C, int N, int D, int H, int W,
                      hipStream_t s);
 void launch_pool_bwd(const uint16_t* dout, int ocs, uint16_t* din, int ics, int ico, int C, int N, int D, int H, int W,
-                     int accumulate, hipStream_t s);
+                     const uint16_t* post, hipStream_t s);
 void launch_up_fwd(const uint16_t* in, int ics, uint16_t* out, int ocs, int oco, int C, int N, int D, int H, int W,
                    hipStream_t s);
 void launch_up_bwd(const uint16_t* dfine, int fcs, int fco, uint16_t* dcoarse, int ccs, int C, int N, int D, int H,
-                   int W, hipStream_t s);
+                   int W, const uint16_t* post, hipStream_t s);
+void launch_pack_patches(const PatchArgs& a, int n, hipStream_t s);
 void launch_pack_input(const InputArgs& a, hipStream_t s);
 int launch_head(const HeadArgs& a, hipStream_t s);
 int launch_head_bwd(const HeadArgs& a, uint16_t* dd1, float* partial, hipStream_t s);
@@ -128,7 +152,5 @@ void launch_f32_to_bf16(const float* src, uint16_t* dst, size_t n, hipStream_t s
 void launch_bf16_to_f32(const uint16_t* src, float* dst, size_t n, hipStream_t s);
 void launch_zero_u16(uint16_t* p, size_t n, hipStream_t s);
 int launch_wsum_partials(const InputArgs& a, size_t n, double2* partial, hipStream_t s);
-void launch_gather_target(const float* src, const int N[3], const int o[3], int P, float invScale, float* dst,
-                          hipStream_t s);
 
 }  // namespace mvr

@@ -203,12 +203,31 @@ __device__ __forceinline__ Weights ring_weights(const ConvArgs& a, int co0, int 
 //     the order of k_pool_fwd, z, then y, then x, so the fused pooling rounds exactly as the pooling kernel; pool[ky]
 //     carries the sums from an even plane to the odd one after it;
 //   - the output head of an inference (NG = 1, 16 channels): psi of voxel (row 4 wave + l/16, l%16) per lane, the
-//     activations themselves not stored.
-enum Epilogue { kPlain, kPool, kHead };
+//     activations themselves not stored;
+//   - the ReLU of a backward pass: values whose activation (mask_values) was not positive
+//     are stored as zeros (ten passes over the gradients before, 121 us of a step of four 64^3 patches).
+enum Epilogue { kPlain, kPool, kHead, kMask };
+
+// this lane's activations of output plane z, in the order of ring_store
+template <int NG>
+__device__ __forceinline__ void mask_values(const ConvArgs& a, int n, int z, int x0, int y0, int co0,
+                                            uint2 (&act)[4][NG]) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int x = min(x0 + (lane & 15), a.W - 1);
+  const uint16_t* plane = a.mask + ((size_t)n * a.D + z) * a.H * a.W * a.mask_cs + co0 + 4 * (lane >> 4);
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const int y = min(y0 + 4 * wave + m, a.H - 1);
+#pragma unroll
+    for (int t = 0; t < NG; ++t)
+      act[m][t] = *reinterpret_cast<const uint2*>(plane + ((size_t)y * a.W + x) * a.mask_cs + t * 16);
+  }
+}
+
 template <int NG, int EPI>
 __device__ __forceinline__ void ring_store(const ConvArgs& a, int n, int z, int x0, int y0, int co0,
                                            const f32x4 (&acc)[4][NG], const f32x4 (&bias)[NG], const f32x4& hw,
-                                           float hb, float avg, float (*pool)[NG][4]) {
+                                           float hb, float avg, float (*pool)[NG][4], const uint2 (*act)[NG]) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i = lane & 15, g = lane >> 4;
   const int x = x0 + i;
@@ -235,6 +254,10 @@ __device__ __forceinline__ void ring_store(const ConvArgs& a, int n, int z, int 
         float v = acc[m][t][r] + bias[t][r];
         if (a.relu) v = fmaxf(v, 0.f);
         b[r] = f2bf_rne(v);
+        if constexpr (EPI == kMask) {
+          const uint32_t p = r < 2 ? act[m][t].x : act[m][t].y;
+          if (bf2f(r & 1 ? p >> 16 : p & 0xffffu) <= 0.f) b[r] = 0;
+        }
       }
       if constexpr (EPI == kHead) {
         float h = 0.f;
@@ -358,11 +381,13 @@ __device__ __forceinline__ void column_step(const ConvArgs& a, const RingSrc& sr
   if (more) ring_issue(src, z + 3, a.D, wave, nxt);
   __builtin_amdgcn_sched_barrier(0);  // the DMA goes out before the products, not behind them
   ring_products<NG, false, NG == 1 ? 0 : 1>(s0, s1, s2, wf, acc, Weights{});
+  uint2 act[4][NG];
+  if constexpr (EPI == kMask) mask_values<NG>(a, T.n, z, T.x0, T.y0, co0, act);  // ahead of them its registers spill
   if (more)
     ring_wait<kDma>();
   else if (z + 1 < ze)
     ring_wait<0>();
-  ring_store<NG, EPI>(a, T.n, z, T.x0, T.y0, co0, acc, bias, hw, hb, avg, pool);
+  ring_store<NG, EPI>(a, T.n, z, T.x0, T.y0, co0, acc, bias, hw, hb, avg, pool, act);
 }
 
 // One chunk: a column of zp planes through a ring of five (unrolled by five, so that the ring positions are known at
@@ -473,7 +498,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_chunks4(ConvArgs a) {
   ring_bias<1>(a, co0, bias);
 #pragma unroll
   for (int o = 0; o < 4; ++o)
-    if (T.zs + o < a.D) ring_store<1, kPlain>(a, T.n, T.zs + o, T.x0, T.y0, co0, acc[o], bias, f32x4{}, 0.f, 0.f, nullptr);
+    if (T.zs + o < a.D) ring_store<1, kPlain>(a, T.n, T.zs + o, T.x0, T.y0, co0, acc[o], bias, f32x4{}, 0.f, 0.f, nullptr, nullptr);
 }
 
 // Several chunks, NG = 2: two planes' accumulators; a chunk's four input planes take the ring positions 4 c .. 4 c + 3
@@ -542,8 +567,12 @@ __global__ __launch_bounds__(256, 2) void k_conv_chunks2(ConvArgs a) {
   ring_bias<2>(a, co0, bias);
   float pool[2][2][4];
 #pragma unroll
-  for (int o = 0; o < 2; ++o)
-    if (T.zs + o < a.D) ring_store<2, EPI>(a, T.n, T.zs + o, T.x0, T.y0, co0, acc[o], bias, f32x4{}, 0.f, 0.f, pool);
+  for (int o = 0; o < 2; ++o) {
+    if (T.zs + o >= a.D) continue;
+    uint2 act[4][2];
+    if constexpr (EPI == kMask) mask_values<2>(a, T.n, T.zs + o, T.x0, T.y0, co0, act);
+    ring_store<2, EPI>(a, T.n, T.zs + o, T.x0, T.y0, co0, acc[o], bias, f32x4{}, 0.f, 0.f, pool, act);
+  }
 }
 
 template <int NG>
@@ -561,6 +590,8 @@ void launch_ng(const ConvArgs& a, hipStream_t s) {
       hipLaunchKernelGGL((k_conv_column<1, kHead>), grid, dim3(256), 0, s, a, zp);
     else if (a.pool_out)
       hipLaunchKernelGGL((k_conv_column<NG, kPool>), grid, dim3(256), 0, s, a, zp);
+    else if (a.mask)
+      hipLaunchKernelGGL((k_conv_column<1, kMask>), grid, dim3(256), 0, s, a, zp);
     else
       hipLaunchKernelGGL((k_conv_column<NG, kPlain>), grid, dim3(256), 0, s, a, zp);
     return;
@@ -575,6 +606,10 @@ void launch_ng(const ConvArgs& a, hipStream_t s) {
     const dim3 grid(columns(2), groups);
     if (a.pool_out)
       hipLaunchKernelGGL((k_conv_chunks2<2, kPool>), grid, dim3(256), 0, s, a);
+    else if (a.mask && a.cin == 32)
+      hipLaunchKernelGGL((k_conv_chunks2<2, kMask>), grid, dim3(256), 0, s, a);
+    else if (a.mask)
+      hipLaunchKernelGGL((k_conv_chunks2<4, kMask>), grid, dim3(256), 0, s, a);
     else if (a.cin == 32)
       hipLaunchKernelGGL((k_conv_chunks2<2, kPlain>), grid, dim3(256), 0, s, a);
     else if (a.cin == 64)
@@ -602,6 +637,8 @@ bool launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
   if (a.up_c && (a.up_c % 16 != 0 || a.up_cs % 16 != 0 || !a.up_in || (a.W | a.H | a.D) & 1)) return false;
   if (a.in_half && a.cin != 16) return false;
   if (a.pool_out && !conv_fuses_pool(a)) return false;
+  // the backward ReLU behind the layers of as many inputs as outputs
+  if (a.mask && (a.cin != a.cout || a.cin > 64 || a.pool_out || a.psi.out || a.mask_cs % 4 != 0)) return false;
   if (a.psi.out && (a.cin != 16 || a.cout != 16 || a.N != 1)) return false;
   if (pairs)
     launch_ng<2>(a, s);

@@ -26,8 +26,6 @@ struct UNet {
     size_t count = 0;
     float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;
     uint16_t *wbf = nullptr, *wt = nullptr;
-    int alloc(bool conv);
-    void release();
   };
   struct Acts {
     int N = 0, D = 0, H = 0, W = 0;
@@ -54,10 +52,12 @@ struct UNet {
   long long step = 0;
   hipStream_t stream = nullptr;
   Param layer[kLayers], bias[kLayers], head;
+  float* params = nullptr;         // the masters, moments and gradients of all of them
   Acts train, inf;
   std::vector<TrainVolume> vols;
   float *wpart = nullptr, *bpart = nullptr;
   double* lossPart = nullptr;
+  int lossParts = 0;               // partial losses of the last training forward pass
   bool convFailed = false;         // a convolution launch was refused since the last check
   long long inferWindow = 1ll << 28;  // voxel budget of one inference window (z slab + halos)
 
@@ -77,7 +77,7 @@ struct UNet {
 
   int ensure_acts(Acts& a, int N, int D, int H, int W, bool grads);
   int ensure_scratch();
-  int pack(Acts& a, int sample, const std::vector<float*>& img, const std::vector<float*>& w, const int N3[3],
+  int pack(Acts& a, const std::vector<float*>& img, const std::vector<float*>& w, const int N3[3],
            const int o[3], float invScale);
   // up != nullptr: input channels [0, up_c) are nearest x2 upsampled from up (channel stride up_cs), the
   // rest come from in + in_co
@@ -87,14 +87,15 @@ struct UNet {
   bool conv(int l, const uint16_t* in, int in_cs, int in_co, uint16_t* out, int out_cs, int out_co, int N, int D,
             int H, int W, bool relu, const uint16_t* up = nullptr, int up_cs = 0, int up_c = 0,
             uint16_t* pool = nullptr, int pool_cs = 0, const PsiArgs* psi = nullptr);
-  void dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t* din, int din_cs, int din_co, int N,
-             int D, int H, int W);
+  void dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t* din, int din_cs, int N, int D,
+             int H, int W, const uint16_t* post = nullptr);
   void wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int dout_cs, int dout_co, int N, int D, int H,
              int W);
-  int forward(Acts& a, bool training, const float* psiScale, float* psiOut, const int* outDims, float minValue,
-              double* loss);
+  int forward(Acts& a, bool training, const float* psiScale, float* psiOut, const int* outDims, float minValue);
+  int read_loss(const Acts& a, double* loss);
   int backward(Acts& a);
   int adam_step(float lr);
+  static void add_tensor(AdamArgs& a, const Param& p, int l);
 };
 
 }  // namespace mvr
