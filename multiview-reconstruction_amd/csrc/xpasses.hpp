@@ -109,6 +109,7 @@ struct XCfg {
   static constexpr int AH = (A + 1) / 2;
   static constexpr int RS_FWD = AH * B + 5;
   static constexpr int BUF_FWD = RW * RS_FWD;
+  static constexpr int BUF_TR = (M + 1) * (RW + 1);  // the rows' spectra of a planar store
   static constexpr int LDS_ROWS_FWD = RW * RS_FWD * 8 + RW * 24;
   static constexpr bool TWL_FWD = !long_rows || (160 * 1024) / (LDS_ROWS_FWD + PX * 4 + LDS_TW) >=
                                                    (160 * 1024) / (LDS_ROWS_FWD + PX * 4);
@@ -260,29 +261,42 @@ __device__ __forceinline__ void x2_forward(float2* buf, const float2* tw, const 
 // R2C post-processing of a row whose complex transform Z lane q holds as z[k2] = Z[q + A k2]:
 // X[k] = (Z[k] + Z*[M - k]) / 2 + W_P0^k (Z[k] - Z*[M - k]) / 2i for k = q + A k2, and X[M] (lane 0), written
 // to dst (the row's start in HBM; cs: values per hx plane) when rowOk
-template <int M, bool TR>
-__device__ __forceinline__ void x2_post_store_regs(const float2* z, int q, const float2* twr, float2* __restrict__ dst,
-                                                   bool rowOk, unsigned cs) {
+// (VIA_LDS, planar spectra: through the work-group's LDS `buf`, (M + 1) (RW + 1) values, and from there with lanes along
+// the rows: rowAt[r] is row r's place in a plane, kNoRow: not stored.  Stored by the lanes of a row, a plane gets runs of
+// 64 / A values: the forward pass of 24 blocks on 120-point grids, 169 MB, takes 78 us so, 60 through the LDS; the
+// quotient pass gains nothing by it, 58 and 61)
+template <int M, bool TR, bool VIA_LDS>
+__device__ __forceinline__ void x2_post_store_regs(const float2* z, const XLane<M>& l, const float2* twr,
+                                                   float2* __restrict__ dst, bool rowOk, float2* buf,
+                                                   const size_t* rowAt, unsigned cs) {
   using C = XCfg<M>;
+  const int q = l.qa;
   float2 zc[C::B];
   x2_mirror_pairs<M>(z, z[0], q, zc);  // Z[M] = Z[0]
-  if (!rowOk || q >= C::A) return;
+  constexpr int TS = C::RW + 1;
+  if (VIA_LDS) __syncthreads();  // the rows' exchange values have been read
+  if ((VIA_LDS || rowOk) && q < C::A) {
+    auto put = [&](int k, float2 zk, float2 c) {
+      const float2 e = make_float2(0.5f * (zk.x + c.x), 0.5f * (zk.y + c.y));
+      const float2 dd = csub(zk, c);
+      const float2 od = make_float2(0.5f * dd.y, -0.5f * dd.x);
+      const float2 x = cadd(e, cmul(twr[k], od));
+      if (VIA_LDS)
+        buf[k * TS + l.ra] = x;
+      else
+        dst[x2_at<TR>(k, cs)] = x;
+    };
 #pragma unroll
-  for (int k2 = 0; k2 < C::B; ++k2) {
-    const int k = q + C::A * k2;
-    const float2 zk = z[k2];
-    const float2 c = cconj(zc[k2]);
-    const float2 e = make_float2(0.5f * (zk.x + c.x), 0.5f * (zk.y + c.y));
-    const float2 dd = csub(zk, c);
-    const float2 od = make_float2(0.5f * dd.y, -0.5f * dd.x);
-    dst[x2_at<TR>(k, cs)] = cadd(e, cmul(twr[k], od));
+    for (int k2 = 0; k2 < C::B; ++k2) put(q + C::A * k2, z[k2], cconj(zc[k2]));
+    if (q == 0) put(M, z[0], cconj(z[0]));
   }
-  if (q == 0) {
-    const float2 zk = z[0], c = cconj(z[0]);
-    const float2 e = make_float2(0.5f * (zk.x + c.x), 0.5f * (zk.y + c.y));
-    const float2 dd = csub(zk, c);
-    const float2 od = make_float2(0.5f * dd.y, -0.5f * dd.x);
-    dst[x2_at<TR>(M, cs)] = cadd(e, cmul(twr[M], od));
+  if (VIA_LDS) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < (M + 1) * C::RW; i += C::NT) {
+      const int k = i / C::RW, r = i % C::RW;
+      const size_t at = rowAt[r];
+      if (at != kNoRow) dst[(size_t)k * cs + at] = buf[k * TS + r];
+    }
   }
 }
 
@@ -358,7 +372,7 @@ template <int M, bool TR>
 __device__ __forceinline__ void x2_fwd_body(const Dom& d, const GatherParams& g, float2* __restrict__ S,
                                             const float2* __restrict__ twM, const float2* __restrict__ wr, int wg) {
   using C = XCfg<M>;
-  __shared__ float2 buf[C::BUF_FWD];
+  __shared__ float2 buf[TR && C::BUF_TR > C::BUF_FWD ? C::BUF_TR : C::BUF_FWD];
   __shared__ float2 twS[C::TWL_FWD ? M : 1];
   __shared__ float2 twrS[C::TWL_FWD ? M + 1 : 1];
   const float2* tw = C::TWL_FWD ? twS : twM;
@@ -450,7 +464,8 @@ __device__ __forceinline__ void x2_fwd_body(const Dom& d, const GatherParams& g,
   float2 z[C::B];
   x2_forward_regs_half<M>(buf, tw, l, v, z);
   const size_t o = dstRow[l.ra];
-  x2_post_store_regs<M, TR>(z, l.qa, twr, S + (o == kNoRow ? 0 : o), o != kNoRow, (unsigned)(d.P[1] * d.P[2]));
+  x2_post_store_regs<M, TR, TR>(z, l, twr, TR ? S : S + (o == kNoRow ? 0 : o), o != kNoRow, buf, dstRow,
+                            (unsigned)(d.P[1] * d.P[2]));
 }
 
 template <int M, bool TR>
@@ -599,8 +614,8 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
   __syncthreads();
   float2 zf[C::B];
   x2_forward<M>(buf, tw, l, zf);
-  x2_post_store_regs<M, TR>(zf, l.qa, twr, Sout + (so == kNoRow ? 0 : so),
-                            so != kNoRow && !(q_.skipOnes && rowOnes), cs);
+  x2_post_store_regs<M, TR, false>(zf, l, twr, Sout + (so == kNoRow ? 0 : so),
+                                   so != kNoRow && !(q_.skipOnes && rowOnes), buf, outOff, cs);
 }
 
 // ------------------------------------------------------------------ inverse + psi update (output rows only)
