@@ -356,6 +356,16 @@ int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
   }
   plan.wy = tunedW[0];
   plan.wz = tunedW[1];
+  viewBatch = 1;
+  if (scheme == SCHEME_MUL) {
+    // Views of one launch, while their work spectra are at most kBatchBytes: launches over a small grid neither fill the
+    // chip nor hide their ends, and spectra beyond the last-level cache gain nothing.  One view a launch and so, us an
+    // iteration: 4 views of 48^3 163 and 79, 3 of 100^3 209 and 123, 8 of 120^3 589 and 323, 4 of 160^3 430 and 342, of
+    // 200^3 772 and 712; with no bound 4 of 256^3 take 1425 in place of 1362, 3 of 320^3 2137 in place of 2004.
+    constexpr size_t kBatchBytes = 256u << 20;
+    viewBatch = (int)std::max<size_t>(1, std::min<size_t>({(size_t)V, (size_t)kViewBatch, kBatchBytes / (plan.ncpx() * 8)}));
+    nS = std::max(nS, viewBatch);
+  }
   // buffers of another size, or of views this call leaves out, go first
   const size_t specN = plan.ncpx();
   for (auto* specs : {&spec1, &spec2}) {
@@ -653,42 +663,51 @@ void Decon::reduce_slots(int n, double2* out) {
 
 // One Mul iteration (ComputeBlockMulThreadCPU.runIteration semantics on the whole volume).
 int Decon::iteration_mul(double2* statOut) {
-  const Dom& d = plan.dom;
+  Dom d = plan.dom;
+  d.blockStride = plan.ncpx();
   // both convolutions are read on the output rows (the quotient and the stored result)
   const int zero[3] = {0, 0, 0};
-  Plan::Mid m1 = plan.mid();
-  plan.restrict_rows(zero, zero, m1);
-  const Plan::Mid rows = m1;
   GatherParams g{};
   g.src = psi;
   for (int k = 0; k < 3; ++k) { g.N[k] = N[k]; g.org[k] = -d.m[k]; }
   g.mode = GATHER_MIRROR;
-  plan.mirror_rows(g, m1);  // psi's mirror copies are read from their sources
+  Plan::Mid fwd = plan.mid();
+  plan.mirror_rows(g, fwd);  // psi's mirror copies are read from their sources
   // the forward transform of psi is shared by all views
   timer.begin(stream, PASS_X_FWD);
   plan.xf(d, g, Spsi, plan.twM, plan.wr, stream);
   timer.end(stream);
-  plan.mid_forward(m1, Spsi, stream, &timer);
+  plan.mid_forward(fwd, Spsi, stream, &timer);
   std::vector<const float*> t2p(V), wp(V);
-  for (int v = 0; v < V; ++v) {
+  for (int v = 0; v < V; ++v) { t2p[v] = T2 + nvox() * v; wp[v] = w[v]; }
+  for (int v = 0; v < V; v += viewBatch) {
+    const int nb = std::min(viewBatch, V - v);
+    timer.views = nb;
+    Plan::Mid m1 = plan.mid();
+    plan.set_views(m1, nb, spec1.data() + v, true);
+    plan.restrict_rows(zero, zero, m1);
+    plan.mirror_rows(g, m1);
     plan.mid_rest(m1, Spsi, S, spec1[v], stream, &timer);
     RatioParams q{};
+    q.views.n = nb;
+    for (int b = 0; b < nb; ++b) q.views.at[b] = img[v + b] - img[v];
     q.img = img[v];
     for (int k = 0; k < 3; ++k) { q.N[k] = N[k]; q.o[k] = 0; }
-    Plan::Mid m2 = rows;
+    Plan::Mid m2 = plan.mid();
+    plan.set_views(m2, nb, spec2.data() + v, false);
+    plan.restrict_rows(zero, zero, m2);
     plan.skip_ones_rows(q, m2);
     timer.begin(stream, PASS_X_RATIO);
     plan.xr(d, q, S, S, plan.twM, plan.wr, stream);
     timer.end(stream);
     plan.mid_forward(m2, S, stream, &timer);
     plan.mid_rest(m2, S, S, spec2[v], stream, &timer);
-    StoreParams st{T2 + nvox() * v};
+    StoreParams st{T2 + nvox() * v, nb};
     timer.begin(stream, PASS_X_STORE);
     plan.xs(d, st, S, plan.twM, plan.wr, stream);
     timer.end(stream);
-    t2p[v] = T2 + nvox() * v;
-    wp[v] = w[v];
   }
+  timer.views = 1;
   double m = 0;
   for (int v = 0; v < V; ++v) m += maxI[v];
   m /= (double)V;

@@ -69,7 +69,17 @@ struct XFwdGroup {
 // the work-groups are dealt over the quotient rows only: grid rows (y, z) in [rowLo, rowLo + rowN) per axis
 // (k = 1, 2), which are exactly the rows the quotient region selects.  For batched blocks (planar spectra only) each
 // block's rows are formed from its entry in the block table, and rowN are the most rows of any block.
-struct RatioParams {
+// Batched views: n > 0 of them, the data of view b at at[b] values from the first's.  (Offsets, so that the compiler knows
+// global memory, and a kernel argument of its own: a struct that is indexed stays in memory with all its members, whose
+// loads then wait one by one; 2 % of a y pass.)
+constexpr int kViewBatch = 8;  // the most views of one launch
+struct ViewOffsets {
+  int n = 0;
+  bool inShared = false;  // all read the same input
+  long long at[kViewBatch];
+};
+
+struct RatioPass {
   const float* img;
   int N[3];
   int o[3];
@@ -77,6 +87,9 @@ struct RatioParams {
   int qhi[3];
   int skipOnes;
   int rowLo[3], rowN[3];
+};
+struct RatioParams : RatioPass {
+  ViewOffsets views;  // of their images; their spectra lie Dom::blockStride apart
 };
 
 struct UpdateParams {
@@ -92,7 +105,7 @@ struct UpdateParams {
 
 struct StoreParams {
   float* out;        // compact D[0]*D[1]*D[2] array
-  int n = 1;         // planar spectra: n of them, Dom::blockStride apart, into arrays of D[0]*D[1]*D[2] back to back
+  int n = 1;         // n > 1: as many spectra, Dom::blockStride apart, into arrays of D[0]*D[1]*D[2] back to back
 };
 
 typedef void (*XFwdFn)(const Dom&, const GatherParams&, float2* S, const float2* twM, const float2* wr,
@@ -107,7 +120,7 @@ typedef int (*XUpdateFn)(const Dom&, const UpdateParams&, const float2* S, const
 typedef void (*XStoreFn)(const Dom&, const StoreParams&, const float2* S, const float2* twM, const float2* wr,
                          hipStream_t s);
 // strided passes: y (plane = z) or z (plane = y)
-struct StridedGeom {
+struct StridedPass {
   size_t planeStride;  // complex elements between consecutive planes
   size_t lineStride;   // complex elements between consecutive pencil elements
   int ncols;           // valid columns (hx) per line
@@ -138,6 +151,9 @@ struct StridedGeom {
   // timing: when set, the launch records the kernel's own start and stop in these events
   hipEvent_t evStart = nullptr, evStop = nullptr;
 };
+struct StridedGeom : StridedPass {
+  ViewOffsets views;  // batched views, as blocks: of their kernel spectra
+};
 // mode: 0 forward, 1 inverse, 2 forward * spec * inverse (spec layout = data layout),
 // 3 forward then scale
 typedef void (*StridedFn)(const StridedGeom&, int mode, const float2* in, float2* out, const float2* spec,
@@ -165,6 +181,7 @@ struct PlaneGeom {
   const int* onesTab = nullptr;            // per batch entry {yLo, yHi, zLo, zHi} instead
   int lo[2] = {0, 0}, hi[2] = {1 << 30, 1 << 30};  // rows (y, z) stored
   hipEvent_t evStart = nullptr, evStop = nullptr;
+  ViewOffsets views;                       // batched views: entry b takes spec + views.at[b] instead
 };
 constexpr int kPlaneMax = 128;     // y and z lengths
 constexpr int kPlanarMaxM = 128;   // x passes with planar spectra are compiled for half lengths up to this

@@ -59,6 +59,9 @@ struct Plan {
   Mid mid() const;
   // batched blocks: nb spectra, blockStride complex values apart
   void set_blocks(Mid& m, int nb, size_t blockStride) const;
+  // batched views: nb spectra, ncpx() complex values apart, each with its kernel spectrum (the
+  // passes are given specs[0]); shared: all read one input
+  void set_views(Mid& m, int nb, float2* const* specs, bool shared) const;
   // Narrows a convolution to what the next x pass reads: the grid rows (y, z) in [m - lo, m + D + hi) per axis (within
   // the grid).  The y pass then stores only those y, and the inverse z pass transforms only those y planes and
   // stores only those z.
@@ -132,10 +135,12 @@ struct Timer {
   void begin(hipStream_t s, int c);
   void end(hipStream_t s);
   // a start / stop pair for a launch that records its own kernel's execution (both null when c is off)
-  void kernel(int c, hipEvent_t* start, hipEvent_t* stop) { kernel(&c, 1, start, stop); }
-  // the same for a launch that does the work of n passes: each is counted, with an nth of the time
-  void kernel(const int* c, int n, hipEvent_t* start, hipEvent_t* stop);
-  bool zForward = false;  // planar plans: the next plane pass does a forward z pass's work too
+  void kernel(int c, hipEvent_t* start, hipEvent_t* stop) { kernel(&c, &views, 1, start, stop); }
+  // the same for a launch that does the work of n passes, pass c[i] times[i] times: each is counted, with its share of the
+  // time
+  void kernel(const int* c, const int* times, int n, hipEvent_t* start, hipEvent_t* stop);
+  int zForward = 0;  // planar plans: forward z passes whose work the next plane pass does too
+  int views = 1;     // views of a batched launch, which counts as a launch for each
   int collect(double* ms, long long* n);  // accumulates into arrays of PASS_COUNT
   void release();
   // enable the categories in mask (bit c = category c), timing the first launch of every group of `every`;
@@ -163,6 +168,7 @@ struct Decon {
   float* psi0 = nullptr;
   Plan plan;
   std::vector<float2*> spec1, spec2;
+  int viewBatch = 1;                // MUL: views of one launch, a work spectrum each
   size_t specLen = 0, workLen = 0;  // complex values of a kernel spectrum, of S
   float2* S = nullptr;
   float2* Spsi = nullptr;

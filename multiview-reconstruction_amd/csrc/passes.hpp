@@ -260,8 +260,8 @@ int strided_span() {
 
 template <int L, int W, int MODE>
 __global__ __launch_bounds__(W * split2(L).A, (s2_min_waves<L, W, MODE>())) void k_strided2(
-    StridedGeom gm, const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ spec,
-    float scale, const float2* __restrict__ twg) {
+    const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ spec,
+    const float2* __restrict__ twg, float scale, StridedPass gm, ViewOffsets views) {
   constexpr Split2 S = split2(L);
   constexpr int A = S.A, B = S.B;
   constexpr int NT = W * A;
@@ -288,13 +288,14 @@ __global__ __launch_bounds__(W * split2(L).A, (s2_min_waves<L, W, MODE>())) void
     const int b = plane / gm.blockPlanes;
     plane -= b * gm.blockPlanes;
     blockOff = (size_t)b * gm.blockStride;
+    if (MODE == 2 && views.n) spec += views.at[b];
   }
   plane += gm.plane0;
   if (MODE == 0 && gm.planeMod > 0 && plane >= gm.planeMod) plane -= gm.planeMod;
   // Lanes of columns beyond ncols (the last tile) read the row pitch's padding (pitch = 16-column multiple) and
   // compute values that are never stored.
   const size_t ls = gm.lineStride;
-  const float2* sb = in + blockOff + (size_t)plane * gm.planeStride + col0;
+  const float2* sb = in + (MODE == 2 && views.inShared ? 0 : blockOff) + (size_t)plane * gm.planeStride + col0;
   float2* db = out + blockOff + (size_t)plane * gm.planeStride + col0;
   const unsigned lo = (unsigned)((w + (size_t)q * ls) * sizeof(float2));
   float2 v[A];
@@ -470,10 +471,10 @@ void launch_strided2_mode(const StridedGeom& gm, const float2* in, float2* out, 
     return;
   }
   if (gm.evStart)  // timed: the events hold the kernel's own start and stop
-    hipExtLaunchKernelGGL((k_strided2<L, W, MODE>), g2, dim3(NT), 0, s, gm.evStart, gm.evStop, 0u, gm, in, out, spec,
-                          scale, tw);
+    hipExtLaunchKernelGGL((k_strided2<L, W, MODE>), g2, dim3(NT), 0, s, gm.evStart, gm.evStop, 0u, in, out, spec, tw,
+                          scale, gm, gm.views);
   else
-    hipLaunchKernelGGL((k_strided2<L, W, MODE>), g2, dim3(NT), 0, s, gm, in, out, spec, scale, tw);
+    hipLaunchKernelGGL((k_strided2<L, W, MODE>), g2, dim3(NT), 0, s, in, out, spec, tw, scale, gm, gm.views);
 }
 
 template <int L, int W>

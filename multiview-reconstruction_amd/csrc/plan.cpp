@@ -109,6 +109,14 @@ void Plan::set_blocks(Mid& m, int nb, size_t blockStride) const {
   m.pl.inStride = m.pl.outStride = blockStride;
 }
 
+void Plan::set_views(Mid& m, int nb, float2* const* specs, bool shared) const {
+  set_blocks(m, nb, ncpx());
+  m.y.views.n = m.pl.views.n = nb;
+  for (int b = 0; b < nb; ++b) m.y.views.at[b] = m.pl.views.at[b] = specs[b] - specs[0];
+  m.y.views.inShared = shared;
+  if (shared) m.pl.inStride = 0;
+}
+
 void Plan::restrict_rows(const int lo[3], const int hi[3], Mid& m) const {
   int a[3], b[3];
   for (int k = 1; k < 3; ++k) {
@@ -161,8 +169,10 @@ void Plan::constant_rows(const int lo[3], const int hi[3], float value, Mid& m) 
   m.zf.onesPlaneHi = hi[1];
   m.zf.onesLo = lo[2];
   m.zf.onesHi = hi[2];
+  const int nb = m.zf.blockPlanes ? m.zf.nplanes / m.zf.blockPlanes : 1;
   m.zf.plane0 = lo[1];
-  m.zf.nplanes = std::max(0, hi[1] - lo[1]);
+  m.zf.nplanes = std::max(0, hi[1] - lo[1]) * nb;
+  if (m.zf.blockPlanes) m.zf.blockPlanes = std::max(0, hi[1] - lo[1]);
   m.y.onesDC = value * (float)dom.P[0] * (float)dom.P[2];  // the xz transform of a constant plane
   m.y.onesDCPlane = 0;
   m.y.onesPlaneLo = 0;
@@ -204,7 +214,7 @@ static G timed(Timer* t, G g, int c) {
 
 void Plan::mid_forward(const Mid& m, float2* S, hipStream_t s, Timer* t) const {
   if (planar) {
-    if (t) t->zForward = true;
+    if (t) t->zForward += t->views;
     return;
   }
   sz(timed(t, m.zf, PASS_Z_FWD), 0, S, S, nullptr, 1.f, twZ, s);
@@ -214,9 +224,9 @@ void Plan::mid_rest(const Mid& m, const float2* in, float2* out, const float2* s
   if (planar) {
     PlaneGeom g = m.pl;
     if (t) {
-      const int passes[3] = {PASS_Y_CONV, PASS_Z_INV, PASS_Z_FWD};
-      t->kernel(passes, t->zForward ? 3 : 2, &g.evStart, &g.evStop);
-      t->zForward = false;
+      const int passes[3] = {PASS_Y_CONV, PASS_Z_INV, PASS_Z_FWD}, times[3] = {t->views, t->views, t->zForward};
+      t->kernel(passes, times, 3, &g.evStart, &g.evStop);
+      t->zForward = 0;
     }
     launch_plane(g, in, out, spec, twY, twZ, s);
     return;
@@ -313,18 +323,26 @@ void Timer::grow() {
   for (size_t i = old; i < ev.size(); ++i) (void)hipEventCreate(&ev[i]);
 }
 void Timer::begin(hipStream_t s, int c) {
-  pending = on && ((mask >> c) & 1u) && seen[c]++ % every == 0;
+  pending = false;
+  if (!on || !((mask >> c) & 1u)) return;
+  for (int i = 0; i < views; ++i)
+    if (seen[c]++ % every == 0) {
+      shots.push_back({used, c, 1.0 / views});
+      pending = true;
+    }
   if (!pending) return;
   grow();
   (void)hipEventRecord(ev[used], s);
-  shots.push_back({used, c, 1.0});
 }
-void Timer::kernel(const int* c, int n, hipEvent_t* start, hipEvent_t* stop) {
+void Timer::kernel(const int* c, const int* times, int n, hipEvent_t* start, hipEvent_t* stop) {
   *start = *stop = nullptr;
   if (!on) return;
   const size_t before = shots.size();
+  int all = 0;
+  for (int i = 0; i < n; ++i) all += times[i];
   for (int i = 0; i < n; ++i)
-    if (((mask >> c[i]) & 1u) && seen[c[i]]++ % every == 0) shots.push_back({used, c[i], 1.0 / n});
+    for (int j = 0; j < times[i]; ++j)
+      if (((mask >> c[i]) & 1u) && seen[c[i]]++ % every == 0) shots.push_back({used, c[i], 1.0 / all});
   if (shots.size() == before) return;
   grow();
   *start = ev[used];

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(NT) void k_plane(PlaneGeom g, PlaneDivs dv, const f
   if (!in) return;
   float2* dst = out + (size_t)b * g.outStride + plane;
   const float2* sp = g.kin ? g.specOut + b * g.kStride + plane
-                           : spec + (g.specIdx ? g.specIdx[b] : 0) * g.specStride + plane;
+                           : spec + (g.views.n ? g.views.at[b] : (long long)((g.specIdx ? g.specIdx[b] : 0) * g.specStride)) + plane;
   with_length(Py, [&](auto len) {
     constexpr int L = decltype(len)::value, A = split2(L).A, B = split2(L).B;
     for (unsigned t = threadIdx.x; t < (unsigned)(Pz * A); t += NT) {

@@ -20,6 +20,7 @@
 // directly; the quotient and the psi update work on rows parked in LDS.  Index arithmetic that depends on
 // runtime sizes is done once per row (row tables in LDS), never per element with '/' or '%'.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "passes.hpp"
@@ -88,8 +89,8 @@ struct XCfg {
   static constexpr int TA = RPW > 64 / T ? A : T;             // lanes from row to row
   static constexpr int RW = NT / 64 * RPW;   // rows per work-group
   static constexpr int TQ = NT / RW;         // lanes per row where rows are walked with every thread (>= A >= B)
-  // lanes from row to row on the B side: dense if that leaves a wave without tasks
-  static constexpr int TB = TA == A || (RW * B + 63) / 64 < NT / 64 ? B : T;
+  // lanes from row to row on the B side: dense where the A side is, and on long rows if that leaves a wave without tasks
+  static constexpr int TB = TA == A || (B > 16 && (RW * B + 63) / 64 < NT / 64) ? B : T;
   static constexpr int RS = M + 5;                 // LDS row stride (complex): M used, +5 against bank conflicts
   static constexpr int PX = 2 * M;
   // the exchange rows, at least as large as the stats reduction that reuses them (2 x 256 doubles)
@@ -140,6 +141,10 @@ struct XLane {
     qa = a ? lane - r * C::TA : C::A;
     rb = b ? (int)threadIdx.x / C::TB : 0;
     qb = b ? (int)threadIdx.x % C::TB : C::B;
+    if (C::TA == C::T && C::TB == C::T) {  // the same lanes on both sides, in the same registers
+      ra = rb;
+      qa = qb;
+    }
   }
 };
 
@@ -494,10 +499,9 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_fwd_groups(Dom d, XFwdGroup 
 // ratio = img > 0 ? img / blurred : 1 on the quotient region, 1 elsewhere
 // (DeconvolutionMethods.computeQuotient, D/iteration/sequential/DeconvolutionMethods.java:46-98)
 template <int M, bool TR>
-__global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(Dom d, RatioParams q_, const float2* __restrict__ Sin,
-                                                           float2* __restrict__ Sout,
-                                                           const float2* __restrict__ twM,
-                                                           const float2* __restrict__ wr) {
+__global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(
+    const float2* __restrict__ Sin, float2* __restrict__ Sout, const float2* __restrict__ twM,
+    const float2* __restrict__ wr, Dom d, RatioPass q_, ViewOffsets views) {
   using C = XCfg<M>;
   __shared__ float2 buf[C::BUF];
   __shared__ float2 twS[C::TWL_RATIO ? M : 1];
@@ -517,6 +521,14 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
     wg -= b * d.wgPerBlock;
     const int* t = d.btab + kBlockTabInts * b;
     for (int k = 0; k < 3; ++k) { o[k] = t[k]; D[k] = t[3 + k]; }
+    Sin += (size_t)b * d.blockStride;
+    Sout += (size_t)b * d.blockStride;
+  }
+  const float* img = q_.img;
+  if (views.n > 1) {  // batched views: this work-group's spectrum and image
+    const int b = wg / d.wgPerBlock;
+    wg -= b * d.wgPerBlock;
+    img += views.at[b];
     Sin += (size_t)b * d.blockStride;
     Sout += (size_t)b * d.blockStride;
   }
@@ -564,7 +576,7 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(D
   if (C::RW * C::TQ == C::NT || r < C::RW) {
     const long long ir = imgRow[r];
     const bool rowIn = ir != kOuterRow;
-    const float* imr = q_.img + (rowIn ? ir : 0);  // image value of FFT position x: imr[x], x in [x0f, x1f)
+    const float* imr = img + (rowIn ? ir : 0);  // image value of FFT position x: imr[x], x in [x0f, x1f)
     if constexpr (!C::long_rows) {
       float* fr = reinterpret_cast<float*>(buf + r * C::RS);
       constexpr int NI = (C::PX + C::TQ - 1) / C::TQ;
@@ -746,11 +758,16 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_UPDATE) void k_x2_update
 #pragma unroll
         for (int j = 0; j < U; ++j) {
           if (!ok[j]) continue;
-          float2 next;
-          next.x = one(last[j].x, fb[at[j]], wt[j].x);
+          const float* f = fb + at[j];
+          const float2 next = make_float2(rl_next_value(last[j].x, f[0], wt[j].x, rc),
+                                          two[j] ? rl_next_value(last[j].y, f[1], wt[j].y, rc) : 0.f);
+          const float c0 = next.x - last[j].x, c1 = next.y - last[j].y;
+          sum += (double)c0;
+          mx = java_maxf(mx, c0);
           if (two[j]) {
-            next.y = one(last[j].y, fb[at[j] + 1], wt[j].y);
             st_pair(u.psi + gi[j], next);
+            sum += (double)c1;
+            mx = java_maxf(mx, c1);
           } else {
             u.psi[gi[j]] = next.x;
           }
@@ -785,7 +802,7 @@ __global__ __launch_bounds__(XCfg<M>::NT) void k_x2_store(Dom d, StoreParams st,
   if (C::TWL) x2_load_twiddles<M>(twS, twrS, twM, wr);
   const int nrows = d.D[1] * d.D[2];
   unsigned wg = blockIdx.x;
-  if (TR && st.n > 1) {  // this work-group's spectrum and output array
+  if (st.n > 1) {  // this work-group's spectrum and output array
     const unsigned b = wg / d.wgPerBlock;
     wg -= b * d.wgPerBlock;
     S += b * d.blockStride;
@@ -859,8 +876,8 @@ void launch_x_ratio(const Dom& d, const RatioParams& q, const float2* Sin, float
   const int rows = q.skipOnes ? q.rowN[1] * q.rowN[2] : d.P[1] * d.P[2];
   if (rows == 0) return;  // no quotient rows: every row is a row of ones, put in by the z pass
   dd.wgPerBlock = (rows + C::RW - 1) / C::RW;
-  const int nb = d.btab ? d.nb : 1;
-  hipLaunchKernelGGL((k_x2_ratio<M, TR>), dim3(dd.wgPerBlock * nb), dim3(C::NT), 0, s, dd, q, Sin, Sout, twM, wr);
+  const int nb = d.btab ? d.nb : std::max(1, q.views.n);
+  hipLaunchKernelGGL((k_x2_ratio<M, TR>), dim3(dd.wgPerBlock * nb), dim3(C::NT), 0, s, Sin, Sout, twM, wr, dd, q, q.views);
 }
 template <int M, bool TR>
 int launch_x_update(const Dom& d, const UpdateParams& u, const float2* S, const float2* twM, const float2* wr,
