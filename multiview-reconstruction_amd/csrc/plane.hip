@@ -11,11 +11,11 @@
 // kernel spectrum is stored in it, [hx][y slot][z slot]) and undone by the inverse steps.  Rows of the plane are
 // padded by one value, so that both directions' accesses (lanes along y or along z) are free of bank conflicts.
 //
-// Bound by the LDS round trips (eleven over a plane) and, at one plane per CU, by their latency (an 80 x 72 plane
-// takes 12 us on its CU, of which its VALU work is 5).  A 48 x 40 x 33 convolution: 43.6 us with three strided passes per
-// transform and direction, 35.0 with this one; two views of 64 x 60 x 52, 5 iterations: 527 -> 480 us; 24 batched blocks
-// on 120-point grids: 141 -> 92 us per convolution.  Single grids gain 12-20 % at 48 points, 4-6 % at 96 and nothing at
-// 128, where the range ends with the LDS.
+// Bound by the LDS round trips (eleven over a plane) and, at one plane per CU, by their latency: an 80 x 72 plane takes
+// 12 us on its CU, of which its VALU work is 5.  A 48 x 40 x 33 convolution with its kernel: 43.6 us with three strided
+// passes per transform and direction, 35.0 with this one, 20.5 with the kernel's plane transformed beside the data's.
+// Two views of 64 x 60 x 52, 5 iterations: 527 -> 480 us; 24 batched blocks on 120-point grids, 340 MB: 141 -> 80 us per
+// convolution.  Single grids gain 12-20 % at 48 points, 4-6 % at 96 and nothing at 128, where the range ends with the LDS.
 #include <type_traits>
 
 #include "passes.hpp"

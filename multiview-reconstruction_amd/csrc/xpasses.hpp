@@ -6,8 +6,8 @@
 // The passes are bound by their vector instructions as much as by HBM (at M = 432 these took 75 % of the update's time,
 // 65 % of the quotient's), so lanes are packed: where it holds more rows than rows at multiples of 16 or 32 lanes would,
 // a wave of the A side holds rows side by side (a row never straddles a wave), and the B side's tasks lie densely over
-// the work-group where that leaves a wave without any.  Where neither is so the aligned rows are 10 % faster (M = 225:
-// their exchange has fewer LDS conflicts).  Values next to one another in the real rows move in pairs; whether a pair
+// the work-group then, and on long rows (B > 16) where that leaves a wave without any.  Elsewhere the aligned rows are
+// faster, at M = 225 by 10 %: their exchange has fewer LDS conflicts.  Values next to one another in the real rows move in pairs; whether a pair
 // lies inside the row is a question of the register index, not of the lane, except at the row's ends.  Measured, one
 // iteration of two views: M = 200 1.08 x, 288 1.06, 400 1.13, 480 1.08, 640 1.11; M = 432, 767 x 700 x 321: forward
 // 197 -> 144 us, quotient 852 -> 690, update 851 -> 701 (2.9 -> 3.3 TB/s).
