@@ -101,13 +101,12 @@ int mvr_fft_convolve(int dev, const float* img, const int n[3], int ext, float e
     }
     if (hipMemcpyAsync(dImg, img, nv * 4, hipMemcpyDefault, s) || hipMemcpyAsync(dK, kernel, nk * 4, hipMemcpyDefault, s))
       break;
-    if (plan.kernel_spectrum(dK, spec, s)) break;
     GatherParams g{};
     g.src = dImg;
     for (int d = 0; d < 3; ++d) { g.N[d] = n[d]; g.org[d] = -plan.dom.m[d]; }
     g.mode = ext == MVR_EXT_MIRROR_SINGLE ? GATHER_MIRROR : GATHER_VALUE;
     g.value = extValue;
-    if (plan.convolve(g, spec, work, dOut, s)) break;
+    if (plan.convolve_once(dK, g, spec, work, dOut, s)) break;
     if (hipMemcpyAsync(out, dOut, nv * 4, hipMemcpyDefault, s) || hipStreamSynchronize(s)) {
       set_error("mvr_fft_convolve: readback failed");
       break;

@@ -161,7 +161,8 @@ typedef void (*StridedFn)(const StridedGeom&, int mode, const float2* in, float2
 
 // One pass of y and z transforms over planar spectra [hx][z][y] (plane.hip), in place or not: forward, times spec
 // ([hx][y slot][z slot]), inverse.  With a kernel (kin) its x transform is first turned into that spectrum, scaled, in
-// specOut (which may be kin), to be used as spec or, without data (in null), on its own.
+// specOut (which may be kin), to be used as spec or, without data (in null), on its own; or, for planes of at most
+// kPlanePairMax, with specOut null, used and dropped.
 struct PlaneGeom {
   int Py, Pz;          // at most kPlaneMax each
   int ncols;           // planes (hx)
@@ -184,6 +185,7 @@ struct PlaneGeom {
   ViewOffsets views;                       // batched views: entry b takes spec + views.at[b] instead
 };
 constexpr int kPlaneMax = 128;     // y and z lengths
+constexpr int kPlanePairMax = 96;  // the largest for a kernel's and the data's plane in the LDS together
 constexpr int kPlanarMaxM = 128;   // x passes with planar spectra are compiled for half lengths up to this
 void launch_plane(const PlaneGeom& g, const float2* in, float2* out, const float2* spec, const float2* twY,
                    const float2* twZ, hipStream_t s);

@@ -304,7 +304,8 @@ int Plan::convolve_once(const float* dKernel, const GatherParams& g, float2* spe
   Mid m = convolve_geometry(gg);
   const XFwdGroup groups[2] = {{kernel_gather(dKernel), spec, 1, 0, 0}, {gg, work, 1, 0, 0}};
   xfg(dom, groups, 2, twM, wr, s);
-  m.pl.kin = m.pl.specOut = spec;
+  m.pl.kin = spec;
+  m.pl.specOut = dom.P[1] <= kPlanePairMax && dom.P[2] <= kPlanePairMax ? nullptr : spec;
   m.pl.kScale = inv_scale();
   m.pl.kK[0] = K[1];
   m.pl.kK[1] = K[2];

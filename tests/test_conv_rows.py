@@ -19,10 +19,12 @@ def rel(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
-# the last three grids have strided passes: 135 and 144 points along y or z, 288 along x
+# (130, 7, 9) to (12, 9, 260) have strided passes: 135 and 144 points along y or z, 288 along x; after them planes of 64
+# and 96 points, whose kernel's plane is transformed beside the data's, and of 100, whose kernel's plane goes first
 @pytest.mark.parametrize("shape,k", [((9, 10, 11), (1, 1, 1)), ((13, 6, 17), (4, 6, 2)), ((1, 5, 8), (8, 1, 12)),
                                      ((1, 1, 2), (16, 16, 16)), ((130, 7, 9), (4, 1, 6)), ((6, 131, 20), (3, 12, 4)),
-                                     ((12, 9, 260), (10, 7, 20))])
+                                     ((12, 9, 260), (10, 7, 20)), ((48, 50, 12), (17, 15, 5)),
+                                     ((80, 82, 20), (15, 15, 9)), ((50, 80, 20), (15, 17, 9)), ((86, 50, 12), (15, 15, 5))])
 @pytest.mark.parametrize("ext,value", [("mirror", 0.0), ("value", 0.0), ("value", -2.5)])
 def test_convolution(oracle, shape, k, ext, value):
     rng = np.random.default_rng(sum(shape) * 31 + sum(k))
@@ -30,6 +32,11 @@ def test_convolution(oracle, shape, k, ext, value):
     ker = rng.uniform(0.0, 1.0, k).astype(np.float32)
     ref = oracle.fft_convolve(img.astype(np.float64), ker.astype(np.float64), ext, value, dtype=np.float64)
     assert rel(hip.fft_convolve(img, ker, ext, value), ref) <= 3e-6
+    ti, tk = torch.from_numpy(img).cuda(), torch.from_numpy(ker).cuda()
+    to = torch.full_like(ti, float("nan"))
+    hip.fft_convolve_noalloc(ti.data_ptr(), img.shape, tk.data_ptr(), k, to.data_ptr(), ext, value)
+    torch.cuda.synchronize()
+    assert rel(to.cpu().numpy(), ref) <= 3e-6
 
 
 @pytest.mark.parametrize("shape", [(20, 20, 20), (140, 9, 10)])
