@@ -195,7 +195,8 @@ int mvr_decon_get_geometry(mvr_decon* d, int out[4]);
  * events recorded by the launch itself (the kernel's own execution), the others with events recorded around
  * the launch.  mask bit c enables category c (0 x_fwd, 1 z_fwd, 2 y_conv, 3 z_inv, 4 x_ratio, 5 x_update,
  * 6 x_store, 7 update_mul, 8 reduce); 0 disables.  Small grids run z_fwd, y_conv and z_inv as one launch, which
- * counts for each of them with an equal share of its time.  Totals are cleared by every call. */
+ * counts for each of them with an equal share of its time; so does a launch that serves several views (Mul scheme on
+ * small grids).  Totals are cleared by every call. */
 int mvr_decon_profile(mvr_decon* d, unsigned mask);
 /* the same, timing only the first launch of every group of `every` launches of each enabled category (every
  * >= 1): the events of a timed launch delay the stream by a few microseconds, so a throughput measured over
