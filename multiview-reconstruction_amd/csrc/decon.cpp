@@ -335,6 +335,7 @@ int Decon::init(int psiInit, const float* psiIn) {
 // work spectra.
 int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
   int nS = 1;  // work spectra: one per block of the largest view list
+  plan.planeMax = blocked() || (scheme == SCHEME_MUL && img.size() > 1) ? kPlaneMax : kPlaneMaxSingle;
   if (blocked()) {
     // a block's domain holds its output region plus both kernels' reach on either side, so that both chained
     // convolutions are exact on the effective region: P >= E + 2 (K - 1), output region at m = m1 + m2
@@ -915,6 +916,7 @@ int BlockThread::set_view_kernels(int v, const float* K1, const float* K2, const
   MVR_HIP(hipSetDevice(dev));
   if (plan.xf == nullptr) {
     for (int d = 0; d < 3; ++d) K[d] = Kd[d];
+    plan.planeMax = kPlaneMaxSingle;
     if (plan.create(B, K)) return -1;
     MVR_HIP(hipMalloc(&S, plan.ncpx() * 8));
   } else {

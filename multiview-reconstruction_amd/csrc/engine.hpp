@@ -185,6 +185,9 @@ struct PlaneGeom {
   ViewOffsets views;                       // batched views: entry b takes spec + views.at[b] instead
 };
 constexpr int kPlaneMax = 128;     // y and z lengths
+// the largest for iterations on one grid at a time: 5 view updates with strided passes and planar take, at 96 points, 528
+// and 508 us, at 120 626 and 646, at 128 681 and 695
+constexpr int kPlaneMaxSingle = 96;
 constexpr int kPlanePairMax = 96;  // the largest for a kernel's and the data's plane in the LDS together
 constexpr int kPlanarMaxM = 128;   // x passes with planar spectra are compiled for half lengths up to this
 void launch_plane(const PlaneGeom& g, const float2* in, float2* out, const float2* spec, const float2* twY,

@@ -32,6 +32,7 @@ struct Plan {
   int K[3] = {0, 0, 0};
   int M = 0, Hx = 0;
   bool planar = false;    // spectra [hx][z][y], y and z transforms in one plane pass
+  int planeMax = kPlaneMax;  // the longest y and z of planar spectra; set before create
   const float2* twM = nullptr;  // length-M twiddles (x); the tables are the library's (twiddle_table)
   const float2* wr = nullptr;   // exp(-2 pi i k / P0), k = 0..M
   const float2* twY = nullptr;

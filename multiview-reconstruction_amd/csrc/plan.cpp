@@ -59,7 +59,7 @@ int Plan::create_geometry(const int D[3], const int Kd[3], const int* Pmin) {
   M = dom.P[0] / 2;
   Hx = M + 1;
   dom.HxP = (Hx + 15) / 16 * 16;
-  planar = dom.P[1] <= kPlaneMax && dom.P[2] <= kPlaneMax && M <= kPlanarMaxM;
+  planar = dom.P[1] <= planeMax && dom.P[2] <= planeMax && M <= kPlanarMaxM;
   xf = get_x_fwd(M, planar);
   xfg = planar ? get_x_fwd_groups(M) : nullptr;
   xr = get_x_ratio(M, planar);

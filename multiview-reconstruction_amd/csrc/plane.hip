@@ -15,7 +15,8 @@
 // 12 us on its CU, of which its VALU work is 5.  A 48 x 40 x 33 convolution with its kernel: 43.6 us with three strided
 // passes per transform and direction, 35.0 with this one, 17.3 with the kernel's plane transformed beside the data's.
 // Two views of 64 x 60 x 52, 5 iterations: 527 -> 480 us; 24 batched blocks on 120-point grids, 340 MB: 141 -> 80 us per
-// convolution.  Single grids gain 12-20 % at 48 points, 4-6 % at 96 and nothing at 128, where the range ends with the LDS.
+// convolution.  One grid at a time gains 4-12 % up to 96 points and loses 2-3 % at 120 and 128 (kPlaneMaxSingle); 128 is
+// what the LDS holds.
 #include <type_traits>
 
 #include "passes.hpp"

@@ -39,7 +39,8 @@ def test_convolution(oracle, shape, k, ext, value):
 
 
 @pytest.mark.parametrize("scheme", ["SEQ", "MUL"])
-@pytest.mark.parametrize("shape,k", [((14, 33, 30), 7), ((40, 52, 20), 21), ((98, 20, 36), 31)])
+@pytest.mark.parametrize("shape,k", [((14, 33, 30), 7), ((40, 52, 20), 21), ((98, 20, 36), 31), ((82, 20, 30), 15),
+                                     ((86, 20, 30), 15)])
 def test_deconvolution(oracle, scheme, shape, k):
     w = syn.small_workload(shape=shape, views=3, k=k, psf_type="EFFICIENT_BAYESIAN", weights="zramp")
     inp = syn.make_inputs(w)
