@@ -296,7 +296,8 @@ int mvr_unet_add_volume(mvr_unet* u, const float* const* imgs, const float* cons
                         const int n[3]);
 int mvr_unet_clear_volumes(mvr_unet* u);
 /* one step on batch patches of patch^3 voxels (volume volIdx[b], origin origins[3b..3b+2] as {x, y, z}):
- * forward, mean squared error to the normalised target in *loss, backward; Adam step when update != 0 */
+ * forward, mean squared error to the normalised target in *loss (loss may be NULL), backward; Adam step when
+ * update != 0 */
 int mvr_unet_train_step(mvr_unet* u, const int* volIdx, const int* origins, int batch, int patch, float lr,
                         int update, double* loss);
 /* psiOut[n] = max(minValue, network estimate) for the given views and weights */

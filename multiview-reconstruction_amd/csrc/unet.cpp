@@ -436,7 +436,9 @@ int UNet::train_step(const int* volIdx, const int* origins, int batch, int P, fl
   if (forward(train, true, nullptr, nullptr, nullptr, 0.f)) return -1;
   if (backward(train)) return -1;
   if (update && adam_step(lr)) return -1;
-  return read_loss(train, loss);
+  if (loss) return read_loss(train, loss);
+  MVR_HIP(hipStreamSynchronize(stream));
+  return 0;
 }
 
 // weighted mean intensity sum w_v img_v / sum w_v over voxels and views (FP64 device partials,
