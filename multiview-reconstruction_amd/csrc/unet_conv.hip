@@ -637,8 +637,8 @@ bool launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
   if (a.up_c && (a.up_c % 16 != 0 || a.up_cs % 16 != 0 || !a.up_in || (a.W | a.H | a.D) & 1)) return false;
   if (a.in_half && a.cin != 16) return false;
   if (a.pool_out && !conv_fuses_pool(a)) return false;
-  // the backward ReLU behind the layers of as many inputs as outputs
-  if (a.mask && (a.cin != a.cout || a.cin > 64 || a.pool_out || a.psi.out || a.mask_cs % 4 != 0)) return false;
+  // the backward ReLU behind the layers of 16, 32 or 64 inputs and as many outputs (the kernel of 48 inputs has none)
+  if (a.mask && (a.cin != a.cout || a.cin == 48 || a.cin > 64 || a.pool_out || a.psi.out || a.mask_cs % 4 != 0)) return false;
   if (a.psi.out && (a.cin != 16 || a.cout != 16 || a.N != 1)) return false;
   if (pairs)
     launch_ng<2>(a, s);
