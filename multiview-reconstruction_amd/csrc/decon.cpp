@@ -378,7 +378,9 @@ int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
     specs->resize(V, nullptr);
   }
   specLen = specN;
-  if (S && specN * nS != workLen) {
+  bool complete = true;
+  for (int v = 0; v < nviews; ++v) complete = complete && spec1[v] && spec2[v];
+  if (S && (specN * nS != workLen || (viewBatch > 1 && !complete))) {  // what has to be there comes before a batch
     (void)hipFree(S);
     S = nullptr;
   }
@@ -403,14 +405,26 @@ int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
   if (hipStreamSynchronize(stream) != hipSuccess) rc = -1;
   (void)hipFree(dk);
   if (rc) { set_error("kernel spectra: allocation, copy or transform failed"); return -1; }
-  if (!S) MVR_HIP(hipMalloc(&S, specN * 8 * (size_t)nS));
-  workLen = specN * nS;
   if (scheme == SCHEME_MUL) {
     if (Spsi) (void)hipFree(Spsi);
     if (T2) (void)hipFree(T2);
+    Spsi = nullptr;
+    T2 = nullptr;
     MVR_HIP(hipMalloc(&Spsi, plan.ncpx() * 8));
     MVR_HIP(hipMalloc(&T2, nvox() * 4 * V));
   }
+  // a device without the memory for a whole batch of views runs smaller ones, down to one view a launch
+  // (a host-side failure injection for tests of this: with MVR_TEST_MAX_VIEW_SPECTRA=k larger batches fail)
+  const char* inj = std::getenv("MVR_TEST_MAX_VIEW_SPECTRA");
+  while (!S) {
+    const bool fail = inj && viewBatch > std::max(1, std::atoi(inj));
+    if (!fail && hipMalloc(&S, specN * 8 * (size_t)nS) == hipSuccess) break;
+    S = nullptr;
+    if (viewBatch == 1) { set_error("work spectra: allocation failed"); return -1; }
+    (void)hipGetLastError();
+    nS = viewBatch = viewBatch / 2;
+  }
+  workLen = specN * nS;
   return 0;
 }
 
