@@ -331,6 +331,15 @@ int Decon::init(int psiInit, const float* psiIn) {
   return 0;
 }
 
+// Views of one Mul launch on the plan's grid, while their work spectra are at most kBatchBytes: launches over a small
+// grid neither fill the chip nor hide their ends, and spectra beyond the last-level cache gain nothing.  One view a launch
+// and so, us an iteration: 4 views of 48^3 163 and 79, 3 of 100^3 209 and 123, 8 of 120^3 589 and 323, 4 of 160^3 430 and
+// 342, of 200^3 772 and 712; with no bound 4 of 256^3 take 1425 in place of 1362, 3 of 320^3 2137 in place of 2004.
+int Decon::views_per_launch() const {
+  constexpr size_t kBatchBytes = 256u << 20;
+  return (int)std::max<size_t>(1, std::min<size_t>({(size_t)V, (size_t)kViewBatch, kBatchBytes / (plan.ncpx() * 8)}));
+}
+
 // Plan for the whole volume (FFT lengths >= Pmin where given), kernel spectra of the first nviews views,
 // work spectra.
 int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
@@ -358,15 +367,7 @@ int Decon::build_plan_and_spectra(const int* Pmin, int nviews) {
   plan.wy = tunedW[0];
   plan.wz = tunedW[1];
   viewBatch = 1;
-  if (scheme == SCHEME_MUL) {
-    // Views of one launch, while their work spectra are at most kBatchBytes: launches over a small grid neither fill the
-    // chip nor hide their ends, and spectra beyond the last-level cache gain nothing.  One view a launch and so, us an
-    // iteration: 4 views of 48^3 163 and 79, 3 of 100^3 209 and 123, 8 of 120^3 589 and 323, 4 of 160^3 430 and 342, of
-    // 200^3 772 and 712; with no bound 4 of 256^3 take 1425 in place of 1362, 3 of 320^3 2137 in place of 2004.
-    constexpr size_t kBatchBytes = 256u << 20;
-    viewBatch = (int)std::max<size_t>(1, std::min<size_t>({(size_t)V, (size_t)kViewBatch, kBatchBytes / (plan.ncpx() * 8)}));
-    nS = std::max(nS, viewBatch);
-  }
+  if (scheme == SCHEME_MUL) nS = viewBatch = views_per_launch();
   // buffers of another size, or of views this call leaves out, go first
   const size_t specN = plan.ncpx();
   for (auto* specs : {&spec1, &spec2}) {
@@ -439,9 +440,9 @@ int Decon::set_graph(bool on) {
   return 0;
 }
 
-// Coordinate descent over the compiled FFT lengths of each axis.  A trial rebuilds the plan and view 0's
-// spectra and times view updates (Seq) or iterations (Mul) of view 0 with HIP events; psi is restored
-// from psi0 afterwards.  On any failure the handle is put back on its previous schedule (plan, every view's
+// Coordinate descent over the compiled FFT lengths of each axis.  A trial rebuilds the plan and the spectra of
+// view 0 (Seq) or of the views of one launch (Mul), and times view updates or iterations of them with HIP events;
+// psi is restored from psi0 afterwards.  On any failure the handle is put back on its previous schedule (plan, every view's
 // spectra, work buffers), so that later runs use a complete plan; if even that fails, run() refuses until the
 // next init.
 int Decon::autotune(int candidates, int chosen[3], double* msOut) {
@@ -470,7 +471,7 @@ int Decon::autotune(int candidates, int chosen[3], double* msOut) {
       set_error("autotune: injected trial failure");
       return -1;
     }
-    if (build_plan_and_spectra(P, 1)) return -1;
+    if (build_plan_and_spectra(P, scheme == SCHEME_MUL ? V : 1)) return -1;
     const bool timing = timer.on;
     timer.on = false;
     int rc = scheme == SCHEME_SEQ ? view_seq(0, st) : iteration_mul(st);
@@ -494,7 +495,7 @@ int Decon::autotune(int candidates, int chosen[3], double* msOut) {
     }
     timer.on = timing;
     if (rc) return -1;
-    *ms = best;
+    *ms = scheme == SCHEME_MUL ? best / V : best;
     return 0;
   };
   int rc = 0;
@@ -509,7 +510,7 @@ int Decon::autotune(int candidates, int chosen[3], double* msOut) {
   }
   if (!rc) {
     for (int d = 0; d < 3; ++d) best[d] = plan.dom.P[d];
-    if (scheme == SCHEME_MUL) V = 1;  // time the shared forward transform + one view
+    if (scheme == SCHEME_MUL) V = views_per_launch();  // time the shared forward transform + a launch's views
     tunedW[0] = tunedW[1] = 0;
     if (trial(best, &bestMs)) rc = -1;
   }

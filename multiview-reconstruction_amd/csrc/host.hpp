@@ -233,6 +233,7 @@ struct Decon {
 
   size_t nvox() const { return (size_t)N[0] * N[1] * N[2]; }
   int ensure_partials(int n);
+  int views_per_launch() const;
   int build_plan_and_spectra(const int* Pmin, int nviews);
   void drop_graph();
   // one Seq view update; slot < 0: its statistics reduced into statOut now; slot >= 0: its partials left at
