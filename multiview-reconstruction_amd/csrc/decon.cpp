@@ -727,11 +727,10 @@ int Decon::iteration_mul(double2* statOut) {
   double m = 0;
   for (int v = 0; v < V; ++v) m += maxI[v];
   m /= (double)V;
-  const int o[3] = {0, 0, 0};
   int np = 0;
   if (ensure_partials(2048)) return -1;
   timer.begin(stream, PASS_UPDATE_MUL);
-  launch_update_mul(psi, t2p.data(), wp.data(), V, N, o, N, (double)lambda, minValue, (float)m, partial, &np, stream);
+  launch_update_mul(psi, t2p.data(), wp.data(), V, nvox(), (double)lambda, minValue, (float)m, partial, &np, stream);
   timer.end(stream);
   timer.begin(stream, PASS_REDUCE);
   launch_reduce_stats(partial, np, statOut, stream);
@@ -1091,11 +1090,9 @@ int BlockThread::iterate_mul(int nv, const float* maxIs) {
   double m = 0;
   for (int v = 0; v < nv; ++v) m += maxIs[v];
   m /= (double)nv;
-  const int o[3] = {0, 0, 0};
   int np = 0;
   if (ensure_partials(2048)) return -1;
-  launch_update_mul(psiB, t2p.data(), wp.data(), nv, B, o, B, (double)lambda, minValue, (float)m, partial, &np,
-                    stream);
+  launch_update_mul(psiB, t2p.data(), wp.data(), nv, nb, (double)lambda, minValue, (float)m, partial, &np, stream);
   launch_reduce_stats(partial, np, statDev, stream);
   MVR_HIP(hipGetLastError());
   return 0;

@@ -217,9 +217,8 @@ void launch_reduce_stats_batched(const double2* partial, size_t stride, const in
                                  hipStream_t s);
 int launch_psi_init_partials(const float* const* imgs, int V, size_t n, double* psum, unsigned long long* pcount,
                              float* pmax, hipStream_t s);  // returns #partials
-void launch_update_mul(float* psi, const float* const* T2, const float* const* w, int V, const int N[3],
-                       const int o[3], const int D[3], double lambda, float minValue, float maxI, double2* partial,
-                       int* nPartialOut, hipStream_t s);
+void launch_update_mul(float* psi, const float* const* T2, const float* const* w, int V, size_t n, double lambda,
+                       float minValue, float maxI, double2* partial, int* nPartialOut, hipStream_t s);
 void launch_copy_block_zero(const float* src, const int N[3], const long long off[3], float* dst, const int B[3],
                             hipStream_t s);
 void launch_blocks_with_content(const float* w, const int N[3], const int* tab, int nblocks, int* flags,
@@ -229,7 +228,6 @@ int launch_final_values(float* psi, const float* integral, const float* weight, 
                         float minValue, float maxI, double2* partial, int maxPartials, hipStream_t s);
 // out[v] = factors[v][nf - 1] * ... * factors[v][0] * first[v], multiplied in the order of the factors, arrays of nk
 void launch_psf_products(const float* first, const float* factors, int V, int nf, size_t nk, float* out, hipStream_t s);
-void launch_scale_copy_kernel_spectrum(const float2* in, float2* out, size_t n, float scale, hipStream_t s);
 void launch_rel_l2(const float* a, const float* b, size_t n, double2* partial, double2* out, hipStream_t s);
 int launch_psi_approx_slice(const float* img, const int N[3], double2* partial, hipStream_t s);
 void launch_fused_nonzero(const float* const* imgs, const float* const* ws, int V, size_t n, float* out,

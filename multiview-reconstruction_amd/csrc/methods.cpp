@@ -107,9 +107,8 @@ int mvr_compute_final_values_mul(int dev, float* psi, int numViews, const float*
   }
   MVR_HIP(hipMalloc(&part.p, sizeof(double2) * kMaxPartials));
   MVR_HIP(hipMalloc(&out.p, sizeof(double2)));
-  const int N[3] = {(int)n, 1, 1}, o[3] = {0, 0, 0}, D[3] = {(int)n, 1, 1};
   int np = 0;
-  launch_update_mul(dp.f(), ip.data(), wp.data(), numViews, N, o, D, lambda, minIntensity, maxIntensity,
+  launch_update_mul(dp.f(), ip.data(), wp.data(), numViews, (size_t)n, lambda, minIntensity, maxIntensity,
                     static_cast<double2*>(part.p), &np, st.s);
   launch_reduce_stats(static_cast<double2*>(part.p), np, static_cast<double2*>(out.p), st.s);
   MVR_HIP(hipGetLastError());

@@ -276,29 +276,20 @@ __device__ __forceinline__ double nth_root(double x, int V, double invV) {
   return x == 0.0 ? 0.0 : x == -__builtin_inf() ? -x : x < 0.0 ? __builtin_nan("") : x;
 }
 
-// Bound by HBM (4 (2 V + 2) bytes a voxel): the views' values are loaded four views at a time ahead of their products, a
-// whole volume's voxels (WHOLE) need no coordinates, and the root takes a fifth of pow's instructions.
+// Bound by HBM (4 (2 V + 2) bytes a voxel): the views' values are loaded four views at a time ahead of their products, and
+// the root takes a fifth of pow's instructions.
 // 160 x 150 x 140, 4 views: 53.7 us with pow and a coordinate division per voxel, 27.7 (4.8 TB/s) so.
-template <bool WHOLE>
-__global__ __launch_bounds__(kThreads) void k_update_mul(float* __restrict__ psi, ViewPtrsW vp, int V, int3 N,
-                                                         int3 o, int3 D, double lambda, float minI, float maxI,
+__global__ __launch_bounds__(kThreads) void k_update_mul(float* __restrict__ psi, ViewPtrsW vp, int V, size_t n,
+                                                         double lambda, float minI, float maxI,
                                                          double2* __restrict__ partial) {
   // Java rounds every float and double operation: no FMA contraction in the update
 #pragma clang fp contract(off)
-  const size_t nvox = (size_t)D.x * D.y * D.z;
   double sumc = 0.0;
   float mxc = -1.f;
   const double invV = 1.0 / (double)V;
   const RLConsts rc = rl_consts(lambda, minI, maxI);
-  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < nvox; i += (size_t)gridDim.x * kThreads) {
-    size_t gi = i;
-    if (!WHOLE) {
-      const int lx = (int)(i % D.x);
-      const size_t r = i / D.x;
-      const int ly = (int)(r % D.y), lz = (int)(r / D.y);
-      gi = ((size_t)(o.z + lz) * N.y + (o.y + ly)) * N.x + (o.x + lx);
-    }
-    const float last = psi[gi];
+  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads) {
+    const float last = psi[i];
     double sumW = 0.0, prod = 1.0;
     for (int v0 = 0; v0 < V; v0 += 4) {
       float t[4], w[4];
@@ -306,7 +297,7 @@ __global__ __launch_bounds__(kThreads) void k_update_mul(float* __restrict__ psi
       for (int j = 0; j < 4; ++j) {
         const int v = min(v0 + j, V - 1);
         t[j] = vp.t2[v][i];
-        w[j] = vp.w[v][gi];
+        w[j] = vp.w[v][i];
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -319,7 +310,7 @@ __global__ __launch_bounds__(kThreads) void k_update_mul(float* __restrict__ psi
     sumW = fmin(1.0, sumW);
     const float next = rl_tikhonov_adjust(last * (float)prod, rc);
     const float res = last + (next - last) * (float)sumW;
-    psi[gi] = res;
+    psi[i] = res;
     const float ch = res - last;
     sumc += (double)ch;
     mxc = java_maxf(mxc, ch);
@@ -327,17 +318,12 @@ __global__ __launch_bounds__(kThreads) void k_update_mul(float* __restrict__ psi
   block_reduce_stats(sumc, mxc, partial + blockIdx.x);
 }
 
-void launch_update_mul(float* psi, const float* const* T2, const float* const* w, int V, const int N[3],
-                       const int o[3], const int D[3], double lambda, float minValue, float maxI, double2* partial,
-                       int* nPartialOut, hipStream_t s) {
+void launch_update_mul(float* psi, const float* const* T2, const float* const* w, int V, size_t n, double lambda,
+                       float minValue, float maxI, double2* partial, int* nPartialOut, hipStream_t s) {
   ViewPtrsW vp{};
   for (int v = 0; v < V && v < kMaxViews; ++v) { vp.t2[v] = T2[v]; vp.w[v] = w[v]; }
-  const size_t nvox = (size_t)D[0] * D[1] * D[2];
-  const int nb = (int)std::min<size_t>((nvox + kThreads - 1) / kThreads, 2048);
-  bool whole = true;
-  for (int k = 0; k < 3; ++k) whole = whole && o[k] == 0 && D[k] == N[k];
-  hipLaunchKernelGGL(whole ? k_update_mul<true> : k_update_mul<false>, dim3(nb), dim3(kThreads), 0, s, psi, vp, V,
-                     make_int3(N[0], N[1], N[2]), make_int3(o[0], o[1], o[2]), make_int3(D[0], D[1], D[2]), lambda, minValue, maxI, partial);
+  const int nb = (int)std::min<size_t>((n + kThreads - 1) / kThreads, 2048);
+  hipLaunchKernelGGL(k_update_mul, dim3(nb), dim3(kThreads), 0, s, psi, vp, V, n, lambda, minValue, maxI, partial);
   *nPartialOut = nb;
 }
 
@@ -485,16 +471,6 @@ void launch_rel_l2(const float* a, const float* b, size_t n, double2* partial, d
   const int nb = (int)std::max<size_t>(1, std::min<size_t>((n + kThreads - 1) / kThreads, 1024));
   hipLaunchKernelGGL(k_rel_l2_partials, dim3(nb), dim3(kThreads), 0, s, a, b, n, partial);
   hipLaunchKernelGGL(k_sum2, dim3(1), dim3(kThreads), 0, s, partial, nb, out);
-}
-
-__global__ void k_scale_copy(const float2* __restrict__ in, float2* __restrict__ out, size_t n, float scale) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    out[i] = cscale(in[i], scale);
-}
-
-void launch_scale_copy_kernel_spectrum(const float2* in, float2* out, size_t n, float scale, hipStream_t s) {
-  const int nb = (int)std::min<size_t>((n + kThreads - 1) / kThreads, 4096);
-  hipLaunchKernelGGL(k_scale_copy, dim3(nb > 0 ? nb : 1), dim3(kThreads), 0, s, in, out, n, scale);
 }
 
 }  // namespace mvr

@@ -35,25 +35,6 @@ __device__ __forceinline__ int mirror_index(int p, int n) {
   return p >= n ? period - p : p;
 }
 
-__device__ __forceinline__ float gather_value(const GatherParams& g, const Dom& d, int x, int y, int z) {
-  if (g.mode == GATHER_MIRROR) {
-    const int gx = mirror_index(g.org[0] + x, g.N[0]);
-    const int gy = mirror_index(g.org[1] + y, g.N[1]);
-    const int gz = mirror_index(g.org[2] + z, g.N[2]);
-    return g.src[((size_t)gz * g.N[1] + gy) * g.N[0] + gx];
-  } else if (g.mode == GATHER_VALUE) {
-    const int gx = g.org[0] + x, gy = g.org[1] + y, gz = g.org[2] + z;
-    if (gx < 0 || gy < 0 || gz < 0 || gx >= g.N[0] || gy >= g.N[1] || gz >= g.N[2]) return g.value;
-    return g.src[((size_t)gz * g.N[1] + gy) * g.N[0] + gx];
-  } else {
-    const int jx = (x + g.N[0] / 2) % d.P[0];
-    const int jy = (y + g.N[1] / 2) % d.P[1];
-    const int jz = (z + g.N[2] / 2) % d.P[2];
-    if (jx >= g.N[0] || jy >= g.N[1] || jz >= g.N[2]) return 0.f;
-    return g.src[((size_t)jz * g.N[1] + jy) * g.N[0] + jx];
-  }
-}
-
 // ------------------------------------------------------------------ update of psi
 // DeconvolutionMethods.computeNextValue (D/iteration/sequential/DeconvolutionMethods.java:320-358),
 // float operations in Java order; Tikhonov in double.  Java rounds every float and double operation, so the

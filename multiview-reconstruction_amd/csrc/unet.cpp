@@ -186,7 +186,7 @@ bool UNet::conv(int l, const uint16_t* in, int in_cs, int in_co, uint16_t* out, 
   c.pool_cs = pool_cs;
   const bool fused = pool && conv_fuses_pool(c);
   if (!fused) c.pool_out = nullptr;
-  if (!launch_conv_fwd(c, stream)) convFailed = true;
+  if (!launch_conv_tiled(c, stream)) convFailed = true;
   return fused;
 }
 
@@ -208,7 +208,7 @@ void UNet::dgrad(int l, const uint16_t* dout, int dout_cs, int dout_co, uint16_t
   c.N = N; c.D = D; c.H = H; c.W = W;
   c.taps = 27;
   c.relu = 0;
-  if (!launch_conv_fwd(c, stream)) convFailed = true;
+  if (!launch_conv_tiled(c, stream)) convFailed = true;
 }
 
 void UNet::wgrad(int l, const uint16_t* in, int in_cs, const uint16_t* dout, int dout_cs, int dout_co, int N, int D,

@@ -24,12 +24,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
   return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);  // round to nearest even
 }
 
-// ------------------------------------------------------------------ convolution (forward and data gradient)
-// The 3^3 convolutions run in the LDS-tiled kernel of unet_conv.hip (launch_conv_tiled).
-
-// ------------------------------------------------------------------ weight gradient
-// Weight and bias gradients: unet_wgrad.hip.
-
 // ------------------------------------------------------------------ elementwise pieces
 // All work on units of 8 channels (16 bytes); channel counts, strides and offsets are multiples of 16.
 typedef __attribute__((ext_vector_type(8))) unsigned short u16x8;
@@ -278,20 +272,6 @@ __global__ __launch_bounds__(256) void k_adam(AdamArgs a) {
   }
 }
 
-__global__ void k_f32_to_bf16(const float* __restrict__ src, uint16_t* __restrict__ dst, size_t n) {
-  for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (size_t)gridDim.x * blockDim.x)
-    dst[j] = f2bf(src[j]);
-}
-
-__global__ void k_bf16_to_f32(const uint16_t* __restrict__ src, float* __restrict__ dst, size_t n) {
-  for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (size_t)gridDim.x * blockDim.x)
-    dst[j] = bf2f(src[j]);
-}
-
-__global__ void k_zero_u16(uint16_t* __restrict__ p, size_t n) {
-  for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (size_t)gridDim.x * blockDim.x) p[j] = 0;
-}
-
 // normalisation of the network input: partial[b] = {sum w_v img_v, sum w_v} (FP64) over a
 // grid-stride share of the voxels and all views; the scale is the ratio of the totals
 __global__ __launch_bounds__(256) void k_wsum_partials(InputArgs a, size_t n, double2* __restrict__ partial) {
@@ -365,10 +345,6 @@ static inline int grid1(size_t n, int cap = 8192) {
   return (int)(b < 1 ? 1 : (b > (size_t)cap ? (size_t)cap : b));
 }
 
-bool launch_conv_fwd(const ConvArgs& a, hipStream_t s) {
-  // every layer of the network has cin, cout and channel strides that are multiples of 16
-  return launch_conv_tiled(a, s);
-}
 void launch_pool_fwd(const uint16_t* in, int ics, int ico, uint16_t* out, int ocs, int C, int N, int D, int H, int W,
                      hipStream_t s) {
   const int units = W * (C / 8);
@@ -415,19 +391,9 @@ void launch_adam(const AdamArgs& a, hipStream_t s) {
   }
   hipLaunchKernelGGL(k_adam, dim3(nwg), dim3(256), 0, s, b);
 }
-void launch_f32_to_bf16(const float* src, uint16_t* dst, size_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_f32_to_bf16, dim3(grid1(n)), dim3(256), 0, s, src, dst, n);
-}
-void launch_bf16_to_f32(const uint16_t* src, float* dst, size_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_bf16_to_f32, dim3(grid1(n)), dim3(256), 0, s, src, dst, n);
-}
 int launch_wsum_partials(const InputArgs& a, size_t n, double2* partial, hipStream_t s) {
   const int nb = grid1(n, 1024);
   hipLaunchKernelGGL(k_wsum_partials, dim3(nb), dim3(256), 0, s, a, n, partial);
   return nb;
 }
-void launch_zero_u16(uint16_t* p, size_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_u16, dim3(grid1(n)), dim3(256), 0, s, p, n);
-}
-
 }  // namespace mvr

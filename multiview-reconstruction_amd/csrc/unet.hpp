@@ -119,8 +119,7 @@ struct PatchArgs {
   float* target_out;
 };
 
-bool launch_conv_fwd(const ConvArgs& a, hipStream_t s);  // false: shape not supported, nothing launched
-// LDS-tiled 3^3 convolution (unet_conv.hip); false when the shape is not one it covers
+// 3^3 convolution (unet_conv.hip); false when the shape is not one it covers, nothing launched
 bool launch_conv_tiled(const ConvArgs& a, hipStream_t s);
 bool conv_fuses_pool(const ConvArgs& a);  // the launch also writes the pooled output (pool_out set, even dimensions)
 // weight and bias gradient partials of a 3^3 layer (cin and cout multiples of 16); returns how many partitions
@@ -148,9 +147,6 @@ void launch_pack_input(const InputArgs& a, hipStream_t s);
 int launch_head(const HeadArgs& a, hipStream_t s);
 int launch_head_bwd(const HeadArgs& a, uint16_t* dd1, float* partial, hipStream_t s);
 void launch_adam(const AdamArgs& a, hipStream_t s);
-void launch_f32_to_bf16(const float* src, uint16_t* dst, size_t n, hipStream_t s);
-void launch_bf16_to_f32(const uint16_t* src, float* dst, size_t n, hipStream_t s);
-void launch_zero_u16(uint16_t* p, size_t n, hipStream_t s);
 int launch_wsum_partials(const InputArgs& a, size_t n, double2* partial, hipStream_t s);
 
 }  // namespace mvr

@@ -589,7 +589,7 @@ void launch_ng(const ConvArgs& a, hipStream_t s) {
     if (a.psi.out)
       hipLaunchKernelGGL((k_conv_column<1, kHead>), grid, dim3(256), 0, s, a, zp);
     else if (a.pool_out)
-      hipLaunchKernelGGL((k_conv_column<NG, kPool>), grid, dim3(256), 0, s, a, zp);
+      hipLaunchKernelGGL((k_conv_column<1, kPool>), grid, dim3(256), 0, s, a, zp);
     else if (a.mask)
       hipLaunchKernelGGL((k_conv_column<1, kMask>), grid, dim3(256), 0, s, a, zp);
     else
@@ -621,9 +621,9 @@ void launch_ng(const ConvArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// pooling is fused into the one-chunk layers and the 32-channel inputs of even output groups
+// pooling is fused into the layers of 16 inputs and 16 outputs and of 32 inputs and an even number of output blocks
 bool conv_fuses_pool(const ConvArgs& a) {
-  return a.pool_out && !((a.D | a.H | a.W) & 1) && (a.cin == 16 || (a.cin == 32 && a.cout % 32 == 0));
+  return a.pool_out && !((a.D | a.H | a.W) & 1) && ((a.cin == 16 && a.cout == 16) || (a.cin == 32 && a.cout % 32 == 0));
 }
 
 // The network's 3^3 convolutions: cout a multiple of 16; cin 16, or 32 and 48 for an odd number of 16-channel output
