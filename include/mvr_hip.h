@@ -77,7 +77,8 @@ int mvr_fft_lengths(int* out, int cap);
  * device memory (code under HIP graph capture, tight serving loops).  img, kernel and out must be device memory
  * of `dev` (refused otherwise); the kernel spectrum and the work spectrum live in one static device array
  * of MVR_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends, so FFT grids up to about 180^3 fit (e.g. a
- * 128^3 block with a 41^3 kernel; the two spectra and the sizes of the four twiddle tables are counted); larger ones are refused with an error before any device work.
+ * 128^3 block with a 41^3 kernel; the two spectra and the sizes of the four twiddle tables are counted); larger
+ * ones are refused with an error before any device work.
  * The kernels are enqueued on `stream` (a hipStream_t; NULL = the default stream) and the call returns without
  * waiting: synchronise the stream before reading out.  All calls on one GPU share its array, so calls that
  * overlap on one GPU race: serialise them (one stream). ---- */

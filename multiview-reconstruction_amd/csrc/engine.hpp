@@ -185,8 +185,14 @@ struct PlaneGeom {
   ViewOffsets views;                       // batched views: entry b takes spec + views.at[b] instead
 };
 constexpr int kPlaneMax = 128;     // y and z lengths
-// the largest for iterations on one grid at a time: 5 view updates with strided passes and planar take, at 96 points, 528
-// and 508 us, at 120 626 and 646, at 128 681 and 695
+// the largest for iterations on one grid at a time: 5 view updates with strided passes and planar take, at 96^3 points, 528
+// and 508 us, at 120^3 626 and 646, at 128^3 681 and 695.  The rules look at y and z alone, though a launch has a plane per
+// x frequency, at most P0 / 2 + 1 of them.  8 view updates, us, strided and planar, at P0 points along x:
+//   64 x 64 points (y, z): P0 = 16 362 and 328, 32 387 and 355, 64 399 and 376, 128 459 and 438, 256 529 and 494
+//   96 x 96:               16 398 and 412, 32 445 and 434, 48 452 and 455, 64 473 and 464, 128 578 and 556, 256 773 and 708
+// One convolution, as far as kPlaneMax: 96 x 96 30.5 and 22.1 at P0 = 16, 36.0 and 24.8 at 64; 128 x 128 33.6 and 36.8 at
+// 16, 37.0 and 39.1 at 32, 44.2 and 42.2 at 64, 57.4 and 49.6 at 128.  So nine planes of 96 x 96 (batches of views and
+// blocks multiply the planes) and up to 17 of 128 x 128 would be 3-9 % faster with strided passes.
 constexpr int kPlaneMaxSingle = 96;
 constexpr int kPlanePairMax = 96;  // the largest for a kernel's and the data's plane in the LDS together
 constexpr int kPlanarMaxM = 128;   // x passes with planar spectra are compiled for half lengths up to this

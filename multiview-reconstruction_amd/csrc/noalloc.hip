@@ -1,13 +1,14 @@
 // noalloc.hip -- mvr_fft_convolve_noalloc: one FFT convolution (util.FFTConvolution semantics, as
 // mvr_fft_convolve) that allocates no device memory.
 //
-// The twiddle tables, the kernel spectrum and the work spectrum live in `scratch`, a static device array of
-// MVR_NOALLOC_SCRATCH_BYTES that every GPU the library runs on holds until the process ends.  In host code the
-// array's name is only a stand-in for the symbol: its device address is looked up once per device
+// The kernel spectrum and the work spectrum live in `scratch`, a static device array of MVR_NOALLOC_SCRATCH_BYTES
+// that every GPU the library runs on holds until the process ends; the twiddle tables are the library's own.  In
+// host code the array's name is only a stand-in for the symbol: its device address is looked up once per device
 // (hipGetSymbolAddress with that device current) and that address is what the kernels receive.  Nothing in the
-// array has to start at zero: every byte a call reads was written earlier in the same call (twiddles by
-// k_twiddles, both spectra by the forward x pass over every row and half-spectrum column).  All calls on one GPU
-// share its array, so calls that overlap on one GPU race; the caller serialises them (one stream).
+// array has to start at zero: the forward x pass writes the rows that hold source or kernel values, and the passes
+// after it read those only (mirror copies from their sources, constants and zeros without a read), apart from the
+// row pitch's padding columns, whose results are not stored.  All calls on one GPU share its array, so calls that
+// overlap on one GPU race; the caller serialises them (one stream).
 #include <mutex>
 #include <string>
 
@@ -54,7 +55,8 @@ extern "C" int mvr_fft_convolve_noalloc(int dev, const float* img, const int n[3
   // geometry and the scratch layout first, on the host: sizes beyond the array are refused before device work
   Plan plan;
   if (plan.create_geometry(n, k)) return -1;
-  // (the limit counts the transforms' four twiddle tables with the two spectra)
+  // (the limit counts four twiddle tables with the two spectra, as it did when the array held them: callers choose
+  // this entry point or mvr_fft_convolve by what it refuses)
   const size_t oWork = align256(plan.ncpx() * 8);
   const size_t tables = align256((size_t)plan.M * 8) + align256((size_t)(plan.M + 1) * 8) +
                         align256((size_t)plan.dom.P[1] * 8) + align256((size_t)plan.dom.P[2] * 8);

@@ -14,9 +14,9 @@
 // Bound by the LDS round trips (eleven over a plane) and, at one plane per CU, by their latency: an 80 x 72 plane takes
 // 12 us on its CU, of which its VALU work is 5.  A 48 x 40 x 33 convolution with its kernel: 43.6 us with three strided
 // passes per transform and direction, 35.0 with this one, 17.3 with the kernel's plane transformed beside the data's.
-// Two views of 64 x 60 x 52, 5 iterations: 527 -> 480 us; 24 batched blocks on 120-point grids, 340 MB: 141 -> 80 us per
-// convolution.  One grid at a time gains 4-12 % up to 96 points and loses 2-3 % at 120 and 128 (kPlaneMaxSingle); 128 is
-// what the LDS holds.
+// Two views of 64 x 60 x 52, 5 iterations: 533 -> 492 us; 24 batched blocks on 120-point grids, 340 MB: 141 -> 80 us per
+// convolution.  One cubic grid at a time gains 2-12 % up to 96 points and loses 2-3 % at 120 and 128 (kPlaneMaxSingle,
+// where grids short along x are listed too); 128 is what the LDS holds.
 #include <type_traits>
 
 #include "passes.hpp"

@@ -28,7 +28,7 @@ struct ConvArgs {
   int out_cs, out_co;
   int cout;            // multiple of 16
   int N, D, H, W;
-  int taps;            // 27 (3^3, zero padding 1) or 1
+  int taps;            // 27 (3^3, zero padding 1)
   int relu;
   // optional fused nearest x2 upsampling: input channels [0, up_c) are read from up_in (channel stride
   // up_cs) at half the coordinates, channels [up_c, cin) from in (its channel 0 = input channel up_c)

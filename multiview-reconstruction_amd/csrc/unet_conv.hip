@@ -5,10 +5,10 @@
 // planes) for NG x 16 output channels (grid.y selects the channel group):
 //   - an input may be a concatenation [up(coarse), fine] whose first part is read from the coarse
 //     tensor at half the coordinates (nearest x2 upsampling fused into the staging);
-//   - the input goes through LDS one 16-channel chunk and one 18 x 18 halo plane at a time, in a ring of four planes:
-//     while the products of one output plane run on three of them, LDS-DMA loads (global_load_lds_dwordx4: 16 bytes
-//     per lane straight into LDS at the wave's base + 16 lane) fill the fourth with the next plane, so each input
-//     plane crosses LDS once per work-group.  Halo voxels outside the volume read a zero in device memory.  Each
+//   - the input goes through LDS one 16-channel chunk and one 18 x 18 halo plane at a time, in a ring of five planes
+//     (one chunk) or six (several): while the products of one output plane run on three of them, LDS-DMA loads
+//     (global_load_lds_dwordx4: 16 bytes per lane straight into LDS at the wave's base + 16 lane) fill the others with
+//     the planes that come next, so each input plane crosses LDS once per work-group.  Halo voxels outside the volume read a zero in device memory.  Each
 //     plane is stored as two 8-channel halves [half][voxel][8], so that the 16 lanes reading one half of 16
 //     consecutive voxels touch 256 contiguous bytes (no bank conflicts);
 //   - v_mfma_f32_16x16x32_bf16 takes K = 32 as two taps x 16 channels: lanes 0-31 carry tap 2p,
@@ -25,9 +25,11 @@
 // and over the tap pairs in order within a chunk).
 //
 // Bound by the LDS reads of the voxel fragments: a fragment (1 KB, 8 clocks of the CU's LDS) feeds NG products of 16
-// clocks, so 16 -> 16 layers cannot run faster than 0.75 us per plane tile and CU (191 us at 252 x 250 x 254; 272 measured,
-// 520 with the weights read from LDS and three halo planes staged per output plane); the wide layers lose the rest to
-// the weight reloads between chunks.  One inference at 252 x 250 x 254, 6 views: 4.75 -> 3.05 ms, with the skip tensors
+// clocks, so 16 -> 16 layers that read one for each product take 0.75 us at least per plane tile and CU (191 us at
+// 252 x 250 x 254; 272 measured, 520 with the weights read from LDS and three halo planes staged per output plane); the
+// wide layers lose the rest to the weight reloads between chunks.  Of the 56 fragments that a wave reads per output plane
+// more than half repeat values of the same input plane (25 are distinct over the three outputs it serves); taking each once
+// needs three outputs' accumulators at a time, in the same order of every sum.  One inference at 252 x 250 x 254, 6 views: 4.75 -> 3.05 ms, with the skip tensors
 // stored without the upsampled channels beside them (the pooled layer 734 -> 312 us) and the head fused behind the last
 // layer.
 #include <hip/hip_runtime.h>

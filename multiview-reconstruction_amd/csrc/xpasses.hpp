@@ -9,8 +9,14 @@
 // the work-group then, and on long rows (B > 16) where that leaves a wave without any.  Elsewhere the aligned rows are
 // faster, at M = 225 by 10 %: their exchange has fewer LDS conflicts.  Values next to one another in the real rows move in pairs; whether a pair
 // lies inside the row is a question of the register index, not of the lane, except at the row's ends.  Measured, one
-// iteration of two views: M = 200 1.08 x, 288 1.06, 400 1.13, 480 1.08, 640 1.11; M = 432, 767 x 700 x 321: forward
-// 197 -> 144 us, quotient 852 -> 690, update 851 -> 701 (2.9 -> 3.3 TB/s).
+// iteration of two views: M = 200 1.08 x, 288 1.06; M = 432, 767 x 700 x 321: forward 197 -> 144 us, quotient 852 -> 690,
+// update 851 -> 701 (2.9 -> 3.3 TB/s).  Long rows (B > 16), 2 M - 30 wide, 27300 rows, with the quotient and the update on
+// the registers that the inverse leaves and aligned rows, and so (us a launch, and the whole iteration):
+//   M           360    400    432    450    480    512    540    576    600    640
+//   forward     54 32  59 38  57 42  63 45  66 45  76 56  80 58  78 54  82 55  85 56
+//   quotient    93 70  99 81 107 91 118 96 120 108 136 127 131 108 134 132 174 128 178 131
+//   update     105 83 119 90 118 104 126 104 140 113 112 110 152 119 160 146 183 156 193 161
+//   iteration  1.12x  1.12x  1.08x  1.07x  1.07x  1.02x  1.10x  1.05x  1.11x  1.11x  (M = 300 1.05x, 320 1.07x, 384 1.01x)
 //
 // The R2C post-processing and the C2R pre-processing combine
 // the values k and M - k of a row; after the second forward step (before the first inverse step) lane q holds
@@ -119,7 +125,10 @@ struct XCfg {
   // SIMD allow; bounded to 6 waves it takes 80 without spilling (x_ratio 4 % faster at M = 150).  Other lengths
   // either fit already or would spill under the bound.
   static constexpr int MINW_RATIO = (M == 100 || M == 120 || M == 150 || M == 200) ? 6 : 1;
-  // The update takes 128 VGPRs and two spilled ones in place of 130-148: 4 waves per SIMD (M = 432: 778 -> 701 us)
+  // The update at M = 432, 450, 480 compiles to 130, 130 and 148 VGPRs (this ROCm), over the 128 that 4 waves per SIMD allow;
+  // bounded to 4 waves it takes 128 and spills one (113 -> 104, 114 -> 104, 123 -> 113 us for 27300 rows; M = 432, 225000
+  // rows: 778 -> 701).  The other long rows: M = 300 to 400, 512 and 540 take 96-126 without a bound; 576 and 600 (162, 160)
+  // would spill 22 (146 -> 157 us, 156 -> 156); 640 fits 3 work-groups per CU by its LDS.
   static constexpr int MINW_UPDATE = (M == 432 || M == 450 || M == 480) ? 4 : 1;
 };
 
@@ -569,7 +578,7 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_RATIO) void k_x2_ratio(
   x2_inverse_half_regs<M, TR>(!rowOnes ? Sin + so : nullptr, buf, tw, twr, l, z, cs);
   // park the blurred rows in LDS, form the quotient there with TQ lanes per row, all of a lane's image values in flight
   // at once at offsets from the lane's row pointers known at compile time, and run the forward transform from LDS.
-  // Positions x = q + TQ i, or on long rows pairs (at M = 432 16 % faster than the quotient on the B side's registers;
+  // Positions x = q + TQ i, or on long rows pairs (at M = 432 16 % faster than the quotient on the B side's registers, 1-27 % at the other lengths above;
   // at M = 150 and 225 pairs are 3-5 % slower, a flat mapping over the work-group 4 %, a wave walking its rows 9 %)
   x2_park_inverse<M>(buf, l, z);
   const int r = (int)threadIdx.x / C::TQ, q = (int)threadIdx.x % C::TQ;
@@ -692,7 +701,8 @@ __global__ __launch_bounds__(XCfg<M>::NT, XCfg<M>::MINW_UPDATE) void k_x2_update
   constexpr int U = 4;
   if constexpr (C::long_rows) {
     // long rows: TQ lanes per row at offsets uniform over the work-group; only a row's last pairs test their positions.
-    // At M = 432 778 us for 225 000 rows, 807 with the flat mapping below, 855 on the B side's registers
+    // At M = 432 778 us for 225 000 rows, 807 with the flat mapping below, 855 on the B side's registers (the other lengths:
+    // the head of this file)
     const int r = (int)threadIdx.x / C::TQ, q = (int)threadIdx.x % C::TQ;
     const long long pr = C::RW * C::TQ == C::NT || r < C::RW ? psiRow[r] : -1;
     if (pr >= 0) {
