@@ -232,6 +232,9 @@ void launch_blocks_with_content(const float* w, const int N[3], const int* tab, 
 void launch_quotient(const float* img, float* blurred, size_t n, hipStream_t s);
 int launch_final_values(float* psi, const float* integral, const float* weight, size_t n, double lambda,
                         float minValue, float maxI, double2* partial, int maxPartials, hipStream_t s);
+// The kernels of the second kernels' products, arrays of dims K: of V given ones those as given of the views 1.., those
+// divided by sums[v] of the views 0.., the same mirrored, and those as given mirrored.
+void launch_psf_kernels(const float* given, const double* sums, int V, const int K[3], float* out, hipStream_t s);
 // out[v] = factors[v][nf - 1] * ... * factors[v][0] * first[v], multiplied in the order of the factors, arrays of nk
 void launch_psf_products(const float* first, const float* factors, int V, int nf, size_t nk, float* out, hipStream_t s);
 void launch_rel_l2(const float* a, const float* b, size_t n, double2* partial, double2* out, hipStream_t s);

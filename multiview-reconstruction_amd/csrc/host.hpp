@@ -93,8 +93,8 @@ struct Plan {
 
   // spectrum of a device kernel (K layout), scaled by the inverse-FFT factor
   int kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const;
-  // planar plans: the second half of kernel_spectrum for n x transforms, ncpx() apart, in place
-  void kernel_planes(float2* spec, int n, hipStream_t s) const;
+  // planar plans: the second half of kernel_spectrum for n x transforms, `stride` apart, in place
+  void kernel_planes(float2* spec, int n, size_t stride, hipStream_t s) const;
   // the gather of a kernel
   GatherParams kernel_gather(const float* dKernel) const;
   // one convolution with a kernel used once: kernel_spectrum and convolve, on planar plans in three launches
@@ -112,7 +112,7 @@ struct Plan {
 int init_psfs(int dev, std::vector<std::vector<float>>& k1, const int K[3], int psfType, int nT,
               std::vector<std::vector<float>>& k2, hipStream_t s);
 double sum_img_quirk(const float* a, size_t n, int nT);
-void norm_to_sum1(float* a, size_t n, int nT);
+double norm_to_sum1(float* a, size_t n, int nT);
 void mirror_all(float* a, const int dim[3]);
 
 enum { PSF_OPT_II = 0, PSF_OPT_I = 1, PSF_EFFICIENT_BAYESIAN = 2, PSF_INDEPENDENT = 3 };

@@ -65,6 +65,33 @@ void launch_reduce_stats_batched(const double2* partial, size_t stride, const in
   hipLaunchKernelGGL(k_reduce_stats_batched, dim3(nUpdates), dim3(kThreads), 0, s, partial, stride, c, out);
 }
 
+// Divided as the host normalises, (float)((double)x / sum), and mirrored as the host mirrors: an even axis leaves its middle
+// pair in place (Mirror.mirror, D/util/Mirror.java:55-132).
+__device__ __forceinline__ int psf_mirror(int i, int n) {
+  return n % 2 == 0 && (i == n / 2 || i == n / 2 - 1) ? i : n - 1 - i;
+}
+__global__ __launch_bounds__(kThreads) void k_psf_kernels(const float* __restrict__ given, const double* __restrict__ sums,
+                                                          int V, int3 K, float* __restrict__ out) {
+  const size_t nk = (size_t)K.x * K.y * K.z, i = (size_t)blockIdx.x * kThreads + threadIdx.x, v = blockIdx.y;
+  if (i >= nk) return;
+  const int x = (int)(i % K.x), y = (int)(i / K.x % K.y), z = (int)(i / K.x / K.y);
+  const size_t m = ((size_t)psf_mirror(z, K.z) * K.y + psf_mirror(y, K.y)) * K.x + psf_mirror(x, K.x);
+  const float a = given[v * nk + i], b = given[v * nk + m];
+  const double sum = sums[v];
+  out[(V - 1 + v) * nk + i] = (float)((double)a / sum);
+  out[(2 * V - 1 + v) * nk + i] = (float)((double)b / sum);
+  if (v > 0) {
+    out[(v - 1) * nk + i] = a;
+    out[(3 * V - 2 + v) * nk + i] = b;
+  }
+}
+
+void launch_psf_kernels(const float* given, const double* sums, int V, const int K[3], float* out, hipStream_t s) {
+  const size_t nk = (size_t)K[0] * K[1] * K[2];
+  hipLaunchKernelGGL(k_psf_kernels, dim3((unsigned)((nk + kThreads - 1) / kThreads), V), dim3(kThreads), 0, s, given, sums,
+                     V, make_int3(K[0], K[1], K[2]), out);
+}
+
 __global__ __launch_bounds__(kThreads) void k_psf_products(const float* first, const float* __restrict__ factors, int nf,
                                                            size_t nk, float* out) {
   const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x, v = blockIdx.y;

@@ -235,10 +235,10 @@ void Plan::mid_rest(const Mid& m, const float2* in, float2* out, const float2* s
   sz(timed(t, m.zi, PASS_Z_INV), 1, out, out, nullptr, 1.f, twZ, s);
 }
 
-void Plan::kernel_planes(float2* spec, int n, hipStream_t s) const {
+void Plan::kernel_planes(float2* spec, int n, size_t stride, hipStream_t s) const {
   PlaneGeom g = mid().pl;
   g.nb = n;
-  g.kStride = ncpx();
+  g.kStride = stride;
   g.kin = g.specOut = spec;
   g.kScale = inv_scale();
   g.kK[0] = K[1];
@@ -258,7 +258,7 @@ GatherParams Plan::kernel_gather(const float* dKernel) const {
 int Plan::kernel_spectrum(const float* dKernel, float2* spec, hipStream_t s) const {
   xf(dom, kernel_gather(dKernel), spec, twM, wr, s);
   if (planar) {
-    kernel_planes(spec, 1, s);
+    kernel_planes(spec, 1, ncpx(), s);
   } else {
     Mid m = mid();
     m.y.plane0 = dom.P[2] - K[2] / 2;  // the kernel's z planes, around 0

@@ -1,6 +1,7 @@
 // psf.cpp -- kernel normalisation and the four iteration schemes' second kernels.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "host.hpp"
 
@@ -56,9 +57,11 @@ double sum_img_quirk(const float* a, size_t n, int nT) {
 }
 
 // AdjustInput.normToSum1 (D/normalization/AdjustInput.java:52-58)
-void norm_to_sum1(float* a, size_t n, int nT) {
+// (returns the sum it divided by)
+double norm_to_sum1(float* a, size_t n, int nT) {
   const double sum = sum_img_quirk(a, n, nT);
   for (size_t i = 0; i < n; ++i) a[i] = (float)((double)a[i] / sum);
+  return sum;
 }
 
 // Mirror.mirror on every axis (D/util/Mirror.java:55-132), sequential order:
@@ -81,15 +84,22 @@ void mirror_all(float* a, const int dim[3]) {
     }
 }
 
+// kernels of V views that PsfProducts uses
+static int psf_kernel_count(int V) { return 4 * V - 2; }
+
 // Products of same-size convolutions (the FFTConvolution chains of DeconViewPSF.init, :132-195, :196-242): with a the
 // V kernels, b the mirrored ones and (*) zero-extended,
 //   twice:  out_v = b_v prod_{w != v} ((b_v (*) a_w) (*) b_w)        otherwise:  out_v = a_v prod_{w != v} (a_v (*) b_w)
-// multiplied in the order of w.  kernels holds a then b, 2 V arrays on the device; out V arrays.
+// multiplied in the order of w.  A view's kernel is normalised when its turn comes: a_v, b_v and those of w < v are
+// normalised, those of w > v as they were given.  Their scale goes with the final normalisation, but it decides where the
+// float products leave their range.  kernels holds, on the device, the given a_1.., the normalised a_0.., the normalised
+// b_0.. and the given b_1.., psf_kernel_count(V) arrays; out V arrays.
 //
-// On grids transformed plane by plane all pairs run in one launch per pass: the 2 V kernel spectra and the V data
-// spectra are transformed once and shared by the pairs.  The pairs of as many views as fit kPairBytes go together.
+// On grids transformed plane by plane all pairs run in one launch per pass: the kernel spectra (of both scales) and the V
+// data spectra are transformed once and shared by the pairs.  The pairs of as many views as fit kPairBytes go together.
+// Planar spectra need no row pitch, so they are Hx planes, not HxP (allocations above 64 MiB take 0.35 ms more here).
 // Six 31^3 kernels, twice (60 convolutions): the set-up of a 192 x 176 x 128 frame takes 17.5 ms with allocations and
-// copies for each pair, 1.62 ms so (110 us of it these kernels).
+// copies for each pair, 1.48 ms so.
 // Larger grids run pair by pair in two spectra, as does a device without the memory for the batch.
 class PsfProducts {
  public:
@@ -101,20 +111,27 @@ class PsfProducts {
   }
   int run(const float* kernels, float* out, hipStream_t s) {
     if (plan.create(K, K)) return -1;
-    const size_t n = plan.ncpx(), pairBytes = (size_t)(V - 1) * (n * 8 + nk * 4);
-    const int views = (int)std::max<size_t>(1, std::min<size_t>(V, kPairBytes / pairBytes));
-    const size_t batch = 3 * (size_t)V * n * 8 + views * pairBytes + 3 * (size_t)V * (V - 1) * sizeof(int);
     if (plan.planar) {
+      const size_t n = planes(), pairBytes = (size_t)(V - 1) * (n * 8 + nk * 4);
+      const int views = (int)std::max<size_t>(1, std::min<size_t>(V, kPairBytes / pairBytes));
+      const size_t batch = (size_t)(nkern() + V) * n * 8 + views * pairBytes + 3 * (size_t)V * (V - 1) * sizeof(int);
       if (hipMalloc(&mem, batch) == hipSuccess) return batched(kernels, out, views, s);
       (void)hipGetLastError();
       mem = nullptr;
     }
-    MVR_HIP(hipMalloc(&mem, 2 * n * 8 + 2 * nk * 4));
+    MVR_HIP(hipMalloc(&mem, 2 * plan.ncpx() * 8 + 2 * nk * 4));
     return pair_by_pair(kernels, out, s);
   }
 
  private:
   static constexpr size_t kPairBytes = 256u << 20;
+  // places of the kernels of view w in the pairs of view v, and of its data; the kernels in use (once: the mirrored ones)
+  int kernel_at(int v, int w) const { return w > v ? w - 1 : V - 1 + w; }
+  int mirrored_at(int v, int w) const { return w > v ? 3 * V - 2 + w : 2 * V - 1 + w; }
+  int data_at(int v) const { return (twice ? 2 * V - 1 : V - 1) + v; }
+  int kern0() const { return twice ? 0 : 2 * V - 1; }
+  int nkern() const { return psf_kernel_count(V) - kern0(); }
+  size_t planes() const { return (size_t)plan.Hx * plan.dom.P[1] * plan.dom.P[2]; }
   GatherParams data_gather(const float* src) const {
     GatherParams g{};
     g.src = src;
@@ -124,10 +141,10 @@ class PsfProducts {
   }
 
   int batched(const float* kernels, float* out, int views, hipStream_t s) {
-    const size_t n = plan.ncpx();
-    const int nf = V - 1, npairs = V * nf;
+    const size_t n = planes();
+    const int nf = V - 1, npairs = V * nf, k0 = kern0(), nkernels = nkern();
     float2* kspec = static_cast<float2*>(mem);
-    float2* dspec = kspec + 2 * V * n;
+    float2* dspec = kspec + nkernels * n;
     float2* work = dspec + V * n;
     float* o = reinterpret_cast<float*>(work + (size_t)views * nf * n);
     int* tab = reinterpret_cast<int*>(o + (size_t)views * nf * nk);
@@ -136,18 +153,17 @@ class PsfProducts {
       for (int w = 0; w < V; ++w)
         if (w != v) {
           h[p] = v;
-          h[npairs + p] = twice ? w : V + w;
-          h[2 * npairs + p++] = V + w;
+          h[npairs + p] = (twice ? kernel_at(v, w) : mirrored_at(v, w)) - k0;
+          h[2 * npairs + p++] = mirrored_at(v, w) - k0;
         }
     MVR_HIP(hipMemcpyAsync(tab, h.data(), h.size() * sizeof(int), hipMemcpyHostToDevice, s));
-    // spectra of the kernels (once: of the mirrored ones only) and of the data
-    const int k0 = twice ? 0 : V;
-    GatherParams g = data_gather(kernels + (twice ? V * nk : 0));
+    // spectra of the kernels and of the data
+    GatherParams g = data_gather(kernels + data_at(0) * nk);
     const Plan::Mid conv = plan.convolve_geometry(g);
-    const XFwdGroup first[2] = {{plan.kernel_gather(kernels + k0 * nk), kspec + k0 * n, 2 * V - k0, nk, n},
+    const XFwdGroup first[2] = {{plan.kernel_gather(kernels + k0 * nk), kspec, nkernels, nk, n},
                                 {g, dspec, V, nk, n}};
     plan.xfg(plan.dom, first, 2, plan.twM, plan.wr, s);
-    plan.kernel_planes(kspec + k0 * n, 2 * V - k0, s);
+    plan.kernel_planes(kspec, nkernels, n, s);
     Dom dom = plan.dom;
     dom.blockStride = n;
     for (int v = 0; v < V; v += views) {
@@ -169,7 +185,7 @@ class PsfProducts {
         launch_plane(pl, work, work, kspec, plan.twY, plan.twZ, s);
         plan.xs(dom, st, work, plan.twM, plan.wr, s);
       }
-      launch_psf_products(kernels + ((twice ? V : 0) + v) * nk, o, np / nf, nf, nk, out + v * nk, s);
+      launch_psf_products(kernels + data_at(v) * nk, o, np / nf, nf, nk, out + v * nk, s);
     }
     MVR_HIP(hipGetLastError());
     MVR_HIP(hipStreamSynchronize(s));  // h and the destructor
@@ -182,16 +198,16 @@ class PsfProducts {
     float2* work = spec + n;
     float* o1 = reinterpret_cast<float*>(work + n);
     float* o2 = o1 + nk;
-    const float* mirrored = kernels + V * nk;
     for (int v = 0; v < V; ++v) {
-      const float* data = (twice ? mirrored : kernels) + v * nk;
+      const float* data = kernels + data_at(v) * nk;
       const float* acc = data;
       for (int w = 0; w < V; ++w) {
         if (w == v) continue;
         const float* o = o1;
-        if (plan.convolve_once((twice ? kernels : mirrored) + w * nk, data_gather(data), spec, work, o1, s)) return -1;
+        const float* k2 = kernels + mirrored_at(v, w) * nk;
+        if (plan.convolve_once(twice ? kernels + kernel_at(v, w) * nk : k2, data_gather(data), spec, work, o1, s)) return -1;
         if (twice) {
-          if (plan.convolve_once(mirrored + w * nk, data_gather(o1), spec, work, o2, s)) return -1;
+          if (plan.convolve_once(k2, data_gather(o1), spec, work, o2, s)) return -1;
           o = o2;
         }
         launch_psf_products(acc, o, 1, 1, nk, out + v * nk, s);
@@ -210,24 +226,23 @@ class PsfProducts {
   void* mem = nullptr;
 };
 
-// the products of the kernels k1 and their mirrored copies, in out
-static int psf_products(const std::vector<std::vector<float>>& k1, const std::vector<std::vector<float>>& inv,
-                        const int K[3], bool twice, std::vector<std::vector<float>>& out, hipStream_t s) {
-  const int V = (int)k1.size();
-  const size_t nk = (size_t)K[0] * K[1] * K[2];
-  std::vector<float> h(2 * V * nk);
-  for (int v = 0; v < V; ++v) {
-    std::copy(k1[v].begin(), k1[v].end(), h.begin() + v * nk);
-    std::copy(inv[v].begin(), inv[v].end(), h.begin() + (V + v) * nk);
-  }
+// the products for the V kernels of nk values that follow their normalising sums (V doubles) in `given`; out V arrays
+static int psf_products(std::vector<float>& given, int V, const int K[3], bool twice,
+                        std::vector<std::vector<float>>& out, hipStream_t s) {
+  const size_t nk = (size_t)K[0] * K[1] * K[2], nkern = psf_kernel_count(V) * nk;
+  // what is given, the kernels of both scales, the results
   float* dev = nullptr;
-  MVR_HIP(hipMalloc(&dev, 3 * V * nk * 4));
+  MVR_HIP(hipMalloc(&dev, (given.size() + nkern + V * nk) * 4));
+  float* kernels = dev + given.size();
+  float* res = kernels + nkern;
   int rc = -1;
-  if (hipMemcpyAsync(dev, h.data(), 2 * V * nk * 4, hipMemcpyHostToDevice, s) != hipSuccess)
+  if (hipMemcpyAsync(dev, given.data(), given.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess) {
     set_error("init_psfs: copy failed");
-  else
-    rc = PsfProducts(K, V, twice).run(dev, dev + 2 * V * nk, s);
-  if (!rc && (hipMemcpyAsync(h.data(), dev + 2 * V * nk, V * nk * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+  } else {
+    launch_psf_kernels(dev + 2 * V, reinterpret_cast<const double*>(dev), V, K, kernels, s);
+    rc = PsfProducts(K, V, twice).run(kernels, res, s);
+  }
+  if (!rc && (hipMemcpyAsync(given.data(), res, V * nk * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
               hipStreamSynchronize(s) != hipSuccess)) {
     set_error("init_psfs: readback failed");
     rc = -1;
@@ -235,7 +250,7 @@ static int psf_products(const std::vector<std::vector<float>>& k1, const std::ve
   if (rc) (void)hipStreamSynchronize(s);
   (void)hipFree(dev);
   if (rc) return rc;
-  for (int v = 0; v < V; ++v) out[v].assign(h.begin() + v * nk, h.begin() + (v + 1) * nk);
+  for (int v = 0; v < V; ++v) out[v].assign(given.begin() + v * nk, given.begin() + (v + 1) * nk);
   return 0;
 }
 
@@ -250,18 +265,21 @@ int init_psfs(int dev, std::vector<std::vector<float>>& k1, const int K[3], int 
     mirror_all(r.data(), K);
     return r;
   };
-  std::vector<std::vector<float>> inv(V);
+  const bool bayesian = psfType == PSF_EFFICIENT_BAYESIAN, products = V > 1 && (bayesian || psfType == PSF_OPT_I);
+  std::vector<float> given;
+  given.reserve(products ? 2 * V + V * nk : 0);
+  given.resize(products ? 2 * V : 0);
   for (int v = 0; v < V; ++v) {
-    norm_to_sum1(k1[v].data(), nk, nT);
-    inv[v] = inverted(k1[v]);
+    if (products) given.insert(given.end(), k1[v].begin(), k1[v].end());
+    const double sum = norm_to_sum1(k1[v].data(), nk, nT);
+    if (products) std::memcpy(given.data() + 2 * v, &sum, sizeof(sum));
   }
   if (V == 1 || psfType == PSF_INDEPENDENT) {
-    k2 = inv;
-  } else if (psfType == PSF_EFFICIENT_BAYESIAN || psfType == PSF_OPT_I) {
+    for (int v = 0; v < V; ++v) k2[v] = inverted(k1[v]);
+  } else if (products) {
     // P_v^compound = P_v^* prod_{w != v} (P_v^* (*) P_w (*) P_w^*)   (:132-195)
     // (P_v prod_{w != v} (P_v (*) P_w^*))^*                           (:196-242)
-    const bool bayesian = psfType == PSF_EFFICIENT_BAYESIAN;
-    if (psf_products(k1, inv, K, bayesian, k2, s)) return -1;
+    if (psf_products(given, V, K, bayesian, k2, s)) return -1;
     for (int v = 0; v < V; ++v) {
       norm_to_sum1(k2[v].data(), nk, nT);
       if (!bayesian) mirror_all(k2[v].data(), K);
