@@ -12,7 +12,7 @@
 //     plane is stored as two 8-channel halves [half][voxel][8], so that the 16 lanes reading one half of 16
 //     consecutive voxels touch 256 contiguous bytes (no bank conflicts);
 //   - v_mfma_f32_16x16x32_bf16 takes K = 32 as two taps x 16 channels: lanes 0-31 carry tap 2p,
-//     lanes 32-63 tap 2p+1 (tap 27 = zeros), eight channels per lane;
+//     lanes 32-63 tap 2p+1 (tap 27 = zero weights on tap 26's voxel), eight channels per lane;
 //   - the weights of the chunk stay in registers (14 fragments per output group): only the voxel fragments are read
 //     from LDS;
 //   - the weights are the first operand, the voxels the second: lane l of the result holds channels 4(l/16)..+3 of
