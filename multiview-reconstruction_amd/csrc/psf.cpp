@@ -99,7 +99,7 @@ static int psf_kernel_count(int V) { return 4 * V - 2; }
 // data spectra are transformed once and shared by the pairs.  The pairs of as many views as fit kPairBytes go together.
 // Planar spectra need no row pitch, so they are Hx planes, not HxP (allocations above 64 MiB take 0.35 ms more here).
 // Six 31^3 kernels, twice (60 convolutions): the set-up of a 192 x 176 x 128 frame takes 17.5 ms with allocations and
-// copies for each pair, 1.48 ms so.
+// copies for each pair, 1.40 ms so.
 // Larger grids run pair by pair in two spectra, as does a device without the memory for the batch.
 class PsfProducts {
  public:
@@ -109,18 +109,36 @@ class PsfProducts {
   ~PsfProducts() {
     if (mem) (void)hipFree(mem);
   }
-  int run(const float* kernels, float* out, hipStream_t s) {
+  // given: the kernels' normalising sums (V doubles) and the V kernels, replaced by the products
+  int run(std::vector<float>& given, hipStream_t s) {
     if (plan.create(K, K)) return -1;
+    // what is given, the kernels of both scales and the results lie before the spectra, in one allocation
+    const size_t kernN = psf_kernel_count(V) * nk, head = ((given.size() + kernN + V * nk) * 4 + 255) / 256 * 256;
+    int views = 0;
     if (plan.planar) {
       const size_t n = planes(), pairBytes = (size_t)(V - 1) * (n * 8 + nk * 4);
-      const int views = (int)std::max<size_t>(1, std::min<size_t>(V, kPairBytes / pairBytes));
+      views = (int)std::max<size_t>(1, std::min<size_t>(V, kPairBytes / pairBytes));
       const size_t batch = (size_t)(nkern() + V) * n * 8 + views * pairBytes + 3 * (size_t)V * (V - 1) * sizeof(int);
-      if (hipMalloc(&mem, batch) == hipSuccess) return batched(kernels, out, views, s);
-      (void)hipGetLastError();
-      mem = nullptr;
+      if (hipMalloc(&mem, head + batch) != hipSuccess) {
+        (void)hipGetLastError();
+        mem = nullptr;
+        views = 0;
+      }
     }
-    MVR_HIP(hipMalloc(&mem, 2 * plan.ncpx() * 8 + 2 * nk * 4));
-    return pair_by_pair(kernels, out, s);
+    if (!mem) MVR_HIP(hipMalloc(&mem, head + 2 * plan.ncpx() * 8 + 2 * nk * 4));
+    spectra = reinterpret_cast<float2*>(static_cast<char*>(mem) + head);
+    float* dgiven = static_cast<float*>(mem);
+    float* kernels = dgiven + given.size();
+    float* out = kernels + kernN;
+    MVR_HIP(hipMemcpyAsync(dgiven, given.data(), given.size() * 4, hipMemcpyHostToDevice, s));
+    launch_psf_kernels(dgiven + 2 * V, reinterpret_cast<const double*>(dgiven), V, K, kernels, s);
+    if (views ? batched(kernels, out, views, s) : pair_by_pair(kernels, out, s)) {
+      (void)hipStreamSynchronize(s);  // given is in use
+      return -1;
+    }
+    MVR_HIP(hipMemcpyAsync(given.data(), out, V * nk * 4, hipMemcpyDeviceToHost, s));
+    MVR_HIP(hipStreamSynchronize(s));
+    return 0;
   }
 
  private:
@@ -143,7 +161,7 @@ class PsfProducts {
   int batched(const float* kernels, float* out, int views, hipStream_t s) {
     const size_t n = planes();
     const int nf = V - 1, npairs = V * nf, k0 = kern0(), nkernels = nkern();
-    float2* kspec = static_cast<float2*>(mem);
+    float2* kspec = spectra;
     float2* dspec = kspec + nkernels * n;
     float2* work = dspec + V * n;
     float* o = reinterpret_cast<float*>(work + (size_t)views * nf * n);
@@ -194,7 +212,7 @@ class PsfProducts {
 
   int pair_by_pair(const float* kernels, float* out, hipStream_t s) {
     const size_t n = plan.ncpx();
-    float2* spec = static_cast<float2*>(mem);
+    float2* spec = spectra;
     float2* work = spec + n;
     float* o1 = reinterpret_cast<float*>(work + n);
     float* o2 = o1 + nk;
@@ -224,35 +242,8 @@ class PsfProducts {
   bool twice;
   size_t nk;
   void* mem = nullptr;
+  float2* spectra = nullptr;
 };
-
-// the products for the V kernels of nk values that follow their normalising sums (V doubles) in `given`; out V arrays
-static int psf_products(std::vector<float>& given, int V, const int K[3], bool twice,
-                        std::vector<std::vector<float>>& out, hipStream_t s) {
-  const size_t nk = (size_t)K[0] * K[1] * K[2], nkern = psf_kernel_count(V) * nk;
-  // what is given, the kernels of both scales, the results
-  float* dev = nullptr;
-  MVR_HIP(hipMalloc(&dev, (given.size() + nkern + V * nk) * 4));
-  float* kernels = dev + given.size();
-  float* res = kernels + nkern;
-  int rc = -1;
-  if (hipMemcpyAsync(dev, given.data(), given.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess) {
-    set_error("init_psfs: copy failed");
-  } else {
-    launch_psf_kernels(dev + 2 * V, reinterpret_cast<const double*>(dev), V, K, kernels, s);
-    rc = PsfProducts(K, V, twice).run(kernels, res, s);
-  }
-  if (!rc && (hipMemcpyAsync(given.data(), res, V * nk * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
-              hipStreamSynchronize(s) != hipSuccess)) {
-    set_error("init_psfs: readback failed");
-    rc = -1;
-  }
-  if (rc) (void)hipStreamSynchronize(s);
-  (void)hipFree(dev);
-  if (rc) return rc;
-  for (int v = 0; v < V; ++v) out[v].assign(given.begin() + v * nk, given.begin() + (v + 1) * nk);
-  return 0;
-}
 
 int init_psfs(int dev, std::vector<std::vector<float>>& k1, const int K[3], int psfType, int nT,
               std::vector<std::vector<float>>& k2, hipStream_t s) {
@@ -279,8 +270,9 @@ int init_psfs(int dev, std::vector<std::vector<float>>& k1, const int K[3], int 
   } else if (products) {
     // P_v^compound = P_v^* prod_{w != v} (P_v^* (*) P_w (*) P_w^*)   (:132-195)
     // (P_v prod_{w != v} (P_v (*) P_w^*))^*                           (:196-242)
-    if (psf_products(given, V, K, bayesian, k2, s)) return -1;
+    if (PsfProducts(K, V, bayesian).run(given, s)) return -1;
     for (int v = 0; v < V; ++v) {
+      k2[v].assign(given.begin() + v * nk, given.begin() + (v + 1) * nk);
       norm_to_sum1(k2[v].data(), nk, nT);
       if (!bayesian) mirror_all(k2[v].data(), K);
     }
